@@ -39,6 +39,7 @@ static constexpr u64 KEY_NONE = ~0ull;   // empty slot (rpma.cuh:38)
 // run key of a batch element: pma << 32 | segment, bit 63 the operation
 static constexpr u64 RK_NONE = ~0ull;
 static constexpr u64 RK_OP = 1ull << 63;
+static constexpr u64 RK_SKIP = 1ull << 62;  // located, but without effect (set in RK_NONE too)
 
 // status flags raised on the device during one update
 static constexpr u32 FLAG_INVALID_KEY = 1u;   // src or dst >= V
@@ -267,13 +268,14 @@ __device__ __forceinline__ u32 locate_segment(const u64 *__restrict__ sep, u32 H
     return base;
 }
 
-// is `key` among the live (front-packed) keys of segment s (a binary search:
-// a 4-ary one here, three probes per step, measured slower)
+// is `key` among the keys of segment s: a binary search over all its slots
+// (the gaps after the live keys hold the largest key), so the segment's count
+// is not read first (a 4-ary search, three probes per step, measured slower)
 __device__ __forceinline__ bool segment_holds(const DevState &d, u32 s, u64 key) {
     const u64 *seg = d.keys + ((u64)s << d.log2S);
-    u32 c = d.cnt[s];
-    u64 i = lower_bound_dev<u64>(seg, 0, c, key);
-    return i < c && seg[i] == key;
+    u32 i = 0;
+    for (u32 h = 1u << (d.log2S - 1); h; h >>= 1) i += seg[i + h - 1] < key ? h : 0u;
+    return seg[i] == key;
 }
 
 // --------------------------------------------------------- wave64 scans

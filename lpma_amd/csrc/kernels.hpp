@@ -17,13 +17,13 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
 // update.hip
 struct BatchBufs {
     u64 *ukey;     // n: decoded keys of the sorted batch
-    u64 *useg;     // n: run key pid << 32 | segment (| RK_OP for inserts) of effective updates, else RK_NONE
+    u64 *useg;     // n: run key pid << 32 | segment (| RK_OP for inserts, RK_SKIP without effect); duplicates RK_NONE
     u64 *ckey;     // n: compacted effective updates (sorted by pid, key)
     u64 *cseg;     // n: their run keys
     i32 *pd;       // n+1: exclusive prefix of +1 (insert) / -1 (delete)
     u32 *rlevel;   // n: chosen level per run start
     uint4 *rwin;   // n: per run start, its chosen window's update range [u0, u1) and counts C, M
-    i32 *part;     // 2 * nblocks + 2: block partials (count, delta)
+    u64 *part;     // LOC_GROUPS + nblocks: (count, delta) of groups of locate blocks, then of each block
     Work *work[NUM_CLASSES];  // n each
     u32 *lchunk;   // n+1: chunk prefix over large windows
     u64 *lmbase;   // n: merged-scratch base per large window
@@ -49,10 +49,12 @@ u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const Inli
                          hipStream_t st);
 
 u32 locate_blocks(u64 n);
-// also clears zero[0, nzero) (the sort's digit totals)
-// and resets the update index wfirst
-hipError_t batch_begin(const Group &g, Status *status, const InlineSegs &in, BatchSeg *segs, u32 *zero, u32 nzero,
-                       u32 *wfirst, hipStream_t st);
+// most groups of locate blocks
+static constexpr u32 LOC_GROUPS = 1024;
+// also clears zero[0, nzero) (the sort's digit totals) and the locate groups
+// and resets the update index
+hipError_t batch_begin(const Group &g, const BatchBufs &b, const InlineSegs &in, BatchSeg *segs, u32 *zero, u32 nzero,
+                       hipStream_t st);
 hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchBufs &b, hipStream_t st);
 // fixed grids for graph replays (work counts read on the device)
 hipError_t rebalance_fixed(const Group &g, const BatchBufs &b, u32 runs_cap, u64 *merged, hipStream_t st);

@@ -157,7 +157,8 @@ struct Pipeline {
     DBuf<u64> pk0, pk1, ukey, useg, ckey, cseg, merged, lmbase;
     DBuf<u32> sort_scr, rlevel, gpre, scan_scr, lchunk, lhdr, lvmask, wfirst;
     DBuf<uint4> rwin;
-    DBuf<i32> pd, part;
+    DBuf<i32> pd;
+    DBuf<u64> part;
     DBuf<Work> work[NUM_CLASSES];
     DBuf<PmaEntry> tab;
     DBuf<BatchSeg> segs;
@@ -566,7 +567,7 @@ int ensure_batch(Pipeline &pl, u64 n, u32 npma, u32 nsegs, u64 runs) {
     if ((r = ensure(pl, pl.pk0, n)) || (r = ensure(pl, pl.pk1, n)) ||
         (r = ensure(pl, pl.sort_scr, sort_scratch_words(n))) || (r = ensure(pl, pl.ukey, n)) ||
         (r = ensure(pl, pl.useg, n)) || (r = ensure(pl, pl.ckey, n)) || (r = ensure(pl, pl.cseg, n)) ||
-        (r = ensure(pl, pl.pd, n + 1)) || (r = ensure(pl, pl.rlevel, n)) || (r = ensure(pl, pl.rwin, n)) || (r = ensure(pl, pl.part, 2 * nb + 2)) ||
+        (r = ensure(pl, pl.pd, n + 1)) || (r = ensure(pl, pl.rlevel, n)) || (r = ensure(pl, pl.rwin, n)) || (r = ensure(pl, pl.part, LOC_GROUPS + nb)) ||
         (r = ensure(pl, pl.tab, npma)) || (r = ensure(pl, pl.segs, std::max<u32>(nsegs, INLINE_SEGS))) ||
         (r = ensure(pl, pl.lvmask, (u64)npma * LV_REPL)) || (r = ensure(pl, pl.wfirst, WFIRST_N + 1)) ||
         (r = ensure(pl, pl.out, out_words)))
@@ -982,7 +983,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
             h0->pyr_owed = false;
         } else {
             HIPCHECK(pay_owed_pyramids(mem, npma, st));
-            HIPCHECK(batch_begin(g, bb.status, in, pl.segs.p, pl.sort_scr.p, sort_zero_words(), bb.wfirst, st));
+            HIPCHECK(batch_begin(g, bb, in, pl.segs.p, pl.sort_scr.p, sort_zero_words(), st));
             pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
                                pl.ukey.p, pl.sort_scr.p, &bb.status->flags, st);
         }
@@ -1114,7 +1115,7 @@ int graph_for(Pipeline &pl, u64 cap, u32 npma, u32 pshift, u32 hi_bit, u32 log2S
         bool ok = hipMemcpyAsync(pl.rhdr.p, pl.h_rhdr, sizeof(RoundHdr), hipMemcpyHostToDevice, cs) == hipSuccess &&
                   hipMemcpyAsync(pl.segs.p, pl.h_segs, nsegs * sizeof(BatchSeg), hipMemcpyHostToDevice, cs) ==
                       hipSuccess &&
-                  batch_begin(g, bb.status, none, pl.segs.p, pl.sort_scr.p, sort_zero_words(), bb.wfirst, cs) == hipSuccess;
+                  batch_begin(g, bb, none, pl.segs.p, pl.sort_scr.p, sort_zero_words(), cs) == hipSuccess;
         if (ok) {
             u64 *pk = pack_and_sort(pl.segs.p, nsegs, cap, &pl.rhdr.p->n, pshift, 0, 0, hi_bit, pl.pk0.p, pl.pk1.p,
                                     pl.ukey.p, pl.sort_scr.p, &bb.status->flags, cs);

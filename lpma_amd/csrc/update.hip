@@ -31,7 +31,8 @@
 namespace pma {
 
 static constexpr int LOC_TPB = 256;
-static constexpr int LOC_TILE = LOC_TPB;  // one batch element per thread
+static constexpr int LOC_TILE = LOC_TPB;  // batch elements of a prefix word
+static constexpr int LOC_ITEMS = 4;       // elements per thread of a large batch's locate
 
 u32 locate_blocks(u64 n) { return (u32)((n + LOC_TILE - 1) / LOC_TILE); }
 
@@ -41,11 +42,11 @@ u32 locate_blocks(u64 n) { return (u32)((n + LOC_TILE - 1) / LOC_TILE); }
 // k_pyr_chunk (nseg >> 11 entries and fewer), so no separate launch is
 // needed for them.
 __global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, InlineSegs in, BatchSeg *segs, u32 *zero,
-                                                      u32 nzero, u32 *wfirst);
+                                                      u32 nzero, u32 *wfirst, u64 *grp);
 
-hipError_t batch_begin(const Group &g, Status *status, const InlineSegs &in, BatchSeg *segs, u32 *zero, u32 nzero,
-                       u32 *wfirst, hipStream_t st) {
-    k_batch_begin<<<g.npma, 1024, 0, st>>>(g, status, in, segs, zero, nzero, wfirst);
+hipError_t batch_begin(const Group &g, const BatchBufs &b, const InlineSegs &in, BatchSeg *segs, u32 *zero, u32 nzero,
+                       hipStream_t st) {
+    k_batch_begin<<<g.npma, 1024, 0, st>>>(g, b.status, in, segs, zero, nzero, b.wfirst, b.part);
     return hipGetLastError();
 }
 
@@ -62,153 +63,317 @@ __device__ __forceinline__ DevState geom(const Group &g, u32 pid) {
     return g.tab[pid].d;
 }
 
-template <bool ONE>
+// last segment whose separator is <= key, by one whole wave: each step tests
+// 128 evenly spaced pivots (two a lane), so 2^19 segments take three rounds
+// of loads
+__device__ __forceinline__ u32 wave_locate(const u64 *__restrict__ sep, u32 H, u64 key) {
+    const u32 lane = lane_id();
+    u32 lo = 0, hi = 1u << H;  // sep[lo] <= key throughout (sep[0] = 0)
+    while (hi - lo > 1) {
+        const u32 step = (hi - lo + 127) / 128;
+        const u32 p = lo + lane * step, q = p + 64 * step;
+        const u64 x = p < hi ? sep[p] : KEY_NONE, y = q < hi ? sep[q] : KEY_NONE;
+        const u32 c = (u32)__popcll(__ballot(p < hi && x <= key)) + (u32)__popcll(__ballot(q < hi && y <= key));
+        lo += (c ? c - 1 : 0) * step;  // c >= 1 by the invariant
+        hi = min(lo + step, hi);
+    }
+    return lo;
+}
+
+// separators of a tile's segment range staged in LDS
+static constexpr u32 LOC_RANGE = 2048;
+
+// Tiles of LOC_TPB * ITEMS sorted keys.  NARROW: the keys of a tile land in a
+// narrow range of segments: two waves find the segments of its first and last
+// key, the separators between them are staged in LDS (one coalesced read) and
+// every key searches there, so a key costs no separator request of its own.  A
+// tile whose range exceeds the LDS (few keys over many segments) or that spans
+// two PMAs searches all separators (locate_segment), as every tile does
+// without NARROW.  Bound: the presence probes, a few dependent loads a key.
+template <bool ONE, int ITEMS, bool NARROW>
 __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restrict__ pk, u64 n,
                                                     u64 *__restrict__ ukey, u64 *__restrict__ useg,
-                                                    i32 *__restrict__ part_cnt, i32 *__restrict__ part_dl) {
+                                                    u64 *__restrict__ part, u64 *__restrict__ grp, u32 grp_log,
+                                                    u32 nb) {
+    __shared__ u64 ls[NARROW ? LOC_RANGE : 1];
+    __shared__ u32 ends[2];
+    __shared__ i32 tmp[2][ITEMS][LOC_TPB / 64];
     if (g.rh) n = g.rh->n;
     const u64 pmask = (1ull << g.pshift) - 1;
-    const u64 i = (u64)blockIdx.x * LOC_TILE + threadIdx.x;
-    i32 eff = 0, dl = 0;
-    if (i < n) {
-        const u64 p = pk[i];
-        const u32 ks = 1 + g.sbits;  // key (and pid) above the request order and op
-        const bool dup = (i + 1 < n) && ((pk[i + 1] >> ks) == (p >> ks));
+    const u32 ks = 1 + g.sbits;  // key (and pid) above the request order and op
+    const u64 i0 = (u64)blockIdx.x * (LOC_TPB * ITEMS);
+    const u32 tid = threadIdx.x, wv = tid >> 6;
+    u64 p[ITEMS];
+    bool dup[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u64 i = i0 + r * LOC_TPB + tid;
+        p[r] = i < n ? pk[i] : ~0ull;
+        dup[r] = i + 1 < n && (pk[i + 1] >> ks) == (p[r] >> ks);
+    }
+    u32 a = 0, cr = 0;  // the tile's segment range, when staged
+    if (NARROW && i0 < n) {
+        const u64 i1 = min(n, i0 + LOC_TPB * ITEMS) - 1;
+        const u64 p0 = pk[i0], p1 = pk[i1];
+        const u32 pid = (u32)(p0 >> g.pshift);
         // a PMA id out of range only follows a failed sort (FLAG_SORT_STALL)
-        if (dup || (u32)(p >> g.pshift) >= g.npma) {
-            useg[i] = RK_NONE;
-        } else {
-            const u32 pid = (u32)(p >> g.pshift);
+        if (pid < g.npma && (u32)(p1 >> g.pshift) == pid) {
             const DevState d = geom<ONE>(g, pid);
-            const u64 kk = (p & pmask) >> ks;
-            const u32 op = (u32)(p & 1);
-            const u64 key = ((kk >> d.vbits) << 32) | (kk & ((1ull << d.vbits) - 1));
-            const u32 s = locate_segment(d.sep, d.H, key);
-            const u32 present = segment_holds(d, s, key) ? 1u : 0u;
-            u64 rk = RK_NONE;
-            if (op != present) {
-                eff = 1;
-                dl = op ? 1 : -1;
-                rk = ((u64)pid << 32) | s | (op ? RK_OP : 0ull);
+            if (wv < 2) {
+                const u64 kk = ((wv ? p1 : p0) & pmask) >> ks;
+                const u32 s = wave_locate(d.sep, d.H, ((kk >> d.vbits) << 32) | (kk & ((1ull << d.vbits) - 1)));
+                if (lane_id() == 0) ends[wv] = s;
             }
-            ukey[i] = key;
-            useg[i] = rk;
+            __syncthreads();
+            a = ends[0];
+            cr = ends[1] - a + 1;  // beyond LOC_RANGE too when the sort failed
+            if (cr > LOC_RANGE) cr = 0;
+            for (u32 x = tid; x < cr; x += LOC_TPB) ls[x] = d.sep[a + x];
+            __syncthreads();
         }
     }
-    __shared__ i32 tmp[2][LOC_TPB / 64];
-    i32 ce = wave_sum(eff), cd = wave_sum(dl);
-    if (lane_id() == 0) { tmp[0][threadIdx.x >> 6] = ce; tmp[1][threadIdx.x >> 6] = cd; }
+    u64 key[ITEMS];
+    u32 seg[ITEMS];
+    bool ok[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u64 i = i0 + r * LOC_TPB + tid;
+        const u32 pid = (u32)(p[r] >> g.pshift);
+        ok[r] = i < n && !dup[r] && pid < g.npma;
+        key[r] = 0;
+        seg[r] = 0;
+        if (!ok[r]) continue;
+        const DevState d = geom<ONE>(g, pid);
+        const u64 kk = (p[r] & pmask) >> ks;
+        key[r] = ((kk >> d.vbits) << 32) | (kk & ((1ull << d.vbits) - 1));
+        if (cr) {
+            u32 lo = 0, hi = cr;  // ls[lo] <= key
+            while (hi - lo > 1) {
+                const u32 mid = (lo + hi) >> 1;
+                if (ls[mid] <= key[r]) lo = mid; else hi = mid;
+            }
+            seg[r] = a + lo;
+        } else {
+            seg[r] = locate_segment(d.sep, d.H, key[r]);
+        }
+    }
+    // presence: the items' binary searches step together (their loads are in
+    // flight at once); an item without a key probes its PMA's first segment
+    const u64 *base[ITEMS];
+    u32 at[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u32 pid = (u32)(p[r] >> g.pshift);
+        base[r] = geom<ONE>(g, ok[r] ? pid : 0).keys + ((u64)seg[r] << g.log2S);
+        at[r] = 0;
+    }
+    for (u32 h = 1u << (g.log2S - 1); h; h >>= 1) {
+        u64 v[ITEMS];
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) v[r] = base[r][at[r] + h - 1];
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) at[r] += v[r] < key[r] ? h : 0u;
+    }
+    u64 got[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) got[r] = base[r][at[r]];
+    i32 eff[ITEMS], dl[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u64 i = i0 + r * LOC_TPB + tid;
+        eff[r] = dl[r] = 0;
+        u64 rk = RK_NONE;
+        if (ok[r]) {
+            const u32 pid = (u32)(p[r] >> g.pshift);
+            const u32 op = (u32)(p[r] & 1);
+            // an update without effect keeps its segment (the update index
+            // wants it) and is marked
+            rk = ((u64)pid << 32) | seg[r];
+            if (op != (got[r] == key[r] ? 1u : 0u)) {
+                eff[r] = 1;
+                dl[r] = op ? 1 : -1;
+                rk |= op ? RK_OP : 0ull;
+            } else {
+                rk |= RK_SKIP;
+            }
+            ukey[i] = key[r];
+        }
+        if (i < n) useg[i] = rk;
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const i32 ce = wave_sum(eff[r]), cd = wave_sum(dl[r]);
+        if (lane_id() == 0) { tmp[0][r][wv] = ce; tmp[1][r][wv] = cd; }
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        i32 a = 0, c = 0;
-        for (int w = 0; w < LOC_TPB / 64; ++w) { a += tmp[0][w]; c += tmp[1][w]; }
-        part_cnt[blockIdx.x] = a;
-        part_dl[blockIdx.x] = c;
+    if (tid < 64) {
+        // one word per LOC_TPB keys
+        u64 both = 0;
+        const u32 b = blockIdx.x * ITEMS + tid;
+        if (tid < ITEMS && b < nb) {
+            i32 x = 0, y = 0;
+            for (int w = 0; w < LOC_TPB / 64; ++w) { x += tmp[0][tid][w]; y += tmp[1][tid][w]; }
+            both = ((u64)(u32)y << 32) + (u32)x;
+            part[b] = both;
+        }
+        if (grp) {
+            const u64 sum = wave_sum(both);
+            if (tid == 0 && sum)
+                atomicAdd((unsigned long long *)&grp[(blockIdx.x * ITEMS) >> grp_log], (unsigned long long)sum);
+        }
     }
 }
 
-__global__ __launch_bounds__(1024) void k_scan_parts(i32 *__restrict__ pc, i32 *__restrict__ pdl, u32 nb,
-                                                     Status *__restrict__ status, i32 *__restrict__ pd) {
-    __shared__ i32 tmp[1024 / 64 + 1];
-    i32 carry_c = 0, carry_d = 0;
-    for (u32 b = 0; b < nb; b += 1024) {
-        u32 i = b + threadIdx.x;
-        i32 vc = i < nb ? pc[i] : 0;
-        i32 vd = i < nb ? pdl[i] : 0;
-        i32 tc, td;
-        i32 ec = block_excl_scan<1024, i32>(vc, tc, tmp);
-        i32 ed = block_excl_scan<1024, i32>(vd, td, tmp);
-        if (i < nb) { pc[i] = carry_c + ec; pdl[i] = carry_d + ed; }
-        carry_c += tc;
-        carry_d += td;
-    }
-    if (threadIdx.x == 0) {
-        status->n_eff = (u32)carry_c;
-        status->delta = carry_d;
-        pd[carry_c] = carry_d;
-    }
+// Prefixes of the locate blocks.  A block of LOC_TILE keys leaves its (count,
+// delta) as one 64-bit word (delta in the high half, wrapping) and every
+// compact block adds up the words before its own: all of them up to LOC_DIRECT
+// blocks (at most eight loads a thread), beyond that the sums of the groups of
+// 2^grp_log blocks before its group (added up by the locate tiles, one atomic
+// each) and the words of its own group, about as many of each.  A scan of the
+// words by one workgroup in between took 12 us for 7.8 K blocks and 44 us for
+// 32 K.
+static constexpr u32 LOC_DIRECT = 2048;
+static u32 locate_group_log(u32 nb) {
+    if (nb <= LOC_DIRECT) return 0;
+    u32 lg = 0;
+    while ((1u << lg) < nb) ++lg;
+    u32 g = std::max<u32>(lg / 2, 2);  // at least the LOC_ITEMS blocks of a locate tile
+    while ((((u64)nb + (1u << g) - 1) >> g) > LOC_GROUPS) ++g;
+    return g;
 }
 
-static constexpr u32 COMPACT_SELF_PREFIX_MAX = 2048;  // blocks
-
-// Stream compaction of the effective updates.  With few blocks every block
-// derives its prefix (and the totals) from the per-block partials itself;
-// otherwise k_scan_parts has already scanned them.
+// Stream compaction of the effective updates, ITEMS locate blocks a
+// workgroup.  An element's (count, inserts) are scanned as the halves of one
+// word, and the wave totals meet the prefix sums at the same barrier.
+template <int ITEMS>
 __global__ __launch_bounds__(LOC_TPB) void k_compact(const Group g, const u64 *__restrict__ ukey,
-                                                     const u64 *__restrict__ useg, u64 n, const i32 *__restrict__ pc,
-                                                     const i32 *__restrict__ pdl, u32 nb,
-                                                     int self_prefix, u64 *__restrict__ ckey, u64 *__restrict__ cseg,
+                                                     const u64 *__restrict__ useg, u64 n,
+                                                     const u64 *__restrict__ part, const u64 *__restrict__ grp, u32 nb,
+                                                     u32 grp_log, u64 *__restrict__ ckey, u64 *__restrict__ cseg,
                                                      i32 *__restrict__ pd, u32 *__restrict__ wfirst,
                                                      Status *__restrict__ status) {
-    const RoundHdr *rh = g.rh;
-    __shared__ i32 tmp[LOC_TPB / 64 + 1];
-    __shared__ i32 red[4][LOC_TPB / 64];
-    i32 base_c, base_d;
-    if (rh) n = rh->n;
-    if (self_prefix) {
+    constexpr u32 NW = LOC_TPB / 64;
+    __shared__ i32 red[4][NW];
+    __shared__ u32 wt[ITEMS * NW];
+    if (g.rh) n = g.rh->n;
+    const u32 wv = threadIdx.x >> 6;
+    const u64 i0 = (u64)blockIdx.x * (LOC_TILE * ITEMS) + threadIdx.x;
+    // the elements are loaded first, in flight during the prefix
+    u64 sg[ITEMS], prev[ITEMS], uk[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u64 i = i0 + r * LOC_TILE;
+        sg[r] = i < n ? useg[i] : RK_NONE;
+        prev[r] = i > 0 && i < n ? useg[i - 1] : 0ull;
+        uk[r] = i < n ? ukey[i] : 0ull;
+    }
+    {
         i32 a = 0, b = 0, ta = 0, tb = 0;
-        for (u32 x = threadIdx.x; x < nb; x += LOC_TPB) {
-            i32 v = pc[x], w = pdl[x];
+        const u64 *tot = grp ? grp : part;
+        const u32 nt = grp ? (nb + (1u << grp_log) - 1) >> grp_log : nb;
+        const u32 b0 = blockIdx.x * ITEMS, mine = b0 >> grp_log;
+        for (u32 x = threadIdx.x; x < nt; x += LOC_TPB) {
+            const u64 t = tot[x];
+            const i32 v = (i32)(u32)t, w = (i32)(u32)(t >> 32);
             ta += v;
             tb += w;
-            if (x < blockIdx.x) { a += v; b += w; }
+            if (x < mine) { a += v; b += w; }
         }
+        if (grp)
+            for (u32 x = (mine << grp_log) + threadIdx.x; x < b0; x += LOC_TPB) {
+                const u64 t = part[x];
+                a += (i32)(u32)t;
+                b += (i32)(u32)(t >> 32);
+            }
         a = wave_sum(a); b = wave_sum(b); ta = wave_sum(ta); tb = wave_sum(tb);
-        if (lane_id() == 0) {
-            red[0][threadIdx.x >> 6] = a; red[1][threadIdx.x >> 6] = b;
-            red[2][threadIdx.x >> 6] = ta; red[3][threadIdx.x >> 6] = tb;
-        }
-        __syncthreads();
-        base_c = 0; base_d = 0; ta = 0; tb = 0;
-        for (int w = 0; w < LOC_TPB / 64; ++w) {
-            base_c += red[0][w]; base_d += red[1][w]; ta += red[2][w]; tb += red[3][w];
-        }
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            status->n_eff = (u32)ta;
-            status->delta = tb;
-            pd[ta] = tb;
-        }
-    } else {
-        base_c = pc[blockIdx.x];
-        base_d = pdl[blockIdx.x];
+        if (lane_id() == 0) { red[0][wv] = a; red[1][wv] = b; red[2][wv] = ta; red[3][wv] = tb; }
     }
-    const u64 i = (u64)blockIdx.x * LOC_TILE + threadIdx.x;
-    const u64 sg = i < n ? useg[i] : RK_NONE;
-    i32 ce = 0, cd = 0;
-    if (sg != RK_NONE) { ce = 1; cd = (sg & RK_OP) ? 1 : -1; }
-    i32 t1, t2;
-    i32 ex = block_excl_scan<LOC_TPB, i32>(ce, t1, tmp) + base_c;
-    i32 dx = block_excl_scan<LOC_TPB, i32>(cd, t2, tmp) + base_d;
-    if (sg != RK_NONE) {
-        ckey[ex] = ukey[i];
-        cseg[ex] = sg & ~RK_OP;
-        pd[ex] = dx;
+    u32 inc[ITEMS], own[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        own[r] = sg[r] & RK_SKIP ? 0u : 1u | (sg[r] & RK_OP ? 1u << 16 : 0u);
+        inc[r] = dpp_incl_scan32(own[r]);
+        if (lane_id() == 63) wt[r * NW + wv] = inc[r];
     }
-    if (g.npma == 1) {
-        // update index: the first update of each index-level window.  The
-        // wave's updates are sorted, so only the first of each window in
-        // the wave competes (atomic min) with the other waves'.
-        const u32 H = pma_of(g, 0).H, lb = index_level(H);
-        if (lb <= H) {
-            const bool e = sg != RK_NONE;
-            const u32 w = e ? (u32)sg >> lb : 0u;  // low word of a run key: the segment
-            const u64 below = __ballot(e) & ((1ull << lane_id()) - 1ull);
-            const int p = below ? 63 - __clzll((long long)below) : (int)lane_id();
-            const u32 wp = (u32)__shfl((int)w, p, 64);
-            if (e && (below == 0 || wp != w)) atomicMin(&wfirst[w], (u32)ex);
+    __syncthreads();
+    i32 base_c = 0, base_d = 0, ta = 0, tb = 0;
+    for (u32 w = 0; w < NW; ++w) {
+        base_c += red[0][w]; base_d += red[1][w]; ta += red[2][w]; tb += red[3][w];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        status->n_eff = (u32)ta;
+        status->delta = tb;
+        pd[ta] = tb;
+    }
+    u32 before = 0;  // of the workgroup's earlier waves and blocks
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        u32 pre = before;
+#pragma unroll
+        for (u32 w = 0; w < NW; ++w) {
+            const u32 t = wt[r * NW + w];
+            if (w < wv) pre += t;
+            before += t;
+        }
+        pre += inc[r] - own[r];
+        const i32 c = (i32)(pre & 0xFFFFu), ins = (i32)(pre >> 16);
+        const u32 ex = (u32)(base_c + c);
+        if (!(sg[r] & RK_SKIP)) {
+            ckey[ex] = uk[r];
+            cseg[ex] = sg[r] & ~RK_OP;
+            pd[ex] = base_d + 2 * ins - c;
+        }
+        if (g.npma == 1 && sg[r] != RK_NONE) {
+            // update index: the first update of each index-level window,
+            // written by the first located element of the window (with or
+            // without effect: the compacted index is the same), found by a
+            // look at the element before it.  Where that one is a duplicate,
+            // which was not located, the smallest index wins by an atomic.
+            // (An atomic from every wave that enters a window took 650 us
+            // where 8.4 M keys land in the 128 windows of a PMA about to be
+            // built.)
+            const u32 H = pma_of(g, 0).H, lb = index_level(H);
+            if (lb <= H) {
+                const u32 w = (u32)sg[r] >> lb;  // low word of a run key: the segment
+                const u64 i = i0 + r * LOC_TILE;
+                if (i > 0 && prev[r] == RK_NONE) atomicMin(&wfirst[w], ex);
+                else if (i == 0 || (u32)prev[r] >> lb != w) wfirst[w] = ex;
+            }
         }
     }
 }
 
 hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchBufs &b, hipStream_t st) {
     u32 nb = locate_blocks(n);
-    i32 *pc = b.part, *pdl = b.part + nb + 1;
-    if (g.inline_one) k_locate<true><<<nb, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, pc, pdl);
-    else k_locate<false><<<nb, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, pc, pdl);
-    int self_prefix = nb <= COMPACT_SELF_PREFIX_MAX;
-    if (!self_prefix) k_scan_parts<<<1, 1024, 0, st>>>(pc, pdl, nb, b.status, b.pd);
-    k_compact<<<nb, LOC_TPB, 0, st>>>(g, b.ukey, b.useg, n, pc, pdl, nb, self_prefix, b.ckey, b.cseg, b.pd,
-                                      b.wfirst, b.status);
+    const u32 gl = locate_group_log(nb);
+    u64 *grp = gl ? b.part : nullptr, *part = b.part + LOC_GROUPS;
+    // Large batches take LOC_ITEMS keys a thread (more probes in flight, a
+    // narrower range for each key).  Small ones over many segments (a lone
+    // PMA's, where the height is known here) skip the range: 1000 keys over
+    // 2^19 segments would stage 2^17 separators a tile.
+    // Large batches: LOC_ITEMS keys a thread, searching their tile's staged
+    // range (8.4 M keys into 2^15 segments: 142 -> 73 us; 2 M into 2^19: 54
+    // -> 52-59, the probes' lines bound it).  Below, one key a thread over
+    // all separators: more waves hide the latency (160 K keys over 2^21
+    // segments: 31 us against 35 us, 10^5 over 2^19: 9.2 against 18).
+    if (gl) {
+        const u32 grid = (nb + LOC_ITEMS - 1) / LOC_ITEMS;
+        if (g.inline_one)
+            k_locate<true, LOC_ITEMS, true><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+        else
+            k_locate<false, LOC_ITEMS, true><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+    } else {
+        if (g.inline_one)
+            k_locate<true, 1, false><<<nb, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+        else
+            k_locate<false, 1, false><<<nb, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+    }
+    if (gl)
+        k_compact<LOC_ITEMS><<<(nb + LOC_ITEMS - 1) / LOC_ITEMS, LOC_TPB, 0, st>>>(
+            g, b.ukey, b.useg, n, part, grp, nb, gl, b.ckey, b.cseg, b.pd, b.wfirst, b.status);
+    else
+        k_compact<1><<<nb, LOC_TPB, 0, st>>>(g, b.ukey, b.useg, n, part, grp, nb, gl, b.ckey, b.cseg, b.pd, b.wfirst,
+                                             b.status);
     return hipGetLastError();
 }
 
@@ -1972,8 +2137,9 @@ __global__ __launch_bounds__(256) void k_pyr_chunk_group(Group g) {
 __global__ __launch_bounds__(1024) void k_pyr_top(DevState d) { pyr_top_levels(d); }
 
 __global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, InlineSegs in, BatchSeg *segs, u32 *zero,
-                                                      u32 nzero, u32 *wfirst) {
+                                                      u32 nzero, u32 *wfirst, u64 *grp) {
     if (blockIdx.x == 0 && threadIdx.x < in.n) segs[threadIdx.x] = in.s[threadIdx.x];
+    if (blockIdx.x == 0 && threadIdx.x < LOC_GROUPS) grp[threadIdx.x] = 0;
     batch_first_work(g, s, blockIdx.x, zero, nzero, wfirst);
 }
 

@@ -1,0 +1,65 @@
+"""Batches at the sizes where the update path changes kernels, against the
+oracle (edges, CSR offsets) and its layout model (slots, row offsets)."""
+import numpy as np
+import pytest
+
+import lpma_amd as L
+import oracle
+from gpu_util import Triple, keys_of, say
+
+pytestmark = pytest.mark.gpu
+
+
+def rand_keys(rng, V, n):
+    return keys_of(rng.integers(0, V, n), rng.integers(0, V, n))
+
+
+# 2048 blocks of 256 keys: the last size whose locate and compaction sum the
+# blocks directly, and the first with groups of blocks and staged separators
+@pytest.mark.parametrize("n", [524288, 524289, 700001])
+@pytest.mark.parametrize("V,S,spread", [(3000, 32, 1), (200, 2, 1), (1 << 18, 64, 1), (3000, 32, 7)])
+def test_large_batch_locate(n, V, S, spread):
+    rng = np.random.default_rng(n + V)
+    t = Triple(V, segment_slots=S)
+    say(f"locate n={n} V={V} S={S} spread={spread}")
+    a = np.repeat(rand_keys(rng, V, -(-n // spread)), spread)[:n]  # runs of equal keys
+    t.insert(a)
+    t.compare()
+    b = rand_keys(rng, V, n)
+    t.mixed(b[: n // 2], np.concatenate([a[: n // 3], b[n // 2:]])[: n - n // 2])
+    t.compare()
+    t.close()
+
+
+def test_locate_tile_wider_than_its_stage():
+    """Few keys over many segments: a tile's separators do not fit the LDS."""
+    V, n = 1 << 22, 530001
+    rng = np.random.default_rng(5)
+    say(f"locate wide V={V} n={n}")
+    t = Triple(V, segment_slots=2, model=False)
+    t.insert(rand_keys(rng, V, n))
+    t.compare(layout=False)
+    t.close()
+
+
+def test_locate_tile_over_two_members():
+    """A group round whose tiles hold the end of one member and the start of the next."""
+    rng = np.random.default_rng(6)
+    Vs = (500, 70000, 9)
+    say(f"locate group {Vs}")
+    ps = [L.PMA(V) for V in Vs]
+    g = L.Group(ps)
+    refs = [np.empty(0, dtype=np.uint64) for _ in Vs]
+    for r in range(2):
+        ins = [rand_keys(rng, V, n) for V, n in zip(Vs, (300001, 300077, 33))]
+        dels = [ref[:: 3] for ref in refs]
+        g.update(ins, dels)
+        for i, V in enumerate(Vs):
+            refs[i] = oracle.apply(refs[i], ins[i], dels[i])
+            ek, ro = ps[i].export()
+            assert np.array_equal(L.to_host_u64(ek), refs[i])
+            assert np.array_equal(ro.cpu().numpy().view(np.uint32), oracle.row_offsets(refs[i], V))
+            assert ps[i].check() == 0
+    g.close()
+    for p in ps:
+        p.close()
