@@ -776,7 +776,8 @@ int finish_round(Pipeline &pl, const Member *mem, u32 npma, const Group &g_in, u
         }
         for (u32 p = 0; !r && any_rebuild && p < npma; ++p)
             if (ps[p].flags & (FLAG_ROOT | FLAG_RESIZE)) {
-                r = ensure(pl, pl.gpre, rebuild_index_words(mem[p].h->st));
+                if (rebuild_merges(mem[p].h->live, ps[p].u1 - ps[p].u0)) r = ensure(pl, pl.merged, mem[p].h->live);
+                if (!r) r = ensure(pl, pl.gpre, rebuild_index_words(mem[p].h->st));
                 if (!r) r = alloc_geometry(mem[p].h, newH[p], geo[p], st);
             }
         if (r) return undo(r);
@@ -838,8 +839,8 @@ int finish_round(Pipeline &pl, const Member *mem, u32 npma, const Group &g_in, u
         for (u32 p = 0; p < npma; ++p) {
             if (!(ps[p].flags & (FLAG_ROOT | FLAG_RESIZE))) continue;
             lpma *h = mem[p].h;
-            HIPUNDO(rebuild_scatter(h->st, state_with(h, newH[p], geo[p]), p, ps[p].u0, ps[p].u1, bb, Mnew[p],
-                                    pl.gpre.p, st));
+            HIPUNDO(rebuild_scatter(h->st, state_with(h, newH[p], geo[p]), p, ps[p].u0, ps[p].u1, bb, h->live,
+                                    Mnew[p], pl.gpre.p, pl.merged.p, st));
             const int r = pyramid_and_install(h, newH[p], geo[p], st);
             if (r) return undo(r);
             h->rebuilds++;

@@ -1787,13 +1787,11 @@ __global__ __launch_bounds__(LGP_TPB) void k_large_push(Group g, const Work *__r
 // order (its surviving keys from registers, its inserts from a stash; up to
 // RB_MERGED of them, more than a full chunk holds), and
 // then the destination segments that hold its ranks are written slot by
-// slot, coalesced: a slot of segment x, lane j holds rank
-// spread_first(x) + j if j is below the segment's count.  A chunk writes
-// the slots of its own ranks, the count and separator of the segments whose
-// first rank is its, and the empty tail of the segments whose last rank is
-// its (with the segments left empty after them: fewer keys than segments);
-// markers also write their row offsets.  A chunk whose keys outgrow the
-// LDS (many inserts) places each key by the even spread's inverse instead.
+// slot, coalesced (spread_out): a slot of segment x, lane j holds rank
+// spread_first(x) + j if j is below the segment's count.  A chunk whose keys
+// outgrow the LDS (many inserts) places each key by the even spread's inverse
+// instead.  16.7 M keys into 2^25 slots: 114 us (145 us with one slot a thread
+// in the writer).
 static constexpr u32 RB_STASH = 256;  // inserts a chunk keeps in LDS
 // merged keys a chunk assembles in LDS: the room of its slots, counts and
 // shifts (ChunkLds up to del), read by then
@@ -1819,6 +1817,55 @@ __device__ __forceinline__ u64 spread_segment(u64 o, u64 M, u32 H, double seg_pe
         g = spread_first(++x + 1, M, H);
     }
     return x;
+}
+
+// Writes the destination segments of ranks [r0, r1) (all of the M keys after
+// the batch, spread over t's 2^t.H segments), whose keys lie in LDS in rank
+// order (mk[o - r0]): two slots a thread, 16-byte stores (one slot a thread
+// issued twice the index arithmetic and stores).  The caller writes the slots
+// of its own ranks, the count and separator of the segments whose first rank
+// is its, the empty tail of the segments whose last rank is its and the
+// segments left empty after them; markers also write their row offsets.
+__device__ __forceinline__ void spread_out(const DevState &t, u64 M, double seg_per_key, u64 r0, u64 r1,
+                                           const u64 *mk) {
+    if (r1 <= r0) return;
+    const u32 Ht = t.H, log2S = t.log2S;
+    const u64 nseg_t = nseg_of(t), Nm1 = nseg_t - 1;
+    u64 f, g;
+    const u64 x0 = spread_segment(r0, M, Ht, seg_per_key, f, g);
+    const u64 xk = spread_segment(r1 - 1, M, Ht, seg_per_key, f, g);
+    const u64 xe = r1 < M ? spread_segment(r1, M, Ht, seg_per_key, f, g) : nseg_t;
+    const u64 x1 = xe > xk + 1 ? xe : xk + 1;
+    const u64 npairs = (x1 - x0) << (log2S - 1);
+    const u32 half = (1u << (log2S - 1)) - 1;
+    for (u64 i = threadIdx.x; i < npairs; i += blockDim.x) {
+        const u64 x = x0 + (i >> (log2S - 1));
+        const u32 lane = ((u32)i & half) * 2;
+        const u64 tt = x * M + Nm1;
+        const u64 fx = tt >> Ht, gx = (tt + M) >> Ht;  // spread_first(x), spread_first(x + 1)
+        const u32 c = (u32)(gx - fx);
+        const u64 slot = (x0 << log2S) + 2 * i;
+        const u64 o = fx + lane;
+        // the tail belongs to the caller of the segment's last rank, an empty
+        // segment's to the caller of the rank before (gx >= 1: the first
+        // segment is never empty)
+        const u64 last = gx - 1;
+        const bool tail = last >= r0 && last < r1;
+        const bool w0 = lane < c ? o >= r0 && o < r1 : tail;
+        const bool w1 = lane + 1 < c ? o + 1 >= r0 && o + 1 < r1 : tail;
+        u64 k0 = KEY_NONE, k1 = KEY_NONE;
+        if (w0 && lane < c) k0 = mk[o - r0];
+        if (w1 && lane + 1 < c) k1 = mk[o + 1 - r0];
+        if (w0 && w1) *(ulonglong2 *)(t.keys + slot) = make_ulonglong2(k0, k1);
+        else if (w0) t.keys[slot] = k0;
+        else if (w1) t.keys[slot + 1] = k1;
+        if (is_marker(k0) && (u32)(k0 >> 32) < t.V) t.row_off[(u32)(k0 >> 32) + 1] = (u32)slot;
+        if (is_marker(k1) && (u32)(k1 >> 32) < t.V) t.row_off[(u32)(k1 >> 32) + 1] = (u32)slot + 1;
+        if (lane == 0 && w0) {
+            t.cnt[x] = c;
+            t.sep[x] = x == 0 ? 0ull : (c ? k0 : mk[last - r0] + 1);
+        }
+    }
 }
 
 __global__ __launch_bounds__(LGP_TPB) __attribute__((amdgpu_waves_per_eu(4))) void k_rebuild_scatter(DevState s, DevState t, u64 pb, u32 u0, u32 u1, u64 M,
@@ -1914,44 +1961,7 @@ __global__ __launch_bounds__(LGP_TPB) __attribute__((amdgpu_waves_per_eu(4))) vo
             if (ov[k] != ~0u) mk[ov[k]] = kv[k];
         for (u32 i = threadIdx.x; i < R.n; i += LGP_TPB) mk[R.io[i] - r0] = R.iy[i];
         __syncthreads();
-        if (r1 > r0) {
-            u64 f, g;
-            const u64 x0 = spread_segment(r0, M, Ht, seg_per_key, f, g);
-            const u64 xk = spread_segment(r1 - 1, M, Ht, seg_per_key, f, g);
-            const u64 xe = r1 < M ? spread_segment(r1, M, Ht, seg_per_key, f, g) : nseg_t;
-            const u64 x1 = xe > xk + 1 ? xe : xk + 1;
-            const u64 nslots = (x1 - x0) << log2S;
-            for (u64 i = threadIdx.x; i < nslots; i += LGP_TPB) {
-                const u64 x = x0 + (i >> log2S);
-                const u32 lane = (u32)i & (SL - 1);
-                const u64 tt = x * M + Nm1;
-                const u64 fx = tt >> Ht, gx = (tt + M) >> Ht;  // spread_first(x), spread_first(x + 1)
-                const u64 slot = (x0 << log2S) + i;
-                if (lane < gx - fx) {
-                    const u64 o = fx + lane;
-                    if (o >= r0 && o < r1) {
-                        const u64 key = mk[o - r0];
-                        t.keys[slot] = key;
-                        if (is_marker(key) && (u32)(key >> 32) < t.V) t.row_off[(u32)(key >> 32) + 1] = (u32)slot;
-                        if (lane == 0) {
-                            t.cnt[x] = (u32)(gx - fx);
-                            t.sep[x] = x == 0 ? 0ull : key;
-                        }
-                    }
-                } else {
-                    // the tail belongs to the chunk of the segment's last
-                    // rank, an empty segment's to the chunk of the rank before
-                    const u64 last = gx - 1;  // gx >= 1: fx == gx == 0 is impossible past segment 0
-                    if (last >= r0 && last < r1) {
-                        t.keys[slot] = KEY_NONE;
-                        if (lane == 0 && gx == fx) {
-                            t.cnt[x] = 0;
-                            t.sep[x] = mk[last - r0] + 1;
-                        }
-                    }
-                }
-            }
-        }
+        spread_out(t, M, seg_per_key, r0, r1, mk);
         __syncthreads();  // the LDS arrays are reused by the next chunk
     }
 }
@@ -1981,21 +1991,166 @@ __global__ __launch_bounds__(256) void k_chunk_index(DevState s, u64 pb, u32 u0,
     }
 }
 
+// ------------------------------------------------ rebuild by merging
+//
+// A batch that is large against the PMA (a graph's first load into a PMA of
+// row markers) puts more keys into a chunk of the old arrays than its LDS
+// holds, and a hub's edges all into one chunk: k_rebuild_scatter then places
+// key by key, and one workgroup ends long after the others (4.4 ms for 8.4 M
+// keys into 2^20 markers).  Here the work is cut by the merged order instead:
+// the live keys are first gathered in key order (k_gather_live), then tile t
+// merges the items [t T, (t + 1) T) of the live keys and the updates together,
+// found by a search along the merge's diagonal, so every workgroup has T items
+// whatever the skew.  Bound: the new arrays' stores.
+
+// the live keys of s in key order; a workgroup per chunk of 2^cl segments,
+// its first rank from the chunk index
+__global__ __launch_bounds__(LGP_TPB) void k_gather_live(DevState s, const u64 *__restrict__ cob,
+                                                         u64 *__restrict__ out) {
+    __shared__ u32 pre[LG_SEG_MAX + 1];
+    __shared__ u32 stmp[LGP_TPB / 64 + 1];
+    const u32 cl = chunk_level(s.log2S, s.H);
+    const u32 nsc = 1u << cl, W = nsc << s.log2S;
+    const u64 s0 = (u64)blockIdx.x << cl;
+    for (u32 x = threadIdx.x; x < nsc; x += LGP_TPB) pre[x] = s.cnt[s0 + x];
+    const u64 base = cob[blockIdx.x];
+    __syncthreads();
+    block_scan_runs<LGP_TPB, LGP_PER>(pre, nsc, stmp);
+    const u64 *keys = s.keys + (s0 << s.log2S);
+    for (u32 t = threadIdx.x; t < W; t += LGP_TPB) {
+        const u32 seg = t >> s.log2S, lane = t & ((1u << s.log2S) - 1);
+        const u32 p0 = pre[seg];
+        if (lane < pre[seg + 1] - p0) out[base + p0 + lane] = keys[t];
+    }
+}
+
+static constexpr u32 RM_TILE = 2048;  // merged items of a tile
+static constexpr u32 RM_PER = RM_TILE / LGP_TPB;
+
+// live keys among the first D items of the merge of A and U (equal keys: the
+// live key first), by one whole wave
+__device__ __forceinline__ u32 merge_split(const u64 *__restrict__ A, u32 na, const u64 *__restrict__ U, u32 nu,
+                                           u64 D) {
+    const u32 lane = lane_id();
+    u32 lo = D > nu ? (u32)(D - nu) : 0u, hi = D < na ? (u32)D : na;
+    while (lo < hi) {
+        const u32 step = (hi - lo + 63) / 64;
+        const u32 p = lo + lane * step;
+        const u64 below = __ballot(p < hi && A[p] <= U[D - 1 - p]);  // a prefix of the lanes
+        const u32 c = (u32)__popcll(below);
+        if (c == 0) return lo;
+        const u32 nlo = lo + (c - 1) * step + 1;
+        hi = min(lo + c * step, hi);
+        lo = nlo;
+    }
+    return lo;
+}
+
+// U, pd: the PMA's nu updates and their prefix (nu + 1 entries); a delete
+// meets its live key, an insert none.  A tile's output ranks are contiguous:
+// its keys are assembled in LDS in rank order and spread_out writes them.
+__global__ __launch_bounds__(LGP_TPB) void k_rebuild_merge(DevState t, const u64 *__restrict__ A, u32 na,
+                                                           const u64 *__restrict__ U, const i32 *__restrict__ pd,
+                                                           u32 nu, u64 M, double seg_per_key) {
+    __shared__ u64 it[RM_TILE];  // the tile's live keys, then its updates; then its merged keys
+    __shared__ i32 P[RM_TILE + 1];
+    __shared__ u32 spl[2];
+    const u32 tid = threadIdx.x, wv = tid >> 6;
+    const u64 all = (u64)na + nu;
+    const u64 D0 = (u64)blockIdx.x * RM_TILE, D1 = min(all, D0 + RM_TILE);
+    if (wv < 2) {
+        const u32 x = merge_split(A, na, U, nu, wv ? D1 : D0);
+        if (lane_id() == 0) spl[wv] = x;
+    }
+    __syncthreads();
+    const u32 i0 = spl[0], i1 = spl[1];
+    const u32 j0 = (u32)(D0 - i0), j1 = (u32)(D1 - i1);
+    const u32 ca = i1 - i0, cu = j1 - j0, n = ca + cu;
+    const i32 pbase = pd[0];
+    // a boundary between a live key and its delete: the rank prefix there is
+    // the one after the delete
+    const u64 nxt = j1 < nu ? U[j1] : KEY_NONE;
+    const bool del0 = i0 > 0 && j0 < nu && U[j0] == A[i0 - 1];
+    const bool del1 = i1 > 0 && j1 < nu && nxt == A[i1 - 1];
+    const u64 r0 = (u64)i0 + (u64)(i64)(pd[j0 + (del0 ? 1 : 0)] - pbase);
+    const u64 r1 = (u64)i1 + (u64)(i64)(pd[j1 + (del1 ? 1 : 0)] - pbase);
+    u64 v[RM_PER];
+#pragma unroll
+    for (u32 k = 0; k < RM_PER; ++k) {
+        const u32 x = tid + k * LGP_TPB;
+        v[k] = x < n ? (x < ca ? A[i0 + x] : U[j0 + (x - ca)]) : KEY_NONE;
+    }
+    for (u32 x = tid; x <= cu; x += LGP_TPB) P[x] = pd[j0 + x] - pbase;
+#pragma unroll
+    for (u32 k = 0; k < RM_PER; ++k) {
+        const u32 x = tid + k * LGP_TPB;
+        if (x < n) it[x] = v[k];
+    }
+    __syncthreads();
+    // each item's lower bound in the other list; the items' searches step
+    // together
+    u32 pos[RM_PER];
+#pragma unroll
+    for (u32 k = 0; k < RM_PER; ++k) pos[k] = 0;
+    const u32 longer = max(ca, cu);
+    for (u32 h = longer ? 1u << (31 - __clz((int)longer)) : 0u; h; h >>= 1) {
+#pragma unroll
+        for (u32 k = 0; k < RM_PER; ++k) {
+            const bool live = tid + k * LGP_TPB < ca;
+            const u32 off = live ? ca : 0u, len = live ? cu : ca;
+            if (pos[k] + h <= len && it[off + pos[k] + h - 1] < v[k]) pos[k] += h;
+        }
+    }
+    u32 o[RM_PER];
+#pragma unroll
+    for (u32 k = 0; k < RM_PER; ++k) {
+        const u32 x = tid + k * LGP_TPB;
+        o[k] = ~0u;
+        if (x < ca) {
+            const u32 q = pos[k];
+            const bool gone = (q < cu ? it[ca + q] : nxt) == v[k];
+            if (!gone) o[k] = (u32)((u64)(i0 + x) + (u64)(i64)P[q] - r0);
+        } else if (x < n) {
+            const u32 q = x - ca;
+            if (P[q + 1] - P[q] == 1) o[k] = (u32)((u64)(i0 + pos[k]) + (u64)(i64)P[q] - r0);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (u32 k = 0; k < RM_PER; ++k)
+        if (o[k] < RM_TILE) it[o[k]] = v[k];
+    __syncthreads();
+    spread_out(t, M, seg_per_key, r0, r1, it);
+}
+
 u64 rebuild_index_words(const DevState &src) {
     const u64 nch = nseg_of(src) >> chunk_level(src.log2S, src.H);
     return 3 * (nch + 1) + 2;
 }
 
+// By merging when the updates are more than half of the live keys: a chunk
+// (about 1150 live keys) then meets more than 500 of them.  Measured into 2^25
+// slots, keys spread like the graph's: 4 M updates on 16.7 M live keys 179 us
+// by chunks, 245 us by merging (10^5: 119 against 174); 15.6 M on 2^20, a first
+// load: 7.6 ms by chunks (a hub's edges meet in one of 512), 148 us by merging.
+bool rebuild_merges(u64 live, u64 updates) { return 2 * updates > live; }
+
 hipError_t rebuild_scatter(const DevState &src, const DevState &dst, u32 pid, u32 u0, u32 u1, const BatchBufs &b,
-                           u64 m, u32 *index, hipStream_t st) {
+                           u64 live, u64 m, u32 *index, u64 *merged, hipStream_t st) {
     const u64 nch = nseg_of(src) >> chunk_level(src.log2S, src.H);
     u32 *cq = index;                                                 // nch + 1 words
     u64 *cob = (u64 *)(((uintptr_t)(index + nch + 1) + 7) & ~(uintptr_t)7);  // nch u64, 8-byte aligned
     const u64 pb = (u64)pid << 32;
+    const double spk = (double)nseg_of(dst) / (double)m;
     k_chunk_index<<<(u32)((nch + 1 + 3) / 4), 256, 0, st>>>(src, pb, u0, u1, b.cseg, cq, cob);
+    if (rebuild_merges(live, u1 - u0)) {
+        k_gather_live<<<(u32)nch, LGP_TPB, 0, st>>>(src, cob, merged);
+        const u32 tiles = (u32)((live + (u1 - u0) + RM_TILE - 1) / RM_TILE);
+        k_rebuild_merge<<<tiles, LGP_TPB, 0, st>>>(dst, merged, (u32)live, b.ckey + u0, b.pd + u0, u1 - u0, m, spk);
+        return hipGetLastError();
+    }
     const u32 grid = (u32)std::min<u64>(nch, 1024);  // ~33 KB of LDS per block: four per CU
-    k_rebuild_scatter<<<grid, LGP_TPB, 0, st>>>(src, dst, pb, u0, u1, m, (double)nseg_of(dst) / (double)m, b.ckey,
-                                                b.cseg, b.pd, cq, cob);
+    k_rebuild_scatter<<<grid, LGP_TPB, 0, st>>>(src, dst, pb, u0, u1, m, spk, b.ckey, b.cseg, b.pd, cq, cob);
     return hipGetLastError();
 }
 

@@ -63,3 +63,25 @@ def test_locate_tile_over_two_members():
     g.close()
     for p in ps:
         p.close()
+
+
+# a rebuild merges when the updates are more than half of the live keys; tiles
+# of 2048 merged items: sizes at their edges, deletes on a tile's boundary, a
+# hub row, segments from 2 to 1024 slots
+@pytest.mark.parametrize("S", [2, 32, 1024])
+@pytest.mark.parametrize("V,n", [(1, 1), (3, 5), (100, 2048 - 100), (100, 2049 - 100), (700, 4096), (5000, 60000)])
+def test_rebuild_by_merging(V, n, S):
+    rng = np.random.default_rng(V + n)
+    say(f"rebuild merge V={V} n={n} S={S}")
+    t = Triple(V, segment_slots=S)
+    a = rand_keys(rng, V, n)
+    a[: n // 2] &= np.uint64(0xFFFFFFFF)  # half of the edges leave vertex 0
+    t.insert(a)  # grows
+    t.compare()
+    t.delete(t.ref[rng.random(t.ref.size) < 0.9])  # shrinks: most live keys deleted
+    t.compare()
+    t.mixed(rand_keys(rng, V, 3 * n), t.ref)  # grows while every edge goes
+    t.compare()
+    t.delete(t.ref)
+    t.compare()
+    t.close()
