@@ -228,9 +228,10 @@ int lpma_snapshot_set_search_width(lpma_snapshot_t *s, uint32_t workgroups);
 /* PageRank over the gapped layout with nvGraph's formulation
  * (include/pagerank.hxx:66-88): from the uniform vector, until the L1 change
  * is below `tolerance` or `max_iter` iterations, then L1-normalised.  FP32
- * values and accumulation.  d_rank has V entries.  Synchronises the stream
- * once to size the per-call edge bins (V <= 2^27) and once per iteration.
- * Device scratch grows to about 8 B per edge plus 32 B per vertex. */
+ * values; sums exact in 64-bit fixed point (V <= 2^27) or compensated FP32.
+ * The host waits for every iteration's L1 change, and for the stream at the
+ * end.  d_rank has V entries.  Device scratch grows to about 5 B per edge
+ * plus 32 B per vertex. */
 int lpma_pagerank(lpma_t *h, float damping, float tolerance, uint32_t max_iter, float *d_rank, uint32_t *iterations,
                   float *last_delta, void *stream);
 

@@ -435,34 +435,41 @@ hipError_t pr_scale(float *pr, u32 V, const float *red, hipStream_t st) {
     return hipGetLastError();
 }
 
-// ------------------------------------------------- binned push (PageRank)
+// ------------------------------------------------- binned edges (PageRank)
 //
 // The push above sends every edge's contribution to a random destination in
 // HBM: one returning atomic per edge on a 64 MB vector, which no L2 holds.
-// Propagation blocking (Beamer, Asanovic, Patterson, "Reducing PageRank
-// communication via propagation blocking", IPDPS 2017) splits it in two
-// streaming passes over the same gapped layout:
-//   bin pass   the slot array is cut into parts of 2^part_log slots; each
-//              part's workgroup writes (dst mod PB_BIN, contribution) pairs
-//              into per-destination-bin runs, at offsets fixed once per call
-//              by a count pass (bin-major exclusive scan of count[bin][part]);
-//   acc pass   each chunk of a bin's pairs is summed in LDS (PB_BIN vertices,
-//              compensated like the atomics above) and written as one
-//              partial vector; the finish pass adds a bin's partials (Kahan).
-// Every access to HBM is then a stream; the random adds stay in LDS.  The
-// graph does not change during a call, so the count pass runs once.
+// Binning the edges by destination (propagation blocking: Beamer, Asanovic,
+// Patterson, "Reducing PageRank communication via propagation blocking",
+// IPDPS 2017) keeps the random adds in LDS.  The graph does not change during
+// a call, so the edges are binned once, not their contributions every
+// iteration:
+//   count    the slot array is cut into parts of 2^part_log slots; the edges
+//            of each (bin, part) are counted and the bin-major exclusive scan
+//            of the counts fixes where each goes;
+//   bin      each part's workgroup writes its edges into its bins' runs, one
+//            word each: source relative to the part's first row, destination
+//            relative to the bin.  Runs are padded to groups of PB_CHUNK words
+//            and each group has the part's first row beside it;
+// and an iteration is one kernel (k_pr_iter): a workgroup takes a chunk of a
+// bin's edges, reads the source's contribution (a run's sources ascend, so
+// the lanes of a wave share lines and the workgroups of an XCD sweep the
+// vector together), adds it to the destination in LDS, and finishes the bin's
+// vertices: rank, next contribution, dangling mass, L1 change.
 
 static constexpr u32 PB_BIN_LOG = 13;  // destination vertices per bin
 static constexpr u32 PB_BIN = 1u << PB_BIN_LOG;
 static constexpr u32 PB_MAX_BINS = 16384;  // LDS cursors of the bin pass: 64 KB
 static constexpr u32 PB_TPB = 1024;
 static constexpr u32 PB_ITEMS = 8;
-static constexpr u32 PB_MAX_PARTS = 1024;
-static constexpr u32 PB_CHUNK = 4;                // pairs per staged chunk (32 B, one HBM sector)
+static constexpr u32 PB_MAX_PART_LOG = 18;         // slots per part (log2): see pb_word
+static constexpr u32 PB_MAX_PARTS = 1u << (32 - PB_MAX_PART_LOG);
+static constexpr u32 PB_CHUNK = 8;                // words per group and staged chunk (32 B, one HBM sector)
 static constexpr u32 PB_STAGE_MAX_BINS = 2048;    // staged bin pass LDS: 40 B per bin
 static constexpr u32 PBS_TPB = 512;               // staged bin pass: two workgroups per CU (80 KB LDS each)
 static constexpr u32 PBS_ITEMS = 8;
-static constexpr u32 PBA_TPB = 512;               // acc pass: fewer waves per LDS accumulator contend less
+static constexpr u32 PRI_TPB = 1024;              // iteration: two workgroups of 64 KB of LDS fill a CU's waves
+static constexpr u32 PRI_ITEMS = 8;
 
 // Lanes holding a live edge of the same bin form runs (adjacent lanes; keys
 // are sorted, so a row's edges to one bin are adjacent).  Returns the lane
@@ -506,10 +513,36 @@ __device__ __forceinline__ void pb_load(const DevState &d, u64 t0, u64 p1, u64 (
 }
 
 __device__ __forceinline__ bool pb_edge(u64 key) { return key != KEY_NONE && !is_marker(key); }
+// An edge in its bin: its source relative to the part's first row, and its
+// destination within the bin.  Every row has its marker in a slot, so a part
+// of 2^18 slots holds edges of at most 2^18 + 1 rows: 19 bits over the bin's
+// 13, and no edge gives the padding word.
+static constexpr u32 PB_PAD = 0xFFFFFFFFu;
+static_assert((1ull << PB_MAX_PART_LOG) + 1 < (1ull << (32 - PB_BIN_LOG)) - 1, "a source fits above the destination");
+__device__ __forceinline__ u32 pb_word(u64 key, u32 row0) {
+    return (((u32)(key >> 32) - row0) << PB_BIN_LOG) | ((u32)key & (PB_BIN - 1));
+}
+
+// the row that slot p lies in (rows whose marker slots are below p), by one
+// whole wave: 64 pivots a step
+__device__ __forceinline__ u32 row_of_slot(const DevState &d, u64 p) {
+    const u32 lane = lane_id();
+    u32 lo = 0, hi = d.V;  // first r with row_off[r + 1] >= p, V if none
+    while (lo < hi) {
+        const u32 step = (hi - lo + 63) / 64;
+        const u64 q = (u64)lo + (u64)lane * step;
+        const u64 below = __ballot(q < hi && d.row_off[q + 1] < p);  // a prefix of the lanes
+        const u32 c = (u32)__popcll(below);
+        if (c == 0) return lo;
+        const u32 nlo = lo + (c - 1) * step + 1;
+        hi = min((u64)lo + (u64)c * step, (u64)hi);
+        lo = nlo;
+    }
+    return lo;
+}
 
 // pb_load in separate phases, for a loop that prefetches its next step:
-// the segment counts, then the keys (after the counts), then the
-// contributions of the keys' sources (after the keys)
+// the segment counts, then the keys (after the counts)
 template <u32 TPB, u32 ITEMS>
 __device__ __forceinline__ void pb_counts(const DevState &d, u64 t0, u64 p1, u32 (&live)[ITEMS]) {
 #pragma unroll
@@ -533,17 +566,13 @@ __device__ __forceinline__ void pb_keys(const DevState &d, u64 t0, u64 p1, const
     }
 }
 
-template <u32 ITEMS>
-__device__ __forceinline__ void pb_contrib(const float *__restrict__ c, const u64 (&key)[ITEMS], float (&x)[ITEMS]) {
-#pragma unroll
-    for (u32 i = 0; i < ITEMS; ++i) x[i] = c[pb_edge(key[i]) ? (u32)(key[i] >> 32) : 0u];  // always in bounds
-}
-
 // count[bin * P + part] = live edges of `part` into `bin`, rounded up to a
-// multiple of pad + 1 (pad = PB_CHUNK - 1 for the staged bin pass, else 0)
-__global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u32 P, u32 NB, u32 pad,
-                                                     u32 *__restrict__ count) {
+// multiple of PB_CHUNK
+// (and clears the iterations' reductions)
+__global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u32 P, u32 NB,
+                                                     u32 *__restrict__ count, PrSlot *slots) {
     extern __shared__ u32 pb_lds[];
+    if (blockIdx.x == 0 && threadIdx.x < PR_SLOTS) slots[threadIdx.x] = PrSlot{0.0, 0.0, 0.0};
     for (u32 b = threadIdx.x; b < NB; b += PB_TPB) pb_lds[b] = 0;
     __syncthreads();
     const u64 W = nseg_of(d) << d.log2S;
@@ -562,17 +591,24 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u
         }
     }
     __syncthreads();
-    for (u32 b = threadIdx.x; b < NB; b += PB_TPB) count[(u64)b * P + blockIdx.x] = (pb_lds[b] + pad) & ~pad;
+    for (u32 b = threadIdx.x; b < NB; b += PB_TPB) 
+        count[(u64)b * P + blockIdx.x] = (pb_lds[b] + PB_CHUNK - 1) & ~(PB_CHUNK - 1);
 }
 
-// pairs[off[bin * P + part] + rank] = (contribution bits << 32) | (dst mod PB_BIN)
-// Phases per step: all key loads, all contribution loads, all cursor adds,
-// then the stores, so each thread keeps PB_ITEMS loads in flight at a time.
+// words[off[bin * P + part] + rank] = pb_word(edge)
+// Phases per step: all key loads, all cursor adds, then the stores, so each
+// thread keeps PB_ITEMS loads in flight at a time.
 __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32 P, u32 NB, const u32 *__restrict__ off,
-                                                   const float *__restrict__ c, u64 *__restrict__ pairs, u64 npairs) {
+                                                   u32 *__restrict__ words, u32 *__restrict__ rows, u64 room) {
     extern __shared__ u32 pb_lds[];
+    __shared__ u32 s_row0;
     for (u32 b = threadIdx.x; b < NB; b += PB_TPB) pb_lds[b] = off[(u64)b * P + blockIdx.x];
+    if (threadIdx.x < 64) {
+        const u32 r = row_of_slot(d, (u64)blockIdx.x << part_log);
+        if (threadIdx.x == 0) s_row0 = r;
+    }
     __syncthreads();
+    const u32 row0 = s_row0;
     const u64 W = nseg_of(d) << d.log2S;
     const u64 p0 = (u64)blockIdx.x << part_log;
     const u64 p1 = min(W, p0 + (1ull << part_log));
@@ -580,9 +616,6 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32
     for (u64 t0 = p0; t0 < p1; t0 += (u64)PB_TPB * PB_ITEMS) {
         u64 key[PB_ITEMS];
         pb_load(d, t0, p1, key);
-        float x[PB_ITEMS];
-#pragma unroll
-        for (u32 i = 0; i < PB_ITEMS; ++i) x[i] = c[pb_edge(key[i]) ? (u32)(key[i] >> 32) : 0u];  // always in bounds
         u32 lead[PB_ITEMS], base[PB_ITEMS];
 #pragma unroll
         for (u32 i = 0; i < PB_ITEMS; ++i) {
@@ -597,17 +630,21 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32
         for (u32 i = 0; i < PB_ITEMS; ++i) {
             const u32 b0 = __shfl(base[i], lead[i], 64);
             const u64 pos = (u64)b0 + (lane - lead[i]);
-            if (pb_edge(key[i]) && pos < npairs)
-                pairs[pos] = ((u64)__float_as_uint(x[i]) << 32) | ((u32)key[i] & (PB_BIN - 1));
+            if (pb_edge(key[i]) && pos < room) {
+                words[pos] = pb_word(key[i], row0);
+                if (pos % PB_CHUNK == 0) rows[pos / PB_CHUNK] = row0;
+            }
         }
     }
+    __syncthreads();
+    // a run's last group is filled up
+    for (u32 b = threadIdx.x; b < NB; b += PB_TPB)
+        for (u64 pos = pb_lds[b]; pos % PB_CHUNK && pos < room; ++pos) words[pos] = PB_PAD;
 }
 
-// Staged form of the bin pass (bins <= PB_STAGE_MAX_BINS): a bin's pairs
-// reach HBM only as whole aligned chunks of PB_CHUNK pairs (32 B), so no
-// partly written line is evicted from L2 and written twice.  Every run of
-// the count is padded to a multiple of PB_CHUNK; padding pairs are zero (no
-// contribution).  Per step, phase by phase:
+// Staged form of the bin pass (bins <= PB_STAGE_MAX_BINS): a bin's words
+// reach HBM only as whole aligned chunks of PB_CHUNK words (32 B), so no
+// partly written line is evicted from L2 and written twice.  Per step, phase by phase:
 //   1. ranks: each edge takes rank r on its bin's fill counter (run-aggregated);
 //   2. r < PB_CHUNK goes to the bin's LDS chunk, r inside a further complete
 //      chunk straight to HBM (a run's lanes are adjacent: coalesced), the
@@ -616,39 +653,39 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32
 //   4. the waiting edges start the next LDS chunk.
 // At the end of the part each bin's last chunk is written with zero padding.
 __global__ __launch_bounds__(PBS_TPB) void k_pb_bin_staged(DevState d, u32 part_log, u32 P, u32 NB,
-                                                          const u32 *__restrict__ off, const float *__restrict__ c,
-                                                          u64 *__restrict__ pairs, u64 npairs) {
-    extern __shared__ u64 pb_stage[];
-    u64 *buf = pb_stage;                                  // NB * PB_CHUNK staged pairs
-    u32 *fill = (u32 *)(buf + (u64)NB * PB_CHUNK);        // staged pairs per bin (< PB_CHUNK between steps)
-    u32 *gpos = fill + NB;                                // pair index of the bin's LDS chunk in HBM
+                                                          const u32 *__restrict__ off,
+                                                          u32 *__restrict__ words, u32 *__restrict__ rows, u64 room) {
+    extern __shared__ uint4 pb_stage[];
+    __shared__ u32 s_row0;
+    u32 *buf = (u32 *)pb_stage;                           // NB * PB_CHUNK staged words
+    u32 *fill = buf + (u64)NB * PB_CHUNK;                 // staged words per bin (< PB_CHUNK between steps)
+    u32 *gpos = fill + NB;                                // word index of the bin's LDS chunk in HBM
+    if (threadIdx.x < 64) {
+        const u32 r = row_of_slot(d, (u64)blockIdx.x << part_log);
+        if (threadIdx.x == 0) s_row0 = r;
+    }
     for (u32 b = threadIdx.x; b < NB; b += PBS_TPB) {
         fill[b] = 0;
         gpos[b] = off[(u64)b * P + blockIdx.x];
     }
     __syncthreads();
+    const u32 row0 = s_row0;
     const u64 W = nseg_of(d) << d.log2S;
     const u64 p0 = (u64)blockIdx.x << part_log;
     const u64 p1 = min(W, p0 + (1ull << part_log));
     const u32 lane = lane_id();
     // the next step's loads go out one phase ahead of their use: counts
-    // during the ranking, keys during the placement, contributions during
-    // the flush (the barriers wait for LDS only)
+    // during the ranking, keys during the placement (the barriers wait for
+    // LDS only)
     constexpr u64 STEP = (u64)PBS_TPB * PBS_ITEMS;
     u32 live_n[PBS_ITEMS];
     u64 key_n[PBS_ITEMS];
-    float x_n[PBS_ITEMS];
     pb_counts<PBS_TPB, PBS_ITEMS>(d, p0, p1, live_n);
     pb_keys<PBS_TPB, PBS_ITEMS>(d, p0, p1, live_n, key_n);
-    pb_contrib<PBS_ITEMS>(c, key_n, x_n);
     for (u64 t0 = p0; t0 < p1; t0 += STEP) {
         u64 key[PBS_ITEMS];
-        float x[PBS_ITEMS];
 #pragma unroll
-        for (u32 i = 0; i < PBS_ITEMS; ++i) {
-            key[i] = key_n[i];
-            x[i] = x_n[i];
-        }
+        for (u32 i = 0; i < PBS_ITEMS; ++i) key[i] = key_n[i];
         const bool more = t0 + STEP < p1;  // uniform
         if (more) pb_counts<PBS_TPB, PBS_ITEMS>(d, t0 + STEP, p1, live_n);
         u32 rank[PBS_ITEMS];
@@ -671,28 +708,31 @@ __global__ __launch_bounds__(PBS_TPB) void k_pb_bin_staged(DevState d, u32 part_
             full[i] = 0;
             if (!pb_edge(key[i])) continue;
             const u32 bin = (u32)key[i] >> PB_BIN_LOG;
-            const u64 pair = ((u64)__float_as_uint(x[i]) << 32) | ((u32)key[i] & (PB_BIN - 1));
+            const u32 word = pb_word(key[i], row0);
             full[i] = fill[bin] & ~(PB_CHUNK - 1);
             if (rank[i] < PB_CHUNK) {
-                buf[bin * PB_CHUNK + rank[i]] = pair;
+                buf[bin * PB_CHUNK + rank[i]] = word;
             } else if (rank[i] < full[i]) {
                 const u64 pos = (u64)gpos[bin] + rank[i];
-                if (pos < npairs) pairs[pos] = pair;
+                if (pos < room) {
+                    words[pos] = word;
+                    if (pos % PB_CHUNK == 0) rows[pos / PB_CHUNK] = row0;
+                }
             } else {
                 wait |= 1u << i;
             }
         }
         __syncthreads();
-        if (more) pb_contrib<PBS_ITEMS>(c, key_n, x_n);
         for (u32 b = threadIdx.x; b < NB; b += PBS_TPB) {
             const u32 F = fill[b];
             if (F >= PB_CHUNK) {
                 const u64 pos = gpos[b];
-                if (pos + PB_CHUNK <= npairs) {
+                if (pos + PB_CHUNK <= room) {
                     const uint4 *src = (const uint4 *)(buf + b * PB_CHUNK);
-                    uint4 *dst = (uint4 *)(pairs + pos);
+                    uint4 *dst = (uint4 *)(words + pos);
 #pragma unroll
-                    for (u32 k = 0; k < PB_CHUNK / 2; ++k) dst[k] = src[k];
+                    for (u32 k = 0; k < PB_CHUNK / 4; ++k) dst[k] = src[k];
+                    rows[pos / PB_CHUNK] = row0;
                 }
                 gpos[b] = (u32)(pos + (F & ~(PB_CHUNK - 1)));
                 fill[b] = F & (PB_CHUNK - 1);
@@ -703,8 +743,7 @@ __global__ __launch_bounds__(PBS_TPB) void k_pb_bin_staged(DevState d, u32 part_
         for (u32 i = 0; i < PBS_ITEMS; ++i)
             if (wait & (1u << i)) {
                 const u32 bin = (u32)key[i] >> PB_BIN_LOG;
-                buf[bin * PB_CHUNK + (rank[i] - full[i])] =
-                    ((u64)__float_as_uint(x[i]) << 32) | ((u32)key[i] & (PB_BIN - 1));
+                buf[bin * PB_CHUNK + (rank[i] - full[i])] = pb_word(key[i], row0);
             }
         // the next step's ranks read fill (settled before the last barrier);
         // its LDS chunk writes come after its first barrier
@@ -713,188 +752,324 @@ __global__ __launch_bounds__(PBS_TPB) void k_pb_bin_staged(DevState d, u32 part_
     for (u32 b = threadIdx.x; b < NB; b += PBS_TPB) {
         const u32 F = fill[b];
         const u64 pos = gpos[b];
-        if (F && pos + PB_CHUNK <= npairs)
-            for (u32 k = 0; k < PB_CHUNK; ++k) pairs[pos + k] = k < F ? buf[b * PB_CHUNK + k] : 0ull;
+        if (F && pos + PB_CHUNK <= room) {
+            for (u32 k = 0; k < PB_CHUNK; ++k) words[pos + k] = k < F ? buf[b * PB_CHUNK + k] : PB_PAD;
+            rows[pos / PB_CHUNK] = row0;
+        }
     }
 }
 
-// chunks per bin: nch[b] = ceil(pairs of bin b / chunk)
-__global__ void k_pb_nchunks(const u32 *__restrict__ off, u32 P, u32 NB, u32 chunk, u32 *__restrict__ nch) {
-    for (u32 b = blockIdx.x * blockDim.x + threadIdx.x; b < NB; b += gridDim.x * blockDim.x) {
-        const u32 n = off[(u64)(b + 1) * P] - off[(u64)b * P];
-        nch[b] = (n + chunk - 1) / chunk;
+// chunks before each bin (cb[NB]: all): ceil(words of the bin / chunk), at
+// least one, so that every bin has a workgroup to finish its vertices; and
+// before it, the chunks of bins of several (their partial sums): cb[NB + 1 + b]
+__global__ __launch_bounds__(1024) void k_pb_chunks(const u32 *__restrict__ off, u32 P, u32 NB, u32 chunk,
+                                                    u32 *__restrict__ cb) {
+    __shared__ u64 tmp[1024 / 64 + 1];
+    u64 carry = 0;
+    for (u32 b0 = 0; b0 < NB; b0 += 1024) {
+        const u32 b = b0 + threadIdx.x;
+        u64 v = 0;
+        if (b < NB) {
+            const u32 n = max(1u, (off[(u64)(b + 1) * P] - off[(u64)b * P] + chunk - 1) / chunk);
+            v = n | (n > 1 ? (u64)n << 32 : 0ull);
+        }
+        u64 tot;
+        const u64 ex = block_excl_scan<1024, u64>(v, tot, tmp) + carry;
+        if (b < NB) {
+            cb[b] = (u32)ex;
+            cb[NB + 1 + b] = (u32)(ex >> 32);
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) cb[NB] = (u32)carry;
+}
+
+// Sums of contributions are kept in 64-bit fixed point of PR_FIX fractional
+// bits: the ranks of a vector sum to 1 (the recurrence keeps it), so a sum
+// stays below 2^(64 - PR_FIX), the adds are exact and their order does not
+// matter.  An FP32 contribution of 2^-39 or more converts exactly; a smaller
+// one loses less than 2^-62.  LDS adds 64-bit integers natively, where FP32
+// compensated by a compare-and-swap took 428 us an iteration at 6.4e7 edges.
+static constexpr u32 PR_FIX = 62;
+__device__ __forceinline__ u64 pr_fixed(float x) {
+    const u32 bits = __float_as_uint(x), e = bits >> 23;  // x >= 0
+    const u64 m = ((u64)((bits & 0x7FFFFFu) | 0x800000u)) << (PR_FIX - 23);  // mantissa, of value 1 at e = 127
+    return m >> min(127u - min(e, 127u), 63u);  // e = 0 (zero, denormal): shifted out
+}
+__device__ __forceinline__ float pr_float(u64 v) { return (float)((double)v * (1.0 / (double)(1ull << PR_FIX))); }
+
+// the host's word: (iteration, its L1 change)
+__device__ __forceinline__ void pr_report(const PrSlot &s, u32 it, u64 *host) {
+    __hip_atomic_store(host, ((u64)it << 32) | __float_as_uint((float)s.delta), __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static __device__ __forceinline__ double wave_sum_d(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// adds three per-thread sums of the workgroup (PRI_TPB threads at most) to a
+// reduction slot; `lds` holds 3 doubles a wave
+__device__ __forceinline__ void pr_reduce(double dang, double sum, double delta, PrSlot *to, double *lds) {
+    dang = wave_sum_d(dang); sum = wave_sum_d(sum); delta = wave_sum_d(delta);
+    const u32 wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    if (lane_id() == 0) { lds[3 * wv] = dang; lds[3 * wv + 1] = sum; lds[3 * wv + 2] = delta; }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        double t = 0.0;
+        for (u32 w = 0; w < nw; ++w) t += lds[3 * w + threadIdx.x];
+        double *at = threadIdx.x == 0 ? &to->dang : (threadIdx.x == 1 ? &to->sum : &to->delta);
+        if (t != 0.0) unsafeAtomicAdd(at, t);  // native 64-bit float atomic on device memory
     }
 }
 
-// acc[v] += x, compensated: acc[v] packs (hi, lo) as two FP32 halves of one
-// 64-bit LDS word; the new hi is the FP32 sum hi + x and its exact rounding
-// error (TwoSum) goes to lo, both installed by one compare-and-swap.  FP32
-// add atomics on LDS run about 20x slower than integer ones here (0.33 vs
-// 6.5 lanes per clock per CU measured on MI355X), the CAS form at 1.4
-// (uniform addresses) to 0.25 (R-MAT-skewed) and keeps FP32 arithmetic.
-__device__ __forceinline__ u64 add2(u64 cur, float x) {
-    const float hi = __uint_as_float((u32)cur), lo = __uint_as_float((u32)(cur >> 32));
-    const float s = hi + x;
-    const float bp = s - hi;
-    const float e = (hi - (s - bp)) + (x - bp);
-    return ((u64)__float_as_uint(lo + e) << 32) | __float_as_uint(s);
-}
-
-// retry from a failed compare: cur is the word's value the CAS returned
-__device__ __forceinline__ void lds_add2_retry(u64 *acc, u32 v, float x, u64 cur) {
-    while (true) {
-        const u64 prev = atomicCAS((unsigned long long *)&acc[v], (unsigned long long)cur,
-                                   (unsigned long long)add2(cur, x));
-        if (prev == cur) break;
-        cur = prev;
+// start vector 1/V, out-degrees (from marker ranks), contributions, dangling
+// mass
+__global__ __launch_bounds__(PR_TPB) void k_pr_start(DevState d, const u32 *__restrict__ gpre,
+                                                     u32 *__restrict__ outdeg, float *__restrict__ pr,
+                                                     float *__restrict__ c0, float *__restrict__ c1, PrSlot *slot) {
+    __shared__ double lds[3 * PR_TPB / 64];
+    const u32 V = d.V, Smask = (1u << d.log2S) - 1;
+    const float p = 1.f / (float)V;
+    double dang = 0.0;
+    for (u64 r = (u64)blockIdx.x * blockDim.x + threadIdx.x; r < V; r += (u64)gridDim.x * blockDim.x) {
+        const u64 hs = d.row_off[r + 1];
+        const u64 ls = r > 0 ? d.row_off[r] : 0u;
+        const u64 hi = (u64)gpre[hs >> d.log2S] + (hs & Smask);
+        const u64 lo = r > 0 ? (u64)gpre[ls >> d.log2S] + (ls & Smask) + 1 : 0ull;
+        const u32 od = (u32)(hi - lo);
+        outdeg[r] = od;
+        pr[r] = p;
+        c0[r] = od ? p / (float)od : 0.f;
+        if (!od) dang += p;
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c0[V] = c1[V] = 0.f;  // the padding words' source
+        slot->sum = 1.0;
+    }
+    pr_reduce(dang, 0.0, 0.0, slot, lds);
 }
 
-// chunk k of bin b (cb = exclusive scan of nch, cb[NB] = chunks) summed in
-// LDS into partial[k * PB_BIN + v] = (hi, lo)
-__global__ __launch_bounds__(PBA_TPB) void k_pb_acc(const u64 *__restrict__ pairs, const u32 *__restrict__ off, u32 P,
-                                                   u32 NB, const u32 *__restrict__ cb, u32 chunk,
-                                                   float2 *__restrict__ partial) {
-    extern __shared__ u64 pb_acc[];  // PB_BIN words: (lo << 32) | hi
+// Iteration `it` (from 1) is two kernels.  It reads the masses of iteration
+// it - 1 from its slot and leaves its own in slot it (the ring's next slot is
+// cleared).  Once an iteration's L1 change is below tol, the ones queued
+// behind it return at once, which lets the host queue an iteration ahead; the
+// first kernel reports the change of the one before it to the host's word.
+
+// Waits for the LDS adds of f at e with both still in their registers.  A
+// 64-bit LDS add without a result has been seen here to pick up its operand
+// after a later instruction had overwritten the register, when many lanes add
+// to one word and the LDS falls behind (half-converted contributions then
+// ended up in the sums): the operands stay untouched until the adds are done.
+template <u32 N>
+__device__ __forceinline__ void lds_adds_done(const u64 (&f)[N], const u32 (&e)[N]) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (u32 r = 0; r < N; ++r) asm volatile("" ::"v"(f[r]), "v"(e[r]));
+}
+
+// a vertex's new rank pr' = alpha * sum + gamma, gamma = (alpha * dangling +
+// (1 - alpha) * sum(pr)) / n, and what the next iteration needs of it
+struct PrMass {
+    double dang, sum, delta;
+};
+__device__ __forceinline__ void pr_vertex(u32 v, u64 acc, float alpha, float gamma, const float *pr, float *out,
+                                          const u32 *outdeg, float *cnext, PrMass &m) {
+    const float p = alpha * pr_float(acc) + gamma;
+    const u32 od = outdeg[v];
+    m.delta += (double)fabsf(p - pr[v]);
+    m.sum += (double)p;
+    if (!od) m.dang += (double)p;
+    out[v] = p;
+    cnext[v] = od ? p / (float)od : 0.f;
+}
+__device__ __forceinline__ float pr_gamma(const PrSlot &prev, float alpha, u32 V) {
+    return (alpha * (float)prev.dang + (1.f - alpha) * (float)prev.sum) / (float)V;
+}
+
+// Chunk k of a bin's edges (cb = chunks before each bin).  A bin of one chunk
+// is finished here; the chunks of a larger one leave their sums in partial,
+// for k_pr_join.  (Joining them by 64-bit atomics on a vector in HBM instead
+// took 850 us an iteration, against 25 us.)
+// Bound: the random reads of the contributions through L2 (one per edge whose
+// line no other lane asks for), then the edge stream (4.5 B an edge).  6.4e7
+// edges on 2^22 vertices: 195 us an iteration and 30 us for the joins, against
+// 1340 us when every iteration binned contributions and summed them by LDS
+// compare-and-swap; with 8-byte edges 235 us.  The LDS adds are hidden: without
+// them the kernel takes the same time.
+__global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ words,
+                                                     const u32 *__restrict__ rows, const u32 *__restrict__ off, u32 P,
+                                                     u32 NB, const u32 *__restrict__ cb, u32 chunk,
+                                                     const float *__restrict__ c, float *__restrict__ cnext,
+                                                     const float *__restrict__ pr, float *__restrict__ out,
+                                                     const u32 *__restrict__ outdeg, u32 V, float alpha, float tol,
+                                                     u32 it, PrSlot *slots, u64 *__restrict__ partial,
+                                                     u64 *__restrict__ host) {
+    extern __shared__ u64 pb_acc[];  // PB_BIN sums
+    __shared__ double red[3 * PRI_TPB / 64];
+    const PrSlot &prev = slots[(it - 1) % PR_SLOTS];
+    if (blockIdx.x == 0 && threadIdx.x == 0 && it > 1) pr_report(prev, it - 1, host);
+    if (it > 1 && (float)prev.delta < tol) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) slots[(it + 1) % PR_SLOTS] = PrSlot{0.0, 0.0, 0.0};
     const u32 k = blockIdx.x;
     if (k >= cb[NB]) return;  // the grid is an upper bound
-    u32 a = 0, z = NB;        // last b with cb[b] <= k
-    while (z - a > 1) {
-        const u32 m = (a + z) >> 1;
-        if (cb[m] <= k) a = m; else z = m;
+    u32 b = 0, z = NB;        // last b with cb[b] <= k
+    while (z - b > 1) {
+        const u32 m = (b + z) >> 1;
+        if (cb[m] <= k) b = m; else z = m;
     }
-    const u32 b = a;
+    const u32 nch = cb[b + 1] - cb[b];
     const u64 e1 = off[(u64)(b + 1) * P];
     const u64 s0 = (u64)off[(u64)b * P] + (u64)(k - cb[b]) * chunk;
     const u64 s1 = min(e1, s0 + chunk);
-    for (u32 v = threadIdx.x; v < PB_BIN; v += PBA_TPB) pb_acc[v] = 0ull;
+    const u32 v0 = b << PB_BIN_LOG, nv = min(PB_BIN, V - v0);
+    for (u32 v = threadIdx.x; v < PB_BIN; v += PRI_TPB) pb_acc[v] = 0ull;
     __syncthreads();
-    for (u64 i0 = s0; i0 < s1; i0 += (u64)PBA_TPB * PB_ITEMS) {
-        u64 pr[PB_ITEMS];
+    for (u64 i0 = s0; i0 < s1; i0 += (u64)PRI_TPB * PRI_ITEMS) {
+        u32 e[PRI_ITEMS], row0[PRI_ITEMS];
 #pragma unroll
-        for (u32 r = 0; r < PB_ITEMS; ++r) {
-            const u64 i = i0 + (u64)r * PBA_TPB + threadIdx.x;
-            pr[r] = pairs[i < s1 ? i : s1 - 1];  // s1 > s0: a chunk is never empty
-            if (i >= s1) pr[r] = 0ull;           // x = +0 adds nothing
+        for (u32 r = 0; r < PRI_ITEMS; ++r) {
+            const u64 i = i0 + (u64)r * PRI_TPB + threadIdx.x;
+            const u64 j = i < s1 ? i : s1 - 1;  // unconditional loads: all of them in flight together
+            e[r] = words[j];
+            row0[r] = rows[j / PB_CHUNK];
+            if (i >= s1) e[r] = PB_PAD;
         }
-        // all reads, then all first compare-and-swaps, then the retries of
-        // the lanes that lost a race: two LDS round trips per step when
-        // nothing collides
-        u64 cur[PB_ITEMS];
+        float x[PRI_ITEMS];
 #pragma unroll
-        for (u32 r = 0; r < PB_ITEMS; ++r) cur[r] = pb_acc[(u32)pr[r] & (PB_BIN - 1)];
-        u64 got[PB_ITEMS];
+        for (u32 r = 0; r < PRI_ITEMS; ++r) x[r] = c[e[r] == PB_PAD ? V : row0[r] + (e[r] >> PB_BIN_LOG)];
+        u64 f[PRI_ITEMS];
 #pragma unroll
-        for (u32 r = 0; r < PB_ITEMS; ++r) {
-            const float x = __uint_as_float((u32)(pr[r] >> 32));
-            got[r] = cur[r];
-            if (x != 0.f)
-                got[r] = atomicCAS((unsigned long long *)&pb_acc[(u32)pr[r] & (PB_BIN - 1)],
-                                   (unsigned long long)cur[r], (unsigned long long)add2(cur[r], x));
-        }
+        for (u32 r = 0; r < PRI_ITEMS; ++r) f[r] = pr_fixed(x[r]);
 #pragma unroll
-        for (u32 r = 0; r < PB_ITEMS; ++r)
-            if (got[r] != cur[r])
-                lds_add2_retry(pb_acc, (u32)pr[r] & (PB_BIN - 1), __uint_as_float((u32)(pr[r] >> 32)), got[r]);
+        for (u32 r = 0; r < PRI_ITEMS; ++r)
+            atomicAdd((unsigned long long *)&pb_acc[e[r] & (PB_BIN - 1)], (unsigned long long)f[r]);
+        lds_adds_done(f, e);
     }
     __syncthreads();
-    float2 *out = partial + (u64)k * PB_BIN;
-    for (u32 v = threadIdx.x; v < PB_BIN; v += PBA_TPB) {
-        const u64 w = pb_acc[v];
-        out[v] = make_float2(__uint_as_float((u32)w), __uint_as_float((u32)(w >> 32)));
+    if (nch > 1) {
+        u64 *to = partial + (u64)(cb[NB + 1 + b] + (k - cb[b])) * PB_BIN;
+        for (u32 v = threadIdx.x; v < nv; v += PRI_TPB) to[v] = pb_acc[v];
+        return;
     }
+    const float gamma = pr_gamma(prev, alpha, V);
+    PrMass m{0.0, 0.0, 0.0};
+    for (u32 v = threadIdx.x; v < nv; v += PRI_TPB)
+        pr_vertex(v0 + v, pb_acc[v], alpha, gamma, pr, out, outdeg, cnext, m);
+    pr_reduce(m.dang, m.sum, m.delta, &slots[it % PR_SLOTS], red);
 }
 
-// as k_pr_finish, with vertex v's sum taken from its bin's chunk partials
-__global__ __launch_bounds__(PR_TPB) void k_pb_finish(const float2 *__restrict__ partial, const u32 *__restrict__ cb,
-                            const float *__restrict__ pr, float *__restrict__ out, u32 V, float alpha,
-                            const float *__restrict__ red_in, float *__restrict__ red_out) {
-    const float dang = red_in[0] + red_in[1];
-    const float sum_in = red_in[2] + red_in[3];
-    const float gamma = (alpha * dang + (1.f - alpha) * sum_in) / (float)V;
-    float dl = 0.f, sum = 0.f;
-    for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (u64)gridDim.x * blockDim.x) {
-        const u32 b = (u32)(v >> PB_BIN_LOG);
-        const u32 k0 = cb[b], k1 = cb[b + 1];
-        float a = 0.f, comp = 0.f;
-        for (u32 k = k0; k < k1; ++k) {
-            const float2 h = partial[(u64)k * PB_BIN + (v & (PB_BIN - 1))];
-            float y = h.y - comp;  // lo first: the small term
-            float t = a + y;
-            comp = (t - a) - y;
-            a = t;
-            y = h.x - comp;
-            t = a + y;
-            comp = (t - a) - y;
-            a = t;
+// the bins of several chunks: PB_BIN / PRI_TPB workgroups a bin, a thread a
+// vertex, the chunks' sums read PRI_ITEMS at a time
+__global__ __launch_bounds__(PRI_TPB) void k_pr_join(u32 NB, const u32 *__restrict__ cb, const u64 *__restrict__ partial,
+                                                     float *__restrict__ cnext, const float *__restrict__ pr,
+                                                     float *__restrict__ out, const u32 *__restrict__ outdeg, u32 V,
+                                                     float alpha, float tol, u32 it, PrSlot *slots) {
+    __shared__ double red[3 * PRI_TPB / 64];
+    constexpr u32 WPB = PB_BIN / PRI_TPB;
+    const PrSlot &prev = slots[(it - 1) % PR_SLOTS];
+    if (it > 1 && (float)prev.delta < tol) return;
+    const u32 b = blockIdx.x / WPB;
+    const u32 k0 = cb[NB + 1 + b], k1 = k0 + (cb[b + 1] - cb[b]);
+    if (k1 - k0 == 1) return;
+    const u32 w = (blockIdx.x % WPB) * PRI_TPB + threadIdx.x;  // vertex within the bin
+    const u32 v = (b << PB_BIN_LOG) + w;
+    PrMass m{0.0, 0.0, 0.0};
+    if (v < V) {
+        u64 acc = 0;
+        u32 k = k0;
+        for (; k + PRI_ITEMS <= k1; k += PRI_ITEMS) {
+            u64 t[PRI_ITEMS];
+#pragma unroll
+            for (u32 r = 0; r < PRI_ITEMS; ++r) t[r] = partial[(u64)(k + r) * PB_BIN + w];
+#pragma unroll
+            for (u32 r = 0; r < PRI_ITEMS; ++r) acc += t[r];
         }
-        float p = alpha * a + gamma;
-        out[v] = p;
-        dl += fabsf(p - pr[v]);
-        sum += p;
+        for (; k < k1; ++k) acc += partial[(u64)k * PB_BIN + w];
+        pr_vertex(v, acc, alpha, pr_gamma(prev, alpha, V), pr, out, outdeg, cnext, m);
     }
-    __shared__ float tmp[PR_TPB / 64];
-    dl = block_sum(dl, tmp);
-    sum = block_sum(sum, tmp);
-    if (threadIdx.x == 0) {
-        atomic_add2(&red_out[4], &red_out[5], dl);
-        atomic_add2(&red_out[2], &red_out[3], sum);
-    }
+    pr_reduce(m.dang, m.sum, m.delta, &slots[it % PR_SLOTS], red);
+}
+
+// rank = p / sum(p) of iteration `it`, and its report to the host
+__global__ void k_pr_norm(const float *pr, float *rank, u32 V, const PrSlot *slot, u32 it, u64 *host) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) pr_report(*slot, it, host);
+    const float inv = 1.f / (float)slot->sum;
+    for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (u64)gridDim.x * blockDim.x)
+        rank[v] = pr[v] * inv;
 }
 
 bool pr_bins_fit(u32 V) { return ((u64)V + PB_BIN - 1) / PB_BIN <= PB_MAX_BINS; }
 
-PrBins pr_bins_plan(const DevState &d) {
+PrBins pr_bins_plan(const DevState &d, u64 edges) {
     PrBins b{};
     const u64 W = nseg_of(d) << d.log2S;
     u32 lw = 0;
     while ((1ull << lw) < W) ++lw;
-    b.part_log = std::max<u32>(d.log2S, lw > 10 ? lw - 10 : 0);  // at most PB_MAX_PARTS parts
+    // about 1024 parts, of at least one step of the bin pass
+    b.part_log = std::max<u32>(std::max<u32>(d.log2S, 12), lw > 10 ? lw - 10 : 0);
+    b.part_log = std::min(b.part_log, PB_MAX_PART_LOG);
     b.parts = (u32)((W + (1ull << b.part_log) - 1) >> b.part_log);
     b.bins = (u32)(((u64)d.V + PB_BIN - 1) / PB_BIN);
     b.staged = b.bins <= PB_STAGE_MAX_BINS;
+    // every run that holds an edge is padded to whole groups
+    b.words = std::min<u64>(edges * PB_CHUNK, edges + (u64)(PB_CHUNK - 1) * b.bins * b.parts);
+    // about two rounds of chunks over the workgroups the device holds (two a
+    // CU): more chunks have more sums to join, fewer leave a tail
+    b.chunk = (u32)((std::max<u64>(8192, edges / 1024) + 1023) / 1024 * 1024);
+    b.max_multi = (u32)(2 * (b.words / b.chunk));  // chunks of bins of several
+    b.max_chunks = (u32)(b.words / b.chunk) + b.bins;
     return b;
 }
 
 u64 pr_bins_count_words(const PrBins &b) { return (u64)b.bins * b.parts + 1; }
+// the groups' rows follow the words
+static u64 pr_bins_rows_at(const PrBins &b) { return (b.words + PB_CHUNK - 1) / PB_CHUNK * PB_CHUNK; }
+u64 pr_bins_edge_words(const PrBins &b) { return pr_bins_rows_at(b) / PB_CHUNK * (PB_CHUNK + 1) + PB_CHUNK; }
 
-hipError_t pr_bins_count(const DevState &d, const PrBins &b, u32 *off, u32 *scan_scratch, hipStream_t st) {
+hipError_t pr_bins_edges(const DevState &d, const PrBins &b, u32 *off, u32 *cb, u32 *words, u32 *scan_scratch,
+                         PrSlot *slots, hipStream_t st) {
     if (b.parts > PB_MAX_PARTS || b.bins > PB_MAX_BINS || b.bins == 0) return hipErrorInvalidValue;
-    k_pb_count<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins,
-                                                             b.staged ? PB_CHUNK - 1 : 0u, off);
-    return device_excl_scan(off, (u64)b.bins * b.parts, off, scan_scratch, st);
-}
-
-void pr_bins_chunking(PrBins &b, u64 pairs) {
-    b.pairs = pairs;
-    b.chunk = (u32)std::max<u64>(4096, (pairs + 2047) / 2048);
-    b.max_chunks = (u32)((pairs + b.chunk - 1) / b.chunk) + b.bins;
-}
-
-u64 pr_bins_partial_floats(const PrBins &b) { return 2ull * PB_BIN * b.max_chunks; }
-
-hipError_t pr_bins_chunks(const PrBins &b, const u32 *off, u32 *cb, u32 *scan_scratch, hipStream_t st) {
-    k_pb_nchunks<<<grid_for(b.bins, 256, 1024), 256, 0, st>>>(off, b.parts, b.bins, b.chunk, cb);
-    return device_excl_scan(cb, b.bins, cb, scan_scratch, st);
-}
-
-hipError_t pr_iterate_binned(const DevState &d, const PrBins &b, const float *pr, const u32 *outdeg, float *c,
-                             const u32 *off, const u32 *cb, u64 *pairs, float *partial, float *out, float alpha,
-                             float *red, float *red_next, hipStream_t st) {
-    const u32 V = d.V;
-    k_pr_reset<<<1, 64, 0, st>>>(red_next);
-    k_pr_prep<<<grid_for(V, PR_TPB, PR_GRID), PR_TPB, 0, st>>>(pr, outdeg, V, c, nullptr, 0, red);
+    k_pb_count<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, slots);
+    hipError_t e = device_excl_scan(off, (u64)b.bins * b.parts, off, scan_scratch, st);
+    if (e != hipSuccess) return e;
+    k_pb_chunks<<<1, 1024, 0, st>>>(off, b.parts, b.bins, b.chunk, cb);
+    u32 *rows = words + pr_bins_rows_at(b);
     if (b.staged)
-        k_pb_bin_staged<<<b.parts, PBS_TPB, b.bins * (PB_CHUNK * sizeof(u64) + 2 * sizeof(u32)), st>>>(
-            d, b.part_log, b.parts, b.bins, off, c, pairs, b.pairs);
+        k_pb_bin_staged<<<b.parts, PBS_TPB, b.bins * (PB_CHUNK + 2) * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins,
+                                                                                        off, words, rows, b.words);
     else
-        k_pb_bin<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, c, pairs,
-                                                                b.pairs);
-    if (b.max_chunks)
-        k_pb_acc<<<b.max_chunks, PBA_TPB, PB_BIN * sizeof(u64), st>>>(pairs, off, b.parts, b.bins, cb, b.chunk,
-                                                                          (float2 *)partial);
-    k_pb_finish<<<grid_for(V, PR_TPB, PR_GRID), PR_TPB, 0, st>>>((const float2 *)partial, cb, pr, out, V, alpha, red,
-                                                         red_next);
+        k_pb_bin<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, words, rows,
+                                                                b.words);
+    return hipGetLastError();
+}
+
+hipError_t pr_bins_start(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *outdeg, float *pr, float *c0, float *c1,
+                         PrSlot *slots, hipStream_t st) {
+    hipError_t e = device_excl_scan(d.cnt, nseg_of(d), gpre, scan_scratch, st);
+    if (e != hipSuccess) return e;
+    k_pr_start<<<grid_for(d.V, PR_TPB, PR_GRID), PR_TPB, 0, st>>>(d, gpre, outdeg, pr, c0, c1, slots);
+    return hipGetLastError();
+}
+
+u64 pr_bins_partial_words(const PrBins &b) { return std::max<u64>(1, (u64)b.max_multi * PB_BIN); }
+
+hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
+                           const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
+                           float tol, u32 it, PrSlot *slots, u64 *partial, u64 *host, hipStream_t st) {
+    k_pr_iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(u64), st>>>(
+        words, words + pr_bins_rows_at(b), off, b.parts, b.bins, cb, b.chunk, c, cnext, pr, out, outdeg, d.V, alpha, tol, it,
+        slots, partial, host);
+    if (b.max_multi)
+        k_pr_join<<<b.bins * (PB_BIN / PRI_TPB), PRI_TPB, 0, st>>>(b.bins, cb, partial, cnext, pr, out, outdeg, d.V,
+                                                                   alpha, tol, it, slots);
+    return hipGetLastError();
+}
+
+hipError_t pr_bins_norm(const float *pr, float *rank, u32 V, u32 it, const PrSlot *slots, u64 *host, hipStream_t st) {
+    k_pr_norm<<<grid_for(V, 256, 16384), 256, 0, st>>>(pr, rank, V, &slots[it % PR_SLOTS], it, host);
     return hipGetLastError();
 }
 

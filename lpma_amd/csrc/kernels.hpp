@@ -126,25 +126,39 @@ u32 pr_red_floats();
 hipError_t pr_iterate(const DevState &d, const float *pr, const u32 *outdeg, float *c, float *acc, float *out,
                       float alpha, float *red, float *red_next, hipStream_t st);
 hipError_t pr_scale(float *pr, u32 V, const float *red, hipStream_t st);
-// binned push: geometry of one PageRank call
+// binned edges: geometry of one PageRank call
 struct PrBins {
     u32 part_log;    // slots per part (log2)
     u32 parts;       // parts of the slot array (<= 1024)
     u32 bins;        // destination bins of 8192 vertices
-    u32 chunk;       // pairs per accumulation chunk
-    u32 max_chunks;  // bound on the chunks of all bins (the acc grid)
-    u32 staged;      // bin pass stages whole 32-byte chunks in LDS (runs padded)
-    u64 pairs;       // live edges
+    u32 chunk;       // edge words per chunk of an iteration
+    u32 max_chunks;  // bound on the chunks of all bins (the iteration's grid)
+    u32 max_multi;   // bound on the chunks of bins of several chunks
+    u32 staged;      // bin pass stages whole 32-byte chunks in LDS
+    u64 words;       // room for the edge words, padding included
 };
+// masses of one iteration, in a ring of PR_SLOTS
+struct PrSlot {
+    double dang, sum, delta;
+};
+static constexpr u32 PR_SLOTS = 4;
 bool pr_bins_fit(u32 V);
-PrBins pr_bins_plan(const DevState &d);
+PrBins pr_bins_plan(const DevState &d, u64 edges);
 u64 pr_bins_count_words(const PrBins &b);
-hipError_t pr_bins_count(const DevState &d, const PrBins &b, u32 *off, u32 *scan_scratch, hipStream_t st);
-void pr_bins_chunking(PrBins &b, u64 pairs);
-u64 pr_bins_partial_floats(const PrBins &b);
-hipError_t pr_bins_chunks(const PrBins &b, const u32 *off, u32 *cb, u32 *scan_scratch, hipStream_t st);
-hipError_t pr_iterate_binned(const DevState &d, const PrBins &b, const float *pr, const u32 *outdeg, float *c,
-                             const u32 *off, const u32 *cb, u64 *pairs, float *partial, float *out, float alpha,
-                             float *red, float *red_next, hipStream_t st);
+u64 pr_bins_edge_words(const PrBins &b);
+// bins the edges (off: pr_bins_count_words, cb: 2 bins + 1, words: pr_bins_edge_words)
+hipError_t pr_bins_edges(const DevState &d, const PrBins &b, u32 *off, u32 *cb, u32 *words, u32 *scan_scratch,
+                         PrSlot *slots, hipStream_t st);
+// after pr_bins_edges: start vector and contributions (c0, c1: V + 1)
+hipError_t pr_bins_start(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *outdeg, float *pr, float *c0, float *c1,
+                         PrSlot *slots, hipStream_t st);
+// iteration `it` = 1, 2, ...; does nothing once an earlier L1 change is below
+// tol.  (it - 1) << 32 | its L1 change reaches `host`; pr_bins_norm reports the
+// last one's.
+u64 pr_bins_partial_words(const PrBins &b);
+hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
+                           const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
+                           float tol, u32 it, PrSlot *slots, u64 *partial, u64 *host, hipStream_t st);
+hipError_t pr_bins_norm(const float *pr, float *rank, u32 V, u32 it, const PrSlot *slots, u64 *host, hipStream_t st);
 
 }  // namespace pma

@@ -241,9 +241,10 @@ struct lpma {
 
     Pipeline pl;  // plain updates, views and analytics scratch
     // analytics scratch
-    DBuf<u32> aq0, apoff, apcb;
-    DBuf<float> af0, af1, af2, ared, apart;
-    DBuf<u64> apairs;
+    DBuf<u32> aq0, apoff, apcb, apwords;
+    DBuf<float> af0, af1, af2, ared;
+    DBuf<u64> apart, aslots;
+    u64 *h_word = nullptr;  // pinned: a word kernels report to
     u32 *d_err = nullptr;
 
     // host counters
@@ -634,6 +635,26 @@ int spread_and_install(lpma *h, u32 H, Geometry &g, const u64 *merged, u64 m, hi
         return LPMA_ERR_DEVICE;
     }
     return pyramid_and_install(h, H, g, st);
+}
+
+// Waits until a kernel queued on st has stored a word for which done(word)
+// holds (a pinned word, system-scope store): the host sees it a few
+// microseconds before a stream or event wait would return.  The stream is
+// asked now and then, so a failed or finished one ends the wait.
+template <class Done>
+int wait_word(const u64 *word, hipStream_t st, u64 &out, Done done) {
+    for (u64 spin = 0;; ++spin) {
+        out = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (done(out)) return LPMA_OK;
+        if ((spin & 0xFFFF) == 0xFFFF) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            (void)hipGetLastError();
+            out = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+            return e == hipSuccess && done(out) ? LPMA_OK : LPMA_ERR_DEVICE;
+        }
+        __builtin_ia32_pause();
+    }
 }
 
 // One PMA's share of a pipeline run.
@@ -1430,8 +1451,9 @@ int lpma_destroy(lpma_t *h) {
     release(h, h->keys); release(h, h->cnt); release(h, h->pyr); release(h, h->owner);
     release(h, h->row_off); release(h, h->sep);
     release(h, h->aq0); release(h, h->apoff); release(h, h->apcb);
-    release(h, h->af0); release(h, h->af1); release(h, h->af2); release(h, h->ared); release(h, h->apart);
-    release(h, h->apairs);
+    release(h, h->af0); release(h, h->af1); release(h, h->af2); release(h, h->ared);
+    release(h, h->apwords); release(h, h->apart); release(h, h->aslots);
+    if (h->h_word) (void)hipHostFree(h->h_word);
     if (h->d_err) (void)hipFree(h->d_err);
     delete h;
     return LPMA_OK;
@@ -1752,6 +1774,56 @@ int lpma_snapshot_set_search_width(lpma_snapshot_t *s, uint32_t workgroups) {
     return LPMA_OK;
 }
 
+// PageRank over edges binned by destination (V within pr_bins_fit).
+static int pagerank_binned(lpma *h, float damping, float tolerance, u32 max_iter, float *d_rank, u32 &it, float &delta,
+                           hipStream_t st) {
+    const u64 V = h->V, nseg = 1ull << h->st.H;
+    const PrBins bins = pr_bins_plan(h->st, h->live - V);
+    const u64 nc = pr_bins_count_words(bins);
+    CHECKED(ensure(h, h->apoff, nc));
+    CHECKED(ensure(h->pl, h->pl.scan_scr, scan_scratch_words(std::max(nc, nseg)) + 8));
+    CHECKED(ensure(h, h->apcb, 2 * (u64)bins.bins + 1));
+    CHECKED(ensure(h, h->apwords, pr_bins_edge_words(bins)));
+    CHECKED(ensure(h, h->apart, pr_bins_partial_words(bins)));
+    CHECKED(ensure(h, h->af1, V + 1));  // with af0: contributions, and the padding's
+    CHECKED(ensure(h, h->aslots, (PR_SLOTS * sizeof(PrSlot) + 7) / 8));
+    if (!h->h_word) {
+        if (injected_failure()) return LPMA_ERR_OUT_OF_MEMORY;
+        if (hipHostMalloc((void **)&h->h_word, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+            (void)hipGetLastError();
+            h->h_word = nullptr;
+            return LPMA_ERR_OUT_OF_MEMORY;
+        }
+    }
+    __atomic_store_n(h->h_word, 0ull, __ATOMIC_RELEASE);
+    PrSlot *slots = (PrSlot *)h->aslots.p;
+    float *vec[2] = {d_rank, h->af2.p}, *c[2] = {h->af0.p, h->af1.p};
+    HIPCHECK(pr_bins_edges(h->st, bins, h->apoff.p, h->apcb.p, h->apwords.p, h->pl.scan_scr.p, slots, st));
+    HIPCHECK(pr_bins_start(h->st, h->pl.gpre.p, h->pl.scan_scr.p, h->aq0.p, vec[0], c[0], c[1], slots, st));
+    // an iteration reports the L1 change of the one before it, so one more is
+    // always queued (it returns at once when it was not wanted)
+    auto queue = [&](u32 i) {
+        const int a = (i - 1) & 1;
+        return pr_bins_iterate(h->st, bins, h->apwords.p, h->apoff.p, h->apcb.p, c[a], c[a ^ 1], vec[a], vec[a ^ 1],
+                               h->aq0.p, damping, tolerance, i, slots, h->apart.p, h->h_word, st);
+    };
+    u64 w = 0;
+    HIPCHECK(queue(1));
+    for (it = 1; it < max_iter; ++it) {
+        HIPCHECK(queue(it + 1));
+        const u32 want = it;
+        CHECKED(wait_word(h->h_word, st, w, [want](u64 x) { return (u32)(x >> 32) == want; }));
+        const u32 bits = (u32)w;
+        memcpy(&delta, &bits, sizeof(delta));
+        if (delta < tolerance) break;
+    }
+    HIPCHECK(pr_bins_norm(vec[it & 1], d_rank, h->V, it, slots, h->h_word, st));
+    HIPCHECK(hipStreamSynchronize(st));
+    const u32 bits = (u32)__atomic_load_n(h->h_word, __ATOMIC_ACQUIRE);
+    memcpy(&delta, &bits, sizeof(delta));
+    return LPMA_OK;
+}
+
 int lpma_pagerank(lpma_t *h, float damping, float tolerance, uint32_t max_iter, float *d_rank, uint32_t *iterations,
                   float *last_delta, void *stream) {
     if (!h || !d_rank || !(damping >= 0.f && damping <= 1.f) || max_iter == 0) return LPMA_ERR_INVALID_ARGUMENT;
@@ -1763,45 +1835,29 @@ int lpma_pagerank(lpma_t *h, float damping, float tolerance, uint32_t max_iter, 
     h->pl.cur_stream = st;
     CHECKED(ensure(h->pl, h->pl.gpre, nseg + 1));
     CHECKED(ensure(h->pl, h->pl.scan_scr, scan_scratch_words(nseg) + 8));
-    CHECKED(ensure(h, h->aq0, V));   // out-degrees
-    CHECKED(ensure(h, h->af0, V));   // contributions
-    CHECKED(ensure(h, h->af2, V));   // second rank vector
-    CHECKED(ensure(h, h->ared, 2 * pr_red_floats()));
-    HIPCHECK(pr_outdeg(h->st, h->pl.gpre.p, h->pl.scan_scr.p, h->aq0.p, st));
-    // Binned push where the destination bins fit the bin pass's LDS, else
-    // the atomic push into per-XCD accumulators.
-    const bool binned = pr_bins_fit(h->st.V);
-    PrBins bins{};
-    if (binned) {
-        bins = pr_bins_plan(h->st);
-        const u64 nc = pr_bins_count_words(bins);
-        CHECKED(ensure(h, h->apoff, nc));
-        CHECKED(ensure(h->pl, h->pl.scan_scr, scan_scratch_words(nc) + 8));
-        HIPCHECK(pr_bins_count(h->st, bins, h->apoff.p, h->pl.scan_scr.p, st));
-        u32 total = 0;
-        HIPCHECK(hipMemcpyAsync(&total, h->apoff.p + (nc - 1), sizeof(u32), hipMemcpyDeviceToHost, st));
-        HIPCHECK(hipStreamSynchronize(st));
-        pr_bins_chunking(bins, total);
-        CHECKED(ensure(h, h->apcb, (u64)bins.bins + 1));
-        CHECKED(ensure(h, h->apairs, std::max<u64>(1, total)));
-        CHECKED(ensure(h, h->apart, pr_bins_partial_floats(bins)));
-        HIPCHECK(pr_bins_chunks(bins, h->apoff.p, h->apcb.p, h->pl.scan_scr.p, st));
-    } else {
-        CHECKED(ensure(h, h->af1, pr_acc_floats(h->V)));  // compensated accumulators
+    CHECKED(ensure(h, h->aq0, V));      // out-degrees
+    CHECKED(ensure(h, h->af0, V + 1));  // contributions
+    CHECKED(ensure(h, h->af2, V));      // second rank vector
+    u32 it = 0;
+    float delta = 0.f;
+    // binned edges where the destination bins fit the bin pass's LDS, else
+    // the atomic push into per-XCD accumulators
+    if (pr_bins_fit(h->st.V)) {
+        CHECKED(pagerank_binned(h, damping, tolerance, max_iter, d_rank, it, delta, st));
+        if (iterations) *iterations = it;
+        if (last_delta) *last_delta = delta;
+        return LPMA_OK;
     }
+    CHECKED(ensure(h, h->ared, 2 * pr_red_floats()));
+    CHECKED(ensure(h, h->af1, pr_acc_floats(h->V)));  // compensated accumulators
+    HIPCHECK(pr_outdeg(h->st, h->pl.gpre.p, h->pl.scan_scr.p, h->aq0.p, st));
     float *red[2] = {h->ared.p, h->ared.p + pr_red_floats()};
     float *vec[2] = {d_rank, h->af2.p};
     HIPCHECK(pr_init(vec[0], h->V, red[0], st));
-    u32 it = 0;
-    float delta = 0.f;
     int cur = 0;
     while (it < max_iter) {
-        if (binned)
-            HIPCHECK(pr_iterate_binned(h->st, bins, vec[cur], h->aq0.p, h->af0.p, h->apoff.p, h->apcb.p, h->apairs.p,
-                                       h->apart.p, vec[cur ^ 1], damping, red[cur], red[cur ^ 1], st));
-        else
-            HIPCHECK(pr_iterate(h->st, vec[cur], h->aq0.p, h->af0.p, h->af1.p, vec[cur ^ 1], damping, red[cur],
-                                red[cur ^ 1], st));
+        HIPCHECK(pr_iterate(h->st, vec[cur], h->aq0.p, h->af0.p, h->af1.p, vec[cur ^ 1], damping, red[cur],
+                            red[cur ^ 1], st));
         cur ^= 1;
         ++it;
         float r[8];

@@ -200,3 +200,27 @@ def test_tiny_and_empty_graphs(V):
         exp, _ = oracle.pagerank(ref, V, 0.85, iters)
         assert np.abs(got - exp).sum() < 1e-6, (got, exp)
     pma.close()
+
+
+@pytest.mark.parametrize("V,E", [(128, 2400), (8192, 60000), (8193, 60000), (30000, 2500000), (3000, 1200000)])
+def test_pagerank_bins_and_chunks(V, E):
+    """One bin and one vertex more, bins of one chunk of edges and of several,
+    parts of one and of many steps, padded groups in every run, most edges
+    into a few vertices; fixed iteration counts, the last one reported."""
+    say(f"pagerank bins V={V} E={E}")
+    from gpu_util import keys_of
+    rng = np.random.default_rng(V)
+    src = rng.integers(0, V, E)
+    dst = np.where(rng.random(E) < 0.5, rng.integers(0, V, E), rng.integers(0, min(V, 40), E))
+    keys = oracle.sort_unique(keys_of(src, dst))
+    pma = L.PMA(V)
+    pma.insert(keys)
+    for iters in (1, 2, 7):
+        pr, it, delta = pma.pagerank(0.85, 0.0, iters)
+        assert it == iters
+        got = pr.cpu().numpy().astype(np.float64)
+        want, _ = oracle.pagerank(keys, V, 0.85, iters)
+        assert np.abs(got - want).sum() < 1e-6
+    before, _ = oracle.pagerank(keys, V, 0.85, 6)
+    assert abs(delta - np.abs(want - before).sum()) < 1e-6
+    pma.close()
