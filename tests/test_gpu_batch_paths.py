@@ -85,3 +85,26 @@ def test_rebuild_by_merging(V, n, S):
     t.delete(t.ref)
     t.compare()
     t.close()
+
+
+# 3 * 2^16 queries: the first size of the staged search; heights below, at and
+# above its table, lines shorter and longer than 16 words
+@pytest.mark.parametrize("V,E,S", [(1, 1, 2), (5, 12, 2), (50, 300, 1024), (300, 40000, 2), (20000, 300000, 8),
+                                   (20000, 300000, 16), (60000, 1000000, 32), (3000, 900000, 256)])
+def test_edge_query_many(V, E, S):
+    rng = np.random.default_rng(V + S)
+    say(f"edge query V={V} E={E} S={S}")
+    import torch
+    pma = L.PMA(V, segment_slots=S)
+    ref = oracle.sort_unique(rand_keys(rng, V, E))
+    pma.insert(ref)
+    gone = ref[:: 7]
+    pma.delete(gone)
+    live = oracle.apply(ref, np.empty(0, dtype=np.uint64), gone)
+    for n in ((3 << 16) - 1, 3 << 16, (3 << 16) + 5, 700001):
+        q = np.concatenate([rng.choice(ref, n // 2), rand_keys(rng, V, n - n // 2 - 6),
+                            keys_of([0, V, V - 1, 0, 0xFFFFFFFF, 0], [0xFFFFFFFF, 0, V, V - 1, 0xFFFFFFFF, 0])])
+        rng.shuffle(q)
+        got = pma.edge_query(L.to_device(q)).cpu().numpy()
+        assert got.size == n and np.array_equal(got != 0, np.isin(q, live))
+    pma.close()
