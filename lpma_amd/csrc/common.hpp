@@ -140,6 +140,15 @@ struct PmaStat {
     i32 pd0, pd1;  // the update prefix at u0 and u1 (delta = pd1 - pd0)
 };
 
+// A lone PMA's outcome as a kernel stores it in pinned host memory, for a
+// host that waits on seq (the run's epoch, stored last) instead of a copy and
+// an event.
+struct EarlyOut {
+    Status s;
+    PmaStat p;
+    u64 seq;
+};
+
 // claimed-level masks: bit l set when some run of the PMA claimed a window
 // of level l >= 1; LV_REPL copies per PMA (written by workgroup index) so
 // the density check's atomics do not all meet on one word
@@ -188,6 +197,16 @@ struct Group {
     const RoundHdr *rh;  // graph replays: n and epoch come from here
     DevState one;
 };
+
+// by one thread, with s and p complete
+__device__ __forceinline__ void report_early(const Status &s, const PmaStat &p, EarlyOut *out, u32 epoch) {
+    const u32 *a = (const u32 *)&s, *b = (const u32 *)&p;
+    for (u32 i = 0; i < sizeof(Status) / 4; ++i)
+        __hip_atomic_store((u32 *)&out->s + i, a[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (u32 i = 0; i < sizeof(PmaStat) / 4; ++i)
+        __hip_atomic_store((u32 *)&out->p + i, b[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&out->seq, (u64)epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __device__ __forceinline__ u32 group_epoch(const Group &g) { return g.rh ? g.rh->epoch : g.epoch; }
 

@@ -69,8 +69,9 @@ hipError_t rebalance_seg(const Group &g, const BatchBufs &b, u64 windows, hipStr
                          hipEvent_t e1 = nullptr);
 // single-segment and one-wave windows in one launch (a lone PMA's early
 // rebalance), its grid sized for at most `bound` windows, the counts read
-// from the status on the device (queued before the host knows them)
-hipError_t rebalance_seg_wave_bound(const Group &g, const BatchBufs &b, u64 bound, hipStream_t st,
+// from the status on the device (queued before the host knows them); first
+// stores the batch's outcome in `early` when given
+hipError_t rebalance_seg_wave_bound(const Group &g, const BatchBufs &b, u64 bound, EarlyOut *early, hipStream_t st,
                                     hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 u32 seg_lanes_log2(u32 log2S, int slots_log2);
 hipError_t group_pyramid(const Group &g, u32 nblocks, hipStream_t st);

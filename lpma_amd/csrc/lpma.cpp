@@ -201,7 +201,7 @@ struct Pipeline {
     double phase_ms[PH_NUM] = {0};
     u64 launches_wave = 0, launches_block = 0, launches_seg = 0;
 
-    hipEvent_t ev_status = nullptr;  // the round's status has reached the host
+    EarlyOut *h_early = nullptr;  // pinned: a lone PMA's outcome, stored by a kernel
 };
 
 static constexpr u64 STATUS_BYTES = (sizeof(Status) + 15) / 16 * 16;
@@ -382,8 +382,6 @@ void pipeline_free(Pipeline &pl) {
     collect_events(pl);
     for (auto e : pl.ev_pool) (void)hipEventDestroy(e);
     pl.ev_pool.clear();
-    if (pl.ev_status) (void)hipEventDestroy(pl.ev_status);
-    pl.ev_status = nullptr;
     int d = pl.device;
     release_on(d, pl.pk0); release_on(d, pl.pk1); release_on(d, pl.ukey); release_on(d, pl.useg);
     release_on(d, pl.ckey); release_on(d, pl.cseg); release_on(d, pl.merged); release_on(d, pl.lmbase);
@@ -401,7 +399,8 @@ void pipeline_free(Pipeline &pl) {
     if (pl.h_tab) (void)hipHostFree(pl.h_tab);
     if (pl.h_segs) (void)hipHostFree(pl.h_segs);
     if (pl.h_out) (void)hipHostFree(pl.h_out);
-    pl.h_tab = nullptr; pl.h_segs = nullptr; pl.h_out = nullptr;
+    if (pl.h_early) (void)hipHostFree(pl.h_early);
+    pl.h_tab = nullptr; pl.h_segs = nullptr; pl.h_out = nullptr; pl.h_early = nullptr;
     if (pl.d_stats) (void)hipFree(pl.d_stats);
     pl.d_stats = nullptr;
 }
@@ -593,6 +592,16 @@ int ensure_batch(Pipeline &pl, u64 n, u32 npma, u32 nsegs, u64 runs) {
             return LPMA_ERR_OUT_OF_MEMORY;
         }
         pl.h_out_bytes = want;
+    }
+    if (!pl.h_early) {
+        if (injected_failure()) return LPMA_ERR_OUT_OF_MEMORY;
+        if (hipHostMalloc((void **)&pl.h_early, sizeof(EarlyOut), hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            pl.h_early = nullptr;
+            return LPMA_ERR_OUT_OF_MEMORY;
+        }
+        pl.h_early->seq = 0;
     }
     return LPMA_OK;
 }
@@ -1025,21 +1034,25 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     }
     const u64 out_bytes = STATUS_BYTES + (u64)npma * sizeof(PmaStat);
     // A lone PMA's single-segment and wave windows are queued before the
-    // host reads the status, with grids sized for the batch and the window
-    // counts read on the device, so they run while the host waits for the
-    // status and queues the rest: a PMA with a root rebuild or resize has no
-    // windows, so a round that fails after the status changes nothing.
-    HIPCHECK(hipMemcpyAsync(pl.h_out, pl.out.p, out_bytes, hipMemcpyDeviceToHost, st));
+    // host knows the status, with grids sized for the batch and the window
+    // counts read on the device, so they run while the host reads it and
+    // queues the rest: a PMA with a root rebuild or resize has no windows, so
+    // a round that fails after the status changes nothing.  Their kernel
+    // stores the status in pinned memory as it starts, which the host polls
+    // (a copy and an event in between took 4 us of the stream and about as
+    // long again on the host).
     if (early) {
-        if (!pl.ev_status) HIPCHECK(hipEventCreateWithFlags(&pl.ev_status, hipEventDisableTiming));
-        HIPCHECK(hipEventRecord(pl.ev_status, st));
         {
             LaunchTimer t(pl, PH_SEG);
-            HIPCHECK(rebalance_seg_wave_bound(g, bb, n, st, t.a, t.b));
+            HIPCHECK(rebalance_seg_wave_bound(g, bb, n, pl.h_early, st, t.a, t.b));
             pl.launches_seg++;
         }
-        HIPCHECK(hipEventSynchronize(pl.ev_status));
+        u64 w;
+        CHECKED(wait_word(&pl.h_early->seq, st, w, [epoch](u64 x) { return x == epoch; }));
+        memcpy(pl.h_out, &pl.h_early->s, sizeof(Status));
+        memcpy(pl.h_out + STATUS_BYTES, &pl.h_early->p, sizeof(PmaStat));
     } else {
+        HIPCHECK(hipMemcpyAsync(pl.h_out, pl.out.p, out_bytes, hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
     }
     return finish_round(pl, mem, npma, g, pyr_blocks, false, st, early);

@@ -1221,9 +1221,11 @@ __global__ __launch_bounds__(SEG_TPB) void k_rebalance_seg(Group g, const Work *
                                                            const Status *__restrict__ status,
                                                            const u64 *__restrict__ ckey, const i32 *__restrict__ pd,
                                                            u32 log2G, u32 nw_host, const Work *__restrict__ wwork,
-                                                           u32 sgrid) {
+                                                           u32 sgrid, EarlyOut *early) {
     extern __shared__ u64 lds[];
     __shared__ u64 red[4];
+    // the host waits for the batch's outcome while the windows are done
+    if (early && blockIdx.x == 0 && threadIdx.x == 0) report_early(*status, g.pstat[0], early, g.epoch);
     const u32 G = 1u << log2G;
     const u32 S = G * SPL;
     const u32 lane_g = threadIdx.x & (G - 1);
@@ -1364,20 +1366,21 @@ u32 seg_lanes_log2(u32 log2S, int slots_log2) {
 // start and end in them (the kernel's execution time, no separate packets)
 template <int SPL>
 static void seg_dispatch(u32 grid, u32 wgrid, size_t lds, hipStream_t st, hipEvent_t e0, hipEvent_t e1,
-                         const Group &g, const BatchBufs &b, u32 log2G, u32 nw, const Work *wwork) {
+                         const Group &g, const BatchBufs &b, u32 log2G, u32 nw, const Work *wwork, EarlyOut *early) {
     if (e0)
         hipExtLaunchKernelGGL(k_rebalance_seg<SPL>, dim3(grid + wgrid), dim3(SEG_TPB), (u32)lds, st, e0, e1, 0u, g,
                               (const Work *)b.work[CLASS_SEG], (const Status *)b.status, (const u64 *)b.ckey,
-                              (const i32 *)b.pd, log2G, nw, wwork, grid);
+                              (const i32 *)b.pd, log2G, nw, wwork, grid, early);
     else
         k_rebalance_seg<SPL><<<grid + wgrid, SEG_TPB, lds, st>>>(g, b.work[CLASS_SEG], b.status, b.ckey, b.pd, log2G,
-                                                                 nw, wwork, grid);
+                                                                 nw, wwork, grid, early);
 }
 
 // `windows`: the exact window count (eager rounds) or a bound that sizes the
 // grid, the kernel then reading the count from the status (graph replays)
 static hipError_t rebalance_seg_launch(const Group &g, const BatchBufs &b, u64 windows, bool exact, hipStream_t st,
-                                       hipEvent_t e0, hipEvent_t e1, bool with_wave = false) {
+                                       hipEvent_t e0, hipEvent_t e1, bool with_wave = false,
+                                       EarlyOut *early = nullptr) {
     u32 S = 1u << g.log2S;
     u32 log2G = g.seg_log2G;
     u32 groups_per_block = SEG_TPB >> log2G;
@@ -1391,11 +1394,11 @@ static hipError_t rebalance_seg_launch(const Group &g, const BatchBufs &b, u64 w
     u32 grid = (u32)(blocks < 1 ? 1 : (blocks > SEG_GRID_MAX ? SEG_GRID_MAX : blocks));
     u32 nw = exact ? (u32)windows : ~0u;
     switch (S >> log2G) {
-        case 1: seg_dispatch<1>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork); break;
-        case 2: seg_dispatch<2>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork); break;
-        case 4: seg_dispatch<4>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork); break;
-        case 8: seg_dispatch<8>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork); break;
-        case 16: seg_dispatch<16>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork); break;
+        case 1: seg_dispatch<1>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork, early); break;
+        case 2: seg_dispatch<2>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork, early); break;
+        case 4: seg_dispatch<4>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork, early); break;
+        case 8: seg_dispatch<8>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork, early); break;
+        case 16: seg_dispatch<16>(grid, wgrid, lds, st, e0, e1, g, b, log2G, nw, wwork, early); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1406,9 +1409,9 @@ hipError_t rebalance_seg(const Group &g, const BatchBufs &b, u64 windows, hipStr
     return rebalance_seg_launch(g, b, windows, true, st, e0, e1);
 }
 
-hipError_t rebalance_seg_wave_bound(const Group &g, const BatchBufs &b, u64 bound, hipStream_t st, hipEvent_t e0,
-                                    hipEvent_t e1) {
-    return rebalance_seg_launch(g, b, bound, false, st, e0, e1, true);
+hipError_t rebalance_seg_wave_bound(const Group &g, const BatchBufs &b, u64 bound, EarlyOut *early, hipStream_t st,
+                                    hipEvent_t e0, hipEvent_t e1) {
+    return rebalance_seg_launch(g, b, bound, false, st, e0, e1, true, early);
 }
 
 hipError_t rebalance_lds(const Group &g, const BatchBufs &b, int cls, u32 grid, hipStream_t st, hipEvent_t e0,
