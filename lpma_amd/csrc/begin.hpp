@@ -1,6 +1,6 @@
-// begin.hpp -- a batch's first device work (status, update index, the count
-// pyramid's top levels), shared by the batch-begin kernel and the sort
-// kernel that carries it for a lone PMA.
+// begin.hpp -- device code that several of the update's kernels share: a
+// batch's first work (status, update index, the count pyramid), its elements'
+// sort keys, and the searches of the density check.
 #pragma once
 #include "common.hpp"
 
@@ -14,21 +14,19 @@ static constexpr u32 PYR_CHL = 11;
 static constexpr u32 PYR_CH = 1u << PYR_CHL;
 
 // Levels 1..PYR_CHL of one chunk of 2^PYR_CHL segments (all levels of a
-// smaller PMA), by one workgroup of 256 threads, through LDS.
-__device__ inline void pyr_chunk(const DevState &d, u64 chunk) {
-    __shared__ u32 v0[PYR_CH];
-    __shared__ u32 v1[PYR_CH / 2];
+// smaller PMA), by one workgroup, through LDS (v0: PYR_CH words, v1: half).
+__device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1) {
     const u64 nseg = nseg_of(d);
     const u32 levels = d.H < PYR_CHL ? d.H : PYR_CHL;
     const u32 n = (u32)(nseg < PYR_CH ? nseg : PYR_CH);
     const u64 c0 = chunk * n;
-    for (u32 i = threadIdx.x; i < n; i += 256) v0[i] = d.cnt[c0 + i];
+    for (u32 i = threadIdx.x; i < n; i += blockDim.x) v0[i] = d.cnt[c0 + i];
     __syncthreads();
     u32 *in = v0, *tmp = v1;
     for (u32 l = 1; l <= levels; ++l) {
         u32 nw = n >> l;
         u32 *out = d.pyr + pyr_off(nseg, l) + (c0 >> l);
-        for (u32 x = threadIdx.x; x < nw; x += 256) {
+        for (u32 x = threadIdx.x; x < nw; x += blockDim.x) {
             u32 s = in[2 * x] + in[2 * x + 1];
             tmp[x] = s;
             out[x] = s;
@@ -46,8 +44,8 @@ __device__ inline void pyr_chunk(const DevState &d, u64 chunk) {
 // through global memory.
 static constexpr u32 PYR_TOP_LDS = 4096;
 
-__device__ inline void pyr_top_levels(const DevState &d) {
-    __shared__ u32 v[2 * PYR_TOP_LDS];
+// v: 2 * PYR_TOP_LDS words of LDS
+__device__ inline void pyr_top_levels(const DevState &d, u32 *v) {
     const u64 nseg = nseg_of(d);
     if (d.H <= PYR_CHL) return;
     const u64 nc = nseg >> PYR_CHL;
@@ -78,11 +76,11 @@ __device__ inline void pyr_top_levels(const DevState &d) {
 
 // One workgroup's share of a batch's first work for PMA pid: its per-batch
 // record and claimed-level masks cleared, its pyramid's top levels summed
-// (unless top is false: then a later kernel sums them); the workgroup of
+// (unless v is null: then a later kernel sums them); the workgroup of
 // PMA 0 also clears the status, zero[0, nzero) and, for a lone PMA, resets
-// the update index wfirst.
+// the update index wfirst.  v: the LDS of pyr_top_levels.
 __device__ inline void batch_first_work(const Group &g, Status *s, u32 pid, u32 *zero, u32 nzero, u32 *wfirst,
-                                        bool top = true) {
+                                        u32 *v) {
     if (pid == 0) {
         for (u32 i = threadIdx.x; i < nzero; i += blockDim.x) zero[i] = 0;
         if (g.npma == 1)
@@ -100,7 +98,78 @@ __device__ inline void batch_first_work(const Group &g, Status *s, u32 pid, u32 
         g.pstat[pid] = z;
     }
     if (threadIdx.x < LV_REPL) g.lvmask[(u64)pid * LV_REPL + threadIdx.x] = 0;
-    if (top) pyr_top_levels(pma_of(g, pid));
+    if (v) pyr_top_levels(pma_of(g, pid), v);
+}
+
+// ------------------------------------------------------- batch elements
+
+// Batch element i comes from the source whose [off, off + n) holds it.
+// Sources are few and sorted by off; each thread finds its first source by
+// binary search and walks forward from there.
+__device__ __forceinline__ u32 source_of(const BatchSeg *__restrict__ segs, u32 nsegs, u64 i) {
+    u32 lo = 0, hi = nsegs;
+    while (hi - lo > 1) {
+        u32 mid = (lo + hi) >> 1;
+        if (segs[mid].off <= i) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// element i of the batch, a source's, as its sort key (src or dst >= V: bad)
+__device__ __forceinline__ u64 pack_element(const BatchSeg &sg, u64 i, u32 pshift, u32 sbits, bool &bad) {
+    u64 k = sg.keys[i - sg.off];
+    u32 src = (u32)(k >> 32), dst = (u32)k;
+    if (src >= sg.V || dst >= sg.V) { bad = true; src = 0; dst = 0; }
+    return ((u64)sg.pid << pshift) | ((((((u64)src) << sg.vbits) | dst) << sbits | sg.seq) << 1) | sg.op;
+}
+
+// ------------------------------------------------ searches near a position
+
+// first index >= start with a[idx] >= target, given a[start-1] < target;
+// the exponential search starts with strides of `step` (a guess of the
+// distance)
+template <class T>
+__device__ __forceinline__ u32 gallop_fwd(const T *__restrict__ a, u32 start, u32 n, typename std::remove_cv<T>::type target,
+                                          u32 step) {
+    u32 lo = start;
+    if (lo >= n || a[lo] >= target) return lo;
+    u32 hi = (n - lo > step) ? lo + step : n;
+    while (hi < n && a[hi] < target) {
+        lo = hi;
+        step <<= 1;
+        hi = (n - lo > step) ? lo + step : n;
+    }
+    // a[lo] < target, hi == n or a[hi] >= target
+    u32 l = lo + 1, h = hi;
+    while (l < h) {
+        u32 m = (l + h) >> 1;
+        if (a[m] < target) l = m + 1; else h = m;
+    }
+    return l;
+}
+
+// smallest index <= start whose suffix [idx, start] is >= target, given
+// a[start] >= target; strides start at `step` as above
+template <class T>
+__device__ __forceinline__ u32 gallop_back(const T *__restrict__ a, u32 start, typename std::remove_cv<T>::type target,
+                                           u32 step) {
+    if (start == 0 || a[start - 1] < target) return start;
+    u32 hi = start - 1;  // a[hi] >= target
+    u32 lo;
+    while (true) {
+        lo = hi >= step ? hi - step : 0;
+        if (a[lo] < target) break;
+        if (lo == 0) return 0;
+        hi = lo;
+        step <<= 1;
+    }
+    // a[lo] < target <= a[hi]
+    u32 l = lo + 1, h = hi;
+    while (l < h) {
+        u32 m = (l + h) >> 1;
+        if (a[m] < target) l = m + 1; else h = m;
+    }
+    return l;
 }
 
 }  // namespace pma

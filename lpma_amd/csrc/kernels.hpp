@@ -48,6 +48,15 @@ u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const Inli
                          u32 sbits, u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 pyr_chunks,
                          hipStream_t st);
 
+// A lone PMA's batch of at most SMALL_MAX_N keys from inline sources, from its
+// keys to the elected windows in one kernel, with the pyramid's levels owed by
+// the last batch (chunks: its chunk levels, 0 if none) summed beside it; the
+// outcome goes to the status and to `early`.  arrive: two words, zero.
+static constexpr u32 SMALL_MAX_N = 2048;
+static constexpr u32 SMALL_ARRIVE_WORDS = 2;
+hipError_t small_batch(const Group &g, const BatchBufs &b, const InlineSegs &in, u64 n, u32 chunks, u32 *arrive,
+                       EarlyOut *early, hipStream_t st);
+
 u32 locate_blocks(u64 n);
 // most groups of locate blocks
 static constexpr u32 LOC_GROUPS = 1024;

@@ -354,12 +354,14 @@ int ensure_host(T *&p, u32 &cap, u64 n, hipStream_t sync_st) {
 int pipeline_init(Pipeline &pl, int device, hipStream_t st) {
     pl.device = device;
     pl.cur_stream = st;
-    if (hipMalloc(&pl.d_stats, ST_ROWS * ST_NUM * sizeof(u64)) != hipSuccess) {
+    // the counters, then the small batch's arrival words
+    static_assert(SMALL_ARRIVE_WORDS <= 2, "one word of 64 bits");
+    if (hipMalloc(&pl.d_stats, (ST_ROWS * ST_NUM + 1) * sizeof(u64)) != hipSuccess) {
         (void)hipGetLastError();
         pl.d_stats = nullptr;
         return LPMA_ERR_OUT_OF_MEMORY;
     }
-    if (fill_u64(pl.d_stats, (u64)ST_ROWS * ST_NUM, 0, st) != hipSuccess) {
+    if (fill_u64(pl.d_stats, (u64)ST_ROWS * ST_NUM + 1, 0, st) != hipSuccess) {
         (void)hipGetLastError();
         return LPMA_ERR_DEVICE;
     }
@@ -1000,51 +1002,62 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     g.defer_rebuild = 0;
     g.one = mem[0].h->st;
     BatchBufs bb = batch_bufs(pl);
-    // bit 0 of a packed key is the operation (with the request order above
-    // it): sorted only when a member mixes them or merges requests
-    const u32 lo_bit = (mixed || sbits) ? 0 : 1;
-    u64 *pk;
-    {
+    // a small batch reaches its windows in one kernel (which needs the early
+    // path's scratch, and reports to the host itself)
+    const bool small = early && nsegs <= INLINE_SEGS && n <= SMALL_MAX_N;
+    if (small) {
         PhaseTimer t(pl, st, PH_SORT);
-        if (npma == 1 && nsegs <= INLINE_SEGS && sort_carries_first(n)) {
-            lpma *h0 = mem[0].h;
-            const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
-            pk = pack_and_sort_first(g, bb.status, bb.wfirst, in, n, pshift, sbits, hi_bit, pl.pk0.p, pl.pk1.p,
-                                     pl.ukey.p, pl.sort_scr.p, chunks, st);
-            h0->pyr_owed = false;
-        } else {
-            HIPCHECK(pay_owed_pyramids(mem, npma, st));
-            HIPCHECK(batch_begin(g, bb, in, pl.segs.p, pl.sort_scr.p, sort_zero_words(), st));
-            pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
-                               pl.ukey.p, pl.sort_scr.p, &bb.status->flags, st);
+        lpma *h0 = mem[0].h;
+        const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
+        HIPCHECK(small_batch(g, bb, in, n, chunks, (u32 *)(pl.d_stats + ST_ROWS * ST_NUM), pl.h_early, st));
+        h0->pyr_owed = false;
+    } else {
+        // bit 0 of a packed key is the operation (with the request order above
+        // it): sorted only when a member mixes them or merges requests
+        const u32 lo_bit = (mixed || sbits) ? 0 : 1;
+        u64 *pk;
+        {
+            PhaseTimer t(pl, st, PH_SORT);
+            if (npma == 1 && nsegs <= INLINE_SEGS && sort_carries_first(n)) {
+                lpma *h0 = mem[0].h;
+                const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
+                pk = pack_and_sort_first(g, bb.status, bb.wfirst, in, n, pshift, sbits, hi_bit, pl.pk0.p, pl.pk1.p,
+                                         pl.ukey.p, pl.sort_scr.p, chunks, st);
+                h0->pyr_owed = false;
+            } else {
+                HIPCHECK(pay_owed_pyramids(mem, npma, st));
+                HIPCHECK(batch_begin(g, bb, in, pl.segs.p, pl.sort_scr.p, sort_zero_words(), st));
+                pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
+                                   pl.ukey.p, pl.sort_scr.p, &bb.status->flags, st);
+            }
+            HIPCHECK(hipGetLastError());
         }
-        HIPCHECK(hipGetLastError());
-    }
-    {
-        PhaseTimer t(pl, st, PH_LOCATE);
-        HIPCHECK(locate_and_compact(g, pk, n, bb, st));
-        HIPCHECK(density_check(g, n, bb, st));
-    }
-    {
-        // window election before the single host synchronisation, so the
-        // host learns the exact work of every rebalance class and sizes each
-        // grid to it (idle workgroups still cost dispatch time)
-        PhaseTimer t(pl, st, PH_ELECT);
-        HIPCHECK(elect_windows(g, n, bb, st));
+        {
+            PhaseTimer t(pl, st, PH_LOCATE);
+            HIPCHECK(locate_and_compact(g, pk, n, bb, st));
+            HIPCHECK(density_check(g, n, bb, st));
+        }
+        {
+            // window election before the single host synchronisation, so the
+            // host learns the exact work of every rebalance class and sizes each
+            // grid to it (idle workgroups still cost dispatch time)
+            PhaseTimer t(pl, st, PH_ELECT);
+            HIPCHECK(elect_windows(g, n, bb, st));
+        }
     }
     const u64 out_bytes = STATUS_BYTES + (u64)npma * sizeof(PmaStat);
     // A lone PMA's single-segment and wave windows are queued before the
     // host knows the status, with grids sized for the batch and the window
     // counts read on the device, so they run while the host reads it and
     // queues the rest: a PMA with a root rebuild or resize has no windows, so
-    // a round that fails after the status changes nothing.  Their kernel
-    // stores the status in pinned memory as it starts, which the host polls
+    // a round that fails after the status changes nothing.  Their kernel (or
+    // the small batch's) stores the status in pinned memory, which the host polls
     // (a copy and an event in between took 4 us of the stream and about as
     // long again on the host).
     if (early) {
         {
             LaunchTimer t(pl, PH_SEG);
-            HIPCHECK(rebalance_seg_wave_bound(g, bb, n, pl.h_early, st, t.a, t.b));
+            HIPCHECK(rebalance_seg_wave_bound(g, bb, n, small ? nullptr : pl.h_early, st, t.a, t.b));
             pl.launches_seg++;
         }
         u64 w;

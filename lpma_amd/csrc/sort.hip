@@ -25,18 +25,6 @@ static constexpr int RS_TPB = 256;
 static constexpr int RS_ITEMS_BIG = 16;   // keys per thread per tile, large inputs
 static constexpr int RS_ITEMS_SMALL = 4;  // smaller tiles for more workgroups on mid-size batches
 
-// Batch element i comes from the source whose [off, off + n) holds it.
-// Sources are few and sorted by off; each thread finds its first source by
-// binary search and walks forward from there.
-__device__ __forceinline__ u32 source_of(const BatchSeg *__restrict__ segs, u32 nsegs, u64 i) {
-    u32 lo = 0, hi = nsegs;
-    while (hi - lo > 1) {
-        u32 mid = (lo + hi) >> 1;
-        if (segs[mid].off <= i) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
 // Packs a group batch into sort keys pid << pshift | (src << vbits | dst) << 1 | op
 // (keys with src or dst >= V raise FLAG_INVALID_KEY) and counts the first
 // radix digit of every tile (digit-major: hist[d * nblocks + tile]).
@@ -435,13 +423,6 @@ static u32 ss_buckets(u64 n) {
     return nb;
 }
 
-__device__ __forceinline__ u64 pack_element(const BatchSeg &sg, u64 i, u32 pshift, u32 sbits, bool &bad) {
-    u64 k = sg.keys[i - sg.off];
-    u32 src = (u32)(k >> 32), dst = (u32)k;
-    if (src >= sg.V || dst >= sg.V) { bad = true; src = 0; dst = 0; }
-    return ((u64)sg.pid << pshift) | ((((((u64)src) << sg.vbits) | dst) << sbits | sg.seq) << 1) | sg.op;
-}
-
 // Splitters and bucket choice work on 32-bit projections of the packed
 // keys, x >> psh with psh >= the bits below the key (request order,
 // operation): equal keys project equally, so they share a bucket, and any
@@ -463,6 +444,7 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
     __shared__ u32 cnt[SS_MAX_BUCKETS];
     __shared__ u32 base[SS_MAX_BUCKETS];
     __shared__ BatchSeg lsegs[INLINE_SEGS];
+    __shared__ u32 pyr_v0[FIRST ? PYR_CH : 1], pyr_v1[FIRST ? PYR_CH / 2 : 1];
     if (n_dev) n = *n_dev;
     const u32 t = blockIdx.x;
     const u32 ntiles = (u32)((n + SS_TILE - 1) / SS_TILE);
@@ -470,9 +452,9 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
     if (FIRST) {
         if (t >= ntiles) {
             if (t == ntiles)
-                batch_first_work(g, status, 0, nullptr, 0, wfirst, false);
+                batch_first_work(g, status, 0, nullptr, 0, wfirst, nullptr);
             else
-                pyr_chunk(pma_of(g, 0), t - ntiles - 1);
+                pyr_chunk(pma_of(g, 0), t - ntiles - 1, pyr_v0, pyr_v1);
             return;
         }
         if (tid < in.n) lsegs[tid] = in.s[tid];
@@ -624,7 +606,8 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
                                                        u64 *__restrict__ aux, u64 n, const u64 *n_dev, u32 nb,
                                                        const u32 *__restrict__ bc, u32 *__restrict__ flags,
                                                        bool top, DevState topd) {
-    __shared__ u64 kb[1][SB_CAP];
+    __shared__ u64 kb[1][SB_CAP];  // (also the pyramid's top levels)
+    static_assert(sizeof(kb) >= 2 * PYR_TOP_LDS * sizeof(u32), "room for the top levels");
     __shared__ u32 whist[SB_NW][256];
     __shared__ u32 dofs[256];
     __shared__ u32 run[256];
@@ -637,7 +620,7 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
     const u32 tid = threadIdx.x;
     const u32 ntiles = (u32)((n + SS_TILE - 1) / SS_TILE);
     if (top && b == nb) {
-        pyr_top_levels(topd);
+        pyr_top_levels(topd, (u32 *)kb);
         return;
     }
     if (b >= nb || ntiles == 0) return;

@@ -379,49 +379,6 @@ hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchB
 
 // ------------------------------------------------------------ density check
 
-// first index >= start with a[idx] >= target, given a[start-1] < target;
-// the exponential search starts with strides of `step` (a guess of the
-// distance)
-__device__ __forceinline__ u32 gallop_fwd(const u64 *__restrict__ a, u32 start, u32 n, u64 target, u32 step) {
-    u32 lo = start;
-    if (lo >= n || a[lo] >= target) return lo;
-    u32 hi = (n - lo > step) ? lo + step : n;
-    while (hi < n && a[hi] < target) {
-        lo = hi;
-        step <<= 1;
-        hi = (n - lo > step) ? lo + step : n;
-    }
-    // a[lo] < target, hi == n or a[hi] >= target
-    u32 l = lo + 1, h = hi;
-    while (l < h) {
-        u32 m = (l + h) >> 1;
-        if (a[m] < target) l = m + 1; else h = m;
-    }
-    return l;
-}
-
-// smallest index <= start whose suffix [idx, start] is >= target, given
-// a[start] >= target; strides start at `step` as above
-__device__ __forceinline__ u32 gallop_back(const u64 *__restrict__ a, u32 start, u64 target, u32 step) {
-    if (start == 0 || a[start - 1] < target) return start;
-    u32 hi = start - 1;  // a[hi] >= target
-    u32 lo;
-    while (true) {
-        lo = hi >= step ? hi - step : 0;
-        if (a[lo] < target) break;
-        if (lo == 0) return 0;
-        hi = lo;
-        step <<= 1;
-    }
-    // a[lo] < target <= a[hi]
-    u32 l = lo + 1, h = hi;
-    while (l < h) {
-        u32 m = (l + h) >> 1;
-        if (a[m] < target) l = m + 1; else h = m;
-    }
-    return l;
-}
-
 // levels climbed with galloping searches before the lock-step searches (a
 // group of PMAs; a lone PMA switches to its update index at index_level(H))
 static constexpr u32 DENSITY_GALLOP_LEVELS = 8;
@@ -877,6 +834,10 @@ hipError_t elect_windows(const Group &g, u64 n, const BatchBufs &b, hipStream_t 
                                                                        b.work[2], b.work[3], b.status);
     return hipGetLastError();
 }
+
+// ------------------------------------------------------------ small batches
+
+#include "small.hpp"
 
 // ------------------------------------------------------- LDS window rebalance
 //
@@ -2268,13 +2229,17 @@ hipError_t rebuild_spread(const DevState &dst, const u64 *merged, u64 m, hipStre
 // segments through LDS (levels 1..11), a single workgroup finishes the
 // levels above.  O(nseg) streaming work, no atomics.
 
-__global__ __launch_bounds__(256) void k_pyr_chunk(DevState d) { pyr_chunk(d, blockIdx.x); }
+__global__ __launch_bounds__(256) void k_pyr_chunk(DevState d) {
+    __shared__ u32 v0[PYR_CH], v1[PYR_CH / 2];
+    pyr_chunk(d, blockIdx.x, v0, v1);
+}
 
 // the chunks of every PMA of the run that took window rebalances
 // the chunks of every PMA of the run that took window rebalances; the
 // workgroups stride over the group's chunk list (its length is read from
 // the table, so the grid does not depend on the members' heights)
 __global__ __launch_bounds__(256) void k_pyr_chunk_group(Group g) {
+    __shared__ u32 v0[PYR_CH], v1[PYR_CH / 2];
     const PmaEntry &last = g.tab[g.npma - 1];
     const u32 total = last.pyr_blk0 + last.pyr_nblk;
     for (u32 c = blockIdx.x; c < total; c += gridDim.x) {
@@ -2287,18 +2252,22 @@ __global__ __launch_bounds__(256) void k_pyr_chunk_group(Group g) {
         if (ps.u1 == ps.u0 || (ps.flags & (FLAG_ROOT | FLAG_RESIZE))) continue;
         const DevState d = pma_of(g, lo);
         if (d.H == 0) continue;
-        pyr_chunk(d, c - g.tab[lo].pyr_blk0);
+        pyr_chunk(d, c - g.tab[lo].pyr_blk0, v0, v1);
         __syncthreads();
     }
 }
 
-__global__ __launch_bounds__(1024) void k_pyr_top(DevState d) { pyr_top_levels(d); }
+__global__ __launch_bounds__(1024) void k_pyr_top(DevState d) {
+    __shared__ u32 v[2 * PYR_TOP_LDS];
+    pyr_top_levels(d, v);
+}
 
 __global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, InlineSegs in, BatchSeg *segs, u32 *zero,
                                                       u32 nzero, u32 *wfirst, u64 *grp) {
+    __shared__ u32 v[2 * PYR_TOP_LDS];
     if (blockIdx.x == 0 && threadIdx.x < in.n) segs[threadIdx.x] = in.s[threadIdx.x];
     if (blockIdx.x == 0 && threadIdx.x < LOC_GROUPS) grp[threadIdx.x] = 0;
-    batch_first_work(g, s, blockIdx.x, zero, nzero, wfirst);
+    batch_first_work(g, s, blockIdx.x, zero, nzero, wfirst, v);
 }
 
 // chunk levels of the PMAs of a run (their top levels follow in the next

@@ -108,3 +108,58 @@ def test_edge_query_many(V, E, S):
         got = pma.edge_query(L.to_device(q)).cpu().numpy()
         assert got.size == n and np.array_equal(got != 0, np.isin(q, live))
     pma.close()
+
+
+# up to 2048 keys: one kernel to the windows; sizes around its sort's powers of
+# two, duplicates, mixed and merged requests, growth, shrink, empty effects,
+# heights below and above the staged separators and the pyramid's chunk levels
+@pytest.mark.parametrize("V,S,fill", [(1, 2, 0), (3, 32, 4), (700, 2, 6000), (700, 1024, 6000), (4096, 32, 40000),
+                                      (60000, 2, 200000), (300000, 16, 300000)])
+def test_small_batches(V, S, fill):
+    rng = np.random.default_rng(V + S)
+    say(f"small batches V={V} S={S}")
+    t = Triple(V, segment_slots=S)
+    if fill:
+        t.insert(rand_keys(rng, V, fill))
+    for n in (1, 2, 63, 64, 65, 500, 1023, 1024, 1025, 2047, 2048, 2049):
+        a = rand_keys(rng, V, n)
+        a[: n // 4] = a[n - n // 4: n]  # duplicates
+        t.insert(a)
+        t.insert(a)  # no effect
+        t.compare()
+        d = rng.choice(t.ref, min(n, t.ref.size)) if t.ref.size else a
+        t.delete(d)
+        t.compare()
+        k = n // 2
+        t.mixed(rand_keys(rng, V, n - k), np.concatenate([a[: k // 2], d[: k - k // 2]])[:k])
+        t.compare()
+    row = keys_of(np.full(2048, V // 2), rng.integers(0, V, 2048))  # one row: wide windows
+    for _ in range(3):
+        t.insert(row)
+        t.compare()
+        t.delete(row)
+        t.compare()
+    t.close()
+
+
+def test_small_batch_refused_and_merged():
+    V = 5000
+    rng = np.random.default_rng(8)
+    say("small batches: invalid keys, merged requests")
+    t = Triple(V)
+    t.insert(rand_keys(rng, V, 30000))
+    for n in (1, 64, 2048):
+        bad = rand_keys(rng, V, n)
+        bad[n // 2] = keys_of([V], [0])[0]
+        with pytest.raises(L.LpmaError):
+            t.pma.insert(bad)
+        t.compare()
+    for _ in range(4):
+        a, b = rand_keys(rng, V, 700), rand_keys(rng, V, 600)
+        b[:300] = a[:300]
+        t.pma.update_sequence([(a, b), (b, a[:500])])
+        t.mixed(a, b)
+        t.mixed(b, a[:500])
+        # the layout is that of one batch; the edges are those of two
+        t.compare(layout=False)
+    t.close()
