@@ -13,8 +13,18 @@ static constexpr u32 PYR_CHL = 11;
 
 static constexpr u32 PYR_CH = 1u << PYR_CHL;
 
+// A store other workgroups of the same kernel read (COH): written through to
+// where every XCD sees it, so its writer needs no write-back of its L2 before
+// it signals them.
+template <bool COH, class T>
+__device__ __forceinline__ void put(T *p, T v) {
+    if (COH) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+
 // Levels 1..PYR_CHL of one chunk of 2^PYR_CHL segments (all levels of a
 // smaller PMA), by one workgroup, through LDS (v0: PYR_CH words, v1: half).
+template <bool COH = false>
 __device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1) {
     const u64 nseg = nseg_of(d);
     const u32 levels = d.H < PYR_CHL ? d.H : PYR_CHL;
@@ -29,7 +39,7 @@ __device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1)
         for (u32 x = threadIdx.x; x < nw; x += blockDim.x) {
             u32 s = in[2 * x] + in[2 * x + 1];
             tmp[x] = s;
-            out[x] = s;
+            put<COH>(&out[x], s);
         }
         __syncthreads();
         u32 *sw = in; in = tmp; tmp = sw;
@@ -45,6 +55,7 @@ __device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1)
 static constexpr u32 PYR_TOP_LDS = 4096;
 
 // v: 2 * PYR_TOP_LDS words of LDS
+template <bool COH = false>
 __device__ inline void pyr_top_levels(const DevState &d, u32 *v) {
     const u64 nseg = nseg_of(d);
     if (d.H <= PYR_CHL) return;
@@ -62,14 +73,15 @@ __device__ inline void pyr_top_levels(const DevState &d, u32 *v) {
         }
         // levels PYR_CHL + 1 .. H: v[nc, 2 nc - 1), contiguous in the pyramid too
         u32 *out = d.pyr + pyr_off(nseg, PYR_CHL + 1);
-        for (u32 x = threadIdx.x; x < (u32)nc - 1; x += blockDim.x) out[x] = v[nc + x];
+        for (u32 x = threadIdx.x; x < (u32)nc - 1; x += blockDim.x) put<COH>(&out[x], v[nc + x]);
         return;
     }
     for (u32 l = PYR_CHL + 1; l <= d.H; ++l) {
         u64 nw = nseg >> l;
         const u32 *in = d.pyr + pyr_off(nseg, l - 1);
         u32 *out = d.pyr + pyr_off(nseg, l);
-        for (u64 x = threadIdx.x; x < nw; x += blockDim.x) out[x] = in[2 * x] + in[2 * x + 1];
+        for (u64 x = threadIdx.x; x < nw; x += blockDim.x) put<COH>(&out[x], in[2 * x] + in[2 * x + 1]);
+        if (COH) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
 }
@@ -170,6 +182,46 @@ __device__ __forceinline__ u32 gallop_back(const T *__restrict__ a, u32 start, t
         if (a[m] < target) l = m + 1; else h = m;
     }
     return l;
+}
+
+// ------------------------------------------- lines read by rows of lanes
+//
+// A lane that searches its own line of 16 words alone asks the memory pipe for
+// it at every step.  Here a row of 16 lanes reads the lines of its 16 lanes'
+// queries one after the other, a word a lane: one request a line.
+
+// lane J of every row of 16 lanes, in all lanes of the row
+template <int J>
+__device__ __forceinline__ u32 row_lane(u32 x) {
+    return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + J, 0xF, 0xF, false);  // row_newbcast
+}
+template <int J>
+__device__ __forceinline__ u64 row_lane(u64 x) {
+    return ((u64)row_lane<J>((u32)(x >> 32)) << 32) | row_lane<J>((u32)x);
+}
+
+// a[at .. at + w) of the row's queries J0 .. J0 + 7 (w <= 16): every lane loads
+// one word of each, KEY_NONE past w
+template <int J0>
+__device__ __forceinline__ void row_lines(const u64 *a, u64 at, u32 w, u64 (&v)[8]) {
+    const u32 gl = lane_id() & 15;
+#define LPMA_LINE(K)                                                  \
+    {                                                                 \
+        const u64 x = row_lane<J0 + K>(at); /* by every lane */       \
+        v[K] = gl < w ? a[x + gl] : KEY_NONE;                         \
+    }
+    LPMA_LINE(0) LPMA_LINE(1) LPMA_LINE(2) LPMA_LINE(3) LPMA_LINE(4) LPMA_LINE(5) LPMA_LINE(6) LPMA_LINE(7)
+#undef LPMA_LINE
+}
+
+// bit J0 + K of the row's answers: how many of the words are <= (LE) or equal
+// to query J0 + K's key
+template <int J0, bool LE>
+__device__ __forceinline__ void row_counts(const u64 (&v)[8], u64 key, u32 &mine) {
+    const u32 gl = lane_id() & 15, sh = lane_id() & 48;
+#define LPMA_COUNT(K)                                                                                    {                                                                                                        const u64 k = row_lane<J0 + K>(key);                                                                 const u32 c = (u32)__popc((u32)(__ballot(LE ? v[K] <= k : v[K] == k) >> sh) & 0xFFFFu);             if (gl == J0 + K) mine = c;                                                                      }
+    LPMA_COUNT(0) LPMA_COUNT(1) LPMA_COUNT(2) LPMA_COUNT(3) LPMA_COUNT(4) LPMA_COUNT(5) LPMA_COUNT(6) LPMA_COUNT(7)
+#undef LPMA_COUNT
 }
 
 }  // namespace pma

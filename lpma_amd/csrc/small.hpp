@@ -7,12 +7,16 @@
 // in LDS, while the others sum the count pyramid's levels the last batch left
 // owing; the last of the two to arrive checks the density and elects (nothing
 // waits inside the kernel), and stores the outcome for the host.  The rebalance
-// kernel follows.  Up to SMALL_MAX_N keys: two a thread.
+// kernel follows.  Up to SMALL_MAX_N keys: two a thread.  Bound: latency.  256
+// keys on 4096 vertices 15 us (load 1.4, sort 4.1, locate 1.4, presence 1.9,
+// store and arrival 1.5, density 3, election and report 1.5); 1000 on 2^20
+// 27 us (load 3, sort 6.4, locate 8 to 11 over 2^19 segments).  One call with
+// everything around it: 50 -> 26 us and 60 -> 40 us.
 #pragma once
 
 static constexpr u32 SM_TPB = 1024;
 static constexpr u32 SM_ITEMS = SMALL_MAX_N / SM_TPB;
-static constexpr u32 SM_TAB_LOG = 10;        // separators staged in LDS
+static constexpr u32 SM_TAB_LOG = 12;        // separators staged in LDS
 static constexpr u32 SM_PYR_GRID = 1024;     // workgroups of the pyramid's chunk levels
 static_assert(SM_ITEMS == 2, "the sort holds two keys a thread");
 
@@ -30,58 +34,100 @@ struct SmallLds {
     u64 tab[1u << SM_TAB_LOG];  // every 2^(H - SM_TAB_LOG)-th separator
     u32 seg[SMALL_MAX_N];       // segments of the compacted updates
     i32 pd[SMALL_MAX_N + 1];    // their prefix
+    u32 c0[SMALL_MAX_N];        // their segments' counts
+    Density dn;
     u32 wt[SM_ITEMS][SM_TPB / 64];
     u32 cls[NUM_CLASSES];
     u32 flags, mask, n_eff, last;
     BatchSeg segs[INLINE_SEGS];
 };
 
-// Bitonic sort of M keys (a power of two, 64 to SMALL_MAX_N), key i of thread
-// i mod SM_TPB: partners less than a wave apart meet by lane exchange, the
-// others through LDS, one barrier a step (the two buffers take turns).  1024
-// keys: about 2.5 us, where radix passes over the 41 bits take 1.8 us each.
-__device__ __forceinline__ void small_sort(u64 (&a)[SM_ITEMS], u32 M, u64 *b0, u64 *b1) {
-    const u32 t = threadIdx.x;
-    for (u32 k = 2; k <= M; k <<= 1) {
-        for (u32 j = k >> 1; j; j >>= 1) {
-            u64 b[SM_ITEMS];
-            if (j >= SM_TPB) {
-                b[0] = a[1];
-                b[1] = a[0];
-            } else if (j >= 64) {
-                b0[t] = a[0];
-                if (M > SM_TPB) b0[t + SM_TPB] = a[1];
-                __syncthreads();
-                b[0] = b0[t ^ j];
-                b[1] = M > SM_TPB ? b0[(t ^ j) + SM_TPB] : 0ull;
-                u64 *x = b0; b0 = b1; b1 = x;
-            } else {
-                b[0] = __shfl_xor(a[0], j, 64);
-                b[1] = M > SM_TPB ? __shfl_xor(a[1], j, 64) : 0ull;
-            }
-#pragma unroll
-            for (u32 r = 0; r < SM_ITEMS; ++r) {
-                const u32 i = t + r * SM_TPB;
-                const bool low = ((i & j) == 0) == ((i & k) == 0);  // keeps the smaller
-                a[r] = (a[r] < b[r]) == low ? a[r] : b[r];
-            }
-        }
+// lane ^ J's value
+template <u32 J>
+__device__ __forceinline__ u32 lane_xor(u32 x) {
+    if constexpr (J == 1) return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
+    if constexpr (J == 2) return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false);  // quad_perm 2,3,0,1
+    if constexpr (J == 4) {  // xor 7 (row_half_mirror), then xor 3 (quad_perm 3,2,1,0)
+        const int m = __builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, false);
+        return (u32)__builtin_amdgcn_update_dpp(0, m, 0x1B, 0xF, 0xF, false);
     }
+    if constexpr (J == 8) return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror:8
+    if constexpr (J == 16) {  // odd rows of the one against even rows of the other
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return lane_id() & 16 ? r[0] : r[1];
+    }
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return lane_id() & 32 ? r[0] : r[1];
+}
+template <u32 J>
+__device__ __forceinline__ u64 lane_xor(u64 x) {
+    return ((u64)lane_xor<J>((u32)(x >> 32)) << 32) | lane_xor<J>((u32)x);
+}
+
+// steps J, J / 2, ..., 1 of a bitonic merge of runs of K / 2
+template <u32 K, u32 J>
+__device__ __forceinline__ void small_merge(u64 (&a)[SM_ITEMS], bool two, u64 *&b0, u64 *&b1) {
+    const u32 t = threadIdx.x;
+    u64 b[SM_ITEMS];
+    if constexpr (J >= SM_TPB) {
+        b[0] = a[1];
+        b[1] = a[0];
+    } else if constexpr (J >= 64) {
+        b0[t] = a[0];
+        if (two) b0[t + SM_TPB] = a[1];
+        __syncthreads();
+        b[0] = b0[t ^ J];
+        b[1] = two ? b0[(t ^ J) + SM_TPB] : 0ull;
+        u64 *x = b0; b0 = b1; b1 = x;
+    } else {
+        b[0] = lane_xor<J>(a[0]);
+        b[1] = two ? lane_xor<J>(a[1]) : 0ull;
+    }
+#pragma unroll
+    for (u32 r = 0; r < SM_ITEMS; ++r) {
+        const u32 i = t + r * SM_TPB;
+        const bool low = ((i & J) == 0) == ((i & K) == 0);  // keeps the smaller
+        a[r] = (a[r] < b[r]) == low ? a[r] : b[r];
+    }
+    if constexpr (J > 1) small_merge<K, J / 2>(a, two, b0, b1);
+}
+template <u32 K>
+__device__ __forceinline__ void small_merges(u64 (&a)[SM_ITEMS], u32 n, u64 *&b0, u64 *&b1) {
+    small_merge<K, K / 2>(a, n > SM_TPB, b0, b1);
+    if constexpr (K < SMALL_MAX_N) {
+        if (K < n || K < 64) small_merges<K * 2>(a, n, b0, b1);
+    }
+}
+
+// Bitonic sort of the n <= SMALL_MAX_N keys of the workgroup, key i in thread
+// i mod SM_TPB (~0 past n), in ascending order: partners less than a wave
+// apart meet by DPP and lane swaps, the others through LDS, one barrier a step
+// (the two buffers take turns).  1000 keys 6.4 us, 256 keys 4.1 us; with every
+// lane exchange through LDS 10.2 and 6.5 us.
+__device__ __forceinline__ void small_sort(u64 (&a)[SM_ITEMS], u32 n, u64 *b0, u64 *b1) {
+    small_merges<2>(a, n, b0, b1);
     __syncthreads();  // the buffers are free
 }
 
-// The workgroup's stores so far become visible device-wide, then one arrival is
-// counted: true in every thread of the workgroup that arrives last of `of`,
-// which then sees the stores of all.  Nothing waits.
+// Counts one arrival, after the workgroup's stores so far have been written
+// (through, by put<true>: a write-back of the L2 for each of 256 workgroups took
+// 18 us): true in every thread of the workgroup that arrives last of `of`, which
+// then sees the stores of all.  Nothing waits.
 __device__ __forceinline__ bool arrive_last(u32 *count, u32 of, SmallLds &S) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        S.last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == of - 1 ? 1u : 0u;
-        __threadfence();
-    }
+    if (threadIdx.x == 0)
+        S.last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == of - 1 ? 1u : 0u;
     __syncthreads();
-    return S.last != 0;
+    if (!S.last) return false;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    return true;
+}
+
+// the density bounds into LDS
+__device__ __forceinline__ void small_density(const Group &g, SmallLds &S) {
+    static_assert(sizeof(Density) % 8 == 0 && sizeof(Density) / 8 <= SM_TPB, "one word a thread");
+    if (threadIdx.x < sizeof(Density) / 8) ((u64 *)&S.dn)[threadIdx.x] = ((const u64 *)&g.tab[0].dn)[threadIdx.x];
 }
 
 // Density check and election of the compacted batch (S.seg, S.pd, n_eff): as
@@ -92,7 +138,7 @@ __device__ __forceinline__ bool arrive_last(u32 *count, u32 of, SmallLds &S) {
 __device__ __forceinline__ void small_settle(const Group &g, const BatchBufs &bb, SmallLds &S, u32 n_eff, u32 flags,
                                              EarlyOut *early) {
     const DevState &d = g.one;
-    const Density &dn = g.tab[0].dn;
+    const Density &dn = S.dn;
     const u64 nseg = nseg_of(d);
     const u64 tag = (u64)g.epoch << 32;
     const u32 t = threadIdx.x;
@@ -123,7 +169,7 @@ __device__ __forceinline__ void small_settle(const Group &g, const BatchBufs &bb
             const u64 w = (u64)s >> l;
             const u64 a = w << l, e = a + (1ull << l);
             const u32 guess = max(1u, u1[r] - u0[r]);
-            const u32 C = *count_ptr(d, l, w);
+            const u32 C = l == 0 ? S.c0[j] : *count_ptr(d, l, w);
             u0[r] = gallop_back(S.seg, u0[r], (u32)a, guess);
             u1[r] = e < nseg ? gallop_fwd(S.seg, u1[r], n_eff, (u32)e, guess) : n_eff;
             const i64 m = (i64)C + (i64)(S.pd[u1[r]] - S.pd[u0[r]]);
@@ -147,7 +193,7 @@ __device__ __forceinline__ void small_settle(const Group &g, const BatchBufs &bb
         if (f) atomicOr(&S.flags, f);
         if (mk) atomicOr(&S.mask, mk);
     }
-    __threadfence();  // the claims, before they are read
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the claims, before they are read
     __syncthreads();
     flags = S.flags;
     const u32 mask = S.mask;
@@ -213,23 +259,32 @@ __global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineS
     if (blockIdx.x > 0) {
         const u32 np = gridDim.x - 1;
         for (u32 c = blockIdx.x - 1; c < chunks; c += np) {
-            pyr_chunk(d, c, S.v0, S.v1);
+            pyr_chunk<true>(d, c, S.v0, S.v1);
             __syncthreads();
         }
         if (np > 1 && !arrive_last(&arrive[0], np, S)) return;
-        pyr_top_levels(d, S.top);
+        pyr_top_levels<true>(d, S.top);
         if (!arrive_last(&arrive[1], 2, S)) return;
         // the batch arrived first: its compacted updates from memory
         n_eff = bb.status->n_eff;
         flags = bb.status->flags;
         for (u32 j = t; j < n_eff; j += SM_TPB) S.seg[j] = (u32)bb.cseg[j];
         for (u32 j = t; j <= n_eff; j += SM_TPB) S.pd[j] = bb.pd[j];
+        for (u32 j = t; j < n_eff; j += SM_TPB) S.c0[j] = d.cnt[S.seg[j]];  // (its own entries)
+        small_density(g, S);
         __syncthreads();
     } else {
-        // keys and staged separators: one round of loads
+        // keys and staged separators: one round of loads (the separators are
+        // wanted after the sort)
         if (t < in.n) S.segs[t] = in.s[t];
+        constexpr u32 TPT = (1u << SM_TAB_LOG) / SM_TPB;
         const u32 tl = min(d.H, SM_TAB_LOG), sh = d.H - tl;
-        const u64 sepv = t < (1u << tl) ? d.sep[(u64)t << sh] : 0ull;
+        u64 sepv[TPT];
+#pragma unroll
+        for (u32 k = 0; k < TPT; ++k) {
+            const u32 i = t + k * SM_TPB;
+            sepv[k] = d.sep[(u64)(i < (1u << tl) ? i : 0u) << sh];
+        }
         __syncthreads();
         bool bad = false;
         u64 p[SM_ITEMS];
@@ -239,20 +294,24 @@ __global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineS
             p[r] = ~0ull;
             if (i < n) p[r] = pack_element(S.segs[source_of(S.segs, in.n, i)], i, g.pshift, g.sbits, bad);
         }
-        if (t < (1u << tl)) S.tab[t] = sepv;
-        u32 M = 64;
-        while (M < n) M <<= 1;
+        small_density(g, S);
         const bool anybad = __syncthreads_or(bad);
         flags = anybad ? FLAG_INVALID_KEY : 0u;
-        small_sort(p, M, S.ex, S.sp);
+        small_sort(p, n, S.ex, S.sp);
 #pragma unroll
         for (u32 r = 0; r < SM_ITEMS; ++r)
-            if (t + r * SM_TPB < M) S.sp[t + r * SM_TPB] = p[r];
+            if (t + r * SM_TPB < n) S.sp[t + r * SM_TPB] = p[r];
+#pragma unroll
+        for (u32 k = 0; k < TPT; ++k) S.tab[t + k * SM_TPB] = sepv[k];
         __syncthreads();
-        // dedup (the last of equal keys), locate, presence: both items together
+        // dedup (the last of equal keys), locate, presence, as the staged edge
+        // queries search: staged separators, probes down to a line, the line
+        // read by the row of lanes (one compute unit's gathers bound this: 64
+        // clocks a wave and probe)
         const u32 ks = 1 + g.sbits;
+        const u32 sw = min(16u, 1u << sh), SS = 1u << d.log2S, kw = min(16u, SS);
         u64 key[SM_ITEMS];
-        u32 seg[SM_ITEMS], at[SM_ITEMS];
+        u32 seg[SM_ITEMS], c0[SM_ITEMS], there[SM_ITEMS];
         bool ok[SM_ITEMS];
 #pragma unroll
         for (u32 r = 0; r < SM_ITEMS; ++r) {
@@ -260,50 +319,36 @@ __global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineS
             ok[r] = i < n && !(i + 1 < n && (S.sp[i + 1] >> ks) == (p[r] >> ks));
             const u64 kk = (p[r] & ((1ull << g.pshift) - 1)) >> ks;
             key[r] = ok[r] ? ((kk >> d.vbits) << 32) | (kk & ((1ull << d.vbits) - 1)) : 0ull;
-            seg[r] = 0;
-            for (u32 h = (1u << tl) >> 1; h; h >>= 1) seg[r] += S.tab[seg[r] + h] <= key[r] ? h : 0u;
-            seg[r] <<= sh;
-        }
-        u32 q = 1u << sh;
-        for (; q >= 4; q >>= 2) {
-            const u32 e = q >> 2;
-            u64 x[SM_ITEMS], y[SM_ITEMS], z[SM_ITEMS];
-#pragma unroll
-            for (u32 r = 0; r < SM_ITEMS; ++r) {
-                x[r] = d.sep[seg[r] + e];
-                y[r] = d.sep[seg[r] + 2 * e];
-                z[r] = d.sep[seg[r] + 3 * e];
+            seg[r] = c0[r] = there[r] = 0;
+            if ((t & ~63u) + r * SM_TPB >= n) continue;  // whole waves
+            u32 at = 0;
+            for (u32 h = (1u << tl) >> 1; h; h >>= 1) at += S.tab[at + h] <= key[r] ? h : 0u;
+            at <<= sh;
+            for (u32 h = (1u << sh) >> 1; h >= 16; h >>= 1) at += d.sep[at + h] <= key[r] ? h : 0u;
+            u64 v[8], w[8];
+            if (sh) {
+                u32 c = 0;
+                row_lines<0>(d.sep, at, sw, v);
+                row_lines<8>(d.sep, at, sw, w);
+                row_counts<0, true>(v, key[r], c);
+                row_counts<8, true>(w, key[r], c);
+                at += min(c, sw) - 1;
             }
-#pragma unroll
-            for (u32 r = 0; r < SM_ITEMS; ++r)
-                seg[r] += (x[r] <= key[r] ? e : 0u) + (y[r] <= key[r] ? e : 0u) + (z[r] <= key[r] ? e : 0u);
+            seg[r] = at;
+            c0[r] = d.cnt[at];
+            u64 base = (u64)at << d.log2S;
+            for (u32 h = SS >> 1; h >= 16; h >>= 1) base += d.keys[base + h - 1] < key[r] ? h : 0u;
+            row_lines<0>(d.keys, base, kw, v);
+            row_lines<8>(d.keys, base, kw, w);
+            row_counts<0, false>(v, key[r], there[r]);
+            row_counts<8, false>(w, key[r], there[r]);
         }
-        if (q == 2) {
-#pragma unroll
-            for (u32 r = 0; r < SM_ITEMS; ++r) seg[r] += d.sep[seg[r] + 1] <= key[r] ? 1u : 0u;
-        }
-        const u64 *base[SM_ITEMS];
-#pragma unroll
-        for (u32 r = 0; r < SM_ITEMS; ++r) {
-            base[r] = d.keys + ((u64)seg[r] << d.log2S);
-            at[r] = 0;
-        }
-        for (u32 h = 1u << (d.log2S - 1); h; h >>= 1) {
-            u64 v[SM_ITEMS];
-#pragma unroll
-            for (u32 r = 0; r < SM_ITEMS; ++r) v[r] = base[r][at[r] + h - 1];
-#pragma unroll
-            for (u32 r = 0; r < SM_ITEMS; ++r) at[r] += v[r] < key[r] ? h : 0u;
-        }
-        u64 got[SM_ITEMS];
-#pragma unroll
-        for (u32 r = 0; r < SM_ITEMS; ++r) got[r] = base[r][at[r]];
         // compaction: (count, inserts) as the halves of one word
         u32 own[SM_ITEMS], inc[SM_ITEMS];
 #pragma unroll
         for (u32 r = 0; r < SM_ITEMS; ++r) {
             const u32 op = (u32)(p[r] & 1);
-            own[r] = ok[r] && op != (got[r] == key[r] ? 1u : 0u) ? 1u | op << 16 : 0u;
+            own[r] = ok[r] && op != there[r] ? 1u | op << 16 : 0u;
             inc[r] = dpp_incl_scan32(own[r]);
             if (lane_id() == 63) S.wt[r][wv] = inc[r];
         }
@@ -323,18 +368,19 @@ __global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineS
                 const i32 x = 2 * (i32)(pre >> 16) - (i32)j;
                 S.seg[j] = seg[r];
                 S.pd[j] = x;
+                S.c0[j] = c0[r];
                 bb.ckey[j] = key[r];
-                bb.cseg[j] = seg[r];
-                bb.pd[j] = x;
+                put<true>(&bb.cseg[j], (u64)seg[r]);
+                put<true>(&bb.pd[j], x);
             }
         }
         n_eff = before & 0xFFFFu;
         if (t == 0) {
             const i32 x = 2 * (i32)(before >> 16) - (i32)n_eff;
             S.pd[n_eff] = x;
-            bb.pd[n_eff] = x;
-            bb.status->n_eff = n_eff;
-            bb.status->flags = flags;
+            put<true>(&bb.pd[n_eff], x);
+            put<true>(&bb.status->n_eff, n_eff);
+            put<true>(&bb.status->flags, flags);
         }
         if (!arrive_last(&arrive[1], 2, S)) return;
     }

@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "begin.hpp"
 
 namespace pma {
 
@@ -121,40 +122,6 @@ __global__ __launch_bounds__(256) void k_edge_query(DevState d, const u64 *__res
 static constexpr u32 EQ_TAB_LOG = 12;
 static constexpr u32 EQ_TPB = 1024;
 static constexpr u32 EQ_GRID = 512;  // two workgroups a CU
-
-// lane J of every row of 16 lanes, in all lanes of the row
-template <int J>
-__device__ __forceinline__ u32 row_lane(u32 x) {
-    return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + J, 0xF, 0xF, false);  // row_newbcast
-}
-template <int J>
-__device__ __forceinline__ u64 row_lane(u64 x) {
-    return ((u64)row_lane<J>((u32)(x >> 32)) << 32) | row_lane<J>((u32)x);
-}
-
-// a[at .. at + w) of the row's queries J0 .. J0 + 7 (w <= 16): every lane loads
-// one word of each, KEY_NONE past w
-template <int J0>
-__device__ __forceinline__ void row_lines(const u64 *a, u64 at, u32 w, u64 (&v)[8]) {
-    const u32 gl = lane_id() & 15;
-#define LPMA_LINE(K)                                                  \
-    {                                                                 \
-        const u64 x = row_lane<J0 + K>(at); /* by every lane */       \
-        v[K] = gl < w ? a[x + gl] : KEY_NONE;                         \
-    }
-    LPMA_LINE(0) LPMA_LINE(1) LPMA_LINE(2) LPMA_LINE(3) LPMA_LINE(4) LPMA_LINE(5) LPMA_LINE(6) LPMA_LINE(7)
-#undef LPMA_LINE
-}
-
-// bit J0 + K of the row's answers: how many of the words are <= (LE) or equal
-// to query J0 + K's key
-template <int J0, bool LE>
-__device__ __forceinline__ void row_counts(const u64 (&v)[8], u64 key, u32 &mine) {
-    const u32 gl = lane_id() & 15, sh = lane_id() & 48;
-#define LPMA_COUNT(K)                                                                                    {                                                                                                        const u64 k = row_lane<J0 + K>(key);                                                                 const u32 c = (u32)__popc((u32)(__ballot(LE ? v[K] <= k : v[K] == k) >> sh) & 0xFFFFu);             if (gl == J0 + K) mine = c;                                                                      }
-    LPMA_COUNT(0) LPMA_COUNT(1) LPMA_COUNT(2) LPMA_COUNT(3) LPMA_COUNT(4) LPMA_COUNT(5) LPMA_COUNT(6) LPMA_COUNT(7)
-#undef LPMA_COUNT
-}
 
 __global__ __launch_bounds__(EQ_TPB) void k_edge_query_staged(DevState d, const u64 *__restrict__ q, u64 n,
                                                                u32 *__restrict__ res) {
