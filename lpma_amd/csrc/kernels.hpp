@@ -9,7 +9,7 @@ u64 scan_scratch_words(u64 n);
 hipError_t device_excl_scan(const u32 *in, u64 n, u32 *out, u32 *scratch, hipStream_t st);
 u64 sort_scratch_words(u64 n);
 u32 sort_zero_words();
-// k0, k1, k2: n keys each (k2 only for batches of up to 2^17 keys, as the
+// k0, k1, k2: n keys each (k2 only for batches of up to 2^19 keys, as the
 // second buffer of an oversized bucket)
 u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32 pshift, u32 sbits, u32 lo_bit,
                    u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 *flags, hipStream_t st);
@@ -39,7 +39,7 @@ struct InlineSegs {
     u32 n;
 };
 
-// sort.hip: a lone PMA's batch of at most 2^17 keys from inline sources is
+// sort.hip: a lone PMA's batch of at most 2^19 keys from inline sources is
 // sorted with the batch's first work (batch_begin's, without clearing the
 // sort scratch) carried by the sort kernels: no batch_begin launch, and the
 // pyramid's pyr_chunks chunk levels owed by the last batch summed there too

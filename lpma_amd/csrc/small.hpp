@@ -42,73 +42,6 @@ struct SmallLds {
     BatchSeg segs[INLINE_SEGS];
 };
 
-// lane ^ J's value
-template <u32 J>
-__device__ __forceinline__ u32 lane_xor(u32 x) {
-    if constexpr (J == 1) return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
-    if constexpr (J == 2) return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false);  // quad_perm 2,3,0,1
-    if constexpr (J == 4) {  // xor 7 (row_half_mirror), then xor 3 (quad_perm 3,2,1,0)
-        const int m = __builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, false);
-        return (u32)__builtin_amdgcn_update_dpp(0, m, 0x1B, 0xF, 0xF, false);
-    }
-    if constexpr (J == 8) return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror:8
-    if constexpr (J == 16) {  // odd rows of the one against even rows of the other
-        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-        return lane_id() & 16 ? r[0] : r[1];
-    }
-    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    return lane_id() & 32 ? r[0] : r[1];
-}
-template <u32 J>
-__device__ __forceinline__ u64 lane_xor(u64 x) {
-    return ((u64)lane_xor<J>((u32)(x >> 32)) << 32) | lane_xor<J>((u32)x);
-}
-
-// steps J, J / 2, ..., 1 of a bitonic merge of runs of K / 2
-template <u32 K, u32 J>
-__device__ __forceinline__ void small_merge(u64 (&a)[SM_ITEMS], bool two, u64 *&b0, u64 *&b1) {
-    const u32 t = threadIdx.x;
-    u64 b[SM_ITEMS];
-    if constexpr (J >= SM_TPB) {
-        b[0] = a[1];
-        b[1] = a[0];
-    } else if constexpr (J >= 64) {
-        b0[t] = a[0];
-        if (two) b0[t + SM_TPB] = a[1];
-        __syncthreads();
-        b[0] = b0[t ^ J];
-        b[1] = two ? b0[(t ^ J) + SM_TPB] : 0ull;
-        u64 *x = b0; b0 = b1; b1 = x;
-    } else {
-        b[0] = lane_xor<J>(a[0]);
-        b[1] = two ? lane_xor<J>(a[1]) : 0ull;
-    }
-#pragma unroll
-    for (u32 r = 0; r < SM_ITEMS; ++r) {
-        const u32 i = t + r * SM_TPB;
-        const bool low = ((i & J) == 0) == ((i & K) == 0);  // keeps the smaller
-        a[r] = (a[r] < b[r]) == low ? a[r] : b[r];
-    }
-    if constexpr (J > 1) small_merge<K, J / 2>(a, two, b0, b1);
-}
-template <u32 K>
-__device__ __forceinline__ void small_merges(u64 (&a)[SM_ITEMS], u32 n, u64 *&b0, u64 *&b1) {
-    small_merge<K, K / 2>(a, n > SM_TPB, b0, b1);
-    if constexpr (K < SMALL_MAX_N) {
-        if (K < n || K < 64) small_merges<K * 2>(a, n, b0, b1);
-    }
-}
-
-// Bitonic sort of the n <= SMALL_MAX_N keys of the workgroup, key i in thread
-// i mod SM_TPB (~0 past n), in ascending order: partners less than a wave
-// apart meet by DPP and lane swaps, the others through LDS, one barrier a step
-// (the two buffers take turns).  1000 keys 6.4 us, 256 keys 4.1 us; with every
-// lane exchange through LDS 10.2 and 6.5 us.
-__device__ __forceinline__ void small_sort(u64 (&a)[SM_ITEMS], u32 n, u64 *b0, u64 *b1) {
-    small_merges<2>(a, n, b0, b1);
-    __syncthreads();  // the buffers are free
-}
-
 // Counts one arrival, after the workgroup's stores so far have been written
 // (through, by put<true>: a write-back of the L2 for each of 256 workgroups took
 // 18 us): true in every thread of the workgroup that arrives last of `of`, which
@@ -297,7 +230,7 @@ __global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineS
         small_density(g, S);
         const bool anybad = __syncthreads_or(bad);
         flags = anybad ? FLAG_INVALID_KEY : 0u;
-        small_sort(p, n, S.ex, S.sp);
+        block_bitonic<u64, SM_TPB, SM_ITEMS>(p, n, S.ex, S.sp);
 #pragma unroll
         for (u32 r = 0; r < SM_ITEMS; ++r)
             if (t + r * SM_TPB < n) S.sp[t + r * SM_TPB] = p[r];

@@ -8,8 +8,8 @@
 // merged sequence, so equal keys end up ordered delete before insert, earlier
 // request before later; the dedup that follows keeps the last of each run.
 // Three paths by batch size:
-//   <= 2^17 keys   sample-split sort: two kernels, buckets chosen from a
-//                  sample, each sorted in LDS on the bits that vary in it;
+//   <= 2^19 keys   sample-split sort: two kernels, buckets chosen from a
+//                  sample, each sorted by a bitonic network;
 //   <= 2^22 keys   LSD radix, one kernel per 10/11-bit digit (decoupled
 //                  look-back), the digit counts of every pass taken at pack;
 //   larger         LSD radix, 8-bit digits, histogram + scan + scatter.
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(RS_TPB) void k_rs_scatter(const u64 *__restrict__ i
 
 // ------------------------------------------------- one kernel per pass
 //
-// Batches of 8K..4M keys sort with DB = 10 or 11-bit digits (four passes
+// Batches of 512K..4M keys sort with DB = 10 or 11-bit digits (four passes
 // for the 40-41 bits of a lone PMA with 2^20 vertices), one kernel each,
 // over tiles of 4096 keys (1024 threads, 4 keys each): few enough tiles that
 // a tile finds the counts of all tiles before it in few look-back steps,
@@ -383,30 +383,36 @@ __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, 
 //
 // Batches of up to SS_MAX_N keys sort in two kernels, whatever their key
 // width.  k_ss_split: every workgroup draws the same regular sample of the
-// batch (SS_SAMPLE packed keys), sorts it in LDS by counting, and takes its
-// quantiles as the splitters of nb buckets (rounded down to a key boundary,
-// so that equal keys of any request order and operation share a bucket);
-// then it packs its tile of SS_TILE keys, assigns each to its bucket, and
-// writes the tile back grouped by bucket (tile-major: no global offsets are
-// needed), with its per-bucket counts.  k_ss_bucket: one workgroup per
-// bucket gathers the bucket's keys from every tile into registers, finds
-// the bits on which they differ (AND / OR over the bucket), sorts them by
-// LSD radix passes of 8 bits over those bits only, ranked in LDS (wave64
-// "match any" ballots, per-wave digit counts joined by a DPP scan), and
-// writes them at the bucket's offset.  A sample-chosen split keeps buckets
-// even under R-MAT skew, where a split on the top key bits puts a hub's keys
-// in one bucket.  A bucket beyond the workgroup's SB_CAP keys (many equal
-// keys) is LSD-radix-sorted through global memory, chunk by chunk, on the
-// bits on which its keys differ (AND / OR of the keys), with wave64 ranking
-// (the k_os_pass scheme).
+// batch (SS_OVER packed keys a bucket), sorts it (bitonic, on 32-bit
+// projections), and takes its quantiles as the splitters of nb buckets
+// (rounded down to a key boundary, so that equal keys of any request order and
+// operation share a bucket); then it packs its tile, assigns each key to its
+// bucket, and writes the tile back grouped by bucket (tile-major: no global
+// offsets are needed), with its per-bucket counts and offsets.  k_ss_bucket:
+// one workgroup per bucket gathers the bucket's keys from every tile into
+// registers, sorts them by a bitonic network (lane swaps within a wave, LDS
+// between waves), and writes them at the bucket's offset.  A sample-chosen
+// split keeps buckets even under R-MAT skew, where a split on the top key bits
+// puts a hub's keys in one bucket.  A bucket beyond the workgroup's SB_CAP keys
+// (many equal keys) is LSD-radix-sorted through global memory, chunk by chunk,
+// on the bits on which its keys differ (AND / OR of the keys), with wave64
+// ranking (the k_os_pass scheme).
+//
+// Bound: the sample's sort in every tile (vector issue: 1024 samples 5 us, 2048
+// 10 us with one tile a compute unit) and the largest bucket.  10^5 R-MAT keys:
+// 13 us + 12 us with 512 buckets of 2 samples each; 256 buckets of 4: 10.6 +
+// 15; of 8: 16 + 10; of 128 buckets, ranked by counting 256 samples, and 8-bit
+// radix passes in LDS (an earlier form): 10.5 + 26.  3.2*10^5 keys: 22 + 26,
+// against 14 + 5 * 15 in the one-kernel passes below.
 
-static constexpr int SS_TPB = 256;
-static constexpr int SS_ITEMS = 4;
-static constexpr u32 SS_TILE = SS_TPB * SS_ITEMS;  // keys per tile
-static constexpr u32 SS_SAMPLE = SS_TPB;            // sample keys (one per thread)
-static constexpr u32 SS_MAX_BUCKETS = 128;
-static constexpr u64 SS_MAX_N = 1ull << 17;
-static constexpr u32 SS_MAX_TILES = (u32)(SS_MAX_N / SS_TILE);
+static constexpr int SS_TPB = 1024;
+static constexpr u32 SS_MAX_TILES = 256;  // a tile a compute unit: every tile sorts the sample
+static constexpr u32 SS_MAX_BUCKETS = 1024;
+static constexpr u32 SS_LSEGS = 128;                 // sources staged in LDS
+static constexpr u32 SS_OVER = 2;                   // sample keys per bucket
+static constexpr u32 SS_MAX_SAMPLE = SS_MAX_BUCKETS * SS_OVER;
+static constexpr int SS_SITEMS = (int)((SS_MAX_SAMPLE + SS_TPB - 1) / SS_TPB);
+static constexpr u64 SS_MAX_N = 1ull << 19;
 static constexpr int SB_TPB = 1024;                 // bucket sort workgroup
 static constexpr int SB_ITEMS = 4;
 static constexpr u32 SB_CAP = SB_TPB * SB_ITEMS;    // keys sorted in LDS
@@ -414,12 +420,18 @@ static constexpr u32 SB_NW = SB_TPB / 64;
 // a tile's count entry: offset << 16 | count, bit 31 on bucket 0's entry
 // when the tile met an invalid key
 static constexpr u32 SS_BAD = 1u << 31;
-static_assert(SS_TILE <= (1u << 15), "a tile's offsets and counts stay below the bad-key bit");
+// keys a thread: 1 up to 2^18 keys, 2 above
+static int ss_items(u64 n) { return n <= (u64)SS_MAX_TILES * SS_TPB ? 1 : 2; }
+static u32 ss_tiles(u64 n) { return (u32)((n + ss_items(n) * SS_TPB - 1) / (ss_items(n) * SS_TPB)); }
+static_assert(SS_MAX_N <= 2ull * SS_MAX_TILES * SS_TPB && 2 * SS_TPB <= (1 << 15),
+              "the tiles hold a batch, and their offsets and counts stay below the bad-key bit");
 
-// buckets of a batch of n keys: about a thousand keys each, a power of two
+// buckets of a batch of n keys, a power of two: of at most 256 keys on average
+// up to 2^18 keys, so that the largest of R-MAT keys (about four times the
+// average) still sorts with one key a thread
 static u32 ss_buckets(u64 n) {
     u32 nb = 1;
-    while (nb < SS_MAX_BUCKETS && (u64)nb * SS_TILE < n) nb <<= 1;
+    while (nb < SS_MAX_BUCKETS && (u64)nb * 256 < n) nb <<= 1;
     return nb;
 }
 
@@ -434,20 +446,21 @@ static u32 ss_buckets(u64 n) {
 // bucket kernel); the sources come from the kernel arguments.  A tile that
 // met an invalid key marks its count of bucket 0 (bit 31): the bucket
 // kernel raises the flag, after the status is cleared.
-template <bool FIRST>
+template <bool FIRST, int ITEMS>
 __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict__ segs, u32 nsegs, u64 n,
                                                       const u64 *n_dev, u32 pshift, u32 sbits, u32 psh, u32 nb,
                                                       u64 *__restrict__ tmp, u32 *__restrict__ bc, InlineSegs in,
                                                       Group g, Status *status, u32 *wfirst) {
-    __shared__ u64 smp[SS_SAMPLE];  // projection << 32 | sample index: distinct
+    constexpr u32 TILE = SS_TPB * ITEMS;
+    __shared__ u32 smp[2][SS_MAX_SAMPLE];
     __shared__ u32 spl[SS_MAX_BUCKETS];
     __shared__ u32 cnt[SS_MAX_BUCKETS];
     __shared__ u32 base[SS_MAX_BUCKETS];
-    __shared__ BatchSeg lsegs[INLINE_SEGS];
+    __shared__ BatchSeg lsegs[FIRST ? INLINE_SEGS : SS_LSEGS];
     __shared__ u32 pyr_v0[FIRST ? PYR_CH : 1], pyr_v1[FIRST ? PYR_CH / 2 : 1];
     if (n_dev) n = *n_dev;
     const u32 t = blockIdx.x;
-    const u32 ntiles = (u32)((n + SS_TILE - 1) / SS_TILE);
+    const u32 ntiles = (u32)((n + TILE - 1) / TILE);
     const u32 tid = threadIdx.x;
     if (FIRST) {
         if (t >= ntiles) {
@@ -462,19 +475,26 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
         segs = lsegs;
     }
     if (t >= ntiles) return;  // whole workgroup: grids sized for a capacity
+    if (!FIRST && nsegs <= SS_LSEGS) {
+        // the sources in LDS: a key's is found by a search over them
+        constexpr u32 W = sizeof(BatchSeg) / 8;
+        for (u32 i = tid; i < nsegs * W; i += SS_TPB) ((u64 *)lsegs)[i] = ((const u64 *)segs)[i];
+        __syncthreads();
+        segs = lsegs;
+    }
 
     // the tile's keys and the sample key are loaded first, all in flight
     // while the sample is ranked
     bool bad = false;
-    const u64 tbase = (u64)t * SS_TILE;
-    u64 key[SS_ITEMS];
-    bool valid[SS_ITEMS];
+    const u64 tbase = (u64)t * TILE;
+    u64 key[ITEMS];
+    bool valid[ITEMS];
     {
         const u64 i0 = tbase + tid;
         u32 s = source_of(segs, nsegs, i0 < n ? i0 : n - 1);
         BatchSeg sg = segs[s];
 #pragma unroll
-        for (int r = 0; r < SS_ITEMS; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const u64 i = i0 + (u64)r * SS_TPB;
             valid[r] = i < n;
             key[r] = 0;
@@ -484,35 +504,32 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
             }
         }
     }
-    {
-        const u64 p = ((2ull * tid + 1) * n) / (2ull * SS_SAMPLE);
-        bool ignore = false;
-        const u64 x = pack_element(segs[source_of(segs, nsegs, p)], p, pshift, sbits, ignore);
-        smp[tid] = ((u64)(u32)(x >> psh) << 32) | tid;
+    // the sample's projections, sorted; its quantiles are the splitters
+    const u32 ns = nb * SS_OVER;
+    u32 sm[SS_SITEMS];
+#pragma unroll
+    for (int r = 0; r < SS_SITEMS; ++r) {
+        const u32 i = tid + r * SS_TPB;
+        sm[r] = ~0u;
+        if (i < ns) {
+            const u64 p = ((2ull * i + 1) * n) / (2ull * ns);
+            bool ignore = false;
+            sm[r] = (u32)(pack_element(segs[source_of(segs, nsegs, p)], p, pshift, sbits, ignore) >> psh);
+        }
     }
     if (tid < SS_MAX_BUCKETS) cnt[tid] = 0;
-    __syncthreads();
-    // rank of each (distinct) sample entry by counting, two entries per LDS read
-    {
-        const u64 x = smp[tid];
-        const ulonglong2 *s2 = (const ulonglong2 *)smp;
-        u32 r = 0;
-#pragma unroll 16
-        for (u32 q = 0; q < SS_SAMPLE / 2; ++q) {
-            const ulonglong2 y = s2[q];
-            r += (y.x < x ? 1u : 0u) + (y.y < x ? 1u : 0u);
-        }
-        __syncthreads();
-        smp[r] = x;
+    block_bitonic<u32, SS_TPB, SS_SITEMS>(sm, ns, smp[0], smp[1]);
+#pragma unroll
+    for (int r = 0; r < SS_SITEMS; ++r) {
+        const u32 i = tid + r * SS_TPB;
+        if (i < ns && i > 0 && i % SS_OVER == 0) spl[i / SS_OVER - 1] = sm[r];
     }
-    __syncthreads();
-    if (tid + 1 < nb) spl[tid] = (u32)(smp[(tid + 1) * (SS_SAMPLE / nb)] >> 32);
     __syncthreads();
 
     // bucket = number of splitters <= the key's projection
-    u32 bk[SS_ITEMS], loc[SS_ITEMS];
+    u32 bk[ITEMS], loc[ITEMS];
 #pragma unroll
-    for (int r = 0; r < SS_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const u32 x = (u32)(key[r] >> psh);
         u32 lo = 0, hi = nb - 1;
         while (lo < hi) {
@@ -524,16 +541,26 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
     }
     const bool tbad = __syncthreads_or(bad);
     if (tid < 64) {
-        // exclusive scan of the bucket counts (nb <= 128: two per lane)
-        const u32 c0 = 2 * tid < nb ? cnt[2 * tid] : 0u, c1 = 2 * tid + 1 < nb ? cnt[2 * tid + 1] : 0u;
-        const u32 ex = wave_incl_scan(c0 + c1) - (c0 + c1);
-        if (2 * tid < nb) base[2 * tid] = ex;
-        if (2 * tid + 1 < nb) base[2 * tid + 1] = ex + c0;
+        // exclusive scan of the bucket counts, four a lane
+        constexpr u32 PER = SS_MAX_BUCKETS / 64;
+        u32 c[PER], sum = 0;
+#pragma unroll
+        for (u32 k = 0; k < PER; ++k) {
+            c[k] = PER * tid + k < nb ? cnt[PER * tid + k] : 0u;
+            sum += c[k];
+        }
+        u32 ex = wave_incl_scan(sum) - sum;
+#pragma unroll
+        for (u32 k = 0; k < PER; ++k) {
+            if (PER * tid + k < nb) base[PER * tid + k] = ex;
+            ex += c[k];
+        }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < SS_ITEMS; ++r)
+    for (int r = 0; r < ITEMS; ++r)
         if (valid[r]) tmp[tbase + base[bk[r]] + loc[r]] = key[r];
+    static_assert(SS_MAX_BUCKETS <= (u32)SS_TPB, "one bucket a thread");
     if (tid < nb) bc[(u64)tid * ntiles + t] = (base[tid] << 16) | cnt[tid] | (tid == 0 && tbad ? SS_BAD : 0u);
 }
 
@@ -603,62 +630,63 @@ __device__ __forceinline__ void sb_rank(const u64 (&x)[SB_ITEMS], u32 m, u32 R, 
 // top: one more workgroup, past the buckets, sums the lone PMA's pyramid
 // top levels (after the split kernel's chunk levels)
 __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tmp, u64 *__restrict__ out,
-                                                       u64 *__restrict__ aux, u64 n, const u64 *n_dev, u32 nb,
+                                                       u64 *__restrict__ aux, u64 n, const u64 *n_dev, u32 tile, u32 nb,
                                                        const u32 *__restrict__ bc, u32 *__restrict__ flags,
                                                        bool top, DevState topd) {
-    __shared__ u64 kb[1][SB_CAP];  // (also the pyramid's top levels)
-    static_assert(sizeof(kb) >= 2 * PYR_TOP_LDS * sizeof(u32), "room for the top levels");
-    __shared__ u32 whist[SB_NW][256];
-    __shared__ u32 dofs[256];
-    __shared__ u32 run[256];
+    // the bucket's sort, or an oversized bucket's radix passes, or the
+    // pyramid's top levels
+    __shared__ union {
+        u64 kb[2][SB_CAP];
+        struct {
+            u32 whist[SB_NW][256], dofs[256], run[256];
+        };
+        u32 pyr[2 * PYR_TOP_LDS];
+    } L;
     __shared__ u32 toff[SS_MAX_TILES + 1], tb[SS_MAX_TILES];
     __shared__ u32 stmp[SB_NW + 1];
     __shared__ u64 red[2][SB_NW];
-    (void)kb;
+    u32(*const whist)[256] = L.whist;
+    u32 *const dofs = L.dofs, *const run = L.run;
     if (n_dev) n = *n_dev;
     const u32 b = blockIdx.x;
     const u32 tid = threadIdx.x;
-    const u32 ntiles = (u32)((n + SS_TILE - 1) / SS_TILE);
+    const u32 ntiles = (u32)((n + tile - 1) / tile);
     if (top && b == nb) {
-        pyr_top_levels(topd, (u32 *)kb);
+        pyr_top_levels(topd, L.pyr);
         return;
     }
     if (b >= nb || ntiles == 0) return;
-    // the bucket's offset: the keys of the buckets before it, whose
-    // per-tile counts are the first b rows of bc
-    u64 obase;
-    {
-        // at most SS_MAX_BUCKETS * SS_MAX_TILES / SB_TPB = 16 words a thread,
-        // all loads in flight at once
-        constexpr u32 PER = SS_MAX_BUCKETS * SS_MAX_TILES / SB_TPB;
-        const u32 lim = b * ntiles;
-        u32 part[PER];
-#pragma unroll
-        for (u32 q = 0; q < PER; ++q) {
-            const u32 i = q * SB_TPB + tid;
-            part[q] = i < lim ? bc[i] & 0xFFFFu : 0u;
+    // where the bucket lies in each tile and inside the bucket; its offset in
+    // the batch is the sum of its offsets in the tiles (a tile's keys of the
+    // buckets before it)
+    constexpr u32 TW = SS_MAX_TILES / 64;  // waves that hold the tiles' entries
+    static_assert(SS_MAX_TILES % 64 == 0 && SS_MAX_TILES <= SB_TPB, "one entry a thread");
+    __shared__ u32 sums[2][TW];
+    u32 e = 0, inc = 0;
+    if (tid < SS_MAX_TILES) {
+        e = tid < ntiles ? bc[(u64)b * ntiles + tid] : 0u;
+        inc = dpp_incl_scan32(e & 0xFFFFu);
+        const u32 off = wave_sum((e & ~SS_BAD) >> 16);
+        if (lane_id() == 63) {
+            sums[0][tid >> 6] = inc;
+            sums[1][tid >> 6] = off;
         }
-        u32 sum = 0;
+    }
+    __syncthreads();
+    if (b == 0 && (e & SS_BAD)) atomicOr(flags, FLAG_INVALID_KEY);
+    u32 m = 0, pre = 0;
+    u64 obase = 0;
 #pragma unroll
-        for (u32 q = 0; q < PER; ++q) sum += part[q];
-        u32 tot;
-        (void)block_excl_scan<SB_TPB, u32>(sum, tot, stmp);
-        obase = tot;
+    for (u32 w = 0; w < TW; ++w) {
+        if (w < tid >> 6) pre += sums[0][w];
+        m += sums[0][w];
+        obase += sums[1][w];
     }
-    // where the bucket lies in each tile: offsets inside the bucket
-    u32 m;
-    {
-        const u32 e = tid < ntiles ? bc[(u64)b * ntiles + tid] : 0u;
-        if (b == 0 && __syncthreads_or((e & SS_BAD) != 0u) && tid == 0) atomicOr(flags, FLAG_INVALID_KEY);
-        u32 tot;
-        const u32 ex = block_excl_scan<SB_TPB, u32>(e & 0xFFFFu, tot, stmp);
-        if (tid < ntiles) {
-            toff[tid] = ex;
-            tb[tid] = (e & ~SS_BAD) >> 16;
-        }
-        if (tid == 0) toff[ntiles] = tot;
-        m = tot;
+    if (tid < ntiles) {
+        toff[tid] = inc - (e & 0xFFFFu) + pre;
+        tb[tid] = (e & ~SS_BAD) >> 16;
     }
+    if (tid == 0) toff[ntiles] = m;
     if (m == 0) return;
     __syncthreads();
     const u32 lane = lane_id();
@@ -669,67 +697,26 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
             const u32 mid = (lo + hi) >> 1;
             if (toff[mid] <= j) lo = mid; else hi = mid;
         }
-        return (u64)lo * SS_TILE + tb[lo] + (j - toff[lo]);
+        return (u64)lo * tile + tb[lo] + (j - toff[lo]);
     };
 
     if (m <= SB_CAP) {
-        // gather: element j = sb_index(w, r, lane, R) into x[r] (addresses
-        // first, then the loads), and the bits on which the keys differ
-        const u32 R = sb_rounds(m);
+        // gather (addresses first, then the loads), and a bitonic sort
         u64 x[SB_ITEMS];
-        u32 rk[SB_ITEMS];
         {
             u64 ad[SB_ITEMS];
 #pragma unroll
             for (int r = 0; r < SB_ITEMS; ++r) {
-                const u32 j = r < (int)R ? sb_index(w, r, lane, R) : m;
+                const u32 j = r * SB_TPB + tid;
                 ad[r] = j < m ? addr_of(j) : ~0ull;
             }
 #pragma unroll
-            for (int r = 0; r < SB_ITEMS; ++r) x[r] = ad[r] != ~0ull ? tmp[ad[r]] : 0ull;
+            for (int r = 0; r < SB_ITEMS; ++r) x[r] = ad[r] != ~0ull ? tmp[ad[r]] : ~0ull;
         }
-        u64 andv = ~0ull, orv = 0;
+        block_bitonic<u64, SB_TPB, SB_ITEMS>(x, m, L.kb[0], L.kb[1]);
 #pragma unroll
         for (int r = 0; r < SB_ITEMS; ++r) {
-            const u32 j = r < (int)R ? sb_index(w, r, lane, R) : m;
-            if (j < m) {
-                andv &= x[r];
-                orv |= x[r];
-            }
-        }
-        andv = wave_and64(andv);
-        orv = wave_or64(orv);
-        if (lane == 0) { red[0][w] = andv; red[1][w] = orv; }
-        __syncthreads();
-        andv = ~0ull;
-        orv = 0;
-#pragma unroll
-        for (u32 q = 0; q < SB_NW; ++q) { andv &= red[0][q]; orv |= red[1][q]; }
-        const u64 diff = andv ^ orv;
-        const u32 lo_bit = diff ? (u32)__builtin_ctzll(diff) : 64u;
-        const u32 hi_bit = diff ? 64u - (u32)__builtin_clzll(diff) : 0u;
-        u64 *kbuf = kb[0];
-        for (u32 shift = lo_bit; shift < hi_bit; shift += 8) {
-            sb_rank(x, m, R, shift, whist, dofs, stmp, rk);
-#pragma unroll
-            for (int r = 0; r < SB_ITEMS; ++r) {
-                const u32 j = r < (int)R ? sb_index(w, r, lane, R) : m;
-                if (j < m) {
-                    const u32 dg = (u32)(x[r] >> shift) & 255u;
-                    kbuf[dofs[dg] + whist[w][dg] + rk[r]] = x[r];
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int r = 0; r < SB_ITEMS; ++r) {
-                const u32 j = r < (int)R ? sb_index(w, r, lane, R) : m;
-                if (j < m) x[r] = kbuf[j];
-            }
-            // (the next pass's first barrier keeps kbuf until every thread has read it)
-        }
-#pragma unroll
-        for (int r = 0; r < SB_ITEMS; ++r) {
-            const u32 j = r < (int)R ? sb_index(w, r, lane, R) : m;
+            const u32 j = r * SB_TPB + tid;
             if (j < m) out[obase + j] = x[r];
         }
         return;
@@ -897,7 +884,8 @@ u64 sort_scratch_words(u64 n) {
     u64 two = (u64)RS_RADIX * nb + 1 + scan_scratch_words((u64)RS_RADIX * nb);
     u64 tile = (u64)os_items(n) * OS_TPB;
     u64 one = 2 * ((n + tile - 1) / tile) * 2048;
-    return OS_GH_WORDS + (n <= OS_MAX_N ? std::max(two, one) : two);
+    u64 split = n <= SS_MAX_N ? (u64)ss_buckets(n) * ss_tiles(n) : 0;
+    return OS_GH_WORDS + std::max(n <= OS_MAX_N ? std::max(two, one) : two, split);
 }
 
 u32 sort_zero_words() { return OS_GH_WORDS; }
@@ -939,13 +927,18 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
         // result, k2 the second buffer of oversized buckets; the tiles'
         // bucket counts go to the scratch after its cleared words
         const u32 nb = ss_buckets(n);
-        const u32 ntiles = (u32)((n + SS_TILE - 1) / SS_TILE);
+        const u32 ntiles = ss_tiles(n);
         u32 *bc = scratch + OS_GH_WORDS;
         const u32 ks = 1 + sbits;
         const u32 psh = hi_bit > 32 + ks ? hi_bit - 32 : ks;
-        k_ss_split<false><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
-                                                      InlineSegs{}, Group{}, nullptr, nullptr);
-        k_ss_bucket<<<nb, SB_TPB, 0, st>>>(k1, k0, k2, n, n_dev, nb, bc, flags, false, DevState{});
+        if (ss_items(n) == 1)
+            k_ss_split<false, 1><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
+                                                             InlineSegs{}, Group{}, nullptr, nullptr);
+        else
+            k_ss_split<false, 2><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
+                                                             InlineSegs{}, Group{}, nullptr, nullptr);
+        k_ss_bucket<<<nb, SB_TPB, 0, st>>>(k1, k0, k2, n, n_dev, (u32)ss_items(n) * SS_TPB, nb, bc, flags, false,
+                                           DevState{});
         return k0;
     }
     if (n <= OS_MAX_N) {
@@ -991,13 +984,18 @@ u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const Inli
                          u32 sbits, u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 pyr_chunks,
                          hipStream_t st) {
     const u32 nb = ss_buckets(n);
-    const u32 ntiles = (u32)((n + SS_TILE - 1) / SS_TILE);
+    const u32 ntiles = ss_tiles(n);
     u32 *bc = scratch + OS_GH_WORDS;
     const u32 ks = 1 + sbits;
     const u32 psh = hi_bit > 32 + ks ? hi_bit - 32 : ks;
-    k_ss_split<true><<<ntiles + 1 + pyr_chunks, SS_TPB, 0, st>>>(nullptr, in.n, n, nullptr, pshift, sbits, psh, nb,
-                                                                  k1, bc, in, g, status, wfirst);
-    k_ss_bucket<<<nb + 1, SB_TPB, 0, st>>>(k1, k0, k2, n, nullptr, nb, bc, &status->flags, true, g.one);
+    if (ss_items(n) == 1)
+        k_ss_split<true, 1><<<ntiles + 1 + pyr_chunks, SS_TPB, 0, st>>>(nullptr, in.n, n, nullptr, pshift, sbits, psh,
+                                                                         nb, k1, bc, in, g, status, wfirst);
+    else
+        k_ss_split<true, 2><<<ntiles + 1 + pyr_chunks, SS_TPB, 0, st>>>(nullptr, in.n, n, nullptr, pshift, sbits, psh,
+                                                                         nb, k1, bc, in, g, status, wfirst);
+    k_ss_bucket<<<nb + 1, SB_TPB, 0, st>>>(k1, k0, k2, n, nullptr, (u32)ss_items(n) * SS_TPB, nb, bc, &status->flags,
+                                           true, g.one);
     return k0;
 }
 

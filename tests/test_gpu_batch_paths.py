@@ -163,3 +163,41 @@ def test_small_batch_refused_and_merged():
         # the layout is that of one batch; the edges are those of two
         t.compare(layout=False)
     t.close()
+
+
+# the sample-split sort: bucket counts double at powers of two, a thread takes
+# two keys above 2^18, buckets of equal keys outgrow their workgroup
+@pytest.mark.parametrize("n", [2049, 65537, 131073, 262144, 262145, 400003])
+@pytest.mark.parametrize("V,equal", [(1 << 14, 0.0), (1 << 14, 0.5), (40, 0.0)])
+def test_sample_split_sort(n, V, equal):
+    rng = np.random.default_rng(n)
+    say(f"sort n={n} V={V} equal={equal}")
+    t = Triple(V)
+    a = rand_keys(rng, V, n)
+    a[rng.random(n) < equal] = keys_of([V // 3], [V // 2])[0]
+    t.insert(a)
+    t.compare()
+    t.mixed(rand_keys(rng, V, n // 2), a[: n - n // 2])
+    t.compare()
+    t.close()
+
+
+def test_many_sources():
+    """More requests than the split kernel stages, and as many as it does."""
+    V = 3000
+    rng = np.random.default_rng(3)
+    for requests in (64, 65, 100):
+        say(f"sources {2 * requests}")
+        pma = L.PMA(V)
+        ref = rand_keys(rng, V, 50000)
+        pma.insert(ref)
+        ref = oracle.sort_unique(ref)
+        batches = [(rand_keys(rng, V, 1500), rand_keys(rng, V, int(rng.integers(0, 1500)))) for _ in range(requests)]
+        pma.update_sequence(batches)
+        for a, d in batches:
+            ref = oracle.apply(ref, a, d)
+        ek, ro = pma.export()
+        assert np.array_equal(L.to_host_u64(ek), ref)
+        assert np.array_equal(ro.cpu().numpy().view(np.uint32), oracle.row_offsets(ref, V))
+        assert pma.check() == 0
+        pma.close()
