@@ -47,8 +47,8 @@ static constexpr u32 FLAG_ROOT = 2u;          // a run chose the root window
 static constexpr u32 FLAG_RESIZE = 4u;        // the root window does not fit
 static constexpr u32 FLAG_SORT_STALL = 8u;    // a sort tile waited too long (the batch fails)
 
-// most passes of the batch sort (11-bit digits over 64 bits)
-static constexpr u32 SORT_MAX_PASSES = 6;
+// most passes of the batch sort (8-bit digits over 64 bits)
+static constexpr u32 SORT_MAX_PASSES = 8;
 
 // rebalance work classes
 static constexpr int CLASS_WAVE = 0;   // one wave64 per window

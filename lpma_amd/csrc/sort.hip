@@ -7,159 +7,37 @@
 // above it for a group and the request order between key and operation for a
 // merged sequence, so equal keys end up ordered delete before insert, earlier
 // request before later; the dedup that follows keeps the last of each run.
-// Three paths by batch size:
+// Two paths by batch size:
 //   <= 2^19 keys   sample-split sort: two kernels, buckets chosen from a
 //                  sample, each sorted by a bitonic network;
-//   <= 2^22 keys   LSD radix, one kernel per 10/11-bit digit (decoupled
-//                  look-back), the digit counts of every pass taken at pack;
-//   larger         LSD radix, 8-bit digits, histogram + scan + scatter.
+//   larger         LSD radix, one kernel per 7/8-bit digit (decoupled
+//                  look-back), the digit counts of every pass taken at pack.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "begin.hpp"
 
 namespace pma {
 
-static constexpr int RS_BITS = 8;
-static constexpr int RS_RADIX = 1 << RS_BITS;
-static constexpr int RS_TPB = 256;
-static constexpr int RS_ITEMS_BIG = 16;   // keys per thread per tile, large inputs
-static constexpr int RS_ITEMS_SMALL = 4;  // smaller tiles for more workgroups on mid-size batches
-
-// Packs a group batch into sort keys pid << pshift | (src << vbits | dst) << 1 | op
-// (keys with src or dst >= V raise FLAG_INVALID_KEY) and counts the first
-// radix digit of every tile (digit-major: hist[d * nblocks + tile]).
-__global__ __launch_bounds__(RS_TPB) void k_pack_group(const BatchSeg *__restrict__ segs, u32 nsegs, u64 n,
-                                                        const u64 *n_dev, u32 pshift, u32 sbits, u64 *__restrict__ out,
-                                                        u32 *__restrict__ flags, u32 shift, u32 items,
-                                                        u32 *__restrict__ hist, u32 nblocks) {
-    __shared__ u32 h[RS_RADIX];
-    if (n_dev) n = *n_dev;
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const u64 base = (u64)blockIdx.x * items * RS_TPB + threadIdx.x;
-    bool bad = false;
-    if (base < n) {
-        u32 s = source_of(segs, nsegs, base);
-        BatchSeg sg = segs[s];
-        for (u32 r = 0; r < items; ++r) {
-            u64 i = base + (u64)r * RS_TPB;
-            if (i >= n) break;
-            while (i >= sg.off + sg.n) sg = segs[++s];
-            u64 k = sg.keys[i - sg.off];
-            u32 src = (u32)(k >> 32), dst = (u32)k;
-            if (src >= sg.V || dst >= sg.V) { bad = true; src = 0; dst = 0; }
-            u64 p = ((u64)sg.pid << pshift) | ((((((u64)src) << sg.vbits) | dst) << sbits | sg.seq) << 1) | sg.op;
-            out[i] = p;
-            atomicAdd(&h[(p >> shift) & (RS_RADIX - 1)], 1u);
-        }
-    }
-    if (__any(bad) && lane_id() == 0) atomicOr(flags, FLAG_INVALID_KEY);
-    __syncthreads();
-    hist[(u64)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
-}
-
-// ------------------------------------------------------------ stable ranking
-//
-// One round ranks NT consecutive keys of a tile by their digit: lanes with
-// equal digits are found with 8 wave ballots (a wave64 "match any"), a
-// lane's rank inside its wave is the popcount of its lower peers, and
-// per-wave digit counts in LDS give the offset of the waves before it.
-
-template <int NT>
-struct RankLds {
-    u32 running[RS_RADIX];
-    u32 wcnt[NT / 64][RS_RADIX];
-};
-
-template <int NT>
-__device__ __forceinline__ void rank_init(RankLds<NT> &s) {
-    for (u32 i = threadIdx.x; i < RS_RADIX; i += NT) s.running[i] = 0;
-    for (u32 i = threadIdx.x; i < (NT / 64) * RS_RADIX; i += NT) (&s.wcnt[0][0])[i] = 0;
-}
-
-template <int NT>
-__device__ __forceinline__ void rank_round(bool valid, u32 digit, RankLds<NT> &s, u32 &pos) {
-    const u32 lane = lane_id();
-    const u32 w = threadIdx.x >> 6;
-    u64 peers = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < RS_BITS; ++b) {
-        u32 bit = (digit >> b) & 1u;
-        u64 bb = __ballot(bit);
-        peers &= bit ? bb : ~bb;
-    }
-    const u32 rank = __popcll(peers & ((1ull << lane) - 1ull));
-    const bool leader = valid && rank == 0;
-    const u32 cnt = __popcll(peers);
-    if (leader) s.wcnt[w][digit] = cnt;
-    __syncthreads();
-    if (valid) {
-        u32 off = s.running[digit];
-        for (u32 v = 0; v < w; ++v) off += s.wcnt[v][digit];
-        pos = off + rank;
-    }
-    __syncthreads();
-    // only the entries written this round change: their leaders fold them in
-    if (leader) {
-        atomicAdd(&s.running[digit], cnt);
-        s.wcnt[w][digit] = 0;
-    }
-    __syncthreads();
-}
-
-// per-tile digit histogram, digit-major (hist[d * nblocks + tile])
-__global__ __launch_bounds__(RS_TPB) void k_rs_hist(const u64 *__restrict__ keys, u64 n, const u64 *n_dev, u32 shift,
-                                                     u32 items, u32 *__restrict__ hist, u32 nblocks) {
-    __shared__ u32 h[RS_RADIX];
-    if (n_dev) n = *n_dev;
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    u64 base = (u64)blockIdx.x * items * RS_TPB;
-    for (u32 r = 0; r < items; ++r) {
-        u64 i = base + (u64)r * RS_TPB + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & (RS_RADIX - 1)], 1u);
-    }
-    __syncthreads();
-    hist[(u64)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
-}
-
-// Scatter of one pass; hist holds the device-wide exclusive scan of the
-// digit-major histograms (each tile's offset of each digit).
-__global__ __launch_bounds__(RS_TPB) void k_rs_scatter(const u64 *__restrict__ in, u64 *__restrict__ out, u64 n,
-                                                        const u64 *n_dev, u32 shift, u32 items,
-                                                        const u32 *__restrict__ hist, u32 nblocks) {
-    __shared__ RankLds<RS_TPB> s;
-    __shared__ u32 gofs[RS_RADIX];
-    if (n_dev) n = *n_dev;
-    gofs[threadIdx.x] = hist[(u64)threadIdx.x * nblocks + blockIdx.x];
-    rank_init<RS_TPB>(s);
-    __syncthreads();
-    u64 base = (u64)blockIdx.x * items * RS_TPB;
-    for (u32 r = 0; r < items; ++r) {
-        u64 i = base + (u64)r * RS_TPB + threadIdx.x;
-        bool valid = i < n;
-        u64 key = valid ? in[i] : 0;
-        u32 digit = (u32)(key >> shift) & (RS_RADIX - 1);
-        u32 pos = 0;
-        rank_round<RS_TPB>(valid, digit, s, pos);
-        if (valid) out[gofs[digit] + pos] = key;
-    }
-}
-
 // ------------------------------------------------- one kernel per pass
 //
-// Batches of 512K..4M keys sort with DB = 10 or 11-bit digits (four passes
-// for the 40-41 bits of a lone PMA with 2^20 vertices), one kernel each,
-// over tiles of 4096 keys (1024 threads, 4 keys each): few enough tiles that
-// a tile finds the counts of all tiles before it in few look-back steps,
-// small enough that a tile's 16 waves rank it in 4 rounds each:
-// the pack kernel counts the digits of every pass at once (global digit
-// totals), and a pass kernel ranks its tile in LDS, publishes the tile's
-// digit counts, reads the counts of the tiles before it (decoupled look-back,
-// Merrill & Garland, "Single-pass Parallel Prefix Scan with Decoupled
-// Look-back", NVR-2016-002) and scatters.  A published word is the count in
-// bits 0..29 with OS_AGG (this tile only) or OS_PRE (this tile and every
-// tile before it) in bits 30..31; 0 means not yet published.
+// Batches of more than 512K keys sort by LSD radix with digits of DB = 7 or 8 bits
+// (six passes for the 41 bits of a lone PMA with 2^20 vertices), one kernel
+// each, over tiles of OS_TPB * ITEMS keys: the pack kernel counts the digits of
+// every pass at once (global digit totals); a pass kernel ranks its tile in
+// LDS, publishes the tile's digit counts, reads the counts of the tiles before
+// it (decoupled look-back, Merrill & Garland, "Single-pass Parallel Prefix Scan
+// with Decoupled Look-back", NVR-2016-002), brings the tile into digit order in
+// LDS and writes it out, a digit's keys side by side.  A published word with
+// OS_PRE set carries the count of this tile and every tile before it in bits
+// 0..30 (a batch has fewer than 2^31 keys); without it, this tile's count plus
+// one; 0 means not yet published.
+//
+// Bound: HBM and the look-back's latency.  Small digits make a tile's keys of
+// one digit a run of 32 to 64 keys (256 to 512 B).  2*10^6 keys of 41 bits:
+// six passes of 17.6 us; four passes over 11-bit digits, written from registers
+// with two keys a digit and tile, took 43 us each.  8.4*10^6 keys of 41 bits:
+// 38 us to pack and six passes of 55 us (2.4 TB/s); 8-bit passes of a
+// histogram, a scan and a scatter kernel took 550 us in all.
 //
 // Tile t waits only on tiles < t.  Workgroups are dispatched in index order,
 // so every tile it waits on is running or done; the wait is still bounded
@@ -167,13 +45,13 @@ __global__ __launch_bounds__(RS_TPB) void k_rs_scatter(const u64 *__restrict__ i
 // and fails without changing anything.
 
 static constexpr int OS_TPB = 1024;  // large tiles: few tiles, short look-back walks
-static constexpr u32 OS_AGG = 1u << 30;
-static constexpr u32 OS_PRE = 2u << 30;
-static constexpr u32 OS_CNT = (1u << 30) - 1;
+static constexpr u32 OS_PRE = 1u << 31;
 static constexpr u32 OS_SPIN_LIMIT = 1u << 20;
-static constexpr u64 OS_MAX_N = 1ull << 22;       // larger batches: the two-kernel passes
-static constexpr u32 OS_GH_WORDS = SORT_MAX_PASSES * 2048;
-static constexpr int OS_ITEMS = 4;   // keys per thread: tiles of 4096
+static constexpr u32 OS_MAX_R = 256;
+// copies of the digit totals: their atomics meet on few lines otherwise
+static constexpr u32 OS_COPIES = 8;
+static constexpr u32 OS_GH_WORDS = SORT_MAX_PASSES * OS_MAX_R * OS_COPIES;
+static constexpr u32 OS_PACK_GRID = 512;
 static constexpr int OS_LOOK = 32;   // look-back loads in flight per thread
 
 __device__ __forceinline__ u32 os_load(const u32 *p) {
@@ -183,77 +61,74 @@ __device__ __forceinline__ void os_store(u32 *p, u32 v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Pack (as k_pack_group) and count the digits of all npass passes:
-// gh[p * R + d] += keys whose pass-p digit is d (gh zeroed by the caller);
-// also clears the look-back row of this tile for the first pass.
+// Pack (keys with src or dst >= V raise FLAG_INVALID_KEY) and count the digits of all npass passes:
+// gh[(copy * npass + p) * R + d] += keys whose pass-p digit is d (gh zeroed by
+// the caller); also clears the tiles' look-back rows for the first pass.  Few
+// workgroups take several tiles each, so that their counts reach memory once.
 template <int DB>
 __global__ __launch_bounds__(OS_TPB) void k_pack_count(const BatchSeg *__restrict__ segs, u32 nsegs, u64 n,
                                                         const u64 *n_dev, u32 pshift, u32 sbits, u64 *__restrict__ out,
                                                         u32 *__restrict__ flags, u32 lo_bit, u32 npass, u32 items,
-                                                        u32 *__restrict__ gh, u32 *__restrict__ look0) {
+                                                        u32 ntiles, u32 *__restrict__ gh, u32 *__restrict__ look0) {
     constexpr u32 R = 1u << DB;
-    __shared__ u32 h[SORT_MAX_PASSES][R];
+    __shared__ u32 h[SORT_MAX_PASSES * R];
     if (n_dev) n = *n_dev;
-    for (u32 i = threadIdx.x; i < npass * R; i += OS_TPB) (&h[0][0])[i] = 0;
-    for (u32 i = threadIdx.x; i < R; i += OS_TPB) look0[(u64)blockIdx.x * R + i] = 0;
+    for (u32 i = threadIdx.x; i < npass * R; i += OS_TPB) h[i] = 0;
     __syncthreads();
-    const u64 base = (u64)blockIdx.x * items * OS_TPB + threadIdx.x;
     bool bad = false;
-    if (base < n) {
+    for (u32 t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        if (threadIdx.x < R) look0[(u64)t * R + threadIdx.x] = 0;
+        const u64 base = (u64)t * items * OS_TPB + threadIdx.x;
+        if (base >= n) continue;
         u32 s = source_of(segs, nsegs, base);
         BatchSeg sg = segs[s];
         for (u32 r = 0; r < items; ++r) {
             u64 i = base + (u64)r * OS_TPB;
             if (i >= n) break;
             while (i >= sg.off + sg.n) sg = segs[++s];
-            u64 k = sg.keys[i - sg.off];
-            u32 src = (u32)(k >> 32), dst = (u32)k;
-            if (src >= sg.V || dst >= sg.V) { bad = true; src = 0; dst = 0; }
-            u64 p = ((u64)sg.pid << pshift) | ((((((u64)src) << sg.vbits) | dst) << sbits | sg.seq) << 1) | sg.op;
+            const u64 p = pack_element(sg, i, pshift, sbits, bad);
             out[i] = p;
-            for (u32 q = 0; q < npass; ++q) atomicAdd(&h[q][(u32)(p >> (lo_bit + q * DB)) & (R - 1)], 1u);
+            for (u32 q = 0; q < npass; ++q) atomicAdd(&h[q * R + ((u32)(p >> (lo_bit + q * DB)) & (R - 1))], 1u);
         }
     }
     if (__any(bad) && lane_id() == 0) atomicOr(flags, FLAG_INVALID_KEY);
     __syncthreads();
+    u32 *to = gh + (u64)(blockIdx.x % OS_COPIES) * npass * R;
     for (u32 i = threadIdx.x; i < npass * R; i += OS_TPB) {
-        u32 v = (&h[0][0])[i];
-        if (v) atomicAdd(&gh[i], v);
+        u32 v = h[i];
+        if (v) atomicAdd(&to[i], v);
     }
 }
 
 // One pass over bits [shift, shift + DB).  Tile t = keys [t*T, t*T + T),
 // T = OS_TPB * ITEMS; wave w holds the 64*ITEMS consecutive keys from
 // t*T + w*64*ITEMS, one per lane per round, so (wave, round, lane) order is
-// input order and the ranking is stable.  W predecessors are read per
-// look-back step.
-template <int DB, int ITEMS, int W>
+// input order and the ranking is stable.  gh: the pass's digit totals, copies
+// gstride apart.
+template <int DB, int ITEMS>
 __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, u64 *__restrict__ out, u64 n,
                                                      const u64 *n_dev, u32 shift, const u32 *__restrict__ gh,
-                                                     u32 *__restrict__ look, u32 *__restrict__ look_next,
-                                                     u32 *__restrict__ flags) {
+                                                     u32 gstride, u32 *__restrict__ look,
+                                                     u32 *__restrict__ look_next, u32 *__restrict__ flags) {
     constexpr u32 R = 1u << DB;
     constexpr u32 NW = OS_TPB / 64;
-    constexpr u32 DPT = R / OS_TPB;  // digits per thread
-    extern __shared__ u32 os_lds[];
-    u32(*whist)[R] = (u32(*)[R])os_lds;  // per-wave digit counts, then per-wave offsets
-    u32 *gofs = os_lds + NW * R;          // keys of smaller digits in the whole batch
-    u32 *tofs = gofs + R;                 // keys of this digit in earlier tiles
-    __shared__ u32 stmp[NW + 1];
+    constexpr u32 DW = R / 64;  // waves that hold the digits
+    extern __shared__ u64 os_lds[];
+    u64 *buf = os_lds;  // the tile in digit order
+    // per-wave digit counts, then per-wave offsets (a tile has at most 2^13 keys)
+    unsigned short(*whist)[R] = (unsigned short(*)[R])(buf + OS_TPB * ITEMS);
+    __shared__ u32 lofs[R];  // the tile's keys of smaller digits
+    __shared__ u32 gofs[R];  // a digit's first place in the batch, less lofs
+    __shared__ u32 sums[2][DW];
     if (n_dev) n = *n_dev;
-    const u32 t = blockIdx.x;
-    if (look_next)
-        for (u32 i = threadIdx.x; i < R; i += OS_TPB) look_next[(u64)t * R + i] = 0;
+    const u32 t = blockIdx.x, tid = threadIdx.x;
+    if (look_next && tid < R) look_next[(u64)t * R + tid] = 0;
     const u64 tbase = (u64)t * OS_TPB * ITEMS;
     if (tbase >= n) return;  // whole workgroup: grids sized for a capacity
     const u32 lane = lane_id();
-    const u32 w = threadIdx.x >> 6;
+    const u32 w = tid >> 6;
     const u64 lt = (1ull << lane) - 1ull;
 
-    // batch-wide digit totals of this pass, contiguous per thread
-    u32 gv[DPT];
-#pragma unroll
-    for (u32 j = 0; j < DPT; ++j) gv[j] = gh[threadIdx.x * DPT + j];
     u64 key[ITEMS];
     const u64 wbase = tbase + (u64)w * 64 * ITEMS + lane;
 #pragma unroll
@@ -261,7 +136,12 @@ __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, 
         u64 i = wbase + (u64)r * 64;
         key[r] = i < n ? in[i] : 0ull;
     }
-    for (u32 i = threadIdx.x; i < NW * R; i += OS_TPB) os_lds[i] = 0;
+    u32 gv = 0;  // batch-wide total of digit tid
+    if (tid < R) {
+#pragma unroll
+        for (u32 c = 0; c < OS_COPIES; ++c) gv += gh[(u64)c * gstride + tid];
+    }
+    for (u32 i = tid; i < NW * R / 2; i += OS_TPB) ((u32 *)whist)[i] = 0;
     __syncthreads();
 
     // rank inside the wave: lanes of equal digit found with DB ballots; the
@@ -287,95 +167,94 @@ __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, 
     }
     __syncthreads();
 
-    // per digit: offsets of the waves, the tile's count, published at once
-    u32 cnt[DPT];
+    // digit tid: offsets of the waves, the tile's count, published at once,
+    // and the scans of the tile's counts and of the totals
+    u32 cnt = 0, li = 0, gi = 0;
+    if (tid < R) {
+        u32 c[NW];
 #pragma unroll
-    for (u32 j = 0; j < DPT; ++j) {
-        const u32 d = j * OS_TPB + threadIdx.x;
-        u32 run = 0;
+        for (u32 v = 0; v < NW; ++v) c[v] = whist[v][tid];
 #pragma unroll
         for (u32 v = 0; v < NW; ++v) {
-            u32 c = whist[v][d];
-            whist[v][d] = run;
-            run += c;
+            whist[v][tid] = (unsigned short)cnt;
+            cnt += c[v];
         }
-        cnt[j] = run;
-        os_store(&look[(u64)t * R + d], (t == 0 ? OS_PRE : OS_AGG) | run);
-    }
-    // exclusive scan of the digit totals
-    {
-        u32 sum = 0;
-#pragma unroll
-        for (u32 j = 0; j < DPT; ++j) sum += gv[j];
-        u32 tot;
-        u32 ex = block_excl_scan<OS_TPB, u32>(sum, tot, stmp);
-#pragma unroll
-        for (u32 j = 0; j < DPT; ++j) { gofs[threadIdx.x * DPT + j] = ex; ex += gv[j]; }
-    }
-
-    // look-back: keys of each digit in tiles < t
-    u32 excl[DPT];
-    int p[DPT];
-#pragma unroll
-    for (u32 j = 0; j < DPT; ++j) { excl[j] = 0; p[j] = (int)t - 1; }
-    bool stalled = false;
-    for (u32 spin = 0;; ++spin) {
-        u32 s[DPT][W];
-#pragma unroll
-        for (u32 j = 0; j < DPT; ++j) {
-            const u32 d = j * OS_TPB + threadIdx.x;
-            // unconditional loads (row 0 stands in past the first tile) so
-            // that all W * DPT of them are in flight together
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                const int q = p[j] - k;
-                s[j][k] = os_load(&look[(u64)(q > 0 ? q : 0) * R + d]);
-            }
-        }
-        // consume predecessors in order until one is unpublished (read it
-        // again next round) or carries the prefix of all before it (done);
-        // branch-free so that s stays in registers
-        bool pending = false;
-#pragma unroll
-        for (u32 j = 0; j < DPT; ++j) {
-            int q = p[j];
-            bool go = q >= 0;
-            u32 acc = 0;
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                const u32 v = s[j][k];
-                const u32 f = v & ~OS_CNT;
-                const bool use = go && f != 0;
-                acc += use ? (v & OS_CNT) : 0u;
-                q = use ? (f == OS_PRE ? -1 : q - 1) : q;
-                go = use && f != OS_PRE;
-            }
-            excl[j] += acc;
-            p[j] = q;
-            pending |= q >= 0;
-        }
-        if (!pending) break;
-        if (spin >= OS_SPIN_LIMIT) {
-            stalled = true;
-            break;
+        os_store(&look[(u64)t * R + tid], t == 0 ? OS_PRE | cnt : cnt + 1);
+        li = dpp_incl_scan32(cnt);
+        gi = dpp_incl_scan32(gv);
+        if (lane == 63) {
+            sums[0][w] = li;
+            sums[1][w] = gi;
         }
     }
-    if (stalled) atomicOr(flags, FLAG_SORT_STALL);
-#pragma unroll
-    for (u32 j = 0; j < DPT; ++j) {
-        const u32 d = j * OS_TPB + threadIdx.x;
-        tofs[d] = excl[j];
-        if (t != 0) os_store(&look[(u64)t * R + d], OS_PRE | ((excl[j] + cnt[j]) & OS_CNT));
+    __syncthreads();
+    if (tid < R) {
+        for (u32 v = 0; v < w; ++v) {
+            li += sums[0][v];
+            gi += sums[1][v];
+        }
+        lofs[tid] = li - cnt;
     }
     __syncthreads();
 
+    // the tile in digit order
 #pragma unroll
     for (int r = 0; r < ITEMS; ++r) {
-        if (wbase + (u64)r * 64 >= n) break;
         const u32 dg = (u32)(key[r] >> shift) & (R - 1);
-        u64 pos = (u64)gofs[dg] + tofs[dg] + whist[w][dg] + rk[r];
-        if (pos >= n) pos = n - 1;  // only after a stall (flagged): stay in bounds
-        out[pos] = key[r];
+        if (wbase + (u64)r * 64 < n) buf[lofs[dg] + whist[w][dg] + rk[r]] = key[r];
+    }
+
+    // look-back: keys of digit tid in tiles < t
+    if (tid < R) {
+        u32 excl = 0;
+        int p = (int)t - 1;
+        bool stalled = false;
+        for (u32 spin = 0; p >= 0; ++spin) {
+            u32 s[OS_LOOK];
+            // unconditional loads (row 0 stands in past the first tile) so
+            // that all of them are in flight together
+#pragma unroll
+            for (int k = 0; k < OS_LOOK; ++k) {
+                const int q = p - k;
+                s[k] = os_load(&look[(u64)(q > 0 ? q : 0) * R + tid]);
+            }
+            // consume predecessors in order until one is unpublished (read it
+            // again next round) or carries the prefix of all before it (done);
+            // branch-free so that s stays in registers
+            int q = p;
+            bool go = true;
+            u32 acc = 0;
+#pragma unroll
+            for (int k = 0; k < OS_LOOK; ++k) {
+                const u32 v = s[k];
+                const bool pre = v >> 31;
+                const bool use = go && q >= 0 && v != 0;
+                acc += use ? (pre ? v & ~OS_PRE : v - 1) : 0u;
+                q = use ? (pre ? -1 : q - 1) : q;
+                go = use && !pre;
+            }
+            excl += acc;
+            p = q;
+            if (p >= 0 && spin >= OS_SPIN_LIMIT) {
+                stalled = true;
+                break;
+            }
+        }
+        if (stalled) atomicOr(flags, FLAG_SORT_STALL);
+        if (t != 0) os_store(&look[(u64)t * R + tid], OS_PRE | (excl + cnt));
+        gofs[tid] = (gi - gv) + excl - (li - cnt);
+    }
+    __syncthreads();
+
+    const u32 m = (u32)min((u64)(OS_TPB * ITEMS), n - tbase);
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const u32 i = tid + r * OS_TPB;
+        if (i >= m) break;
+        const u64 k = buf[i];
+        u32 pos = gofs[(u32)(k >> shift) & (R - 1)] + i;
+        if (pos >= n) pos = (u32)n - 1;  // only after a stall (flagged): stay in bounds
+        out[pos] = k;
     }
 }
 
@@ -871,46 +750,43 @@ hipError_t device_excl_scan(const u32 *in, u64 n, u32 *out, u32 *scratch, hipStr
 
 // ------------------------------------------------------------ radix driver
 
-// small tiles keep >= ~2000 workgroups in flight up to 8M keys
-static u32 rs_items(u64 n) { return n <= (1ull << 23) ? RS_ITEMS_SMALL : RS_ITEMS_BIG; }
+// Keys a thread in a tile of the one-kernel passes: 4 up to one tile per CU, 8
+// beyond, for longer runs and fewer tiles to look back over (2*10^6 keys: 17.6
+// against 19.9 us a pass; 8.4*10^6: 55 and 54).
+static u32 os_items(u64 n) { return n <= (1ull << 20) ? 4 : 8; }
 
-static u32 os_items(u64) { return OS_ITEMS; }
-
-// digit width for a sort over `width` bits: 10 unless 11 saves a pass
-static u32 os_digit_bits(u32 width) { return (width + 9) / 10 == (width + 10) / 11 ? 10 : 11; }
+// digit width for a sort over `width` bits: as many passes as 8-bit digits take
+static u32 os_digit_bits(u32 width) { return (width + 7) / 8 * 7 >= width ? 7 : 8; }
 
 u64 sort_scratch_words(u64 n) {
-    u64 nb = (n + (u64)rs_items(n) * RS_TPB - 1) / ((u64)rs_items(n) * RS_TPB);
-    u64 two = (u64)RS_RADIX * nb + 1 + scan_scratch_words((u64)RS_RADIX * nb);
-    u64 tile = (u64)os_items(n) * OS_TPB;
-    u64 one = 2 * ((n + tile - 1) / tile) * 2048;
-    u64 split = n <= SS_MAX_N ? (u64)ss_buckets(n) * ss_tiles(n) : 0;
-    return OS_GH_WORDS + std::max(n <= OS_MAX_N ? std::max(two, one) : two, split);
+    const u64 tile = (u64)os_items(n) * OS_TPB;
+    const u64 look = 2 * ((n + tile - 1) / tile) * OS_MAX_R;
+    const u64 split = (u64)ss_buckets(n) * ss_tiles(n);
+    return OS_GH_WORDS + (n <= SS_MAX_N ? split : look);
 }
 
 u32 sort_zero_words() { return OS_GH_WORDS; }
 
-template <int DB>
-static void os_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32 pshift, u32 sbits, u32 lo_bit,
-                    u32 npass, u64 *k0, u64 *k1, u32 *scratch, u32 *flags, u64 **result, hipStream_t st) {
+template <int DB, int ITEMS>
+static u64 *os_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32 pshift, u32 sbits, u32 lo_bit,
+                    u32 npass, u64 *k0, u64 *k1, u32 *scratch, u32 *flags, hipStream_t st) {
     constexpr u32 R = 1u << DB;
-    const u32 items = os_items(n);
-    const u64 tile = (u64)items * OS_TPB;
+    constexpr u64 tile = (u64)ITEMS * OS_TPB;
     const u32 ntiles = (u32)((n + tile - 1) / tile);
     u32 *gh = scratch;
     u32 *look[2] = {scratch + OS_GH_WORDS, scratch + OS_GH_WORDS + (u64)ntiles * R};
-    k_pack_count<DB><<<ntiles, OS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, k0, flags, lo_bit, npass, items,
-                                                gh, look[0]);
+    k_pack_count<DB><<<std::min(ntiles, OS_PACK_GRID), OS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, k0, flags,
+                                                                       lo_bit, npass, ITEMS, ntiles, gh, look[0]);
     u64 *src = k0, *dst = k1;
+    const size_t lds = tile * sizeof(u64) + (size_t)(OS_TPB / 64) * R * sizeof(unsigned short);
     for (u32 q = 0; q < npass; ++q) {
         const u32 shift = lo_bit + q * DB;
         u32 *nxt = q + 1 < npass ? look[(q + 1) & 1] : nullptr;
-        const size_t lds = ((size_t)(OS_TPB / 64) * R + 2 * R) * sizeof(u32);
-        k_os_pass<DB, OS_ITEMS, OS_LOOK / (R / OS_TPB)><<<ntiles, OS_TPB, lds, st>>>(src, dst, n, n_dev, shift,
-                                                                                   gh + q * R, look[q & 1], nxt, flags);
+        k_os_pass<DB, ITEMS><<<ntiles, OS_TPB, lds, st>>>(src, dst, n, n_dev, shift, gh + q * R, npass * R, look[q & 1],
+                                                          nxt, flags);
         u64 *t = src; src = dst; dst = t;
     }
-    *result = src;
+    return src;
 }
 
 // Packs a group batch (n elements from nsegs sources) and sorts the packed
@@ -941,35 +817,15 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
                                            DevState{});
         return k0;
     }
-    if (n <= OS_MAX_N) {
-        const u32 width = hi_bit - lo_bit;
-        const u32 db = os_digit_bits(width);
-        const u32 npass = (width + db - 1) / db;
-        u64 *res = k0;
-        if (db == 10)
-            os_sort<10>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, &res, st);
-        else
-            os_sort<11>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, &res, st);
-        return res;
-    }
-    scratch += OS_GH_WORDS;
-    const u32 items = rs_items(n);
-    const u64 tile = (u64)items * RS_TPB;
-    const u32 nblk = (u32)((n + tile - 1) / tile);
-    u32 *hist = scratch;
-    u32 *sscr = scratch + (u64)RS_RADIX * nblk + 1;
-    u64 *src = k0, *dst = k1;
-    for (u32 shift = lo_bit; shift < hi_bit; shift += RS_BITS) {
-        if (shift == lo_bit)
-            k_pack_group<<<nblk, RS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, k0, flags, shift, items,
-                                                  hist, nblk);
-        else
-            k_rs_hist<<<nblk, RS_TPB, 0, st>>>(src, n, n_dev, shift, items, hist, nblk);
-        (void)device_excl_scan(hist, (u64)RS_RADIX * nblk, hist, sscr, st);
-        k_rs_scatter<<<nblk, RS_TPB, 0, st>>>(src, dst, n, n_dev, shift, items, hist, nblk);
-        u64 *t = src; src = dst; dst = t;
-    }
-    return src;
+    const u32 width = hi_bit - lo_bit;
+    const u32 db = os_digit_bits(width);
+    const u32 npass = (width + db - 1) / db;
+    const bool big = os_items(n) == 8;
+    if (db == 7)
+        return big ? os_sort<7, 8>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, st)
+                   : os_sort<7, 4>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, st);
+    return big ? os_sort<8, 8>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, st)
+               : os_sort<8, 4>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, st);
 }
 
 bool sort_carries_first(u64 n) { return n > 0 && n <= SS_MAX_N; }

@@ -182,6 +182,24 @@ def test_sample_split_sort(n, V, equal):
     t.close()
 
 
+# the radix sort: its smallest batch, 4 keys a thread up to 2^20 and 8 above
+# (whole tiles and one key more), digits of 7 bits (V = 2^20: 41 bits; 40: 13)
+# and of 8 (2^14: 29), half of the keys equal
+@pytest.mark.parametrize("n", [(1 << 19) + 1, 1 << 20, (1 << 20) + 1, (1 << 20) + (3 << 13), 1500001])
+@pytest.mark.parametrize("V,equal", [(1 << 20, 0.0), (1 << 14, 0.5), (40, 0.0)])
+def test_radix_sort(n, V, equal):
+    rng = np.random.default_rng(n)
+    say(f"sort n={n} V={V} equal={equal}")
+    t = Triple(V)
+    a = rand_keys(rng, V, n)
+    a[rng.random(n) < equal] = keys_of([V // 3], [V // 2])[0]
+    t.insert(a)
+    t.compare()
+    t.mixed(rand_keys(rng, V, n // 2), a[: n - n // 2])
+    t.compare()
+    t.close()
+
+
 def test_many_sources():
     """More requests than the split kernel stages, and as many as it does."""
     V = 3000
