@@ -204,6 +204,8 @@ struct Pipeline {
     EarlyOut *h_early = nullptr;  // pinned: a lone PMA's outcome, stored by a kernel
 };
 
+// the lone PMA's outcome stands before the copied one in its pinned block
+static constexpr u64 EARLY_BYTES = (sizeof(EarlyOut) + 127) / 128 * 128;
 static constexpr u64 STATUS_BYTES = (sizeof(Status) + 15) / 16 * 16;
 
 // ------------------------------------------------------------------ handle
@@ -400,7 +402,6 @@ void pipeline_free(Pipeline &pl) {
     pl.h_rhdr = nullptr;
     if (pl.h_tab) (void)hipHostFree(pl.h_tab);
     if (pl.h_segs) (void)hipHostFree(pl.h_segs);
-    if (pl.h_out) (void)hipHostFree(pl.h_out);
     if (pl.h_early) (void)hipHostFree(pl.h_early);
     pl.h_tab = nullptr; pl.h_segs = nullptr; pl.h_out = nullptr; pl.h_early = nullptr;
     if (pl.d_stats) (void)hipFree(pl.d_stats);
@@ -581,29 +582,25 @@ int ensure_batch(Pipeline &pl, u64 n, u32 npma, u32 nsegs, u64 runs) {
         return r;
     if (!pl.h_out || pl.h_out_bytes < out_words * 8) {
         if (injected_failure()) return LPMA_ERR_OUT_OF_MEMORY;
-        if (pl.h_out) {
+        if (pl.h_early) {
             (void)hipStreamSynchronize(pl.cur_stream);
-            (void)hipHostFree(pl.h_out);
+            (void)hipHostFree(pl.h_early);
+            pl.h_early = nullptr;
             pl.h_out = nullptr;
         }
         u64 want = std::max<u64>(out_words * 8, 2 * pl.h_out_bytes);
-        if (hipHostMalloc((void **)&pl.h_out, want, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            pl.h_out = nullptr;
-            pl.h_out_bytes = 0;
-            return LPMA_ERR_OUT_OF_MEMORY;
-        }
-        pl.h_out_bytes = want;
-    }
-    if (!pl.h_early) {
-        if (injected_failure()) return LPMA_ERR_OUT_OF_MEMORY;
-        if (hipHostMalloc((void **)&pl.h_early, sizeof(EarlyOut), hipHostMallocMapped | hipHostMallocCoherent) !=
+        // one block for both: an allocation of pinned memory costs 100 us of a
+        // store's or group's first batch
+        if (hipHostMalloc((void **)&pl.h_early, EARLY_BYTES + want, hipHostMallocMapped | hipHostMallocCoherent) !=
             hipSuccess) {
             (void)hipGetLastError();
             pl.h_early = nullptr;
+            pl.h_out_bytes = 0;
             return LPMA_ERR_OUT_OF_MEMORY;
         }
         pl.h_early->seq = 0;
+        pl.h_out = (unsigned char *)pl.h_early + EARLY_BYTES;
+        pl.h_out_bytes = want;
     }
     return LPMA_OK;
 }
