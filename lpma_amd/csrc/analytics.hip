@@ -13,6 +13,13 @@ namespace pma {
 
 static constexpr u32 INF_LEVEL = 0xFFFFFFFFu;
 
+// the XCD this wave runs on
+__device__ __forceinline__ u32 xcc_id() {
+    u32 x;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(x));
+    return x & 7u;
+}
+
 __device__ __forceinline__ void slot_range(const DevState &d, u32 r, u64 &lo, u64 &hi) {
     lo = r == 0 ? 0 : (u64)d.row_off[r] + 1;
     hi = d.row_off[r + 1];
@@ -21,240 +28,298 @@ __device__ __forceinline__ void slot_range(const DevState &d, u32 r, u64 &lo, u6
 // ------------------------------------------------------------------ BFS
 //
 // Level-synchronous, top-down.  A level expands the frontier's slot ranges
-// with one thread per slot, so hub vertices are split over many threads:
-//   k_bfs_len   each frontier row's slot count and first slot;
-//   scan        the counts' exclusive prefix: slot t of the level belongs to
-//               the last entry whose offset is <= t;
-//   k_bfs_runs  the first entry of every run of EXP_RUN slots (one binary
-//               search per run, all in parallel);
-//   k_bfs_expand  a workgroup per run stages the run's entries (offsets and
-//               first slots) in LDS; each thread takes EXP_ITEMS slots and
-//               issues their loads phase by phase (segment counts, keys,
-//               visited words), so dead lines of the gapped rows are not read
-//               and a thread has EXP_ITEMS loads in flight per phase.
+// with one lane per slot, so hub vertices are split over many waves:
+//   k_bfs_front   lists the frontier's non-empty rows (the entries): a row's
+//                 first place in the level's slots and what to add to a place
+//                 to get its slot; and the first entry of every run of
+//                 BFS_RUN places;
+//   k_bfs_expand  a wave per run: a bit for each entry's first place (so a
+//                 place finds its entry by counting bits), then segment
+//                 counts, keys and visited words, BFS_ITEMS loads in flight a
+//                 lane at each step, dead lines never read.
+// The sizes stand in device memory, so the host queues BFS_AHEAD levels at a
+// time and then asks once whether the last of them found anything (a level
+// after the end costs two empty launches); a copy and a wait after every
+// level, and a fill, three kernels to scan and one to search before its
+// expansion, took 100 us a level.
 // A visited bitmap (V bits: 2 MB at V = 2^24, held by every XCD's L2) filters
 // the edges; the levels array (32 bits per vertex) is only written.  A vertex
 // is claimed by the atomic OR that sets its bit, so it enters the next
 // frontier once; a plain read of a word another XCD has just changed can only
 // miss bits (they go from 0 to 1), which costs an extra atomic, never a wrong
 // level.
+// Bound: at V = 2^22 and E = 2^26 the two large levels (80 and 70 million
+// places) take 671 and 409 us, 140 of them for the first's keys; the rest are
+// visited words that miss L1 (a miss every 6 to 8 clocks a CU, through L1 or
+// past it) and atomics (6 G/s, with or without their results).  A workgroup
+// per run of 2048 places, with barriers and a binary search per place, took
+// 813 and 510.
 
-__global__ void k_bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *counters, u32 *visited) {
+// per level mod 4: vertices found, and entries (high 31 bits) and places (low
+// 33 bits)
+struct BfsCtl {
+    u64 ent[4];
+    u64 scanned;  // live edges of the frontiers so far
+    u32 qn[4];
+    u32 depth;    // levels with a frontier
+};
+static_assert(sizeof(BfsCtl) <= BFS_CTL_WORDS * 4, "control words");
+
+static constexpr u64 BFS_PLACES = (1ull << 33) - 1;
+static constexpr u32 BFS_ITEMS = 4;
+static constexpr u32 BFS_RUN = 64 * BFS_ITEMS;  // places per run
+
+__global__ void k_bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, BfsCtl *ctl, u32 *visited) {
     for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < V; i += (u64)gridDim.x * blockDim.x)
         levels[i] = i == src ? 0u : INF_LEVEL;
     for (u64 w = (u64)blockIdx.x * blockDim.x + threadIdx.x; w < bfs_visited_words(V); w += (u64)gridDim.x * blockDim.x)
         visited[w] = w == (src >> 5) ? 1u << (src & 31) : 0u;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         queue[0] = src;
-        counters[0] = 0;  // next frontier size
-        counters[1] = 0;  // live edges scanned
+        for (int k = 0; k < 4; ++k) {
+            ctl->ent[k] = 0;
+            ctl->qn[k] = k == 0 ? 1u : 0u;
+        }
+        ctl->scanned = 0;
+        ctl->depth = 0;
     }
 }
 
-__global__ void k_bfs_len(DevState d, const u32 *__restrict__ q, u32 qn, u32 *__restrict__ len,
-                          u64 *__restrict__ first) {
-    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < qn; i += (u64)gridDim.x * blockDim.x) {
-        u64 lo, hi;
-        slot_range(d, q[i], lo, hi);
-        len[i] = (u32)(hi - lo);
-        first[i] = lo;
+static constexpr u32 FRONT_TPB = 1024;
+
+// Entries of a level's frontier, FRONT_TPB vertices at a time.  One atomic
+// gives a chunk its entries and its places together, so places grow with
+// entries whatever order the chunks come in.  A run's first place lies in one
+// chunk, which finds the entry by binary search in LDS.  Bound: random reads
+// of row_off (1.6 million vertices: 40 us).
+__global__ __launch_bounds__(FRONT_TPB) void k_bfs_front(DevState d, u32 level, const u32 *__restrict__ q,
+                                                          BfsCtl *__restrict__ ctl, u32 *__restrict__ off,
+                                                          u32 *__restrict__ adj, u32 *__restrict__ runs) {
+    constexpr u32 NW = FRONT_TPB / 64;
+    __shared__ u32 s_off[FRONT_TPB];
+    __shared__ u32 s_n[NW], s_len[NW];
+    __shared__ u64 s_base;
+    const u32 tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+    const u32 qn = ctl->qn[level & 3];
+    if (blockIdx.x == 0 && tid == 0) {  // words of the level after the next: nothing reads or adds to them yet
+        ctl->qn[(level + 2) & 3] = 0;
+        ctl->ent[(level + 2) & 3] = 0;
+        if (qn) ctl->depth = level + 1;
+    }
+    for (u64 c = (u64)blockIdx.x * FRONT_TPB; c < qn; c += (u64)gridDim.x * FRONT_TPB) {
+        u64 lo = 0, hi = 0;
+        if (c + tid < qn) slot_range(d, q[c + tid], lo, hi);
+        const u32 len = (u32)(hi - lo);
+        const u64 some = __ballot(len != 0);
+        const u32 li = dpp_incl_scan32(len);
+        if (lane == 63) {
+            s_n[w] = __popcll(some);
+            s_len[w] = li;
+        }
+        __syncthreads();
+        u32 n0 = 0, l0 = 0, nt = 0, lt = 0;
+        for (u32 x = 0; x < NW; ++x) {
+            if (x == w) { n0 = nt; l0 = lt; }
+            nt += s_n[x];
+            lt += s_len[x];
+        }
+        if (tid == 0) s_base = nt ? atomicAdd((unsigned long long *)&ctl->ent[level & 3], ((u64)nt << 33) | lt) : 0;
+        __syncthreads();
+        const u32 eb = (u32)(s_base >> 33), pb = (u32)s_base;  // places: fewer than 2^32 slots
+        if (len) {
+            const u32 k = n0 + __popcll(some & ((1ull << lane) - 1ull));
+            const u32 o = l0 + li - len;
+            s_off[k] = o;
+            off[eb + k] = pb + o;
+            adj[eb + k] = (u32)lo - (pb + o);
+        }
+        __syncthreads();
+        const u64 end = (u64)pb + lt;
+        for (u64 r = ((u64)pb + BFS_RUN - 1) / BFS_RUN + tid; r * BFS_RUN < end; r += FRONT_TPB) {
+            const u32 t = (u32)(r * BFS_RUN - pb);
+            u32 x = 0, y = nt;
+            while (y - x > 1) {
+                const u32 m = (x + y) >> 1;
+                if (s_off[m] <= t) x = m; else y = m;
+            }
+            runs[r] = eb + x;
+        }
+        __syncthreads();
     }
 }
 
 static constexpr u32 EXP_TPB = 512;
-static constexpr u32 EXP_ITEMS = 4;
-static constexpr u32 EXP_RUN = EXP_TPB * EXP_ITEMS;  // slots per run
-static constexpr u32 EXP_STAGE = EXP_RUN + 1;        // staged entries: every entry of a run of non-empty
-                                                     // rows; empty rows past it use the global search
+static constexpr u32 EXP_WAVES = EXP_TPB / 64;
+static constexpr u32 EXP_Q = 2 * BFS_RUN;  // discovered vertices a wave holds: flushed before a run could outgrow them
 
-// last entry e in [lo, hi) with off[e] <= t (off[lo] <= t)
-__device__ __forceinline__ u32 entry_of(const u32 *__restrict__ off, u32 lo, u32 hi, u64 t) {
-    while (hi - lo > 1) {
-        const u32 m = (lo + hi) >> 1;
-        if ((u64)off[m] <= t) lo = m; else hi = m;
-    }
-    return lo;
-}
-
-// runs[r] = entry holding slot r * EXP_RUN
-__global__ void k_bfs_runs(const u32 *__restrict__ off, u32 qn, u32 *__restrict__ runs) {
-    const u64 total = off[qn];
-    const u64 nruns = (total + EXP_RUN - 1) / EXP_RUN;
-    for (u64 r = (u64)blockIdx.x * blockDim.x + threadIdx.x; r < nruns; r += (u64)gridDim.x * blockDim.x)
-        runs[r] = entry_of(off, 0, qn, r * EXP_RUN);
-}
-
-// Moves the workgroup's discovered vertices from LDS to the next frontier:
-// one atomic on the frontier size per flush.
-__device__ __forceinline__ void bfs_flush(u32 *s_q, u32 &s_n, u32 &s_base, u32 *__restrict__ qnext,
-                                          u32 *__restrict__ counters) {
-    const u32 n = s_n;  // read by all after the barrier that precedes the call
-    if (threadIdx.x == 0) s_base = atomicAdd(&counters[0], n);
-    __syncthreads();
-    const u32 base = s_base;
-    for (u32 k = threadIdx.x; k < n; k += EXP_TPB) qnext[base + k] = s_q[k];
-    __syncthreads();
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
-}
-
-// entries of a run's stage each thread loads (and later writes to LDS)
-static constexpr u32 EXP_SK = (EXP_STAGE + EXP_TPB - 1) / EXP_TPB;
-
-// the stage of the run starting at entry e0, into registers
-__device__ __forceinline__ void bfs_stage_load(const u32 *__restrict__ off, const u64 *__restrict__ first, u32 qn,
-                                               u32 e0, u32 (&p_off)[EXP_SK], u64 (&p_first)[EXP_SK]) {
-#pragma unroll
-    for (u32 k = 0; k < EXP_SK; ++k) {
-        const u32 kk = threadIdx.x + k * EXP_TPB;
-        const u64 idx = (u64)e0 + kk;
-        p_off[k] = (kk < EXP_STAGE && idx <= qn) ? off[idx] : 0xFFFFFFFFu;
-        p_first[k] = (kk < EXP_STAGE && idx < qn) ? first[idx] : 0ull;
-    }
-}
-
-__global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 qn, const u32 *__restrict__ off,
-                                                         const u64 *__restrict__ first,
-                                                         const u32 *__restrict__ runs, u32 *__restrict__ levels,
-                                                         u32 *__restrict__ visited, u32 level,
-                                                         u32 *__restrict__ qnext, u32 *__restrict__ counters) {
-    __shared__ u32 s_off[EXP_STAGE];
-    __shared__ u64 s_first[EXP_STAGE];
-    __shared__ u32 s_q[2 * EXP_RUN];  // discovered vertices; flushed once it holds EXP_RUN
-    __shared__ u32 s_n, s_base;
-    if (threadIdx.x == 0) s_n = 0;
-    const u64 total = off[qn];
-    const u64 nruns = (total + EXP_RUN - 1) / EXP_RUN;
-    const u32 lane = lane_id();
+__global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, const u32 *__restrict__ off,
+                                                         const u32 *__restrict__ adj, const u32 *__restrict__ runs,
+                                                         u32 *__restrict__ levels, u32 *__restrict__ visited,
+                                                         u32 *__restrict__ qnext, BfsCtl *__restrict__ ctl) {
+    __shared__ u32 s_adj[EXP_WAVES][BFS_RUN];
+    __shared__ u32 s_q[EXP_WAVES][EXP_Q];
+    __shared__ u32 s_first[EXP_WAVES][2 * BFS_ITEMS];  // a bit per place: an entry starts there
+    __shared__ u32 s_n[EXP_WAVES], s_scanned[EXP_WAVES], s_base;
+    const u32 lane = lane_id(), w = threadIdx.x >> 6;
+    const u64 ent = ctl->ent[level & 3];
+    const u64 total = ent & BFS_PLACES;
+    const u32 nent = (u32)(ent >> 33);
+    const u64 nruns = (total + BFS_RUN - 1) / BFS_RUN;
+    const u64 le = ~0ull >> (63 - lane);  // this lane and those below
     const u32 Smask = (1u << d.log2S) - 1;
     const gu64 *keys = (const gu64 *)d.keys;
-    u32 scanned = 0;
-    // a run's entry and stage are loaded one run ahead, into registers, and
-    // written to LDS once the previous run is done with the stage
-    u32 p_off[EXP_SK];
-    u64 p_first[EXP_SK];
-    u32 e0n = 0;
-    if (blockIdx.x < nruns) {
-        e0n = runs[blockIdx.x];
-        bfs_stage_load(off, first, qn, e0n, p_off, p_first);
+    u32 *next_n = &ctl->qn[(level + 1) & 3];
+    u32 scanned = 0, n = 0;
+    const u64 stride = (u64)gridDim.x * EXP_WAVES;
+    u64 run = (u64)blockIdx.x * EXP_WAVES + w;
+    // a run's first entries are loaded one run ahead
+    u32 e0 = 0, p_off = 0, p_adj = 0;
+    auto load = [&](u32 e) {
+        const bool in = e < nent;
+        p_off = in ? off[e] : ~0u;
+        p_adj = in ? adj[e] : 0u;
+    };
+    if (run < nruns) {
+        e0 = runs[run];
+        load(e0 + lane);
     }
-    for (u64 run = blockIdx.x; run < nruns; run += gridDim.x) {
-        const u64 t0 = run * EXP_RUN;
-        const u32 e0 = e0n;
-#pragma unroll
-        for (u32 k = 0; k < EXP_SK; ++k) {
-            const u32 kk = threadIdx.x + k * EXP_TPB;
-            if (kk < EXP_STAGE) {
-                s_off[kk] = p_off[k];
-                s_first[kk] = p_first[k];
+    for (; run < nruns; run += stride) {
+        const bool more = run + stride < nruns;
+        u32 e1 = 0;
+        if (more) e1 = runs[run + stride];
+        const u64 t0 = run * BFS_RUN;
+        if (lane < 2 * BFS_ITEMS) s_first[w][lane] = 0;
+        __builtin_amdgcn_wave_barrier();
+        for (u32 k = lane;; k += 64) {
+            // the first entry may begin before the run
+            const bool in = e0 + k < nent && (u64)p_off < t0 + BFS_RUN;
+            if (in) {
+                const u32 at = p_off > t0 ? (u32)(p_off - t0) : 0u;
+                s_adj[w][k] = p_adj;
+                atomicOr(&s_first[w][at >> 5], 1u << (at & 31));
             }
+            if (!__all(in)) break;
+            load(e0 + k + 64);
         }
-        __syncthreads();
-        const bool more = run + gridDim.x < nruns;  // uniform
-        if (more) e0n = runs[run + gridDim.x];
-        // slot of each item: the staged entry holding it, or the global search
-        // past the stage (only when empty rows fill it)
-        u64 slot[EXP_ITEMS];
-        bool ok[EXP_ITEMS];
-        const bool staged_all = (u64)s_off[EXP_STAGE - 1] > t0 + EXP_RUN - 1;
+        __builtin_amdgcn_wave_barrier();
+        u32 slot[BFS_ITEMS];
+        bool ok[BFS_ITEMS];
+        u32 before = 0;
 #pragma unroll
-        for (u32 i = 0; i < EXP_ITEMS; ++i) {
-            const u64 t = t0 + (u64)i * EXP_TPB + threadIdx.x;
+        for (u32 i = 0; i < BFS_ITEMS; ++i) {
+            const u64 m = (u64)s_first[w][2 * i + 1] << 32 | s_first[w][2 * i];
+            const u64 t = t0 + i * 64 + lane;
             ok[i] = t < total;
-            slot[i] = 0;
-            if (!ok[i]) continue;
-            if (staged_all || (u64)s_off[EXP_STAGE - 1] > t) {
-                u32 lo = 0, hi = EXP_STAGE - 1;  // s_off[0] <= t0 <= t
-                while (hi - lo > 1) {
-                    const u32 m = (lo + hi) >> 1;
-                    if ((u64)s_off[m] <= t) lo = m; else hi = m;
-                }
-                slot[i] = s_first[lo] + (t - s_off[lo]);
-            } else {
-                const u32 e = entry_of(off, e0 + EXP_STAGE - 1, qn, t);
-                slot[i] = first[e] + (t - off[e]);
-            }
+            const u32 k = before + __popcll(m & le) - 1;
+            slot[i] = ok[i] ? (u32)t + s_adj[w][k] : 0u;
+            before += __popcll(m);
         }
-        // the next run's stage: its entry has arrived during the searches
-        if (more) bfs_stage_load(off, first, qn, e0n, p_off, p_first);
-        u32 live[EXP_ITEMS];
+        u32 live[BFS_ITEMS];
 #pragma unroll
-        for (u32 i = 0; i < EXP_ITEMS; ++i) live[i] = d.cnt[slot[i] >> d.log2S];  // slot 0 when !ok: in bounds
-        u64 key[EXP_ITEMS];
+        for (u32 i = 0; i < BFS_ITEMS; ++i) live[i] = d.cnt[slot[i] >> d.log2S];  // slot 0 when !ok: in bounds
+        e0 = e1;
+        if (more) load(e1 + lane);
+        u64 key[BFS_ITEMS];
 #pragma unroll
-        for (u32 i = 0; i < EXP_ITEMS; ++i) {
+        for (u32 i = 0; i < BFS_ITEMS; ++i) {
             u64 k = KEY_NONE;
-            if (ok[i] && (u32)(slot[i] & Smask) < live[i]) k = keys[slot[i]];
+            if (ok[i] && (slot[i] & Smask) < live[i]) k = keys[slot[i]];
             key[i] = k;
         }
-        u32 vw[EXP_ITEMS];
+        u32 vw[BFS_ITEMS];
 #pragma unroll
-        for (u32 i = 0; i < EXP_ITEMS; ++i) vw[i] = key[i] != KEY_NONE ? visited[(u32)key[i] >> 5] : ~0u;
-#pragma unroll
-        for (u32 i = 0; i < EXP_ITEMS; ++i) {
-            bool found = false;
-            if (key[i] != KEY_NONE) {
-                ++scanned;
-                const u32 v = (u32)key[i], bit = 1u << (v & 31);
-                if (!(vw[i] & bit) && !(atomicOr(&visited[v >> 5], bit) & bit)) {
-                    found = true;
-                    levels[v] = level + 1;
-                }
-            }
-            const u64 m = __ballot(found);
-            if (m) {
-                const u32 lead = (u32)__builtin_ctzll(m);
-                u32 base = 0;
-                if (lane == lead) base = atomicAdd(&s_n, (u32)__popcll(m));  // LDS
-                base = __shfl(base, lead, 64);
-                if (found) s_q[base + __popcll(m & ((1ull << lane) - 1ull))] = (u32)key[i];
-            }
+        for (u32 i = 0; i < BFS_ITEMS; ++i) {
+            vw[i] = key[i] != KEY_NONE ? visited[(u32)key[i] >> 5] : ~0u;
+            scanned += key[i] != KEY_NONE;
         }
-        __syncthreads();  // the stage is rewritten by the next run; s_n is final for this run
-        if (s_n >= EXP_RUN) bfs_flush(s_q, s_n, s_base, qnext, counters);  // a run adds at most EXP_RUN
+        u32 old[BFS_ITEMS];
+#pragma unroll
+        for (u32 i = 0; i < BFS_ITEMS; ++i) {
+            const u32 v = (u32)key[i], bit = 1u << (v & 31);
+            old[i] = ~0u;
+            if (!(vw[i] & bit)) old[i] = atomicOr(&visited[v >> 5], bit);
+        }
+#pragma unroll
+        for (u32 i = 0; i < BFS_ITEMS; ++i) {
+            const u32 v = (u32)key[i];
+            const bool found = !((old[i] >> (v & 31)) & 1u);
+            const u64 m = __ballot(found);
+            if (found) {
+                levels[v] = level + 1;
+                s_q[w][n + __popcll(m & le) - 1] = v;
+            }
+            n += __popcll(m);
+        }
+        if (n > EXP_Q - BFS_RUN) {
+            u32 base = 0;
+            if (lane == 0) base = atomicAdd(next_n, n);
+            base = (u32)__builtin_amdgcn_readfirstlane((int)base);
+            __builtin_amdgcn_wave_barrier();
+            for (u32 k = lane; k < n; k += 64) qnext[base + k] = s_q[w][k];
+            __builtin_amdgcn_wave_barrier();
+            n = 0;
+        }
+    }
+    // what is left, with one atomic a workgroup
+    scanned = wave_sum(scanned);
+    if (lane == 0) {
+        s_n[w] = n;
+        s_scanned[w] = scanned;
     }
     __syncthreads();
-    if (s_n) bfs_flush(s_q, s_n, s_base, qnext, counters);
-    scanned = wave_sum(scanned);
-    if (lane == 0 && scanned) atomicAdd(&counters[1], scanned);
+    if (threadIdx.x == 0) {
+        u32 sum = 0, sc = 0;
+        for (u32 v = 0; v < EXP_WAVES; ++v) {
+            const u32 c = s_n[v];
+            s_n[v] = sum;
+            sum += c;
+            sc += s_scanned[v];
+        }
+        s_base = sum ? atomicAdd(next_n, sum) : 0u;
+        if (sc) atomicAdd((unsigned long long *)&ctl->scanned, (u64)sc);
+    }
+    __syncthreads();
+    const u32 base = s_base + s_n[w];
+    for (u32 k = lane; k < n; k += 64) qnext[base + k] = s_q[w][k];
 }
 
-hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *counters, u32 *visited, hipStream_t st) {
-    k_bfs_init<<<grid_for(V, 256, 16384), 256, 0, st>>>(levels, V, src, queue, counters, visited);
+hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visited, hipStream_t st) {
+    k_bfs_init<<<grid_for(V, 256, 16384), 256, 0, st>>>(levels, V, src, queue, (BfsCtl *)ctl, visited);
     return hipGetLastError();
 }
 
-u64 bfs_run_words(u64 slots) { return slots / EXP_RUN + 2; }
+u64 bfs_run_words(u64 slots) { return slots / BFS_RUN + 2; }
+
+void bfs_state(const u32 *ctl, u32 level, u32 &qn, u32 &depth, u64 &scanned) {
+    const BfsCtl *c = (const BfsCtl *)ctl;
+    qn = c->qn[level & 3];
+    depth = c->depth;
+    scanned = c->scanned;
+}
 
 // Default expansion grid: every workgroup resident at once (compute units x
-// workgroups per CU that fit), so the runs are shared out in one round; a
-// grid one resident round larger leaves its last workgroups a tail of their
-// own (2048 workgroups of 512 threads: 9.1 ms per search, 1024: 11.6, one
-// round of 768: 8.1 on MI355X).
+// workgroups per CU that fit), so the runs are shared out in one round.
 static u32 bfs_expand_grid() {
     static std::atomic<u32> cached[64];
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 2048;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 1024;
     u32 g = cached[dev].load(std::memory_order_relaxed);
     if (g) return g;
     int cus = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bfs_expand, EXP_TPB, 0) != hipSuccess || cus <= 0 ||
         per_cu <= 0)
-        return 2048;
+        return 1024;
     g = (u32)(cus * per_cu);
     cached[dev].store(g, std::memory_order_relaxed);
     return g;
 }
 
-hipError_t bfs_level(const DevState &d, const u32 *q, u32 qn, u32 *len, u64 *first, u32 *runs, u32 *scan_scratch,
-                     u32 *levels, u32 *visited, u32 level, u32 *qnext, u32 *counters, u32 expand_grid,
-                     hipStream_t st) {
-    k_bfs_len<<<grid_for(qn, 256, 16384), 256, 0, st>>>(d, q, qn, len, first);
-    (void)device_excl_scan(len, qn, len, scan_scratch, st);
-    k_bfs_runs<<<grid_for(bfs_run_words(nseg_of(d) << d.log2S), 256, 16384), 256, 0, st>>>(len, qn, runs);
-    k_bfs_expand<<<expand_grid ? expand_grid : bfs_expand_grid(), EXP_TPB, 0, st>>>(d, qn, len, first, runs, levels, visited,
-                                                                      level, qnext, counters);
+hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited, u32 level,
+                     u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st) {
+    k_bfs_front<<<grid_for(d.V, FRONT_TPB, 512), FRONT_TPB, 0, st>>>(d, level, q, (BfsCtl *)ctl, off, adj, runs);
+    k_bfs_expand<<<expand_grid ? expand_grid : bfs_expand_grid(), EXP_TPB, 0, st>>>(d, level, off, adj, runs, levels,
+                                                                                  visited, qnext, (BfsCtl *)ctl);
     return hipGetLastError();
 }
 
@@ -276,12 +341,6 @@ hipError_t bfs_level(const DevState &d, const u32 *q, u32 qn, u32 *len, u64 *fir
 // summed (Kahan) when the iteration finishes.
 
 static constexpr u32 PR_COPIES = 8;  // accumulator copies, one per XCD
-
-__device__ __forceinline__ u32 xcc_id() {
-    u32 x;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(x));
-    return x & (PR_COPIES - 1);
-}
 
 // hi += x with the rounding error of that add going to lo
 __device__ __forceinline__ void atomic_add2(float *hi, float *lo, float x) {

@@ -1616,52 +1616,39 @@ int lpma_check(lpma_t *h, uint64_t *violations, void *stream) {
 static int bfs_core(int device, const DevState &d, u32 src, u32 *d_levels, u32 *depth, u64 *edges_scanned,
                     u32 expand_grid, hipStream_t st) {
     const u64 V = d.V;
-    DBuf<u32> q0, q1, len, cnt, scan, runs, visited;
-    DBuf<u64> first;
+    DBuf<u32> q0, q1, off, adj, runs, ctl, visited;
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(st);
-        release_on(device, q0); release_on(device, q1); release_on(device, len); release_on(device, cnt);
-        release_on(device, scan); release_on(device, runs); release_on(device, first); release_on(device, visited);
+        release_on(device, q0); release_on(device, q1); release_on(device, off); release_on(device, adj);
+        release_on(device, runs); release_on(device, ctl); release_on(device, visited);
     };
     int r;
     if ((r = ensure_on(device, st, q0, V + 1)) || (r = ensure_on(device, st, q1, V + 1)) ||
-        (r = ensure_on(device, st, len, V + 2)) || (r = ensure_on(device, st, scan, scan_scratch_words(V + 1) + 8)) ||
-        (r = ensure_on(device, st, cnt, 4)) || (r = ensure_on(device, st, first, V + 1)) ||
+        (r = ensure_on(device, st, off, V + 1)) || (r = ensure_on(device, st, adj, V + 1)) ||
         (r = ensure_on(device, st, runs, bfs_run_words(nseg_of(d) << d.log2S))) ||
-        (r = ensure_on(device, st, visited, bfs_visited_words(V)))) {
+        (r = ensure_on(device, st, ctl, BFS_CTL_WORDS)) || (r = ensure_on(device, st, visited, bfs_visited_words(V)))) {
         cleanup();
         return r;
     }
-    if (bfs_init(d_levels, d.V, src, q0.p, cnt.p, visited.p, st) != hipSuccess) {
-        (void)hipGetLastError();
-        cleanup();
-        return LPMA_ERR_DEVICE;
-    }
-    u32 *q = q0.p, *qn_buf = q1.p;
-    u32 qn = 1, level = 0;
+    u32 *q[2] = {q0.p, q1.p};
+    bool ok = bfs_init(d_levels, d.V, src, q[0], ctl.p, visited.p, st) == hipSuccess;
+    u32 level = 0, qn = 1, levels_done = 0;
     u64 scanned = 0;
-    u32 c[2];
-    int rc = LPMA_OK;
-    while (qn) {
-        if (bfs_level(d, q, qn, len.p, first.p, runs.p, scan.p, d_levels, visited.p, level, qn_buf, cnt.p, expand_grid,
-                      st) != hipSuccess ||
-            hipMemcpyAsync(c, cnt.p, sizeof(c), hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess || fill_u32(cnt.p, 2, 0, st) != hipSuccess) {
-            (void)hipGetLastError();
-            rc = LPMA_ERR_DEVICE;
-            break;
-        }
-        scanned += c[1];
-        qn = c[0];
-        std::swap(q, qn_buf);
-        ++level;
+    while (ok && qn) {
+        for (u32 k = 0; ok && k < BFS_AHEAD; ++k, ++level)
+            ok = bfs_level(d, q[level & 1], off.p, adj.p, runs.p, d_levels, visited.p, level, q[(level + 1) & 1], ctl.p,
+                           expand_grid, st) == hipSuccess;
+        alignas(8) u32 c[BFS_CTL_WORDS];
+        ok = ok && hipMemcpyAsync(c, ctl.p, sizeof(c), hipMemcpyDeviceToHost, st) == hipSuccess &&
+             hipStreamSynchronize(st) == hipSuccess;
+        if (ok) bfs_state(c, level, qn, levels_done, scanned);
     }
+    if (!ok) (void)hipGetLastError();
     cleanup();
-    if (rc == LPMA_OK) {
-        if (depth) *depth = level;
-        if (edges_scanned) *edges_scanned = scanned;
-    }
-    return rc;
+    if (!ok) return LPMA_ERR_DEVICE;
+    if (depth) *depth = levels_done;
+    if (edges_scanned) *edges_scanned = scanned;
+    return LPMA_OK;
 }
 
 int lpma_bfs(lpma_t *h, uint32_t src, uint32_t *d_levels, uint32_t *depth, uint64_t *edges_scanned, void *stream) {

@@ -173,12 +173,12 @@ int grow_pin(Pin<T> &b, u64 n, hipStream_t st) {
     return LPMA_OK;
 }
 
-// device scratch of one search: per vertex two queues, the counts, the first
-// slots and the levels (32 B) and a visited bit; one run entry per 1024 slots
-// (a snapshot holds at least 8 B per slot, so snapshot bytes / 2048 covers
-// it); the scan
+// device scratch of one search: per vertex two queues, an entry's two words
+// and the level (20 B) and a visited bit; one run entry per 256 slots (a
+// snapshot holds at least 8 B per slot, so snapshot bytes / 512 covers it);
+// the control words
 u64 bfs_bytes(u32 V, u64 snap_bytes) {
-    return 32ull * ((u64)V + 2) + (u64)V / 8 + 64 + snap_bytes / 2048 + (1ull << 20);
+    return 20ull * ((u64)V + 2) + (u64)V / 8 + 64 + snap_bytes / 512 + (1ull << 20);
 }
 
 void finish(lpma_server *s, Request *r, int status) {

@@ -86,6 +86,54 @@ def test_bfs_frontier_of_empty_rows():
     pma.close()
 
 
+def bfs_shape(shape):
+    """(V, edge sources, edge destinations)"""
+    if shape == "lone":  # no edges at all
+        return 1, [], []
+    if shape == "path":  # many more levels than are queued at a time
+        n = 131
+        return n, np.arange(n - 1), np.arange(1, n)
+    if shape == "star":  # one row over many runs, then many empty ones
+        n = 70001
+        return n, np.zeros(n - 1, dtype=np.int64), np.arange(1, n)
+    if shape == "ones":  # rows of one edge: as many entries as places in a run
+        n = 5000
+        return 2 * n + 1, np.concatenate([np.zeros(n, dtype=np.int64), np.arange(1, n + 1)]), np.concatenate(
+            [np.arange(1, n + 1), np.arange(n + 1, 2 * n + 1)])
+    n = 3001  # rows of every length from 0 to 300 and back
+    rng = np.random.default_rng(17)
+    src = np.repeat(np.arange(n), np.abs(np.arange(n) % 601 - 300))
+    return n, src, rng.integers(0, n, src.size)
+
+
+@pytest.mark.parametrize("shape", ["lone", "path", "star", "ones", "ramp"])
+@pytest.mark.parametrize("slots", [16, 128])
+def test_bfs_shapes(shape, slots):
+    """Searches of one live graph and of its snapshot, the latter with the
+    default width and with one workgroup."""
+    from gpu_util import keys_of
+    V, s, d = bfs_shape(shape)
+    say(f"bfs {shape} S={slots}")
+    keys = oracle.sort_unique(keys_of(np.asarray(s, dtype=np.int64), np.asarray(d, dtype=np.int64)))
+    pma = L.PMA(V, segment_slots=slots)
+    if keys.size:
+        pma.insert(keys)
+    snap = L.Snapshot(pma)
+    deg = np.diff(oracle.csr_of(keys, V)[0].astype(np.int64))
+    for src in {0, V // 2, V - 1}:
+        want = oracle.bfs(keys, V, src)
+        reached = want != 0xFFFFFFFF
+        for width in (None, 0, 1):
+            if width is not None:
+                assert L.lib().lpma_snapshot_set_search_width(snap._h, width) == 0
+            lv, depth, scanned = pma.bfs(src) if width is None else snap.bfs(src)
+            assert np.array_equal(lv.cpu().numpy().view(np.uint32), want)
+            assert depth == int(want[reached].max()) + 1
+            assert scanned == int(deg[reached].sum())
+    snap.close()
+    pma.close()
+
+
 def test_pagerank_partial_last_bin():
     """V = 20000: three destination bins of 8192 vertices, the last one
     partial; uniform edges with a tenth of the vertices dangling."""
