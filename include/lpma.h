@@ -186,9 +186,13 @@ int lpma_edge_query(lpma_t *h, const uint64_t *d_keys, uint64_t n, uint32_t *d_r
  * out-degree of d_srcs[i] (0 for ids >= num_vertices). */
 int lpma_neighbor_count(lpma_t *h, const uint32_t *d_srcs, uint64_t n, uint32_t *d_len, void *stream);
 
+/* The exclusive scan of lpma_neighbor_count's lengths, d_offsets[n] included
+ * (modulo 2^32), and their total; waits for the total. */
+int lpma_neighbor_offsets(lpma_t *h, const uint32_t *d_srcs, uint64_t n, uint32_t *d_offsets, uint64_t *total,
+                          void *stream);
+
 /* Writes the neighbors (dst ids, ascending) of d_srcs[i] at
- * d_out[d_offsets[i] ...]; d_offsets typically the exclusive scan of
- * lpma_neighbor_count's lengths. */
+ * d_out[d_offsets[i] ...]; d_offsets typically from lpma_neighbor_offsets. */
 int lpma_neighbor_gather(lpma_t *h, const uint32_t *d_srcs, uint64_t n, const uint32_t *d_offsets, uint32_t *d_out,
                          void *stream);
 
@@ -213,6 +217,8 @@ int lpma_snapshot_destroy(lpma_snapshot_t *s);
 int lpma_snapshot_get_view(const lpma_snapshot_t *s, lpma_view_t *out);
 int lpma_snapshot_neighbor_count(lpma_snapshot_t *s, const uint32_t *d_srcs, uint64_t n, uint32_t *d_len,
                                  void *stream);
+int lpma_snapshot_neighbor_offsets(lpma_snapshot_t *s, const uint32_t *d_srcs, uint64_t n, uint32_t *d_offsets,
+                                   uint64_t *total, void *stream);
 int lpma_snapshot_neighbor_gather(lpma_snapshot_t *s, const uint32_t *d_srcs, uint64_t n, const uint32_t *d_offsets,
                                   uint32_t *d_out, void *stream);
 int lpma_snapshot_edge_query(lpma_snapshot_t *s, const uint64_t *d_keys, uint64_t n, uint32_t *d_result,

@@ -131,6 +131,7 @@ SIGNATURES = [
     ("lpma_to_csr", _int, [_vp, _vp, _vp, _vp]),
     ("lpma_edge_query", _int, [_vp, _vp, _u64, _vp, _vp]),
     ("lpma_neighbor_count", _int, [_vp, _vp, _u64, _vp, _vp]),
+    ("lpma_neighbor_offsets", _int, [_vp, _vp, _u64, _vp, ctypes.POINTER(_u64), _vp]),
     ("lpma_neighbor_gather", _int, [_vp, _vp, _u64, _vp, _vp, _vp]),
     ("lpma_check", _int, [_vp, ctypes.POINTER(_u64), _vp]),
     ("lpma_bfs", _int, [_vp, _u32, _vp, ctypes.POINTER(_u32), ctypes.POINTER(_u64), _vp]),
@@ -163,6 +164,7 @@ SIGNATURES = [
     ("lpma_snapshot_create", _int, [ctypes.POINTER(_vp), _vp, _vp]),
     ("lpma_snapshot_destroy", _int, [_vp]),
     ("lpma_snapshot_get_view", _int, [_vp, ctypes.POINTER(View)]),
+    ("lpma_snapshot_neighbor_offsets", _int, [_vp, _vp, _u64, _vp, ctypes.POINTER(_u64), _vp]),
     ("lpma_snapshot_neighbor_count", _int, [_vp, _vp, _u64, _vp, _vp]),
     ("lpma_snapshot_neighbor_gather", _int, [_vp, _vp, _u64, _vp, _vp, _vp]),
     ("lpma_snapshot_edge_query", _int, [_vp, _vp, _u64, _vp, _vp]),
@@ -475,18 +477,16 @@ class PMA:
         torch = _torch()
         srcs = srcs.to(self.device, torch.int32).contiguous()
         n = srcs.numel()
-        ln = torch.empty(max(n, 1), dtype=torch.int32, device=self.device)
-        _check(lib().lpma_neighbor_count(self._h, srcs.data_ptr(), n, ln.data_ptr(), _stream_ptr(self.stream)),
-               "neighbor_count")
-        offs = torch.zeros(n + 1, dtype=torch.int64, device=self.device)
-        if n:
-            offs[1:] = torch.cumsum(ln[:n].to(torch.int64), 0)
-        total = int(offs[-1].item())
-        offs32 = offs.to(torch.int32)
+        offs = torch.empty(n + 1, dtype=torch.int32, device=self.device)
+        total = _u64(0)
+        st = _stream_ptr(self.stream)
+        _check(lib().lpma_neighbor_offsets(self._h, srcs.data_ptr(), n, offs.data_ptr(), ctypes.byref(total), st),
+               "neighbor_offsets")
+        total = int(total.value)
         out = torch.empty(max(total, 1), dtype=torch.int32, device=self.device)
-        _check(lib().lpma_neighbor_gather(self._h, srcs.data_ptr(), n, offs32.data_ptr(), out.data_ptr(),
-                                          _stream_ptr(self.stream)), "neighbor_gather")
-        return offs32, out[:total]
+        _check(lib().lpma_neighbor_gather(self._h, srcs.data_ptr(), n, offs.data_ptr(), out.data_ptr(), st),
+               "neighbor_gather")
+        return offs, out[:total]
 
     def bfs(self, src):
         """(levels int32 device tensor, depth, live edges scanned); unreached = -1."""
@@ -577,18 +577,16 @@ class Snapshot:
         torch = _torch()
         srcs = srcs.to(self.device, torch.int32).contiguous()
         n = srcs.numel()
-        ln = torch.empty(max(n, 1), dtype=torch.int32, device=self.device)
-        _check(lib().lpma_snapshot_neighbor_count(self._h, srcs.data_ptr(), n, ln.data_ptr(),
-                                                  _stream_ptr(self.stream)), "snapshot_neighbor_count")
-        offs = torch.zeros(n + 1, dtype=torch.int64, device=self.device)
-        if n:
-            offs[1:] = torch.cumsum(ln[:n].to(torch.int64), 0)
-        total = int(offs[-1].item())
-        offs32 = offs.to(torch.int32)
+        offs = torch.empty(n + 1, dtype=torch.int32, device=self.device)
+        total = _u64(0)
+        st = _stream_ptr(self.stream)
+        _check(lib().lpma_snapshot_neighbor_offsets(self._h, srcs.data_ptr(), n, offs.data_ptr(),
+                                                    ctypes.byref(total), st), "snapshot_neighbor_offsets")
+        total = int(total.value)
         out = torch.empty(max(total, 1), dtype=torch.int32, device=self.device)
-        _check(lib().lpma_snapshot_neighbor_gather(self._h, srcs.data_ptr(), n, offs32.data_ptr(), out.data_ptr(),
-                                                   _stream_ptr(self.stream)), "snapshot_neighbor_gather")
-        return offs32, out[:total]
+        _check(lib().lpma_snapshot_neighbor_gather(self._h, srcs.data_ptr(), n, offs.data_ptr(), out.data_ptr(),
+                                                   st), "snapshot_neighbor_gather")
+        return offs, out[:total]
 
     def bfs(self, src):
         torch = _torch()

@@ -119,6 +119,9 @@ u64 export_static_max_segments();
 hipError_t export_compacted_static(int device, const DevState &d, u64 *edge_keys, u32 *row_std, hipStream_t st);
 hipError_t edge_query(const DevState &d, const u64 *q, u64 n, u32 *res, hipStream_t st);
 hipError_t neighbor_count(const DevState &d, const u32 *srcs, u64 n, u32 *len, hipStream_t st);
+hipError_t neighbor_offsets(const DevState &d, const u32 *srcs, u64 n, u32 *offs, u64 *word, u64 *host,
+                            hipStream_t st);
+bool neighbor_total(u64 word, u64 &total);  // of the word neighbor_offsets stores for the host
 hipError_t neighbor_gather(const DevState &d, const u32 *srcs, u64 n, const u32 *offs, u32 *out, hipStream_t st);
 hipError_t check_invariants(const DevState &d, u32 *err, hipStream_t st);
 

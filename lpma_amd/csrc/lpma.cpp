@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <map>
 #include <mutex>
 #include <new>
@@ -279,6 +280,68 @@ struct lpma_snapshot {
 namespace {
 
 std::atomic<u32> g_epoch{0};
+
+// Words of a call that waits for a kernel's result without the stream: a
+// pinned word the kernel stores and the host polls, and a device word that is
+// zero between calls.  A call takes a pair and gives it back once the kernel
+// has stored its result, so calls on any threads and streams have their own; a
+// device has at most WORDS_MAX pairs, and further calls wait for one.
+struct WordPair {
+    u64 *host = nullptr, *dev = nullptr;
+};
+static constexpr size_t WORDS_MAX = 64;
+struct WordPool {
+    std::mutex mu;
+    std::condition_variable cv;
+    WordPair free[WORDS_MAX];
+    size_t nfree = 0, made = 0;
+};
+std::mutex g_words_mu;
+std::map<int, WordPool *> g_words;
+
+WordPool &words_for(int dev) {
+    std::lock_guard<std::mutex> g(g_words_mu);
+    WordPool *&p = g_words[dev];
+    if (!p) p = new WordPool();
+    return *p;
+}
+
+// p null: a pair that must not be used again (a kernel may still store to it)
+void words_give(int dev, const WordPair *p) {
+    WordPool &W = words_for(dev);
+    {
+        std::lock_guard<std::mutex> g(W.mu);
+        if (p) W.free[W.nfree++] = *p; else --W.made;
+    }
+    W.cv.notify_one();
+}
+
+int words_take(int dev, hipStream_t st, WordPair &out) {
+    WordPool &W = words_for(dev);
+    {
+        std::unique_lock<std::mutex> g(W.mu);
+        W.cv.wait(g, [&] { return W.nfree || W.made < WORDS_MAX; });
+        if (W.nfree) {
+            out = W.free[--W.nfree];
+            return LPMA_OK;
+        }
+        ++W.made;
+    }
+    void *p = nullptr;
+    int r = pool_alloc(dev, &p, sizeof(u64));
+    out.dev = (u64 *)p;
+    if (r == LPMA_OK && (injected_failure() || hipHostMalloc((void **)&out.host, sizeof(u64),
+                                                             hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess))
+        r = LPMA_ERR_OUT_OF_MEMORY;
+    else if (r == LPMA_OK && fill_u64(out.dev, 1, 0, st) != hipSuccess)
+        r = LPMA_ERR_DEVICE;
+    if (r == LPMA_OK) return r;
+    (void)hipGetLastError();
+    if (out.host) (void)hipHostFree(out.host);
+    pool_free(dev, out.dev);
+    words_give(dev, nullptr);
+    return r;
+}
 
 struct DevGuard {
     int prev = -1;
@@ -663,6 +726,23 @@ int wait_word(const u64 *word, hipStream_t st, u64 &out, Done done) {
         }
         __builtin_ia32_pause();
     }
+}
+
+// Neighbor lists' offsets, and their total once the kernel has stored it.  A
+// pair whose kernel did not come to its end is not used again.
+int neighbor_offsets_core(int device, const DevState &d, const u32 *srcs, u64 n, u32 *offs, u64 *total,
+                          hipStream_t st) {
+    WordPair p;
+    CHECKED(words_take(device, st, p));
+    __atomic_store_n(p.host, 0ull, __ATOMIC_RELEASE);
+    int r = LPMA_ERR_DEVICE;
+    u64 w;
+    if (neighbor_offsets(d, srcs, n, offs, p.dev, p.host, st) == hipSuccess)
+        r = wait_word(p.host, st, w, [total](u64 x) { return neighbor_total(x, *total); });
+    else
+        (void)hipGetLastError();
+    words_give(device, r == LPMA_OK ? &p : nullptr);
+    return r;
 }
 
 // One PMA's share of a pipeline run.
@@ -1590,6 +1670,13 @@ int lpma_neighbor_count(lpma_t *h, const uint32_t *d_srcs, uint64_t n, uint32_t 
     return LPMA_OK;
 }
 
+int lpma_neighbor_offsets(lpma_t *h, const uint32_t *d_srcs, uint64_t n, uint32_t *d_offsets, uint64_t *total,
+                          void *stream) {
+    if (!h || (!d_srcs && n) || !d_offsets || !total) return LPMA_ERR_INVALID_ARGUMENT;
+    DevGuard guard(h->device);
+    return neighbor_offsets_core(h->device, h->st, d_srcs, n, d_offsets, total, (hipStream_t)stream);
+}
+
 int lpma_neighbor_gather(lpma_t *h, const uint32_t *d_srcs, uint64_t n, const uint32_t *d_offsets, uint32_t *d_out,
                          void *stream) {
     if (!h || ((!d_srcs || !d_offsets || !d_out) && n)) return LPMA_ERR_INVALID_ARGUMENT;
@@ -1750,6 +1837,14 @@ int lpma_snapshot_neighbor_count(lpma_snapshot_t *s, const uint32_t *d_srcs, uin
     CHECKED(snapshot_wait(s, (hipStream_t)stream));
     HIPCHECK(neighbor_count(s->st, d_srcs, n, d_len, (hipStream_t)stream));
     return LPMA_OK;
+}
+
+int lpma_snapshot_neighbor_offsets(lpma_snapshot_t *s, const uint32_t *d_srcs, uint64_t n, uint32_t *d_offsets,
+                                   uint64_t *total, void *stream) {
+    if (!s || (!d_srcs && n) || !d_offsets || !total) return LPMA_ERR_INVALID_ARGUMENT;
+    DevGuard guard(s->device);
+    CHECKED(snapshot_wait(s, (hipStream_t)stream));
+    return neighbor_offsets_core(s->device, s->st, d_srcs, n, d_offsets, total, (hipStream_t)stream);
 }
 
 int lpma_snapshot_neighbor_gather(lpma_snapshot_t *s, const uint32_t *d_srcs, uint64_t n, const uint32_t *d_offsets,

@@ -176,27 +176,115 @@ hipError_t edge_query(const DevState &d, const u64 *q, u64 n, u32 *res, hipStrea
 // Neighbor lists (query_rpma, rpma.cuh:1827-2036, without the time window):
 // row r's edges are the live slots strictly between the markers of rows
 // r-1 and r, i.e. slots (row_off[r], row_off[r+1]) (from slot 0 for r = 0).
-// One wave per queried vertex walks that slot range.
 __device__ __forceinline__ void row_range(const DevState &d, u32 r, u64 &lo, u64 &hi) {
     lo = r == 0 ? 0 : (u64)d.row_off[r] + 1;
     hi = d.row_off[r + 1];
 }
 
-__global__ void k_nbr_count(DevState d, const u32 *__restrict__ srcs, u64 n, u32 *__restrict__ len) {
-    const u64 waves = ((u64)gridDim.x * blockDim.x) >> 6;
+// Live edges of this lane's row r (0 when !ok), from the segment counts: a
+// segment's live slots are its first ones and both markers are live, so a row
+// inside one segment has no gaps, and one over several has the rest of its
+// first segment's live slots, every live slot of the middle ones, and the
+// slots before its marker in the last.  A wave sums a long row together.  Every
+// lane of the wave active.
+__device__ __forceinline__ u32 row_live(const DevState &d, u32 r, bool ok) {
+    const u32 Smask = (1u << d.log2S) - 1;
+    u64 lo = 0, hi = 0;
+    if (ok) row_range(d, r, lo, hi);
+    const u32 a = (u32)(lo >> d.log2S), b = (u32)(hi >> d.log2S);
+    u32 c = (u32)(hi - lo);
+    if (a != b) {
+        c = d.cnt[a] - ((u32)lo & Smask) + ((u32)hi & Smask);
+        if (b - a <= 8)
+            for (u32 k = a + 1; k < b; ++k) c += d.cnt[k];
+    }
     const u32 lane = lane_id();
-    for (u64 i = ((u64)blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < n; i += waves) {
-        u32 r = srcs[i];
-        u32 c = 0;
-        if (r < d.V) {
-            u64 lo, hi;
-            row_range(d, r, lo, hi);
-            for (u64 t = lo + lane; t < hi; t += 64) c += d.keys[t] != KEY_NONE ? 1u : 0u;
-        }
-        c = wave_sum(c);
-        if (lane == 0) len[i] = c;
+    for (u64 m = __ballot(b - a > 8); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const u32 x = (u32)__builtin_amdgcn_readlane((int)a, l), y = (u32)__builtin_amdgcn_readlane((int)b, l);
+        u32 sum = 0;
+#pragma unroll 4
+        for (u32 k = x + 1 + lane; k < y; k += 64) sum += d.cnt[k];
+        sum = wave_sum(sum);
+        if (lane == (u32)l) c += sum;
+    }
+    return c;
+}
+
+__global__ __launch_bounds__(256) void k_nbr_count(DevState d, const u32 *__restrict__ srcs, u64 n,
+                                                    u32 *__restrict__ len) {
+    for (u64 i0 = (u64)blockIdx.x * 256; i0 < n; i0 += (u64)gridDim.x * 256) {
+        const u64 i = i0 + threadIdx.x;
+        const u32 r = i < n ? srcs[i] : 0xFFFFFFFFu;
+        const u32 c = row_live(d, r, r < d.V);
+        if (i < n) len[i] = c;
     }
 }
+
+// Offsets of the rows' neighbor lists: counts and their exclusive prefix, the
+// total stored where the host polls for it.  A workgroup takes `per` rows; with
+// several, each leaves its sum in the place of its first offset (which is 0
+// within the workgroup) and adds it to `word` with its arrival (bits 48 up),
+// and the last to arrive turns the sums into bases, which k_nbr_base adds to
+// the offsets after them.  `word` is 0 between calls.
+// Bound: latency (row offsets, then counts; 512 rows: 6 us with the launch).
+static constexpr u32 NBR_TPB = 1024;  // also the most workgroups: one base a thread
+static constexpr u64 NBR_DONE = 1ull << 63;
+
+__global__ __launch_bounds__(NBR_TPB) void k_nbr_offsets(DevState d, const u32 *__restrict__ srcs, u64 n, u64 per,
+                                                          u32 *__restrict__ offs, u64 *__restrict__ word,
+                                                          u64 *__restrict__ host) {
+    __shared__ u64 tmp[NBR_TPB / 64 + 1];
+    __shared__ u64 s_total;
+    __shared__ u32 s_last;
+    const u32 t = threadIdx.x;
+    const u64 first = blockIdx.x * per;
+    u64 carry = 0;
+    for (u64 k = 0; k < per && first + k < n; k += NBR_TPB) {
+        const u64 i = first + k + t;
+        const u32 r = i < n ? srcs[i] : 0xFFFFFFFFu;
+        const u64 c = row_live(d, r, r < d.V);
+        u64 total;
+        const u64 x = carry + block_excl_scan<NBR_TPB, u64>(c, total, tmp);
+        carry += total;
+        if (i < n && (i != first || gridDim.x == 1)) offs[i] = (u32)x;
+        __syncthreads();
+    }
+    if (gridDim.x > 1) {
+        if (t == 0) {
+            __hip_atomic_store(&offs[first], (u32)carry, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const u64 old = __hip_atomic_fetch_add(word, (1ull << 48) | carry, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+            s_last = (old >> 48) == gridDim.x - 1;
+            s_total = (old & ((1ull << 48) - 1)) + carry;
+        }
+        __syncthreads();
+        if (!s_last) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        carry = s_total;
+        u32 sum = 0;
+        if (t < gridDim.x) sum = __hip_atomic_load(&offs[t * per], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        u32 total;
+        const u32 x = block_excl_scan<NBR_TPB, u32>(sum, total, (u32 *)tmp);
+        if (t < gridDim.x) offs[t * per] = x;
+        if (t == 0) __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (t == 0) {
+        offs[n] = (u32)carry;
+        __hip_atomic_store(host, NBR_DONE | carry, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+__global__ __launch_bounds__(NBR_TPB) void k_nbr_base(u64 n, u64 per, u32 *__restrict__ offs) {
+    const u64 i = (u64)blockIdx.x * NBR_TPB + threadIdx.x;
+    const u64 first = (u64)blockIdx.x * NBR_TPB / per * per;
+    if (i < n && i != first) offs[i] += offs[first];
+}
+
+// A wave per row, NBR_LOADS rounds of 64 slots in flight (one at a time left a
+// row of 20000 slots 300 memory latencies).
+static constexpr u32 NBR_LOADS = 4;
 
 __global__ void k_nbr_gather(DevState d, const u32 *__restrict__ srcs, u64 n, const u32 *__restrict__ offs,
                              u32 *__restrict__ out) {
@@ -208,21 +296,43 @@ __global__ void k_nbr_gather(DevState d, const u32 *__restrict__ srcs, u64 n, co
         u64 lo, hi;
         row_range(d, r, lo, hi);
         u64 o = offs[i];
-        for (u64 t0 = lo; t0 < hi; t0 += 64) {
-            u64 t = t0 + lane;
-            u64 key = t < hi ? d.keys[t] : KEY_NONE;
-            bool live = key != KEY_NONE;
-            u64 m = __ballot(live);
-            if (live) out[o + __popcll(m & ((1ull << lane) - 1ull))] = (u32)key;
-            o += __popcll(m);
+        for (u64 t0 = lo; t0 < hi; t0 += 64 * NBR_LOADS) {
+            u64 key[NBR_LOADS];
+#pragma unroll
+            for (u32 k = 0; k < NBR_LOADS; ++k) {
+                const u64 t = t0 + k * 64 + lane;
+                key[k] = t < hi ? d.keys[t] : KEY_NONE;
+            }
+#pragma unroll
+            for (u32 k = 0; k < NBR_LOADS; ++k) {
+                const bool live = key[k] != KEY_NONE;
+                const u64 m = __ballot(live);
+                if (live) out[o + __popcll(m & ((1ull << lane) - 1ull))] = (u32)key[k];
+                o += __popcll(m);
+            }
         }
     }
 }
 
 hipError_t neighbor_count(const DevState &d, const u32 *srcs, u64 n, u32 *len, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    k_nbr_count<<<grid_for(n * 64, 256, 16384), 256, 0, st>>>(d, srcs, n, len);
+    k_nbr_count<<<grid_for(n, 256, 16384), 256, 0, st>>>(d, srcs, n, len);
     return hipGetLastError();
+}
+
+hipError_t neighbor_offsets(const DevState &d, const u32 *srcs, u64 n, u32 *offs, u64 *word, u64 *host,
+                            hipStream_t st) {
+    const u64 blocks = std::max<u64>(1, (n + NBR_TPB - 1) / NBR_TPB);
+    const u64 per = (blocks + NBR_TPB - 1) / NBR_TPB * NBR_TPB;
+    const u32 grid = (u32)std::max<u64>(1, (n + per - 1) / per);
+    k_nbr_offsets<<<grid, NBR_TPB, 0, st>>>(d, srcs, n, per, offs, word, host);
+    if (grid > 1) k_nbr_base<<<(u32)blocks, NBR_TPB, 0, st>>>(n, per, offs);
+    return hipGetLastError();
+}
+
+bool neighbor_total(u64 word, u64 &total) {
+    total = word & ~NBR_DONE;
+    return word & NBR_DONE;
 }
 
 hipError_t neighbor_gather(const DevState &d, const u32 *srcs, u64 n, const u32 *offs, u32 *out, hipStream_t st) {

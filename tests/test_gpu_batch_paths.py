@@ -219,3 +219,83 @@ def test_many_sources():
         assert np.array_equal(ro.cpu().numpy().view(np.uint32), oracle.row_offsets(ref, V))
         assert pma.check() == 0
         pma.close()
+
+
+# neighbor offsets: one workgroup takes 1024 rows and alone stores its result;
+# rows inside one segment, over a few (a lane sums them) and over many (a wave
+# does), empty ones, ids out of range and repeats
+@pytest.mark.parametrize("n", [0, 1, 63, 1024, 1025, 5000, (1 << 20) + 1])
+@pytest.mark.parametrize("slots", [16, 64])
+def test_neighbor_lists(n, slots):
+    import torch
+    V = 3000
+    rng = np.random.default_rng(n + slots)
+    say(f"neighbors n={n} S={slots}")
+    hub = np.arange(0, V, 2)
+    ref = np.concatenate([rand_keys(rng, V, 30000), keys_of(np.full(hub.size, 7), hub),
+                          keys_of(np.full(200, V - 1), rng.integers(0, V, 200))])
+    ref = oracle.sort_unique(ref[(ref >> np.uint64(32)) % np.uint64(11) != 0])
+    pma = L.PMA(V, segment_slots=slots)
+    pma.insert(ref)
+    gone = rng.choice(ref, 3000, replace=False)  # gaps
+    pma.delete(gone)
+    ref = oracle.apply(ref, (), gone)
+    ro = oracle.row_offsets(ref, V).astype(np.int64)
+    srcs = rng.integers(0, V + 2, n)
+    srcs[: min(n, 8)] = [7, V - 1, 0, V, 7, 11, -1, 1][: min(n, 8)]
+    at = np.where((srcs >= 0) & (srcs < V), srcs, 0)
+    ln = np.where((srcs >= 0) & (srcs < V), ro[at + 1] - ro[at], 0)
+    want = np.concatenate([[0], np.cumsum(ln)])
+    inner = np.arange(want[-1]) - np.repeat(want[:-1], ln)
+    vals = (ref & np.uint64(0xFFFFFFFF)).astype(np.int64)[np.repeat(ro[at], ln) + inner]
+    snap = L.Snapshot(pma)
+    for store in (pma, snap, pma):
+        offs, nb = store.neighbors(torch.from_numpy(srcs.astype(np.int32)))
+        assert offs.dtype == torch.int32 and nb.dtype == torch.int32
+        assert np.array_equal(offs.cpu().numpy(), want)
+        assert np.array_equal(nb.cpu().numpy(), vals)
+    ln_dev = torch.empty(max(n, 1), dtype=torch.int32, device="cuda")
+    s_dev = torch.from_numpy(srcs.astype(np.int32)).cuda()
+    assert L.lib().lpma_neighbor_count(pma._h, s_dev.data_ptr(), n, ln_dev.data_ptr(), None) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(ln_dev.cpu().numpy()[:n], ln)
+    snap.close()
+    pma.close()
+
+
+def test_neighbor_lists_from_threads():
+    """Calls at once on one handle, each on a stream of its own."""
+    import threading
+    import torch
+    V = 2000
+    rng = np.random.default_rng(5)
+    ref = oracle.sort_unique(rand_keys(rng, V, 30000))
+    pma = L.PMA(V)
+    pma.insert(ref)
+    torch.cuda.synchronize()
+    ro = oracle.row_offsets(ref, V).astype(np.int64)
+    bad = []
+
+    def work(k):
+        r = np.random.default_rng(k)
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            for _ in range(20):
+                srcs = r.integers(0, V, int(r.integers(1, 4000)))
+                s = torch.from_numpy(srcs.astype(np.int32)).cuda()
+                offs = torch.empty(srcs.size + 1, dtype=torch.int32, device="cuda")
+                total = L.ctypes.c_uint64(0)
+                rc = L.lib().lpma_neighbor_offsets(pma._h, s.data_ptr(), srcs.size, offs.data_ptr(),
+                                                   L.ctypes.byref(total), st.cuda_stream)
+                st.synchronize()
+                want = np.concatenate([[0], np.cumsum(ro[srcs + 1] - ro[srcs])])
+                if rc or total.value != want[-1] or not np.array_equal(offs.cpu().numpy(), want):
+                    bad.append(k)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for x in ts:
+        x.start()
+    for x in ts:
+        x.join()
+    assert not bad
+    pma.close()
