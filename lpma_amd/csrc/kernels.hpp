@@ -110,8 +110,9 @@ hipError_t copy_device(void *dst, const void *src, u64 bytes, hipStream_t st);
 hipError_t gen_rmat_device(u32 scale, u64 n, double a, double b, double c, u64 seed, u64 *out, hipStream_t st);
 
 // views.hip
-hipError_t export_compacted(const DevState &d, u32 *gpre, u32 *scan_scratch, u64 *edge_keys, u32 *row_std,
-                            u64 *all_keys, u32 *csr_row, u32 *csr_col, hipStream_t st);
+u64 export_scratch_words();
+hipError_t export_compacted(const DevState &d, u32 *sums, u64 *edge_keys, u32 *row_std, u64 *all_keys, u32 *csr_row,
+                            u32 *csr_col, hipStream_t st);
 // the export with its scratch in a static device array (no allocation);
 // setup finds the array's address on the current device
 hipError_t export_scratch_setup(int device);

@@ -1627,10 +1627,8 @@ static int export_common(lpma_t *h, u64 *edges, u32 *row_std, u64 *all, u32 *csr
     hipStream_t st = (hipStream_t)stream;
     h->cur_stream = st;
     h->pl.cur_stream = st;
-    u64 nseg = 1ull << h->st.H;
-    CHECKED(ensure(h->pl, h->pl.gpre, nseg + 1));
-    CHECKED(ensure(h->pl, h->pl.scan_scr, scan_scratch_words(nseg) + 8));
-    HIPCHECK(export_compacted(h->st, h->pl.gpre.p, h->pl.scan_scr.p, edges, row_std, all, csr_row, csr_col, st));
+    CHECKED(ensure(h->pl, h->pl.scan_scr, export_scratch_words()));
+    HIPCHECK(export_compacted(h->st, h->pl.scan_scr.p, edges, row_std, all, csr_row, csr_col, st));
     return LPMA_OK;
 }
 

@@ -221,6 +221,39 @@ def test_many_sources():
         pma.close()
 
 
+# export: fewer segments than a tile has at least (8), one tile a workgroup, and
+# tiles of more segments than are scanned at a time (512: over 2^19 segments)
+@pytest.mark.parametrize("V,E,slots", [(1, 0, 32), (3, 2, 2), (500, 3000, 128), (40000, 300000, 16),
+                                       (1 << 20, 500000, 2), (1 << 20, 2500000, 2)])
+def test_export_tiles(V, E, slots):
+    rng = np.random.default_rng(V + E)
+    say(f"export V={V} E={E} S={slots}")
+    ref = oracle.sort_unique(rand_keys(rng, V, E))
+    pma = L.PMA(V, segment_slots=slots)
+    if E:
+        pma.insert(ref)
+        pma.delete(ref[::7])
+        ref = np.delete(ref, np.arange(0, ref.size, 7))
+    ro = oracle.row_offsets(ref, V)
+    ek, got = pma.export()
+    assert np.array_equal(L.to_host_u64(ek), ref)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), ro)
+    assert np.array_equal(pma.row_offsets().cpu().numpy().view(np.uint32), ro)
+    # every live key, markers at the rows' ends, in the order of the store
+    src = np.concatenate([ref >> np.uint64(32), np.arange(V, dtype=np.uint64)]).astype(np.int64)
+    dst = np.concatenate([ref & np.uint64(0xFFFFFFFF), np.full(V, 0xFFFFFFFF, dtype=np.uint64)])
+    order = np.argsort(src, kind="stable")
+    src, dst = src[order], dst[order].astype(np.int64)
+    data = L.to_host_u64(pma.get_data())
+    assert np.array_equal(data >> np.uint64(32), src.astype(np.uint64))
+    mark = dst == 0xFFFFFFFF
+    assert np.array_equal(data[~mark], ref)
+    row, col = pma.to_csr()
+    assert np.array_equal(col.cpu().numpy().view(np.uint32), np.where(mark, src, dst).astype(np.uint32))
+    assert np.array_equal(row.cpu().numpy().view(np.uint32)[1:], (np.flatnonzero(mark) + 1).astype(np.uint32))
+    pma.close()
+
+
 # neighbor offsets: one workgroup takes 1024 rows and alone stores its result;
 # rows inside one segment, over a few (a lane sums them) and over many (a wave
 # does), empty ones, ids out of range and repeats
