@@ -34,18 +34,21 @@ struct BatchBufs {
 
 // batch descriptors small enough to travel as kernel arguments
 static constexpr u32 INLINE_SEGS = 4;
-struct InlineSegs {
-    BatchSeg s[INLINE_SEGS];
+template <u32 N>
+struct SegArgs {
+    BatchSeg s[N];
     u32 n;
 };
+using InlineSegs = SegArgs<INLINE_SEGS>;
+static constexpr u32 SORT_SEGS = 64;  // of the kernel that sorts (3 KB of arguments)
 
-// sort.hip: a lone PMA's batch of at most 2^19 keys from inline sources is
-// sorted with the batch's first work (batch_begin's, without clearing the
+// sort.hip: a lone PMA's batch of at most 2^19 keys from at most SORT_SEGS
+// sources (segs: on the host, passed as kernel arguments) is sorted with the batch's first work (batch_begin's, without clearing the
 // sort scratch) carried by the sort kernels: no batch_begin launch, and the
 // pyramid's pyr_chunks chunk levels owed by the last batch summed there too
-bool sort_carries_first(u64 n);
-u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const InlineSegs &in, u64 n, u32 pshift,
-                         u32 sbits, u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 pyr_chunks,
+bool sort_carries_first(u64 n, u32 nsegs);
+u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const BatchSeg *segs, u32 nsegs, u64 n,
+                         u32 pshift, u32 sbits, u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 pyr_chunks,
                          hipStream_t st);
 
 // A lone PMA's batch of at most SMALL_MAX_N keys from inline sources, from its

@@ -1027,6 +1027,8 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     CHECKED(begin_epoch(mem, npma, epoch, st));
     CHECKED(upload_table(pl, mem, npma, pyr_blocks, st));
 
+    // the sort carries the batch's first work and takes the sources as arguments
+    const bool carried = npma == 1 && sort_carries_first(n, nsegs);
     // batch sources: each request's deletes (op 0), then its inserts (op 1)
     InlineSegs in;
     memset(&in, 0, sizeof(in));
@@ -1058,7 +1060,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
         if (nsegs <= INLINE_SEGS) {
             for (u32 k2 = 0; k2 < nsegs; ++k2) in.s[k2] = pl.h_segs[k2];
             in.n = nsegs;
-        } else {
+        } else if (!carried) {
             HIPCHECK(hipMemcpyAsync(pl.segs.p, pl.h_segs, nsegs * sizeof(BatchSeg), hipMemcpyHostToDevice, st));
         }
     }
@@ -1095,11 +1097,11 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
         u64 *pk;
         {
             PhaseTimer t(pl, st, PH_SORT);
-            if (npma == 1 && nsegs <= INLINE_SEGS && sort_carries_first(n)) {
+            if (carried) {
                 lpma *h0 = mem[0].h;
                 const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
-                pk = pack_and_sort_first(g, bb.status, bb.wfirst, in, n, pshift, sbits, hi_bit, pl.pk0.p, pl.pk1.p,
-                                         pl.ukey.p, pl.sort_scr.p, chunks, st);
+                pk = pack_and_sort_first(g, bb.status, bb.wfirst, pl.h_segs, nsegs, n, pshift, sbits, hi_bit, pl.pk0.p,
+                                         pl.pk1.p, pl.ukey.p, pl.sort_scr.p, chunks, st);
                 h0->pyr_owed = false;
             } else {
                 HIPCHECK(pay_owed_pyramids(mem, npma, st));

@@ -12,6 +12,8 @@
 //                  sample, each sorted by a bitonic network;
 //   larger         LSD radix, one kernel per 7/8-bit digit (decoupled
 //                  look-back), the digit counts of every pass taken at pack.
+#include <string.h>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "begin.hpp"
@@ -318,24 +320,24 @@ static u32 ss_buckets(u64 n) {
 // keys, x >> psh with psh >= the bits below the key (request order,
 // operation): equal keys project equally, so they share a bucket, and any
 // non-decreasing splitters give a correct split.
-// FIRST: a lone PMA's batch of inline sources, whose first work (status,
+// FIRST: a lone PMA's batch of at most FIRST sources, whose first work (status,
 // update index) one more workgroup, past the tiles, does here instead of a
 // kernel of its own, and the next pyr_chunks workgroups the count pyramid's
 // chunk levels the last batch left owing (its top levels follow in the
 // bucket kernel); the sources come from the kernel arguments.  A tile that
 // met an invalid key marks its count of bucket 0 (bit 31): the bucket
 // kernel raises the flag, after the status is cleared.
-template <bool FIRST, int ITEMS>
+template <u32 FIRST, int ITEMS>
 __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict__ segs, u32 nsegs, u64 n,
                                                       const u64 *n_dev, u32 pshift, u32 sbits, u32 psh, u32 nb,
-                                                      u64 *__restrict__ tmp, u32 *__restrict__ bc, InlineSegs in,
-                                                      Group g, Status *status, u32 *wfirst) {
+                                                      u64 *__restrict__ tmp, u32 *__restrict__ bc,
+                                                      SegArgs<FIRST ? FIRST : 1> in, Group g, Status *status, u32 *wfirst) {
     constexpr u32 TILE = SS_TPB * ITEMS;
     __shared__ u32 smp[2][SS_MAX_SAMPLE];
     __shared__ u32 spl[SS_MAX_BUCKETS];
     __shared__ u32 cnt[SS_MAX_BUCKETS];
     __shared__ u32 base[SS_MAX_BUCKETS];
-    __shared__ BatchSeg lsegs[FIRST ? INLINE_SEGS : SS_LSEGS];
+    __shared__ BatchSeg lsegs[FIRST ? FIRST : SS_LSEGS];
     __shared__ u32 pyr_v0[FIRST ? PYR_CH : 1], pyr_v1[FIRST ? PYR_CH / 2 : 1];
     if (n_dev) n = *n_dev;
     const u32 t = blockIdx.x;
@@ -808,11 +810,11 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
         const u32 ks = 1 + sbits;
         const u32 psh = hi_bit > 32 + ks ? hi_bit - 32 : ks;
         if (ss_items(n) == 1)
-            k_ss_split<false, 1><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
-                                                             InlineSegs{}, Group{}, nullptr, nullptr);
+            k_ss_split<0, 1><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
+                                                             SegArgs<1>{}, Group{}, nullptr, nullptr);
         else
-            k_ss_split<false, 2><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
-                                                             InlineSegs{}, Group{}, nullptr, nullptr);
+            k_ss_split<0, 2><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
+                                                             SegArgs<1>{}, Group{}, nullptr, nullptr);
         k_ss_bucket<<<nb, SB_TPB, 0, st>>>(k1, k0, k2, n, n_dev, (u32)ss_items(n) * SS_TPB, nb, bc, flags, false,
                                            DevState{});
         return k0;
@@ -828,28 +830,44 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
                : os_sort<8, 4>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, st);
 }
 
-bool sort_carries_first(u64 n) { return n > 0 && n <= SS_MAX_N; }
+bool sort_carries_first(u64 n, u32 nsegs) { return n > 0 && n <= SS_MAX_N && nsegs <= SORT_SEGS; }
 
-// The sample-split sort of a lone PMA's batch of at most SS_MAX_N keys from
-// inline sources, with the batch's first work (batch_begin without its
+// The sample-split sort of a lone PMA's batch of at most SS_MAX_N keys from at
+// most SORT_SEGS sources, with the batch's first work (batch_begin without its
 // sort-scratch clearing, which the sample-split sort does not need) in one
 // more workgroup of the split kernel, pyr_chunks more for the pyramid's
 // chunk levels the last batch left owing, and one more of the bucket kernel
-// for the pyramid's top levels.
-u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const InlineSegs &in, u64 n, u32 pshift,
-                         u32 sbits, u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 pyr_chunks,
+// for the pyramid's top levels.  Sources beyond INLINE_SEGS in the arguments
+// instead of a copy of them, a kernel for the first work and two for the
+// pyramid: 32 requests of 5000 + 5000 keys on 2^25 edges @SEQ@.
+template <u32 N>
+static void ss_split_first(u32 grid, const Group &g, Status *status, u32 *wfirst, const BatchSeg *segs, u32 nsegs,
+                           u64 n, u32 pshift, u32 sbits, u32 psh, u32 nb, u64 *tmp, u32 *bc, hipStream_t st) {
+    static_assert(sizeof(SegArgs<N>) + sizeof(Group) + 128 <= 4096, "kernel arguments");
+    SegArgs<N> in;
+    memset(&in, 0, sizeof(in));
+    for (u32 k = 0; k < nsegs; ++k) in.s[k] = segs[k];
+    in.n = nsegs;
+    if (ss_items(n) == 1)
+        k_ss_split<N, 1><<<grid, SS_TPB, 0, st>>>(nullptr, nsegs, n, nullptr, pshift, sbits, psh, nb, tmp, bc, in, g,
+                                                  status, wfirst);
+    else
+        k_ss_split<N, 2><<<grid, SS_TPB, 0, st>>>(nullptr, nsegs, n, nullptr, pshift, sbits, psh, nb, tmp, bc, in, g,
+                                                  status, wfirst);
+}
+
+u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const BatchSeg *segs, u32 nsegs, u64 n,
+                         u32 pshift, u32 sbits, u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 pyr_chunks,
                          hipStream_t st) {
     const u32 nb = ss_buckets(n);
-    const u32 ntiles = ss_tiles(n);
     u32 *bc = scratch + OS_GH_WORDS;
     const u32 ks = 1 + sbits;
     const u32 psh = hi_bit > 32 + ks ? hi_bit - 32 : ks;
-    if (ss_items(n) == 1)
-        k_ss_split<true, 1><<<ntiles + 1 + pyr_chunks, SS_TPB, 0, st>>>(nullptr, in.n, n, nullptr, pshift, sbits, psh,
-                                                                         nb, k1, bc, in, g, status, wfirst);
+    const u32 grid = ss_tiles(n) + 1 + pyr_chunks;
+    if (nsegs <= INLINE_SEGS)
+        ss_split_first<INLINE_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
     else
-        k_ss_split<true, 2><<<ntiles + 1 + pyr_chunks, SS_TPB, 0, st>>>(nullptr, in.n, n, nullptr, pshift, sbits, psh,
-                                                                         nb, k1, bc, in, g, status, wfirst);
+        ss_split_first<SORT_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
     k_ss_bucket<<<nb + 1, SB_TPB, 0, st>>>(k1, k0, k2, n, nullptr, (u32)ss_items(n) * SS_TPB, nb, bc, &status->flags,
                                            true, g.one);
     return k0;

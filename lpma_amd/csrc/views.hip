@@ -20,8 +20,8 @@ namespace pma {
 // sums every tile's counts, and a workgroup of the second adds up the sums
 // before its own and scans its counts EX_SUB segments at a time.
 // Bound: HBM.  8.4*10^6 edges in 2^19 segments: 5 + 34 us (3.9 TB/s of lines
-// read, 2.1
-// written); a three-kernel scan of the counts and a slot a thread took 13 + 38.
+// read, 2.1 written); a three-kernel scan of the counts and a slot a thread
+// took 13 + 38.
 static constexpr u32 EX_TPB = 256;
 static constexpr u32 EX_TILES = 1024;
 static constexpr u32 EX_SUB = 512;
