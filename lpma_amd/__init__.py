@@ -324,6 +324,34 @@ def _stream_ptr(stream):
     return ctypes.c_void_p(s.cuda_stream)
 
 
+def _key_columns(owners, ins, dels):
+    """Pointers and counts of the key arrays of several requests, entry i for
+    owners[i] (None and empty arrays: 0), as C arrays, and the tensors behind
+    them.  Tensors are asked for few attributes: each costs 0.1 to 0.2 us, their
+    len() 1.3 us."""
+    torch = _torch()
+    tensor, i64 = torch.Tensor, torch.int64
+    n = max(len(owners), 1)
+    keep, cols = [], []
+    for arrays in (ins, dels):
+        ptrs, counts = [0] * n, [0] * n
+        for i, owner in enumerate(owners):
+            arr = arrays[i]
+            if arr is None:
+                continue
+            if isinstance(arr, tensor) and arr.dtype is i64 and arr.is_cuda and arr.dim() == 1:
+                t = arr.contiguous()
+            elif len(arr) == 0:
+                continue
+            else:
+                t = owner._dev_keys(arr)
+            keep.append(t)
+            ptrs[i] = t.data_ptr()
+            counts[i] = t.numel()
+        cols += [(ctypes.c_void_p * n)(*ptrs), (_u64 * n)(*counts)]
+    return keep, cols
+
+
 class PMA:
     """One packed-memory-array edge store on a GPU (a handle of the C ABI)."""
 
@@ -393,31 +421,9 @@ class PMA:
 
     def update_sequence(self, batches):
         """Applies [(ins, dels), ...] in order as one pipeline run."""
-        # (tensors are asked for few attributes: each costs 0.1 to 0.2 us, their
-        # len() 1.3 us, once per request here)
-        torch = _torch()
-        tensor, i64 = torch.Tensor, torch.int64
-        n = len(batches)
         pairs = [(a, d) for a, d in batches]
-        keep = []
-        cols = []  # insert pointers, insert counts, delete pointers, delete counts
-        for side in (0, 1):
-            ptrs, counts = [0] * max(n, 1), [0] * max(n, 1)
-            for i in range(n):
-                arr = pairs[i][side]
-                if arr is None:
-                    continue
-                if isinstance(arr, tensor) and arr.dtype is i64 and arr.is_cuda and arr.dim() == 1:
-                    t = arr.contiguous()
-                elif len(arr) == 0:
-                    continue
-                else:
-                    t = self._dev_keys(arr)
-                keep.append(t)
-                ptrs[i] = t.data_ptr()
-                counts[i] = t.numel()
-            cols += [(ctypes.c_void_p * len(ptrs))(*ptrs), (_u64 * len(counts))(*counts)]
-        pi, ni, pd, nd = cols
+        n = len(pairs)
+        keep, (pi, ni, pd, nd) = _key_columns([self] * n, [a for a, _ in pairs], [d for _, d in pairs])
         _check(lib().lpma_update_sequence(self._h, pi, ni, pd, nd, n, _stream_ptr(self.stream)), "update_sequence")
 
     def bulk_load(self, keys):
@@ -641,21 +647,8 @@ class Group:
     def update(self, ins, dels):
         """One round: ins[i] / dels[i] (int64 device tensors, numpy arrays or
         None) for member i."""
-        n = len(self.members)
-        keep = []
-        pi = (ctypes.c_void_p * n)()
-        ni = (_u64 * n)()
-        pd = (ctypes.c_void_p * n)()
-        nd = (_u64 * n)()
-        for i, m in enumerate(self.members):
-            for arr, p_, n_ in ((ins[i] if ins is not None else None, pi, ni),
-                                (dels[i] if dels is not None else None, pd, nd)):
-                if arr is None or len(arr) == 0:
-                    continue
-                t = m._dev_keys(arr)
-                keep.append(t)
-                p_[i] = t.data_ptr()
-                n_[i] = t.numel()
+        none = [None] * len(self.members)
+        keep, (pi, ni, pd, nd) = _key_columns(self.members, none if ins is None else ins, none if dels is None else dels)
         _check(lib().lpma_group_update(self._h, pi, ni, pd, nd, _stream_ptr(self.stream)), "group_update")
 
     def stats(self):
