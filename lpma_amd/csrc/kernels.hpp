@@ -40,9 +40,16 @@ struct SegArgs {
     u32 n;
 };
 using InlineSegs = SegArgs<INLINE_SEGS>;
-static constexpr u32 SORT_SEGS = 64;  // of the kernel that sorts (3 KB of arguments)
+static constexpr u32 ARG_SEGS = 64;  // of the sort's and the batch's first kernel (3 KB of arguments)
+template <u32 N>
+inline SegArgs<N> seg_args(const BatchSeg *segs, u32 n) {
+    SegArgs<N> a = {};
+    for (u32 k = 0; k < n; ++k) a.s[k] = segs[k];
+    a.n = n;
+    return a;
+}
 
-// sort.hip: a lone PMA's batch of at most 2^19 keys from at most SORT_SEGS
+// sort.hip: a lone PMA's batch of at most 2^19 keys from at most ARG_SEGS
 // sources (segs: on the host, passed as kernel arguments) is sorted with the batch's first work (batch_begin's, without clearing the
 // sort scratch) carried by the sort kernels: no batch_begin launch, and the
 // pyramid's pyr_chunks chunk levels owed by the last batch summed there too
@@ -63,10 +70,14 @@ hipError_t small_batch(const Group &g, const BatchBufs &b, const InlineSegs &in,
 u32 locate_blocks(u64 n);
 // most groups of locate blocks
 static constexpr u32 LOC_GROUPS = 1024;
-// also clears zero[0, nzero) (the sort's digit totals) and the locate groups
-// and resets the update index
-hipError_t batch_begin(const Group &g, const BatchBufs &b, const InlineSegs &in, BatchSeg *segs, u32 *zero, u32 nzero,
-                       hipStream_t st);
+// also clears zero[0, nzero) (the sort's digit totals) and the locate groups,
+// resets the update index and, given at most ARG_SEGS sources of the host's in
+// `hsegs`, stores them in segs
+hipError_t batch_begin(const Group &g, const BatchBufs &b, const BatchSeg *hsegs, u32 nsegs, BatchSeg *segs, u32 *zero,
+                       u32 nzero, hipStream_t st);
+// the batch's outcome (words of it, in b.status and after) into pinned memory,
+// then *seq = epoch
+hipError_t report_outcome(const BatchBufs &b, u32 words, u32 *host, u64 *seq, u32 epoch, hipStream_t st);
 hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchBufs &b, hipStream_t st);
 // fixed grids for graph replays (work counts read on the device)
 hipError_t rebalance_fixed(const Group &g, const BatchBufs &b, u32 runs_cap, u64 *merged, hipStream_t st);

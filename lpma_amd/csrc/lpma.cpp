@@ -1030,8 +1030,6 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     // the sort carries the batch's first work and takes the sources as arguments
     const bool carried = npma == 1 && sort_carries_first(n, nsegs);
     // batch sources: each request's deletes (op 0), then its inserts (op 1)
-    InlineSegs in;
-    memset(&in, 0, sizeof(in));
     {
         u64 off = 0;
         u32 k = 0;
@@ -1057,10 +1055,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
                 }
             }
         }
-        if (nsegs <= INLINE_SEGS) {
-            for (u32 k2 = 0; k2 < nsegs; ++k2) in.s[k2] = pl.h_segs[k2];
-            in.n = nsegs;
-        } else if (!carried) {
+        if (nsegs > ARG_SEGS) {
             HIPCHECK(hipMemcpyAsync(pl.segs.p, pl.h_segs, nsegs * sizeof(BatchSeg), hipMemcpyHostToDevice, st));
         }
     }
@@ -1088,7 +1083,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
         PhaseTimer t(pl, st, PH_SORT);
         lpma *h0 = mem[0].h;
         const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
-        HIPCHECK(small_batch(g, bb, in, n, chunks, (u32 *)(pl.d_stats + ST_ROWS * ST_NUM), pl.h_early, st));
+        HIPCHECK(small_batch(g, bb, seg_args<INLINE_SEGS>(pl.h_segs, nsegs), n, chunks, (u32 *)(pl.d_stats + ST_ROWS * ST_NUM), pl.h_early, st));
         h0->pyr_owed = false;
     } else {
         // bit 0 of a packed key is the operation (with the request order above
@@ -1105,7 +1100,8 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
                 h0->pyr_owed = false;
             } else {
                 HIPCHECK(pay_owed_pyramids(mem, npma, st));
-                HIPCHECK(batch_begin(g, bb, in, pl.segs.p, pl.sort_scr.p, sort_zero_words(), st));
+                HIPCHECK(batch_begin(g, bb, pl.h_segs, nsegs <= ARG_SEGS ? nsegs : 0, pl.segs.p, pl.sort_scr.p,
+                                     sort_zero_words(), st));
                 pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
                                    pl.ukey.p, pl.sort_scr.p, &bb.status->flags, st);
             }
@@ -1144,8 +1140,9 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
         memcpy(pl.h_out, &pl.h_early->s, sizeof(Status));
         memcpy(pl.h_out + STATUS_BYTES, &pl.h_early->p, sizeof(PmaStat));
     } else {
-        HIPCHECK(hipMemcpyAsync(pl.h_out, pl.out.p, out_bytes, hipMemcpyDeviceToHost, st));
-        HIPCHECK(hipStreamSynchronize(st));
+        HIPCHECK(report_outcome(bb, (u32)(out_bytes / 4), (u32 *)pl.h_out, &pl.h_early->seq, epoch, st));
+        u64 w;
+        CHECKED(wait_word(&pl.h_early->seq, st, w, [epoch](u64 x) { return x == epoch; }));
     }
     return finish_round(pl, mem, npma, g, pyr_blocks, false, st, early);
 }
@@ -1237,12 +1234,10 @@ int graph_for(Pipeline &pl, u64 cap, u32 npma, u32 pshift, u32 hi_bit, u32 log2S
         hipStream_t cs = pl.cap_stream;
         HIPCHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeRelaxed));
         BatchBufs bb = batch_bufs(pl);
-        InlineSegs none;
-        memset(&none, 0, sizeof(none));
         bool ok = hipMemcpyAsync(pl.rhdr.p, pl.h_rhdr, sizeof(RoundHdr), hipMemcpyHostToDevice, cs) == hipSuccess &&
                   hipMemcpyAsync(pl.segs.p, pl.h_segs, nsegs * sizeof(BatchSeg), hipMemcpyHostToDevice, cs) ==
                       hipSuccess &&
-                  batch_begin(g, bb, none, pl.segs.p, pl.sort_scr.p, sort_zero_words(), cs) == hipSuccess;
+                  batch_begin(g, bb, nullptr, 0, pl.segs.p, pl.sort_scr.p, sort_zero_words(), cs) == hipSuccess;
         if (ok) {
             u64 *pk = pack_and_sort(pl.segs.p, nsegs, cap, &pl.rhdr.p->n, pshift, 0, 0, hi_bit, pl.pk0.p, pl.pk1.p,
                                     pl.ukey.p, pl.sort_scr.p, &bb.status->flags, cs);

@@ -12,8 +12,6 @@
 //                  sample, each sorted by a bitonic network;
 //   larger         LSD radix, one kernel per 7/8-bit digit (decoupled
 //                  look-back), the digit counts of every pass taken at pack.
-#include <string.h>
-
 #include "common.hpp"
 #include "kernels.hpp"
 #include "begin.hpp"
@@ -830,10 +828,10 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
                : os_sort<8, 4>(segs, nsegs, n, n_dev, pshift, sbits, lo_bit, npass, k0, k1, scratch, flags, st);
 }
 
-bool sort_carries_first(u64 n, u32 nsegs) { return n > 0 && n <= SS_MAX_N && nsegs <= SORT_SEGS; }
+bool sort_carries_first(u64 n, u32 nsegs) { return n > 0 && n <= SS_MAX_N && nsegs <= ARG_SEGS; }
 
 // The sample-split sort of a lone PMA's batch of at most SS_MAX_N keys from at
-// most SORT_SEGS sources, with the batch's first work (batch_begin without its
+// most ARG_SEGS sources, with the batch's first work (batch_begin without its
 // sort-scratch clearing, which the sample-split sort does not need) in one
 // more workgroup of the split kernel, pyr_chunks more for the pyramid's
 // chunk levels the last batch left owing, and one more of the bucket kernel
@@ -844,10 +842,7 @@ template <u32 N>
 static void ss_split_first(u32 grid, const Group &g, Status *status, u32 *wfirst, const BatchSeg *segs, u32 nsegs,
                            u64 n, u32 pshift, u32 sbits, u32 psh, u32 nb, u64 *tmp, u32 *bc, hipStream_t st) {
     static_assert(sizeof(SegArgs<N>) + sizeof(Group) + 128 <= 4096, "kernel arguments");
-    SegArgs<N> in;
-    memset(&in, 0, sizeof(in));
-    for (u32 k = 0; k < nsegs; ++k) in.s[k] = segs[k];
-    in.n = nsegs;
+    const SegArgs<N> in = seg_args<N>(segs, nsegs);
     if (ss_items(n) == 1)
         k_ss_split<N, 1><<<grid, SS_TPB, 0, st>>>(nullptr, nsegs, n, nullptr, pshift, sbits, psh, nb, tmp, bc, in, g,
                                                   status, wfirst);
@@ -867,7 +862,7 @@ u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const Batc
     if (nsegs <= INLINE_SEGS)
         ss_split_first<INLINE_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
     else
-        ss_split_first<SORT_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
+        ss_split_first<ARG_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
     k_ss_bucket<<<nb + 1, SB_TPB, 0, st>>>(k1, k0, k2, n, nullptr, (u32)ss_items(n) * SS_TPB, nb, bc, &status->flags,
                                            true, g.one);
     return k0;

@@ -41,12 +41,33 @@ u32 locate_blocks(u64 n) { return (u32)((n + LOC_TILE - 1) / LOC_TILE); }
 // the previous batch: the levels above the per-workgroup chunks of
 // k_pyr_chunk (nseg >> 11 entries and fewer), so no separate launch is
 // needed for them.
-__global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, InlineSegs in, BatchSeg *segs, u32 *zero,
+template <u32 N>
+__global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, SegArgs<N> in, BatchSeg *segs, u32 *zero,
                                                       u32 nzero, u32 *wfirst, u64 *grp);
 
-hipError_t batch_begin(const Group &g, const BatchBufs &b, const InlineSegs &in, BatchSeg *segs, u32 *zero, u32 nzero,
-                       hipStream_t st) {
-    k_batch_begin<<<g.npma, 1024, 0, st>>>(g, b.status, in, segs, zero, nzero, b.wfirst, b.part);
+hipError_t batch_begin(const Group &g, const BatchBufs &b, const BatchSeg *hsegs, u32 nsegs, BatchSeg *segs, u32 *zero,
+                       u32 nzero, hipStream_t st) {
+    if (nsegs <= INLINE_SEGS)
+        k_batch_begin<INLINE_SEGS><<<g.npma, 1024, 0, st>>>(g, b.status, seg_args<INLINE_SEGS>(hsegs, nsegs), segs, zero,
+                                                            nzero, b.wfirst, b.part);
+    else
+        k_batch_begin<ARG_SEGS><<<g.npma, 1024, 0, st>>>(g, b.status, seg_args<ARG_SEGS>(hsegs, nsegs), segs, zero,
+                                                         nzero, b.wfirst, b.part);
+    return hipGetLastError();
+}
+
+// One workgroup.  The host polls seq: it sees the outcome of a group's batch
+// 10 us before a copy and a wait for the stream would return.
+__global__ __launch_bounds__(256) void k_report(const u32 *__restrict__ out, u32 words, u32 *host, u64 *seq, u32 epoch) {
+    for (u32 i = threadIdx.x; i < words; i += blockDim.x)
+        __hip_atomic_store(&host[i], out[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(seq, (u64)epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t report_outcome(const BatchBufs &b, u32 words, u32 *host, u64 *seq, u32 epoch, hipStream_t st) {
+    k_report<<<1, 256, 0, st>>>((const u32 *)b.status, words, host, seq, epoch);
     return hipGetLastError();
 }
 
@@ -2372,7 +2393,8 @@ __global__ __launch_bounds__(1024) void k_pyr_top(DevState d) {
     pyr_top_levels(d, v);
 }
 
-__global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, InlineSegs in, BatchSeg *segs, u32 *zero,
+template <u32 N>
+__global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, SegArgs<N> in, BatchSeg *segs, u32 *zero,
                                                       u32 nzero, u32 *wfirst, u64 *grp) {
     __shared__ u32 v[2 * PYR_TOP_LDS];
     if (blockIdx.x == 0 && threadIdx.x < in.n) segs[threadIdx.x] = in.s[threadIdx.x];

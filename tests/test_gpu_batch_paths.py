@@ -221,6 +221,37 @@ def test_many_sources():
         pma.close()
 
 
+# a group's sources travel as arguments of its first kernel up to 4 and up to
+# 64, and as a copy beyond; a lone PMA's as arguments of its sort up to 64
+@pytest.mark.parametrize("members", [1, 2, 3, 32, 33])
+def test_group_sources(members):
+    say(f"group sources {2 * members}")
+    rng = np.random.default_rng(members)
+    Vs = [int(rng.integers(50, 400)) for _ in range(members)]
+    pmas = [L.PMA(V) for V in Vs]
+    refs = [oracle.sort_unique(rand_keys(rng, V, 2000)) for V in Vs]
+    group = L.Group(pmas)
+    group.update(refs, None)
+    for _ in range(3):
+        ins = [rand_keys(rng, V, 150) for V in Vs]
+        dels = [rng.choice(r, 100) for r in refs]
+        group.update(ins, dels)
+        refs = [oracle.apply(r, a, d) for r, a, d in zip(refs, ins, dels)]
+    for p, r in zip(pmas, refs):
+        assert np.array_equal(L.to_host_u64(p.export()[0]), r)
+        assert p.check() == 0
+    group.close()
+    one = pmas[0]
+    for requests in (2, 3, 32, 33):
+        batches = [(rand_keys(rng, Vs[0], 30), rng.choice(refs[0], 20)) for _ in range(requests)]
+        one.update_sequence(batches)
+        for a, d in batches:
+            refs[0] = oracle.apply(refs[0], a, d)
+    assert np.array_equal(L.to_host_u64(one.export()[0]), refs[0])
+    for p in pmas:
+        p.close()
+
+
 # export: fewer segments than a tile has at least (8), one tile a workgroup, and
 # tiles of more segments than are scanned at a time (512: over 2^19 segments)
 @pytest.mark.parametrize("V,E,slots", [(1, 0, 32), (3, 2, 2), (500, 3000, 128), (40000, 300000, 16),
