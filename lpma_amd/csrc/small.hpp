@@ -3,42 +3,37 @@
 //
 // A batch of a few thousand keys is a chain of latencies: pack, sort, locate,
 // compact, density check and election took eight launches of 3 to 13 us for
-// any size below 10^4.  Here one workgroup takes the batch through all of it,
-// in LDS, while the others sum the count pyramid's levels the last batch left
-// owing; the last of the two to arrive checks the density and elects (nothing
-// waits inside the kernel), and stores the outcome for the host.  The rebalance
-// kernel follows.  Up to SMALL_MAX_N keys: two a thread.  Bound: latency.  256
-// keys on 4096 vertices 15 us (load 1.4, sort 4.1, locate 1.4, presence 1.9,
-// store and arrival 1.5, density 3, election and report 1.5); 1000 on 2^20
-// 27 us (load 3, sort 6.4, locate 8 to 11 over 2^19 segments).  One call with
-// everything around it: 50 -> 26 us and 60 -> 40 us.
+// any size below 10^4.  Here the keys are shared out over the chip, a wave a
+// key, while other workgroups sum the count pyramid's levels the last batch
+// left owing; the last workgroup to arrive compacts the batch, checks the
+// density and elects (nothing waits inside the kernel), and stores the outcome
+// for the host.  The rebalance kernel follows.  Up to SMALL_MAX_N keys, of
+// which the last workgroup holds two a thread.  Bound: latency.  1000 keys on
+// 2^20 vertices 19 us (one workgroup sorting and searching alone: 27), 256 on
+// 4096 13 (13).  One call with everything around it, on 2^20 vertices and 8
+// million edges: 1000 keys 29 us (60 with eight launches, 37 with one
+// workgroup), 2000 keys 34 (55 with one).
 #pragma once
 
 static constexpr u32 SM_TPB = 1024;
 static constexpr u32 SM_ITEMS = SMALL_MAX_N / SM_TPB;
-static constexpr u32 SM_TAB_LOG = 12;        // separators staged in LDS
 static constexpr u32 SM_PYR_GRID = 1024;     // workgroups of the pyramid's chunk levels
-static_assert(SM_ITEMS == 2, "the sort holds two keys a thread");
 
 struct SmallLds {
     union {
-        struct {
-            u64 sp[SMALL_MAX_N];  // the sort's buffers; then the sorted keys (sp)
-            u64 ex[SMALL_MAX_N];
-        };
+        u64 sp[SMALL_MAX_N];  // the batch's keys as they came
         struct {
             u32 v0[PYR_CH], v1[PYR_CH / 2];
         };
         u32 top[2 * PYR_TOP_LDS];
     };
-    u64 tab[1u << SM_TAB_LOG];  // every 2^(H - SM_TAB_LOG)-th separator
-    u32 seg[SMALL_MAX_N];       // segments of the compacted updates
-    i32 pd[SMALL_MAX_N + 1];    // their prefix
-    u32 c0[SMALL_MAX_N];        // their segments' counts
+    u32 seg[SMALL_MAX_N];     // segments of the compacted updates
+    i32 pd[SMALL_MAX_N + 1];  // their prefix
+    u32 c0[SMALL_MAX_N];      // their segments' counts
     Density dn;
     u32 wt[SM_ITEMS][SM_TPB / 64];
     u32 cls[NUM_CLASSES];
-    u32 flags, mask, n_eff, last;
+    u32 flags, mask, last;
     BatchSeg segs[INLINE_SEGS];
 };
 
@@ -180,150 +175,141 @@ __device__ __forceinline__ void small_settle(const Group &g, const BatchBufs &bb
     }
 }
 
-// Workgroup 0: the batch; the others: the pyramid (chunks: the chunk levels
-// owed, 0 if none; its top levels always).  arrive: two counters, zero before
-// and after.
-__global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineSegs in, u32 n, u32 chunks, u32 *arrive,
-                                                  EarlyOut *early) {
+// Compacts the batch, update j's (effective, insert) in own[r] of thread t, j = t
+// + r * SM_TPB (1 and 1 << 16), with its key, segment and count, into LDS and
+// memory.  Returns n_eff.
+__device__ __forceinline__ u32 small_compact(const BatchBufs &bb, SmallLds &S, const u32 (&own)[SM_ITEMS],
+                                             const u64 (&key)[SM_ITEMS], const u32 (&seg)[SM_ITEMS],
+                                             const u32 (&c0)[SM_ITEMS]) {
+    const u32 t = threadIdx.x, wv = t >> 6;
+    u32 inc[SM_ITEMS];
+#pragma unroll
+    for (u32 r = 0; r < SM_ITEMS; ++r) {
+        inc[r] = dpp_incl_scan32(own[r]);
+        if (lane_id() == 63) S.wt[r][wv] = inc[r];
+    }
+    __syncthreads();
+    u32 before = 0;
+#pragma unroll
+    for (u32 r = 0; r < SM_ITEMS; ++r) {
+        u32 pre = before;
+        for (u32 w = 0; w < SM_TPB / 64; ++w) {
+            const u32 x = S.wt[r][w];
+            if (w < wv) pre += x;
+            before += x;
+        }
+        pre += inc[r] - own[r];
+        if (own[r]) {
+            const u32 j = pre & 0xFFFFu;
+            const i32 x = 2 * (i32)(pre >> 16) - (i32)j;
+            S.seg[j] = seg[r];
+            S.pd[j] = x;
+            S.c0[j] = c0[r];
+            bb.ckey[j] = key[r];
+            bb.cseg[j] = seg[r];
+            bb.pd[j] = x;
+        }
+    }
+    const u32 n_eff = before & 0xFFFFu;
+    if (t == 0) {
+        const i32 x = 2 * (i32)(before >> 16) - (i32)n_eff;
+        S.pd[n_eff] = x;
+        bb.pd[n_eff] = x;
+    }
+    return n_eff;
+}
+
+// The first `parts` workgroups: the batch, a wave a key.  A workgroup loads all
+// the keys and takes SPLIT_KEYS of them: it finds each one's place in the
+// batch's order, and whether a later equal one follows, by comparing it with
+// all the keys, searches its segment 128 ways at a step, and leaves its outcome
+// at its place.  The others: the pyramid (chunks: the chunk levels owed, 0 if
+// none; its top levels always).  The last workgroup to arrive compacts, checks
+// and elects.  arrive: two counters, zero before and after.
+static constexpr u32 SPLIT_KEYS = SM_TPB / 64;
+
+// an outcome: segment, its count (at most 1024), effective, insert
+static constexpr u64 SPLIT_EFF = 1ull << 48, SPLIT_INS = 1ull << 49;
+
+__global__ __launch_bounds__(SM_TPB) void k_small(Group g, BatchBufs bb, InlineSegs in, u32 n, u32 parts,
+                                                        u32 chunks, u32 *arrive, EarlyOut *early) {
     __shared__ SmallLds S;
     const DevState &d = g.one;
-    const u32 t = threadIdx.x, wv = t >> 6;
-    u32 n_eff = 0, flags = 0;
-    if (blockIdx.x > 0) {
-        const u32 np = gridDim.x - 1;
-        for (u32 c = blockIdx.x - 1; c < chunks; c += np) {
+    const u32 t = threadIdx.x, lane = lane_id();
+    if (blockIdx.x >= parts) {
+        const u32 np = gridDim.x - parts;
+        for (u32 c = blockIdx.x - parts; c < chunks; c += np) {
             pyr_chunk<true>(d, c, S.v0, S.v1);
             __syncthreads();
         }
         if (np > 1 && !arrive_last(&arrive[0], np, S)) return;
         pyr_top_levels<true>(d, S.top);
-        if (!arrive_last(&arrive[1], 2, S)) return;
-        // the batch arrived first: its compacted updates from memory
-        n_eff = bb.status->n_eff;
-        flags = bb.status->flags;
-        for (u32 j = t; j < n_eff; j += SM_TPB) S.seg[j] = (u32)bb.cseg[j];
-        for (u32 j = t; j <= n_eff; j += SM_TPB) S.pd[j] = bb.pd[j];
-        for (u32 j = t; j < n_eff; j += SM_TPB) S.c0[j] = d.cnt[S.seg[j]];  // (its own entries)
-        small_density(g, S);
-        __syncthreads();
     } else {
-        // keys and staged separators: one round of loads (the separators are
-        // wanted after the sort)
         if (t < in.n) S.segs[t] = in.s[t];
-        constexpr u32 TPT = (1u << SM_TAB_LOG) / SM_TPB;
-        const u32 tl = min(d.H, SM_TAB_LOG), sh = d.H - tl;
-        u64 sepv[TPT];
-#pragma unroll
-        for (u32 k = 0; k < TPT; ++k) {
-            const u32 i = t + k * SM_TPB;
-            sepv[k] = d.sep[(u64)(i < (1u << tl) ? i : 0u) << sh];
-        }
         __syncthreads();
         bool bad = false;
-        u64 p[SM_ITEMS];
 #pragma unroll
         for (u32 r = 0; r < SM_ITEMS; ++r) {
             const u32 i = t + r * SM_TPB;
-            p[r] = ~0ull;
-            if (i < n) p[r] = pack_element(S.segs[source_of(S.segs, in.n, i)], i, g.pshift, g.sbits, bad);
+            if (i < n) S.sp[i] = pack_element(S.segs[source_of(S.segs, in.n, i)], i, g.pshift, g.sbits, bad);
         }
-        small_density(g, S);
         const bool anybad = __syncthreads_or(bad);
-        flags = anybad ? FLAG_INVALID_KEY : 0u;
-        block_bitonic<u64, SM_TPB, SM_ITEMS>(p, n, S.ex, S.sp);
-#pragma unroll
-        for (u32 r = 0; r < SM_ITEMS; ++r)
-            if (t + r * SM_TPB < n) S.sp[t + r * SM_TPB] = p[r];
-#pragma unroll
-        for (u32 k = 0; k < TPT; ++k) S.tab[t + k * SM_TPB] = sepv[k];
-        __syncthreads();
-        // dedup (the last of equal keys), locate, presence, as the staged edge
-        // queries search: staged separators, probes down to a line, the line
-        // read by the row of lanes (one compute unit's gathers bound this: 64
-        // clocks a wave and probe)
-        const u32 ks = 1 + g.sbits;
-        const u32 sw = min(16u, 1u << sh), SS = 1u << d.log2S, kw = min(16u, SS);
-        u64 key[SM_ITEMS];
-        u32 seg[SM_ITEMS], c0[SM_ITEMS], there[SM_ITEMS];
-        bool ok[SM_ITEMS];
-#pragma unroll
-        for (u32 r = 0; r < SM_ITEMS; ++r) {
-            const u32 i = t + r * SM_TPB;
-            ok[r] = i < n && !(i + 1 < n && (S.sp[i + 1] >> ks) == (p[r] >> ks));
-            const u64 kk = (p[r] & ((1ull << g.pshift) - 1)) >> ks;
-            key[r] = ok[r] ? ((kk >> d.vbits) << 32) | (kk & ((1ull << d.vbits) - 1)) : 0ull;
-            seg[r] = c0[r] = there[r] = 0;
-            if ((t & ~63u) + r * SM_TPB >= n) continue;  // whole waves
-            u32 at = 0;
-            for (u32 h = (1u << tl) >> 1; h; h >>= 1) at += S.tab[at + h] <= key[r] ? h : 0u;
-            at <<= sh;
-            for (u32 h = (1u << sh) >> 1; h >= 16; h >>= 1) at += d.sep[at + h] <= key[r] ? h : 0u;
-            u64 v[8], w[8];
-            if (sh) {
-                u32 c = 0;
-                row_lines<0>(d.sep, at, sw, v);
-                row_lines<8>(d.sep, at, sw, w);
-                row_counts<0, true>(v, key[r], c);
-                row_counts<8, true>(w, key[r], c);
-                at += min(c, sw) - 1;
+        if (blockIdx.x == 0 && t == 0) put<true>(&bb.status->flags, anybad ? FLAG_INVALID_KEY : 0u);
+        const u32 i = blockIdx.x * SPLIT_KEYS + (t >> 6);
+        if (i < n) {
+            const u32 ks = 1 + g.sbits;
+            const u64 x = S.sp[i];
+            u32 rank = 0;
+            bool dup = false;
+            for (u32 k = 0; k < n; k += 64) {
+                const u32 j = k + lane;
+                const u64 y = S.sp[min(j, n - 1)];
+                rank += (u32)__popcll(__ballot(j < n && (y < x || (y == x && j < i))));
+                dup = dup || (j < n && (y >> ks) == (x >> ks) && (y > x || (y == x && j > i)));
             }
-            seg[r] = at;
-            c0[r] = d.cnt[at];
-            u64 base = (u64)at << d.log2S;
-            for (u32 h = SS >> 1; h >= 16; h >>= 1) base += d.keys[base + h - 1] < key[r] ? h : 0u;
-            row_lines<0>(d.keys, base, kw, v);
-            row_lines<8>(d.keys, base, kw, w);
-            row_counts<0, false>(v, key[r], there[r]);
-            row_counts<8, false>(w, key[r], there[r]);
-        }
-        // compaction: (count, inserts) as the halves of one word
-        u32 own[SM_ITEMS], inc[SM_ITEMS];
-#pragma unroll
-        for (u32 r = 0; r < SM_ITEMS; ++r) {
-            const u32 op = (u32)(p[r] & 1);
-            own[r] = ok[r] && op != there[r] ? 1u | op << 16 : 0u;
-            inc[r] = dpp_incl_scan32(own[r]);
-            if (lane_id() == 63) S.wt[r][wv] = inc[r];
-        }
-        __syncthreads();
-        u32 before = 0;
-#pragma unroll
-        for (u32 r = 0; r < SM_ITEMS; ++r) {
-            u32 pre = before;
-            for (u32 w = 0; w < SM_TPB / 64; ++w) {
-                const u32 x = S.wt[r][w];
-                if (w < wv) pre += x;
-                before += x;
+            u64 key = 0, out = 0;
+            if (!__any(dup)) {
+                const u64 kk = (x & ((1ull << g.pshift) - 1)) >> ks;
+                key = ((kk >> d.vbits) << 32) | (kk & ((1ull << d.vbits) - 1));
+                const u32 s = wave_locate(d.sep, d.H, key);
+                const u64 base = (u64)s << d.log2S;
+                const u32 c = d.cnt[s];
+                bool there = false;
+                for (u32 k = lane; k < 1u << d.log2S; k += 64) there = there || d.keys[base + k] == key;
+                const u32 op = (u32)(x & 1);
+                out = (u64)s | (u64)c << 32;
+                if (op != (__any(there) ? 1u : 0u)) out |= SPLIT_EFF | (op ? SPLIT_INS : 0ull);
             }
-            pre += inc[r] - own[r];
-            if (own[r]) {
-                const u32 j = pre & 0xFFFFu;
-                const i32 x = 2 * (i32)(pre >> 16) - (i32)j;
-                S.seg[j] = seg[r];
-                S.pd[j] = x;
-                S.c0[j] = c0[r];
-                bb.ckey[j] = key[r];
-                put<true>(&bb.cseg[j], (u64)seg[r]);
-                put<true>(&bb.pd[j], x);
+            if (lane == 0) {
+                put<true>(&bb.ukey[rank], key);
+                put<true>(&bb.useg[rank], out);
             }
         }
-        n_eff = before & 0xFFFFu;
-        if (t == 0) {
-            const i32 x = 2 * (i32)(before >> 16) - (i32)n_eff;
-            S.pd[n_eff] = x;
-            put<true>(&bb.pd[n_eff], x);
-            put<true>(&bb.status->n_eff, n_eff);
-            put<true>(&bb.status->flags, flags);
-        }
-        if (!arrive_last(&arrive[1], 2, S)) return;
     }
+    if (!arrive_last(&arrive[1], parts + 1, S)) return;
     if (t < 2) __hip_atomic_store(&arrive[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    small_density(g, S);
+    u64 key[SM_ITEMS];
+    u32 own[SM_ITEMS], seg[SM_ITEMS], c0[SM_ITEMS];
+#pragma unroll
+    for (u32 r = 0; r < SM_ITEMS; ++r) {
+        const u32 j = t + r * SM_TPB;
+        const u64 out = j < n ? bb.useg[j] : 0ull;
+        key[r] = j < n ? bb.ukey[j] : 0ull;
+        seg[r] = (u32)out;
+        c0[r] = (u32)(out >> 32) & 0xFFFFu;
+        own[r] = out & SPLIT_EFF ? 1u | (out & SPLIT_INS ? 1u << 16 : 0u) : 0u;
+    }
+    const u32 flags = bb.status->flags;
+    const u32 n_eff = small_compact(bb, S, own, key, seg, c0);
+    __syncthreads();
     small_settle(g, bb, S, n_eff, flags, early);
 }
 
 hipError_t small_batch(const Group &g, const BatchBufs &b, const InlineSegs &in, u64 n, u32 chunks, u32 *arrive,
                        EarlyOut *early, hipStream_t st) {
     const u32 np = std::max<u32>(1, std::min<u32>(chunks, SM_PYR_GRID));
-    k_small<<<1 + np, SM_TPB, 0, st>>>(g, b, in, (u32)n, chunks, arrive, early);
+    const u32 parts = ((u32)n + SPLIT_KEYS - 1) / SPLIT_KEYS;
+    k_small<<<parts + np, SM_TPB, 0, st>>>(g, b, in, (u32)n, parts, chunks, arrive, early);
     return hipGetLastError();
 }
