@@ -575,12 +575,11 @@ def run_analytics(args):
         lv, depth, scanned = pma.bfs(0)
         torch.cuda.synchronize()
         bfs_s = time.perf_counter() - t0
-        # algorithmic bytes of the binned push: per iteration the live keys
-        # and row markers (8 B each), per edge its (dst, contribution) pair
-        # written and read back (16 B), per vertex the degree, contribution,
-        # rank and partial-sum vectors (about 28 B); once per call the count
-        # pass over the live keys
-        pr_bytes = iters * (8 * (E + V) + 16 * E + 28 * V) + 8 * (E + V)
+        # algorithmic bytes: per iteration an edge's word (4 B) and its
+        # source's contribution (4 B), per vertex the degree, rank, new rank
+        # and new contribution (16 B); once per call the live keys read by the
+        # count and by the bin pass (8 B each), and the words written (4 B)
+        pr_bytes = iters * (8 * E + 16 * V) + 16 * (E + V) + 4 * E
         reached = int((lv >= 0).sum().item())
         row = {"batch": b, "op": op, "update_ms": upd_ms, "edges": E, "capacity_slots": cap,
                "pagerank_ms": pr_s * 1e3, "pagerank_iterations": iters, "pagerank_last_l1_change": delta,

@@ -315,8 +315,8 @@ static u32 bfs_expand_grid() {
     return g;
 }
 
-hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited, u32 level,
-                     u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st) {
+hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
+                     u32 level, u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st) {
     k_bfs_front<<<grid_for(d.V, FRONT_TPB, 512), FRONT_TPB, 0, st>>>(d, level, q, (BfsCtl *)ctl, off, adj, runs);
     k_bfs_expand<<<expand_grid ? expand_grid : bfs_expand_grid(), EXP_TPB, 0, st>>>(d, level, off, adj, runs, levels,
                                                                                   visited, qnext, (BfsCtl *)ctl);

@@ -146,8 +146,8 @@ static constexpr u32 BFS_CTL_WORDS = 32;  // a search's sizes on the device
 static constexpr u32 BFS_AHEAD = 4;       // levels queued before the host asks for the frontier
 hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visited, hipStream_t st);
 u64 bfs_run_words(u64 slots);
-hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited, u32 level,
-                     u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st);
+hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
+                     u32 level, u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st);
 void bfs_state(const u32 *ctl, u32 level, u32 &qn, u32 &depth, u64 &scanned);
 hipError_t pr_outdeg(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *outdeg, hipStream_t st);
 hipError_t pr_init(float *pr, u32 V, float *red, hipStream_t st);

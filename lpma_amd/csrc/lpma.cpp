@@ -1,8 +1,8 @@
 // lpma.cpp -- host side of the C ABI: handle, device pool allocator, and
 // the update orchestrator that replaces update_rpma (rpma.cuh:1549-1718).
 //
-// One update call = one stream-ordered kernel sequence with exactly one
-// host synchronisation (after the density check, to learn whether the batch
+// One update call = one stream-ordered kernel sequence in which the host waits
+// once, for a word a kernel stores in pinned memory (after the density check, to learn whether the batch
 // is a plain rebalance, a root rebalance or a resize), instead of the
 // reference's per-level host loop with a device sync after every step.
 #include <hip/hip_runtime.h>

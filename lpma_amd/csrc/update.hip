@@ -1,7 +1,7 @@
 // update.hip -- the batched edge-update path on gfx950.
 //
 // Reference pipeline (update_rpma, rpma.cuh:1549-1718) and what replaces it:
-//   sort (:1557)                      -> sort.hip (packed keys, LDS radix)
+//   sort (:1557)                      -> sort.hip (packed keys)
 //   locate_leaf_kernel (:253-316)     -> k_locate: dedup + separator search
 //                                        + presence check (handle_del_mod,
 //                                        gpma.cuh:162-175)
@@ -10,13 +10,17 @@
 //   per-level host loop (:1611-1657)  -> k_density: every run picks the
 //                                        lowest level whose window fits, in
 //                                        one pass, from the count pyramid
-//   window grouping per level          -> k_claim / k_leaders: the maximal
+//   window grouping per level          -> k_leaders: the maximal
 //                                        chosen windows are elected, no host
 //                                        round trip per level
 //   block_rebalancing_kernel (:765-847) and rebalancing_kernel (:1127-1211)
 //                                     -> k_rebalance_{wave,block} (LDS) and
 //                                        the multi-workgroup global path
-//   resize / rebuild (:1301-1530)     -> rebuild_push + rebuild_spread
+//   resize / rebuild (:1301-1530)     -> k_rebuild_scatter, or k_gather_live
+//                                        and k_rebuild_merge for batches of more
+//                                        than half the live keys
+// and for a lone PMA's batch of up to 2048 keys everything up to the elected
+// windows in one kernel, k_small (small.hpp).
 //   row-offset fixup (:652-657, gpma.cuh:340-344) -> fused into the spread.
 //
 // Every kernel works on a Group: one or many independent PMAs whose batch
@@ -48,8 +52,8 @@ __global__ __launch_bounds__(1024) void k_batch_begin(Group g, Status *s, SegArg
 hipError_t batch_begin(const Group &g, const BatchBufs &b, const BatchSeg *hsegs, u32 nsegs, BatchSeg *segs, u32 *zero,
                        u32 nzero, hipStream_t st) {
     if (nsegs <= INLINE_SEGS)
-        k_batch_begin<INLINE_SEGS><<<g.npma, 1024, 0, st>>>(g, b.status, seg_args<INLINE_SEGS>(hsegs, nsegs), segs, zero,
-                                                            nzero, b.wfirst, b.part);
+        k_batch_begin<INLINE_SEGS><<<g.npma, 1024, 0, st>>>(g, b.status, seg_args<INLINE_SEGS>(hsegs, nsegs), segs,
+                                                            zero, nzero, b.wfirst, b.part);
     else
         k_batch_begin<ARG_SEGS><<<g.npma, 1024, 0, st>>>(g, b.status, seg_args<ARG_SEGS>(hsegs, nsegs), segs, zero,
                                                          nzero, b.wfirst, b.part);
@@ -58,7 +62,8 @@ hipError_t batch_begin(const Group &g, const BatchBufs &b, const BatchSeg *hsegs
 
 // One workgroup.  The host polls seq: it sees the outcome of a group's batch
 // 10 us before a copy and a wait for the stream would return.
-__global__ __launch_bounds__(256) void k_report(const u32 *__restrict__ out, u32 words, u32 *host, u64 *seq, u32 epoch) {
+__global__ __launch_bounds__(256) void k_report(const u32 *__restrict__ out, u32 words, u32 *host, u64 *seq,
+                                                u32 epoch) {
     for (u32 i = threadIdx.x; i < words; i += blockDim.x)
         __hip_atomic_store(&host[i], out[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __threadfence_system();

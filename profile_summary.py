@@ -16,9 +16,9 @@
         method.
 
 An update batch is the run of dispatches from its first kernel to the next
-batch's: k_batch_begin, or the sample-split sort's k_ss_split where that
-carries the batch's first work (a lone PMA's batch of up to 2^17 keys).  A
-batch whose sort took the large-batch radix kernels is a bulk load (the
+batch's: k_batch_begin, the sample-split sort's k_ss_split where that
+carries the batch's first work (a lone PMA's batch of up to 2^19 keys), or
+k_small (up to 2048).  A batch whose sort took the large-batch radix kernels is a bulk load (the
 update batches sort with the sample-split kernels) and is left out.
 """
 import argparse
@@ -48,7 +48,8 @@ def batches(dispatches):
     (update batches, bulk batches, dispatches before the first batch)."""
     segs, cur, pre = [], [], []
     for d in dispatches:
-        first = d[0] == "k_batch_begin" or (d[0] == "k_ss_split" and not (cur and cur[-1][0] == "k_batch_begin"))
+        first = d[0] in ("k_batch_begin", "k_small") or (
+            d[0] == "k_ss_split" and not (cur and cur[-1][0] == "k_batch_begin"))
         if first:
             if cur:
                 segs.append(cur)
