@@ -39,7 +39,7 @@ __device__ __forceinline__ void slot_range(const DevState &d, u32 r, u64 &lo, u6
 //                 lane at each step, dead lines never read.
 // The sizes stand in device memory, so the host queues BFS_AHEAD levels at a
 // time and then asks once whether the last of them found anything (a level
-// after the end costs two empty launches); a copy and a wait after every
+// after the end costs its empty launches); a copy and a wait after every
 // level, and a fill, three kernels to scan and one to search before its
 // expansion, took 100 us a level.
 // A visited bitmap (V bits: 2 MB at V = 2^24, held by every XCD's L2) filters
@@ -49,11 +49,11 @@ __device__ __forceinline__ void slot_range(const DevState &d, u32 r, u64 &lo, u6
 // miss bits (they go from 0 to 1), which costs an extra atomic, never a wrong
 // level.
 // Bound: at V = 2^22 and E = 2^26 the two large levels (80 and 70 million
-// places) take 671 and 409 us, 140 of them for the first's keys; the rest are
-// visited words that miss L1 (a miss every 6 to 8 clocks a CU, through L1 or
-// past it) and atomics (6 G/s, with or without their results).  A workgroup
-// per run of 2048 places, with barriers and a binary search per place, took
-// 813 and 510.
+// places) take 671 and 409 us this way, 140 of them for the first's keys; the
+// rest are visited words that miss L1 (a miss every 6 to 8 clocks a CU, through
+// L1 or past it) and atomics (6 G/s, with or without their results).  A
+// workgroup per run of 2048 places, with barriers and a binary search per
+// place, took 813 and 510.  Through lists (below) 300 and 290.
 
 // per level mod 4: vertices found, and entries (high 31 bits) and places (low
 // 33 bits)
@@ -68,6 +68,30 @@ static_assert(sizeof(BfsCtl) <= BFS_CTL_WORDS * 4, "control words");
 static constexpr u64 BFS_PLACES = (1ull << 33) - 1;
 static constexpr u32 BFS_ITEMS = 4;
 static constexpr u32 BFS_RUN = 64 * BFS_ITEMS;  // places per run
+
+// Large levels of a graph of at most BFS_WINDOWS * 2^BFS_WIN_LOG vertices go
+// through lists (BfsLists): the expansion's waves leave their edges'
+// destinations in extents of BFS_EXT, each of one window of the bitmap; a
+// workgroup of k_bfs_windows holds a window in LDS and marks the destinations of
+// its share of the extents there; k_bfs_merge joins the workgroups' windows.
+// The random reads meet LDS instead of L2, and nothing is claimed by atomics in
+// memory: 218 us for the expansion, 76 for the windows, 8 to join them, where
+// the claims in memory took 671 (80 million places; a 2^22-vertex, 2^26-edge
+// search 1340 -> 900 us).  The windows cost 60 us however few destinations there
+// are, as the claims do for some 8 million places.
+static constexpr u32 BFS_WIN_WORDS = 1u << (BFS_WIN_LOG - 5);
+static constexpr u32 BFS_EXT = 128;
+static constexpr u32 BFS_WIN_GRID = 256;
+static constexpr u32 BFS_WIN_EXT = 8;  // extents a wave of k_bfs_windows reads at a time
+static constexpr u64 BFS_LISTED = 1ull << 22;  // places from which a level goes through lists
+
+__device__ __forceinline__ bool bfs_listed(const BfsLists &ls, u64 ent) {
+    return ls.list && (ent & BFS_PLACES) >= BFS_LISTED;
+}
+// extents a wave of the expansion may fill
+__host__ __device__ __forceinline__ u64 bfs_extents(u64 nruns, u32 waves) {
+    return (nruns + waves - 1) / waves * (BFS_RUN / BFS_EXT) + BFS_WINDOWS;
+}
 
 __global__ void k_bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, BfsCtl *ctl, u32 *visited) {
     for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < V; i += (u64)gridDim.x * blockDim.x)
@@ -86,6 +110,7 @@ __global__ void k_bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, BfsCtl *ctl,
 }
 
 static constexpr u32 FRONT_TPB = 1024;
+static constexpr u32 FRONT_ITEMS = 4;  // vertices a lane of a sweep (one from the queue)
 
 // Entries of a level's frontier, FRONT_TPB vertices at a time.  One atomic
 // gives a chunk its entries and its places together, so places grow with
@@ -94,9 +119,10 @@ static constexpr u32 FRONT_TPB = 1024;
 // of row_off (1.6 million vertices: 40 us).
 __global__ __launch_bounds__(FRONT_TPB) void k_bfs_front(DevState d, u32 level, const u32 *__restrict__ q,
                                                           BfsCtl *__restrict__ ctl, u32 *__restrict__ off,
-                                                          u32 *__restrict__ adj, u32 *__restrict__ runs) {
+                                                          u32 *__restrict__ adj, u32 *__restrict__ runs,
+                                                          BfsLists ls, u32 *__restrict__ levels) {
     constexpr u32 NW = FRONT_TPB / 64;
-    __shared__ u32 s_off[FRONT_TPB];
+    __shared__ u32 s_off[FRONT_TPB * FRONT_ITEMS];
     __shared__ u32 s_n[NW], s_len[NW];
     __shared__ u64 s_base;
     const u32 tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
@@ -106,14 +132,49 @@ __global__ __launch_bounds__(FRONT_TPB) void k_bfs_front(DevState d, u32 level, 
         ctl->ent[(level + 2) & 3] = 0;
         if (qn) ctl->depth = level + 1;
     }
-    for (u64 c = (u64)blockIdx.x * FRONT_TPB; c < qn; c += (u64)gridDim.x * FRONT_TPB) {
-        u64 lo = 0, hi = 0;
-        if (c + tid < qn) slot_range(d, q[c + tid], lo, hi);
-        const u32 len = (u32)(hi - lo);
-        const u64 some = __ballot(len != 0);
-        const u32 li = dpp_incl_scan32(len);
+    // after a listed level the frontier is a bitmap, whose waves take vertices 64
+    // at a time from regions far apart: neighboring hubs fall to different
+    // workgroups
+    const bool sweep = qn && level > 0 && bfs_listed(ls, ctl->ent[(level - 1) & 3]);
+    const u32 blocks = (d.V + 63) / 64;
+    const u32 items = sweep ? FRONT_ITEMS : 1;
+    const u32 chunks = sweep ? (blocks + NW * FRONT_ITEMS - 1) / (NW * FRONT_ITEMS) : (qn + FRONT_TPB - 1) / FRONT_TPB;
+    for (u32 c = blockIdx.x; c < chunks; c += gridDim.x) {
+        u32 v[FRONT_ITEMS], lo[FRONT_ITEMS], len[FRONT_ITEMS];
+        bool ok[FRONT_ITEMS];
+#pragma unroll
+        for (u32 k = 0; k < FRONT_ITEMS; ++k) {
+            v[k] = 0;
+            ok[k] = false;
+            if (sweep) {
+                const u64 i = ((u64)(k * NW + w) * chunks + c) * 64 + lane;
+                v[k] = (u32)i;
+                ok[k] = i < d.V && ((ls.fresh[i >> 5] >> (i & 31)) & 1u);
+            } else if (k == 0) {
+                const u64 i = (u64)c * FRONT_TPB + tid;
+                ok[k] = i < qn;
+                if (ok[k]) v[k] = q[i];
+            }
+        }
+        u32 n = 0, sum = 0;
+#pragma unroll
+        for (u32 k = 0; k < FRONT_ITEMS; ++k) {
+            u64 l = 0, h = 0;
+            if (k < items && ok[k]) {
+                slot_range(d, v[k], l, h);
+                if (sweep) levels[v[k]] = level;
+            }
+            lo[k] = (u32)l;
+            len[k] = (u32)(h - l);
+        }
+#pragma unroll
+        for (u32 k = 0; k < FRONT_ITEMS; ++k) {
+            n += len[k] != 0;
+            sum += len[k];
+        }
+        const u32 ni = dpp_incl_scan32(n), li = dpp_incl_scan32(sum);
         if (lane == 63) {
-            s_n[w] = __popcll(some);
+            s_n[w] = ni;
             s_len[w] = li;
         }
         __syncthreads();
@@ -126,13 +187,16 @@ __global__ __launch_bounds__(FRONT_TPB) void k_bfs_front(DevState d, u32 level, 
         if (tid == 0) s_base = nt ? atomicAdd((unsigned long long *)&ctl->ent[level & 3], ((u64)nt << 33) | lt) : 0;
         __syncthreads();
         const u32 eb = (u32)(s_base >> 33), pb = (u32)s_base;  // places: fewer than 2^32 slots
-        if (len) {
-            const u32 k = n0 + __popcll(some & ((1ull << lane) - 1ull));
-            const u32 o = l0 + li - len;
-            s_off[k] = o;
-            off[eb + k] = pb + o;
-            adj[eb + k] = (u32)lo - (pb + o);
-        }
+        u32 e = n0 + ni - n, o = l0 + li - sum;
+#pragma unroll
+        for (u32 k = 0; k < FRONT_ITEMS; ++k)
+            if (len[k]) {
+                s_off[e] = o;
+                off[eb + e] = pb + o;
+                adj[eb + e] = lo[k] - (pb + o);
+                ++e;
+                o += len[k];
+            }
         __syncthreads();
         const u64 end = (u64)pb + lt;
         for (u64 r = ((u64)pb + BFS_RUN - 1) / BFS_RUN + tid; r * BFS_RUN < end; r += FRONT_TPB) {
@@ -155,9 +219,13 @@ static constexpr u32 EXP_Q = 2 * BFS_RUN;  // discovered vertices a wave holds: 
 __global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, const u32 *__restrict__ off,
                                                          const u32 *__restrict__ adj, const u32 *__restrict__ runs,
                                                          u32 *__restrict__ levels, u32 *__restrict__ visited,
-                                                         u32 *__restrict__ qnext, BfsCtl *__restrict__ ctl) {
+                                                         u32 *__restrict__ qnext, BfsCtl *__restrict__ ctl,
+                                                         BfsLists ls) {
     __shared__ u32 s_adj[EXP_WAVES][BFS_RUN];
-    __shared__ u32 s_q[EXP_WAVES][EXP_Q];
+    __shared__ union {
+        u32 q[EXP_Q];
+        u32 b[BFS_WINDOWS][BFS_EXT + 64];  // a listed level's destinations by window
+    } s_w[EXP_WAVES];
     __shared__ u32 s_first[EXP_WAVES][2 * BFS_ITEMS];  // a bit per place: an entry starts there
     __shared__ u32 s_n[EXP_WAVES], s_scanned[EXP_WAVES], s_base;
     const u32 lane = lane_id(), w = threadIdx.x >> 6;
@@ -165,6 +233,22 @@ __global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, c
     const u64 total = ent & BFS_PLACES;
     const u32 nent = (u32)(ent >> 33);
     const u64 nruns = (total + BFS_RUN - 1) / BFS_RUN;
+    const bool listed = bfs_listed(ls, ent);
+    const u32 wave = blockIdx.x * EXP_WAVES + w;
+    const u64 ext0 = wave * bfs_extents(nruns, gridDim.x * EXP_WAVES);  // this wave's extents
+    u32 ne = 0, bn[BFS_WINDOWS] = {};
+    // extent of the first `len` destinations of window x; the others move up
+    auto put_extent = [&](u32 x, u32 len) {
+        __builtin_amdgcn_wave_barrier();
+        u32 *to = ls.list + (ext0 + ne) * BFS_EXT;
+        for (u32 k = lane; k < len; k += 64) to[k] = s_w[w].b[x][k];
+        const u32 rest = s_w[w].b[x][BFS_EXT + lane];
+        if (lane == 0) ls.meta[ext0 + ne] = x << 8 | len;
+        ++ne;
+        __builtin_amdgcn_wave_barrier();
+        s_w[w].b[x][lane] = rest;
+        __builtin_amdgcn_wave_barrier();
+    };
     const u64 le = ~0ull >> (63 - lane);  // this lane and those below
     const u32 Smask = (1u << d.log2S) - 1;
     const gu64 *keys = (const gu64 *)d.keys;
@@ -226,6 +310,26 @@ __global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, c
             if (ok[i] && (slot[i] & Smask) < live[i]) k = keys[slot[i]];
             key[i] = k;
         }
+        if (listed) {
+#pragma unroll
+            for (u32 i = 0; i < BFS_ITEMS; ++i) {
+                const bool edge = key[i] != KEY_NONE;
+                const u32 v = (u32)key[i], win = v >> BFS_WIN_LOG;
+                scanned += edge;
+#pragma unroll
+                for (u32 x = 0; x < BFS_WINDOWS; ++x) {
+                    const u64 m = __ballot(edge && win == x);
+                    if (!m) continue;
+                    if (edge && win == x) s_w[w].b[x][bn[x] + __popcll(m & le) - 1] = v;
+                    bn[x] += (u32)__popcll(m);
+                    if (bn[x] >= BFS_EXT) {
+                        put_extent(x, BFS_EXT);
+                        bn[x] -= BFS_EXT;
+                    }
+                }
+            }
+            continue;
+        }
         u32 vw[BFS_ITEMS];
 #pragma unroll
         for (u32 i = 0; i < BFS_ITEMS; ++i) {
@@ -246,7 +350,7 @@ __global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, c
             const u64 m = __ballot(found);
             if (found) {
                 levels[v] = level + 1;
-                s_q[w][n + __popcll(m & le) - 1] = v;
+                s_w[w].q[n + __popcll(m & le) - 1] = v;
             }
             n += __popcll(m);
         }
@@ -255,10 +359,16 @@ __global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, c
             if (lane == 0) base = atomicAdd(next_n, n);
             base = (u32)__builtin_amdgcn_readfirstlane((int)base);
             __builtin_amdgcn_wave_barrier();
-            for (u32 k = lane; k < n; k += 64) qnext[base + k] = s_q[w][k];
+            for (u32 k = lane; k < n; k += 64) qnext[base + k] = s_w[w].q[k];
             __builtin_amdgcn_wave_barrier();
             n = 0;
         }
+    }
+    if (listed) {
+#pragma unroll
+        for (u32 x = 0; x < BFS_WINDOWS; ++x)
+            if (bn[x]) put_extent(x, bn[x]);
+        if (lane == 0) ls.ne[wave] = ne;
     }
     // what is left, with one atomic a workgroup
     scanned = wave_sum(scanned);
@@ -280,7 +390,83 @@ __global__ __launch_bounds__(EXP_TPB) void k_bfs_expand(DevState d, u32 level, c
     }
     __syncthreads();
     const u32 base = s_base + s_n[w];
-    for (u32 k = lane; k < n; k += 64) qnext[base + k] = s_q[w][k];
+    for (u32 k = lane; k < n; k += 64) qnext[base + k] = s_w[w].q[k];
+}
+
+// Workgroup b: window b % windows, share b / windows of the expansion's waves.
+__global__ __launch_bounds__(1024) void k_bfs_windows(u32 V, u32 level, u32 waves, const u32 *__restrict__ visited,
+                                                       const BfsCtl *__restrict__ ctl, BfsLists ls) {
+    extern __shared__ u32 win[];
+    const u64 ent = ctl->ent[level & 3];
+    if (!bfs_listed(ls, ent)) return;
+    const u32 tid = threadIdx.x, lane = lane_id();
+    const u32 x = blockIdx.x % ls.windows, share = blockIdx.x / ls.windows, shares = gridDim.x / ls.windows;
+    const u64 words = bfs_visited_words(V), w0 = (u64)x * BFS_WIN_WORDS;
+    for (u32 i0 = tid; i0 < BFS_WIN_WORDS; i0 += 1024 * 16) {
+        u32 r[16];
+#pragma unroll
+        for (u32 k = 0; k < 16; ++k) {
+            const u64 i = w0 + i0 + k * 1024;
+            r[k] = visited[i < words ? i : 0];
+            if (i >= words) r[k] = 0;
+        }
+#pragma unroll
+        for (u32 k = 0; k < 16; ++k) win[i0 + k * 1024] = r[k];
+    }
+    __syncthreads();
+    const u64 epw = bfs_extents(((ent & BFS_PLACES) + BFS_RUN - 1) / BFS_RUN, waves);
+    auto mark = [&](u32 v, bool ok) {
+        const u32 i = (v >> 5) & (BFS_WIN_WORDS - 1), bit = 1u << (v & 31);
+        if (ok && !(win[i] & bit)) atomicOr(&win[i], bit);
+    };
+    // (shares beyond the last whole one have none)
+    for (u32 wv = share < shares ? share + (tid >> 6) * shares : waves; wv < waves; wv += 16 * shares) {
+        const u32 ne = ls.ne[wv];
+        for (u32 e0 = 0; e0 < ne; e0 += 64) {
+            const u32 m = e0 + lane < ne ? ls.meta[wv * epw + e0 + lane] : ~0u;
+            u64 mine = __ballot(m >> 8 == x);
+            while (mine) {
+                u32 v[BFS_WIN_EXT][2], len[BFS_WIN_EXT];
+#pragma unroll
+                for (u32 k = 0; k < BFS_WIN_EXT; ++k) {
+                    const u32 l = mine ? (u32)__builtin_ctzll(mine) : 0u;
+                    len[k] = mine ? (u32)__builtin_amdgcn_readlane((int)m, (int)l) & 0xFFu : 0u;
+                    mine &= mine - 1;
+                    const u32 *from = ls.list + (wv * epw + e0 + l) * BFS_EXT;
+#pragma unroll
+                    for (u32 h = 0; h < 2; ++h) v[k][h] = lane + 64 * h < len[k] ? from[lane + 64 * h] : 0u;
+                }
+#pragma unroll
+                for (u32 k = 0; k < BFS_WIN_EXT; ++k)
+#pragma unroll
+                    for (u32 h = 0; h < 2; ++h) mark(v[k][h], lane + 64 * h < len[k]);
+            }
+        }
+    }
+    __syncthreads();
+    for (u32 i = tid; i < BFS_WIN_WORDS; i += 1024) ls.part[(u64)blockIdx.x * BFS_WIN_WORDS + i] = win[i];
+}
+
+// A thread a word: what the workgroups' windows have beyond the bitmap is the
+// next frontier.
+__global__ __launch_bounds__(256) void k_bfs_merge(u32 V, u32 level, u32 *__restrict__ visited,
+                                                    BfsCtl *__restrict__ ctl, BfsLists ls) {
+    if (!bfs_listed(ls, ctl->ent[level & 3])) return;
+    const u64 words = bfs_visited_words(V);
+    const u32 shares = BFS_WIN_GRID / ls.windows;
+    for (u64 i = (u64)blockIdx.x * 256 + threadIdx.x; i < words; i += (u64)gridDim.x * 256) {
+        const u32 x = (u32)(i >> (BFS_WIN_LOG - 5));
+        const u32 *from = ls.part + (u64)x * BFS_WIN_WORDS + (i & (BFS_WIN_WORDS - 1));
+        u32 now = 0;
+#pragma unroll 8
+        for (u32 s = 0; s < shares; ++s) now |= from[(u64)s * ls.windows * BFS_WIN_WORDS];
+        const u32 was = visited[i];
+        ls.fresh[i] = now & ~was;
+        if (now & ~was) {
+            visited[i] = now | was;
+            ctl->qn[(level + 1) & 3] = 1;  // a listed level only tells none from some
+        }
+    }
 }
 
 hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visited, hipStream_t st) {
@@ -315,11 +501,22 @@ static u32 bfs_expand_grid() {
     return g;
 }
 
+u32 bfs_list_waves() { return bfs_expand_grid() * EXP_WAVES; }
+u64 bfs_list_extents(u64 slots, u32 waves) { return bfs_extents((slots + BFS_RUN - 1) / BFS_RUN, waves) * waves; }
+u64 bfs_list_words(u64 extents) { return extents * BFS_EXT; }
+u64 bfs_part_words() { return (u64)BFS_WIN_GRID * BFS_WIN_WORDS; }
+
 hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
-                     u32 level, u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st) {
-    k_bfs_front<<<grid_for(d.V, FRONT_TPB, 512), FRONT_TPB, 0, st>>>(d, level, q, (BfsCtl *)ctl, off, adj, runs);
-    k_bfs_expand<<<expand_grid ? expand_grid : bfs_expand_grid(), EXP_TPB, 0, st>>>(d, level, off, adj, runs, levels,
-                                                                                  visited, qnext, (BfsCtl *)ctl);
+                     u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u32 expand_grid, hipStream_t st) {
+    BfsCtl *c = (BfsCtl *)ctl;
+    const u32 grid = expand_grid ? expand_grid : bfs_expand_grid();
+    k_bfs_front<<<grid_for(d.V, FRONT_TPB, 512), FRONT_TPB, 0, st>>>(d, level, q, c, off, adj, runs, ls, levels);
+    k_bfs_expand<<<grid, EXP_TPB, 0, st>>>(d, level, off, adj, runs, levels, visited, qnext, c, ls);
+    if (ls.list) {
+        k_bfs_windows<<<BFS_WIN_GRID, 1024, BFS_WIN_WORDS * sizeof(u32), st>>>(d.V, level, grid * EXP_WAVES, visited, c,
+                                                                            ls);
+        k_bfs_merge<<<grid_for(bfs_visited_words(d.V), 256, 1024), 256, 0, st>>>(d.V, level, visited, c, ls);
+    }
     return hipGetLastError();
 }
 

@@ -146,8 +146,24 @@ static constexpr u32 BFS_CTL_WORDS = 32;  // a search's sizes on the device
 static constexpr u32 BFS_AHEAD = 4;       // levels queued before the host asks for the frontier
 hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visited, hipStream_t st);
 u64 bfs_run_words(u64 slots);
+// a search's large levels through lists (list null: none)
+static constexpr u32 BFS_WIN_LOG = 20;  // vertices of a window of the bitmap: 128 KB of LDS
+static constexpr u32 BFS_WINDOWS = 4;
+static constexpr u64 BFS_LIST_SLOTS = 1ull << 24;
+struct BfsLists {
+    u32 *list;   // destinations, in extents
+    u32 *meta;   // an extent's window and length
+    u32 *ne;     // extents of each wave of the expansion
+    u32 *part;   // the workgroups' windows
+    u32 *fresh;  // the next frontier's bits
+    u32 windows;
+};
+u32 bfs_list_waves();  // of the default expansion
+u64 bfs_list_extents(u64 slots, u32 waves);
+u64 bfs_list_words(u64 extents);
+u64 bfs_part_words();
 hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
-                     u32 level, u32 *qnext, u32 *ctl, u32 expand_grid, hipStream_t st);
+                     u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u32 expand_grid, hipStream_t st);
 void bfs_state(const u32 *ctl, u32 level, u32 &qn, u32 &depth, u64 &scanned);
 hipError_t pr_outdeg(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *outdeg, hipStream_t st);
 hipError_t pr_init(float *pr, u32 V, float *red, hipStream_t st);

@@ -1698,11 +1698,13 @@ int lpma_check(lpma_t *h, uint64_t *violations, void *stream) {
 static int bfs_core(int device, const DevState &d, u32 src, u32 *d_levels, u32 *depth, u64 *edges_scanned,
                     u32 expand_grid, hipStream_t st) {
     const u64 V = d.V;
-    DBuf<u32> q0, q1, off, adj, runs, ctl, visited;
+    DBuf<u32> q0, q1, off, adj, runs, ctl, visited, list, meta, ne, part, fresh;
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(st);
         release_on(device, q0); release_on(device, q1); release_on(device, off); release_on(device, adj);
         release_on(device, runs); release_on(device, ctl); release_on(device, visited);
+        release_on(device, list); release_on(device, meta); release_on(device, ne); release_on(device, part);
+        release_on(device, fresh);
     };
     int r;
     if ((r = ensure_on(device, st, q0, V + 1)) || (r = ensure_on(device, st, q1, V + 1)) ||
@@ -1712,6 +1714,20 @@ static int bfs_core(int device, const DevState &d, u32 src, u32 *d_levels, u32 *
         cleanup();
         return r;
     }
+    // Lists for the large levels of a graph whose bitmap is a few windows, where
+    // there is memory for them (a destination a slot); a search of a given
+    // width, which runs beside other work in a budget, goes without.  A graph
+    // of fewer slots has no level that gains what their two launches cost.
+    BfsLists ls{};
+    const u64 slots = nseg_of(d) << d.log2S;
+    if (!expand_grid && V <= (u64)BFS_WINDOWS << BFS_WIN_LOG && slots >= BFS_LIST_SLOTS && slots <= 1ull << 28) {
+        const u32 waves = bfs_list_waves();
+        const u64 ext = bfs_list_extents(slots, waves);
+        if (!ensure_on(device, st, list, bfs_list_words(ext)) && !ensure_on(device, st, meta, ext) &&
+            !ensure_on(device, st, ne, waves) && !ensure_on(device, st, part, bfs_part_words()) &&
+            !ensure_on(device, st, fresh, bfs_visited_words(V)))
+            ls = {list.p, meta.p, ne.p, part.p, fresh.p, (u32)((V + (1u << BFS_WIN_LOG) - 1) >> BFS_WIN_LOG)};
+    }
     u32 *q[2] = {q0.p, q1.p};
     bool ok = bfs_init(d_levels, d.V, src, q[0], ctl.p, visited.p, st) == hipSuccess;
     u32 level = 0, qn = 1, levels_done = 0;
@@ -1719,7 +1735,7 @@ static int bfs_core(int device, const DevState &d, u32 src, u32 *d_levels, u32 *
     while (ok && qn) {
         for (u32 k = 0; ok && k < BFS_AHEAD; ++k, ++level)
             ok = bfs_level(d, q[level & 1], off.p, adj.p, runs.p, d_levels, visited.p, level, q[(level + 1) & 1], ctl.p,
-                           expand_grid, st) == hipSuccess;
+                           ls, expand_grid, st) == hipSuccess;
         alignas(8) u32 c[BFS_CTL_WORDS];
         ok = ok && hipMemcpyAsync(c, ctl.p, sizeof(c), hipMemcpyDeviceToHost, st) == hipSuccess &&
              hipStreamSynchronize(st) == hipSuccess;

@@ -134,6 +134,41 @@ def test_bfs_shapes(shape, slots):
     pma.close()
 
 
+# large levels through lists: from 2^24 slots and 2^22 places; a bitmap of one
+# window, of several, of whole ones and with a few vertices over; a vertex
+# beyond the listed sizes; dangling vertices and a hub
+@pytest.mark.parametrize("V,listed", [(1500, True), (1 << 20, True), ((1 << 20) + 33, True), (3 << 20, True),
+                                      (1 << 22, True), ((1 << 22) + 1, False)])
+def test_bfs_large_levels(V, listed):
+    from gpu_util import keys_of
+    say(f"bfs lists V={V}")
+    rng = np.random.default_rng(V)
+    E = 9500000
+    # half of the edges leave a twentieth of the vertices, a quarter lead to few
+    src = rng.integers(0, V, E)
+    src[::2] %= max(1, V // 20)
+    dst = rng.integers(0, V, E)
+    dst[::4] = V - 1 - dst[::4] % max(1, V // 50)
+    if V > 10000:
+        src = np.concatenate([src, np.zeros(50000, dtype=np.int64)])
+        dst = np.concatenate([dst, rng.integers(0, V, 50000)])
+    keys = oracle.sort_unique(keys_of(src, dst))
+    pma = L.PMA(V)
+    pma.bulk_load(keys)
+    if V > 10000:
+        assert pma.view().capacity >= 1 << 24
+    deg = np.diff(oracle.csr_of(keys, V)[0].astype(np.int64))
+    for src in (0, V - 1):
+        want = oracle.bfs(keys, V, src)
+        reached = want != 0xFFFFFFFF
+        for _ in range(2):
+            lv, depth, scanned = pma.bfs(src)
+            assert np.array_equal(lv.cpu().numpy().view(np.uint32), want)
+            assert depth == int(want[reached].max()) + 1
+            assert scanned == int(deg[reached].sum())
+    pma.close()
+
+
 def test_pagerank_partial_last_bin():
     """V = 20000: three destination bins of 8192 vertices, the last one
     partial; uniform edges with a tenth of the vertices dangling."""
