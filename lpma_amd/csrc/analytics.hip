@@ -37,11 +37,11 @@ __device__ __forceinline__ void slot_range(const DevState &d, u32 r, u64 &lo, u6
 //                 place finds its entry by counting bits), then segment
 //                 counts, keys and visited words, BFS_ITEMS loads in flight a
 //                 lane at each step, dead lines never read.
-// The sizes stand in device memory, so the host queues BFS_AHEAD levels at a
-// time and then asks once whether the last of them found anything (a level
-// after the end costs its empty launches); a copy and a wait after every
-// level, and a fill, three kernels to scan and one to search before its
-// expansion, took 100 us a level.
+// The sizes stand in device memory, and a front stores its own where the host
+// polls, so the host keeps BFS_AHEAD levels queued past the last it knows of (a
+// level after the end costs its empty launches) and nothing waits between
+// levels; a copy and a wait after every level, and a fill, three kernels to
+// scan and one to search before its expansion, took 100 us a level.
 // A visited bitmap (V bits: 2 MB at V = 2^24, held by every XCD's L2) filters
 // the edges; the levels array (32 bits per vertex) is only written.  A vertex
 // is claimed by the atomic OR that sets its bit, so it enters the next
@@ -77,7 +77,7 @@ static constexpr u32 BFS_RUN = 64 * BFS_ITEMS;  // places per run
 // The random reads meet LDS instead of L2, and nothing is claimed by atomics in
 // memory: 218 us for the expansion, 76 for the windows, 8 to join them, where
 // the claims in memory took 671 (80 million places; a 2^22-vertex, 2^26-edge
-// search 1340 -> 900 us).  The windows cost 60 us however few destinations there
+// search 1250 -> 800 us).  The windows cost 60 us however few destinations there
 // are, as the claims do for some 8 million places.
 static constexpr u32 BFS_WIN_WORDS = 1u << (BFS_WIN_LOG - 5);
 static constexpr u32 BFS_EXT = 128;
@@ -120,7 +120,7 @@ static constexpr u32 FRONT_ITEMS = 4;  // vertices a lane of a sweep (one from t
 __global__ __launch_bounds__(FRONT_TPB) void k_bfs_front(DevState d, u32 level, const u32 *__restrict__ q,
                                                           BfsCtl *__restrict__ ctl, u32 *__restrict__ off,
                                                           u32 *__restrict__ adj, u32 *__restrict__ runs,
-                                                          BfsLists ls, u32 *__restrict__ levels) {
+                                                          BfsLists ls, u32 *__restrict__ levels, u64 *host) {
     constexpr u32 NW = FRONT_TPB / 64;
     __shared__ u32 s_off[FRONT_TPB * FRONT_ITEMS];
     __shared__ u32 s_n[NW], s_len[NW];
@@ -131,6 +131,9 @@ __global__ __launch_bounds__(FRONT_TPB) void k_bfs_front(DevState d, u32 level, 
         ctl->qn[(level + 2) & 3] = 0;
         ctl->ent[(level + 2) & 3] = 0;
         if (qn) ctl->depth = level + 1;
+        __hip_atomic_store(host + 1, ctl->scanned, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(host + 2, (u64)(qn ? level + 1 : ctl->depth), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(host, (u64)(level + 1) << 32 | qn, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     // after a listed level the frontier is a bitmap, whose waves take vertices 64
     // at a time from regions far apart: neighboring hubs fall to different
@@ -476,13 +479,6 @@ hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visi
 
 u64 bfs_run_words(u64 slots) { return slots / BFS_RUN + 2; }
 
-void bfs_state(const u32 *ctl, u32 level, u32 &qn, u32 &depth, u64 &scanned) {
-    const BfsCtl *c = (const BfsCtl *)ctl;
-    qn = c->qn[level & 3];
-    depth = c->depth;
-    scanned = c->scanned;
-}
-
 // Default expansion grid: every workgroup resident at once (compute units x
 // workgroups per CU that fit), so the runs are shared out in one round.
 static u32 bfs_expand_grid() {
@@ -507,10 +503,11 @@ u64 bfs_list_words(u64 extents) { return extents * BFS_EXT; }
 u64 bfs_part_words() { return (u64)BFS_WIN_GRID * BFS_WIN_WORDS; }
 
 hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
-                     u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u32 expand_grid, hipStream_t st) {
+                     u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u64 *host, u32 expand_grid, hipStream_t st) {
     BfsCtl *c = (BfsCtl *)ctl;
     const u32 grid = expand_grid ? expand_grid : bfs_expand_grid();
-    k_bfs_front<<<grid_for(d.V, FRONT_TPB, 512), FRONT_TPB, 0, st>>>(d, level, q, c, off, adj, runs, ls, levels);
+    k_bfs_front<<<grid_for(d.V, FRONT_TPB, 512), FRONT_TPB, 0, st>>>(d, level, q, c, off, adj, runs, ls, levels,
+                                                                    host);
     k_bfs_expand<<<grid, EXP_TPB, 0, st>>>(d, level, off, adj, runs, levels, visited, qnext, c, ls);
     if (ls.list) {
         k_bfs_windows<<<BFS_WIN_GRID, 1024, BFS_WIN_WORDS * sizeof(u32), st>>>(d.V, level, grid * EXP_WAVES, visited, c,

@@ -143,7 +143,7 @@ hipError_t check_invariants(const DevState &d, u32 *err, hipStream_t st);
 // analytics.hip
 __host__ __device__ __forceinline__ u64 bfs_visited_words(u64 V) { return (V + 31) / 32; }
 static constexpr u32 BFS_CTL_WORDS = 32;  // a search's sizes on the device
-static constexpr u32 BFS_AHEAD = 4;       // levels queued before the host asks for the frontier
+static constexpr u32 BFS_AHEAD = 2;       // levels queued past the last one whose frontier the host knows
 hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visited, hipStream_t st);
 u64 bfs_run_words(u64 slots);
 // a search's large levels through lists (list null: none)
@@ -162,9 +162,10 @@ u32 bfs_list_waves();  // of the default expansion
 u64 bfs_list_extents(u64 slots, u32 waves);
 u64 bfs_list_words(u64 extents);
 u64 bfs_part_words();
+// host: pinned; [0] level + 1 and the size of its frontier (low half), stored
+// last; [1] live edges scanned and [2] levels with a frontier before it
 hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
-                     u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u32 expand_grid, hipStream_t st);
-void bfs_state(const u32 *ctl, u32 level, u32 &qn, u32 &depth, u64 &scanned);
+                     u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u64 *host, u32 expand_grid, hipStream_t st);
 hipError_t pr_outdeg(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *outdeg, hipStream_t st);
 hipError_t pr_init(float *pr, u32 V, float *red, hipStream_t st);
 u64 pr_acc_floats(u32 V);

@@ -16,6 +16,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -281,9 +282,9 @@ namespace {
 
 std::atomic<u32> g_epoch{0};
 
-// Words of a call that waits for a kernel's result without the stream: a
-// pinned word the kernel stores and the host polls, and a device word that is
-// zero between calls.  A call takes a pair and gives it back once the kernel
+// Words of a call that waits for a kernel's result without the stream: pinned
+// words a kernel stores and the host polls (the first last), and a device word
+// that is zero between calls.  A call takes a pair and gives it back once the kernel
 // has stored its result, so calls on any threads and streams have their own; a
 // device has at most WORDS_MAX pairs, and further calls wait for one.
 struct WordPair {
@@ -330,7 +331,7 @@ int words_take(int dev, hipStream_t st, WordPair &out) {
     void *p = nullptr;
     int r = pool_alloc(dev, &p, sizeof(u64));
     out.dev = (u64 *)p;
-    if (r == LPMA_OK && (injected_failure() || hipHostMalloc((void **)&out.host, sizeof(u64),
+    if (r == LPMA_OK && (injected_failure() || hipHostMalloc((void **)&out.host, 64,
                                                              hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess))
         r = LPMA_ERR_OUT_OF_MEMORY;
     else if (r == LPMA_OK && fill_u64(out.dev, 1, 0, st) != hipSuccess)
@@ -724,6 +725,8 @@ int wait_word(const u64 *word, hipStream_t st, u64 &out, Done done) {
             out = __atomic_load_n(word, __ATOMIC_ACQUIRE);
             return e == hipSuccess && done(out) ? LPMA_OK : LPMA_ERR_DEVICE;
         }
+        // a long wait lets other threads have the core
+        if (spin > 4096 && (spin & 63) == 63) std::this_thread::yield();
         __builtin_ia32_pause();
     }
 }
@@ -1728,21 +1731,30 @@ static int bfs_core(int device, const DevState &d, u32 src, u32 *d_levels, u32 *
             !ensure_on(device, st, fresh, bfs_visited_words(V)))
             ls = {list.p, meta.p, ne.p, part.p, fresh.p, (u32)((V + (1u << BFS_WIN_LOG) - 1) >> BFS_WIN_LOG)};
     }
+    WordPair w;
+    if ((r = words_take(device, st, w))) {
+        cleanup();
+        return r;
+    }
+    __atomic_store_n(w.host, 0ull, __ATOMIC_RELEASE);
     u32 *q[2] = {q0.p, q1.p};
     bool ok = bfs_init(d_levels, d.V, src, q[0], ctl.p, visited.p, st) == hipSuccess;
-    u32 level = 0, qn = 1, levels_done = 0;
-    u64 scanned = 0;
-    while (ok && qn) {
-        for (u32 k = 0; ok && k < BFS_AHEAD; ++k, ++level)
+    // every level's first kernel reports its frontier; two levels past the
+    // last reported one are queued
+    u64 seen = 0, word = 0;
+    for (u32 level = 0; ok;) {
+        for (; ok && level < seen + BFS_AHEAD; ++level)
             ok = bfs_level(d, q[level & 1], off.p, adj.p, runs.p, d_levels, visited.p, level, q[(level + 1) & 1], ctl.p,
-                           ls, expand_grid, st) == hipSuccess;
-        alignas(8) u32 c[BFS_CTL_WORDS];
-        ok = ok && hipMemcpyAsync(c, ctl.p, sizeof(c), hipMemcpyDeviceToHost, st) == hipSuccess &&
-             hipStreamSynchronize(st) == hipSuccess;
-        if (ok) bfs_state(c, level, qn, levels_done, scanned);
+                           ls, w.host, expand_grid, st) == hipSuccess;
+        ok = ok && wait_word(w.host, st, word, [seen](u64 x) { return (x >> 32) > seen; }) == LPMA_OK;
+        seen = word >> 32;
+        if (!(u32)word) break;
     }
+    const u64 scanned = __atomic_load_n(w.host + 1, __ATOMIC_RELAXED);
+    const u32 levels_done = (u32)__atomic_load_n(w.host + 2, __ATOMIC_RELAXED);
     if (!ok) (void)hipGetLastError();
-    cleanup();
+    cleanup();  // waits for the levels queued past the end
+    words_give(device, ok ? &w : nullptr);
     if (!ok) return LPMA_ERR_DEVICE;
     if (depth) *depth = levels_done;
     if (edges_scanned) *edges_scanned = scanned;
