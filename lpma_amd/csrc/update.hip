@@ -380,21 +380,24 @@ __global__ __launch_bounds__(LOC_TPB) void k_compact(const Group g, const u64 *_
             cseg[ex] = sg[r] & ~RK_OP;
             pd[ex] = base_d + 2 * ins - c;
         }
+        // update index: the first update of each index-level window, written by
+        // the first located element of the window (with or without effect: the
+        // compacted index is the same), found by a look at the located element
+        // before it.  Where that one is not in the wave, and the element in
+        // front of the wave's first located one is a duplicate, which was not
+        // located, the smallest index wins by an atomic.  (An atomic from every
+        // wave that enters a window took 650 us where 8.4 M keys land in the 128
+        // windows of a PMA about to be built; one from every element behind a
+        // duplicate 15 us of a batch of 60000 keys, a third of them repeats.)
+        const u64 below = __ballot(sg[r] != RK_NONE) & ((1ull << lane_id()) - 1ull);
+        const u32 near = (u32)__shfl((int)(u32)sg[r], below ? 63 - __clzll((long long)below) : 0, 64);
         if (g.npma == 1 && sg[r] != RK_NONE) {
-            // update index: the first update of each index-level window,
-            // written by the first located element of the window (with or
-            // without effect: the compacted index is the same), found by a
-            // look at the element before it.  Where that one is a duplicate,
-            // which was not located, the smallest index wins by an atomic.
-            // (An atomic from every wave that enters a window took 650 us
-            // where 8.4 M keys land in the 128 windows of a PMA about to be
-            // built.)
             const u32 H = pma_of(g, 0).H, lb = index_level(H);
             if (lb <= H) {
                 const u32 w = (u32)sg[r] >> lb;  // low word of a run key: the segment
                 const u64 i = i0 + r * LOC_TILE;
-                if (i > 0 && prev[r] == RK_NONE) atomicMin(&wfirst[w], ex);
-                else if (i == 0 || (u32)prev[r] >> lb != w) wfirst[w] = ex;
+                if (!below && i > 0 && prev[r] == RK_NONE) atomicMin(&wfirst[w], ex);
+                else if (i == 0 || (below ? near : (u32)prev[r]) >> lb != w) wfirst[w] = ex;
             }
         }
     }
