@@ -824,8 +824,8 @@ hipError_t density_check(const Group &g, u64 n, const BatchBufs &b, hipStream_t 
 // workgroup adds to the lists' ends once for 1024 runs (atomics on one line).
 // Bound: scattered reads of claims and of the check's records.  2*10^6 updates
 // over 2^19 segments: 59 us an update a lane, 48 with four at a time, 35 now;
-// 3.2*10^5 over 2^21: 10 us an update a lane, 15 with four.
-static constexpr u64 LEADERS_MANY = 1ull << 20;
+// 7.5*10^5: 20 and 18; 3.2*10^5 over 2^21: 10 us an update a lane, 15 with four.
+static constexpr u64 LEADERS_MANY = 1ull << 19;
 
 template <bool ONE, int ITEMS>
 __global__ __launch_bounds__(1024) void k_leaders(Group g, const u64 *__restrict__ cseg, const i32 *__restrict__ pd,
