@@ -169,6 +169,35 @@ def test_bfs_large_levels(V, listed):
     pma.close()
 
 
+def test_bfs_large_levels_without_lists():
+    """A search that cannot have its lists (a word a slot), and one of a given
+    width, find the same."""
+    from gpu_util import keys_of
+    say("bfs without lists")
+    rng = np.random.default_rng(3)
+    V, E = 200000, 9500000
+    keys = oracle.sort_unique(keys_of(rng.integers(0, V, E) % 150000, rng.integers(0, V, E)))
+    pma = L.PMA(V)
+    pma.bulk_load(keys)
+    assert pma.view().capacity >= 1 << 24
+    want = oracle.bfs(keys, V, 1)
+    snap = L.Snapshot(pma)
+    assert L.lib().lpma_snapshot_set_search_width(snap._h, 64) == 0
+    pma.bfs(1)  # its other scratch is in the pool now
+    L.lib().lpma_pool_trim()
+    try:
+        L.set_pool_budget(L.pool_reserved_bytes() + (8 << 20))
+        got = [pma.bfs(1), snap.bfs(1)]
+    finally:
+        L.set_pool_budget(0)
+    got.append(pma.bfs(1))
+    for lv, depth, scanned in got:
+        assert np.array_equal(lv.cpu().numpy().view(np.uint32), want)
+        assert (depth, scanned) == (got[2][1], got[2][2])
+    snap.close()
+    pma.close()
+
+
 def test_pagerank_partial_last_bin():
     """V = 20000: three destination bins of 8192 vertices, the last one
     partial; uniform edges with a tenth of the vertices dangling."""
