@@ -297,19 +297,12 @@ struct WordPool {
     WordPair free[WORDS_MAX];
     size_t nfree = 0, made = 0;
 };
-std::mutex g_words_mu;
-std::map<int, WordPool *> g_words;
-
-WordPool &words_for(int dev) {
-    std::lock_guard<std::mutex> g(g_words_mu);
-    WordPool *&p = g_words[dev];
-    if (!p) p = new WordPool();
-    return *p;
-}
+static constexpr int WORDS_DEVICES = 64;
+WordPool g_words[WORDS_DEVICES];
 
 // p null: a pair that must not be used again (a kernel may still store to it)
 void words_give(int dev, const WordPair *p) {
-    WordPool &W = words_for(dev);
+    WordPool &W = g_words[dev];
     {
         std::lock_guard<std::mutex> g(W.mu);
         if (p) W.free[W.nfree++] = *p; else --W.made;
@@ -318,7 +311,8 @@ void words_give(int dev, const WordPair *p) {
 }
 
 int words_take(int dev, hipStream_t st, WordPair &out) {
-    WordPool &W = words_for(dev);
+    if (dev < 0 || dev >= WORDS_DEVICES) return LPMA_ERR_DEVICE;
+    WordPool &W = g_words[dev];
     {
         std::unique_lock<std::mutex> g(W.mu);
         W.cv.wait(g, [&] { return W.nfree || W.made < WORDS_MAX; });
