@@ -236,8 +236,9 @@ int lpma_snapshot_set_search_width(lpma_snapshot_t *s, uint32_t workgroups);
  * is below `tolerance` or `max_iter` iterations, then L1-normalised.  FP32
  * values; sums exact in 64-bit fixed point (V <= 2^27) or compensated FP32.
  * The host waits for every iteration's L1 change, and for the stream at the
- * end.  d_rank has V entries.  Device scratch grows to about 5 B per edge
- * plus 32 B per vertex. */
+ * end.  d_rank has V entries.  Device scratch (V <= 2^27): 5 to 8 B per edge
+ * and 32 B per vertex, 4 B for each part of 2^12 to 2^18 slots and 8192
+ * vertices, and partial sums of up to 16 B per edge, at most 134 MB. */
 int lpma_pagerank(lpma_t *h, float damping, float tolerance, uint32_t max_iter, float *d_rank, uint32_t *iterations,
                   float *last_delta, void *stream);
 

@@ -702,8 +702,10 @@ hipError_t pr_scale(float *pr, u32 V, const float *red, hipStream_t st) {
 //            of the counts fixes where each goes;
 //   bin      each part's workgroup writes its edges into its bins' runs, one
 //            word each: source relative to the part's first row, destination
-//            relative to the bin.  Runs are padded to groups of PB_CHUNK words
-//            and each group has the part's first row beside it;
+//            relative to the bin.  Runs are padded to groups of words and each
+//            group has the part's first row beside it.  A group is PB_CHUNK
+//            words, or one word, without padding, where runs are short or their
+//            padding would pass 32-bit offsets (pr_bins_plan);
 // and an iteration is one kernel (k_pr_iter): a workgroup takes a chunk of a
 // bin's edges, reads the source's contribution (a run's sources ascend, so
 // the lanes of a wave share lines and the workgroups of an XCD sweep the
@@ -819,10 +821,9 @@ __device__ __forceinline__ void pb_keys(const DevState &d, u64 t0, u64 p1, const
     }
 }
 
-// count[bin * P + part] = live edges of `part` into `bin`, rounded up to a
-// multiple of PB_CHUNK
-// (and clears the iterations' reductions)
-__global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u32 P, u32 NB,
+// count[bin * P + part] = live edges of `part` into `bin`, rounded up to whole
+// groups (and clears the iterations' reductions)
+__global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u32 P, u32 NB, u32 group,
                                                      u32 *__restrict__ count, PrSlot *slots) {
     extern __shared__ u32 pb_lds[];
     if (blockIdx.x == 0 && threadIdx.x < PR_SLOTS) slots[threadIdx.x] = PrSlot{0.0, 0.0, 0.0};
@@ -844,13 +845,14 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u
         }
     }
     __syncthreads();
-    for (u32 b = threadIdx.x; b < NB; b += PB_TPB) 
-        count[(u64)b * P + blockIdx.x] = (pb_lds[b] + PB_CHUNK - 1) & ~(PB_CHUNK - 1);
+    for (u32 b = threadIdx.x; b < NB; b += PB_TPB)
+        count[(u64)b * P + blockIdx.x] = (pb_lds[b] + group - 1) & ~(group - 1);
 }
 
 // words[off[bin * P + part] + rank] = pb_word(edge)
 // Phases per step: all key loads, all cursor adds, then the stores, so each
-// thread keeps PB_ITEMS loads in flight at a time.
+// thread keeps PB_ITEMS loads in flight at a time.  G: words of a group.
+template <u32 G>
 __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32 P, u32 NB, const u32 *__restrict__ off,
                                                    u32 *__restrict__ words, u32 *__restrict__ rows, u64 room) {
     extern __shared__ u32 pb_lds[];
@@ -885,14 +887,14 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32
             const u64 pos = (u64)b0 + (lane - lead[i]);
             if (pb_edge(key[i]) && pos < room) {
                 words[pos] = pb_word(key[i], row0);
-                if (pos % PB_CHUNK == 0) rows[pos / PB_CHUNK] = row0;
+                if (pos % G == 0) rows[pos / G] = row0;
             }
         }
     }
     __syncthreads();
     // a run's last group is filled up
     for (u32 b = threadIdx.x; b < NB; b += PB_TPB)
-        for (u64 pos = pb_lds[b]; pos % PB_CHUNK && pos < room; ++pos) words[pos] = PB_PAD;
+        for (u64 pos = pb_lds[b]; pos % G && pos < room; ++pos) words[pos] = PB_PAD;
 }
 
 // Staged form of the bin pass (bins <= PB_STAGE_MAX_BINS): a bin's words
@@ -904,7 +906,7 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32
 //      rest waits;
 //   3. full LDS chunks are written out and the bin's position advances;
 //   4. the waiting edges start the next LDS chunk.
-// At the end of the part each bin's last chunk is written with zero padding.
+// At the end of the part each bin's last chunk is filled up with PB_PAD.
 __global__ __launch_bounds__(PBS_TPB) void k_pb_bin_staged(DevState d, u32 part_log, u32 P, u32 NB,
                                                           const u32 *__restrict__ off,
                                                           u32 *__restrict__ words, u32 *__restrict__ rows, u64 room) {
@@ -1023,7 +1025,8 @@ __global__ __launch_bounds__(1024) void k_pb_chunks(const u32 *__restrict__ off,
         const u32 b = b0 + threadIdx.x;
         u64 v = 0;
         if (b < NB) {
-            const u32 n = max(1u, (off[(u64)(b + 1) * P] - off[(u64)b * P] + chunk - 1) / chunk);
+            const u32 len = off[(u64)(b + 1) * P] - off[(u64)b * P];
+            const u32 n = len ? (len - 1) / chunk + 1 : 1u;
             v = n | (n > 1 ? (u64)n << 32 : 0ull);
         }
         u64 tot;
@@ -1142,7 +1145,7 @@ __device__ __forceinline__ float pr_gamma(const PrSlot &prev, float alpha, u32 V
     return (alpha * (float)prev.dang + (1.f - alpha) * (float)prev.sum) / (float)V;
 }
 
-// Chunk k of a bin's edges (cb = chunks before each bin).  A bin of one chunk
+// Chunk k of a bin's edges (cb = chunks before each bin), in groups of G words.  A bin of one chunk
 // is finished here; the chunks of a larger one leave their sums in partial,
 // for k_pr_join.  (Joining them by 64-bit atomics on a vector in HBM instead
 // took 850 us an iteration, against 25 us.)
@@ -1152,6 +1155,7 @@ __device__ __forceinline__ float pr_gamma(const PrSlot &prev, float alpha, u32 V
 // 1340 us when every iteration binned contributions and summed them by LDS
 // compare-and-swap; with 8-byte edges 235 us.  The LDS adds are hidden: without
 // them the kernel takes the same time.
+template <u32 G>
 __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ words,
                                                      const u32 *__restrict__ rows, const u32 *__restrict__ off, u32 P,
                                                      u32 NB, const u32 *__restrict__ cb, u32 chunk,
@@ -1187,7 +1191,7 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
             const u64 i = i0 + (u64)r * PRI_TPB + threadIdx.x;
             const u64 j = i < s1 ? i : s1 - 1;  // unconditional loads: all of them in flight together
             e[r] = words[j];
-            row0[r] = rows[j / PB_CHUNK];
+            row0[r] = rows[j / G];
             if (i >= s1) e[r] = PB_PAD;
         }
         float x[PRI_ITEMS];
@@ -1256,6 +1260,10 @@ __global__ void k_pr_norm(const float *pr, float *rank, u32 V, const PrSlot *slo
 
 bool pr_bins_fit(u32 V) { return ((u64)V + PB_BIN - 1) / PB_BIN <= PB_MAX_BINS; }
 
+// the groups' rows follow the words
+static u64 pr_bins_rows_at(const PrBins &b) { return (b.words + b.group - 1) / b.group * b.group; }
+u64 pr_bins_edge_words(const PrBins &b) { return pr_bins_rows_at(b) / b.group * (b.group + 1) + b.group; }
+
 PrBins pr_bins_plan(const DevState &d, u64 edges) {
     PrBins b{};
     const u64 W = nseg_of(d) << d.log2S;
@@ -1266,9 +1274,16 @@ PrBins pr_bins_plan(const DevState &d, u64 edges) {
     b.part_log = std::min(b.part_log, PB_MAX_PART_LOG);
     b.parts = (u32)((W + (1ull << b.part_log) - 1) >> b.part_log);
     b.bins = (u32)(((u64)d.V + PB_BIN - 1) / PB_BIN);
-    b.staged = b.bins <= PB_STAGE_MAX_BINS;
-    // every run that holds an edge is padded to whole groups
+    // Every run that holds an edge is padded to whole groups, and the offsets
+    // of the words are 32-bit sums: runs whose padding could pass them, or could
+    // take more memory than a row beside every word (8 B an edge), go unpadded.
+    b.group = PB_CHUNK;
     b.words = std::min<u64>(edges * PB_CHUNK, edges + (u64)(PB_CHUNK - 1) * b.bins * b.parts);
+    if (b.words >= 1ull << 32 || pr_bins_edge_words(b) > 2 * edges) {
+        b.group = 1;
+        b.words = edges;  // with a marker a row in 2^32 slots at most
+    }
+    b.staged = b.group == PB_CHUNK && b.bins <= PB_STAGE_MAX_BINS;
     // about two rounds of chunks over the workgroups the device holds (two a
     // CU): more chunks have more sums to join, fewer leave a tail
     b.chunk = (u32)((std::max<u64>(8192, edges / 1024) + 1023) / 1024 * 1024);
@@ -1278,14 +1293,11 @@ PrBins pr_bins_plan(const DevState &d, u64 edges) {
 }
 
 u64 pr_bins_count_words(const PrBins &b) { return (u64)b.bins * b.parts + 1; }
-// the groups' rows follow the words
-static u64 pr_bins_rows_at(const PrBins &b) { return (b.words + PB_CHUNK - 1) / PB_CHUNK * PB_CHUNK; }
-u64 pr_bins_edge_words(const PrBins &b) { return pr_bins_rows_at(b) / PB_CHUNK * (PB_CHUNK + 1) + PB_CHUNK; }
 
 hipError_t pr_bins_edges(const DevState &d, const PrBins &b, u32 *off, u32 *cb, u32 *words, u32 *scan_scratch,
                          PrSlot *slots, hipStream_t st) {
     if (b.parts > PB_MAX_PARTS || b.bins > PB_MAX_BINS || b.bins == 0) return hipErrorInvalidValue;
-    k_pb_count<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, slots);
+    k_pb_count<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, b.group, off, slots);
     hipError_t e = device_excl_scan(off, (u64)b.bins * b.parts, off, scan_scratch, st);
     if (e != hipSuccess) return e;
     k_pb_chunks<<<1, 1024, 0, st>>>(off, b.parts, b.bins, b.chunk, cb);
@@ -1293,9 +1305,12 @@ hipError_t pr_bins_edges(const DevState &d, const PrBins &b, u32 *off, u32 *cb, 
     if (b.staged)
         k_pb_bin_staged<<<b.parts, PBS_TPB, b.bins * (PB_CHUNK + 2) * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins,
                                                                                         off, words, rows, b.words);
+    else if (b.group == PB_CHUNK)
+        k_pb_bin<PB_CHUNK><<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, words,
+                                                                         rows, b.words);
     else
-        k_pb_bin<<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, words, rows,
-                                                                b.words);
+        k_pb_bin<1><<<b.parts, PB_TPB, b.bins * sizeof(u32), st>>>(d, b.part_log, b.parts, b.bins, off, words, rows,
+                                                                  b.words);
     return hipGetLastError();
 }
 
@@ -1312,7 +1327,8 @@ u64 pr_bins_partial_words(const PrBins &b) { return std::max<u64>(1, (u64)b.max_
 hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
                            const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
                            float tol, u32 it, PrSlot *slots, u64 *partial, u64 *host, hipStream_t st) {
-    k_pr_iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(u64), st>>>(
+    const auto iter = b.group == PB_CHUNK ? k_pr_iter<PB_CHUNK> : k_pr_iter<1>;
+    iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(u64), st>>>(
         words, words + pr_bins_rows_at(b), off, b.parts, b.bins, cb, b.chunk, c, cnext, pr, out, outdeg, d.V, alpha, tol, it,
         slots, partial, host);
     if (b.max_multi)

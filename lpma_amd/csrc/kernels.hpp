@@ -176,12 +176,13 @@ hipError_t pr_scale(float *pr, u32 V, const float *red, hipStream_t st);
 // binned edges: geometry of one PageRank call
 struct PrBins {
     u32 part_log;    // slots per part (log2)
-    u32 parts;       // parts of the slot array (<= 1024)
+    u32 parts;       // parts of the slot array (<= 2^14)
     u32 bins;        // destination bins of 8192 vertices
     u32 chunk;       // edge words per chunk of an iteration
     u32 max_chunks;  // bound on the chunks of all bins (the iteration's grid)
     u32 max_multi;   // bound on the chunks of bins of several chunks
     u32 staged;      // bin pass stages whole 32-byte chunks in LDS
+    u32 group;       // words that share a row; a run is padded to whole groups
     u64 words;       // room for the edge words, padding included
 };
 // masses of one iteration, in a ring of PR_SLOTS

@@ -336,3 +336,21 @@ def test_pagerank_bins_and_chunks(V, E):
     before, _ = oracle.pagerank(keys, V, 0.85, 6)
     assert abs(delta - np.abs(want - before).sum()) < 1e-6
     pma.close()
+
+
+@pytest.mark.parametrize("V,E", [((1 << 17) + 3, 2000), (1 << 20, 150000), ((1 << 24) + 5, 20000000)])
+def test_pagerank_runs_of_edges(V, E):
+    """Few edges over many bins and parts, whose runs go without padding, and
+    more bins than the staged bin pass takes with enough edges for padding."""
+    say(f"pagerank runs V={V} E={E}")
+    from gpu_util import keys_of
+    rng = np.random.default_rng(V)
+    dst = rng.integers(0, V, E)
+    dst[::3] = V - 1 - dst[::3] % 5000
+    keys = oracle.sort_unique(keys_of(rng.integers(0, V, E), dst))
+    pma = L.PMA(V)
+    pma.insert(keys)
+    pr, iters, delta = pma.pagerank(0.85, 0.0, 3)
+    want, _ = oracle.pagerank(keys, V, 0.85, 3)
+    assert np.abs(pr.cpu().numpy().astype(np.float64) - want).sum() < 1e-6
+    pma.close()
