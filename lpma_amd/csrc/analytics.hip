@@ -851,7 +851,8 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_count(DevState d, u32 part_log, u
 
 // words[off[bin * P + part] + rank] = pb_word(edge)
 // Phases per step: all key loads, all cursor adds, then the stores, so each
-// thread keeps PB_ITEMS loads in flight at a time.  G: words of a group.
+// thread keeps PB_ITEMS loads in flight at a time.  G: words of a group (of
+// one, the row stands beside its word).
 template <u32 G>
 __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32 P, u32 NB, const u32 *__restrict__ off,
                                                    u32 *__restrict__ words, u32 *__restrict__ rows, u64 room) {
@@ -886,8 +887,12 @@ __global__ __launch_bounds__(PB_TPB) void k_pb_bin(DevState d, u32 part_log, u32
             const u32 b0 = __shfl(base[i], lead[i], 64);
             const u64 pos = (u64)b0 + (lane - lead[i]);
             if (pb_edge(key[i]) && pos < room) {
-                words[pos] = pb_word(key[i], row0);
-                if (pos % G == 0) rows[pos / G] = row0;
+                if (G == 1) {
+                    ((uint2 *)words)[pos] = make_uint2(pb_word(key[i], row0), row0);
+                } else {
+                    words[pos] = pb_word(key[i], row0);
+                    if (pos % G == 0) rows[pos / G] = row0;
+                }
             }
         }
     }
@@ -1190,8 +1195,14 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
         for (u32 r = 0; r < PRI_ITEMS; ++r) {
             const u64 i = i0 + (u64)r * PRI_TPB + threadIdx.x;
             const u64 j = i < s1 ? i : s1 - 1;  // unconditional loads: all of them in flight together
-            e[r] = words[j];
-            row0[r] = rows[j / G];
+            if (G == 1) {
+                const uint2 w = ((const uint2 *)words)[j];
+                e[r] = w.x;
+                row0[r] = w.y;
+            } else {
+                e[r] = words[j];
+                row0[r] = rows[j / G];
+            }
             if (i >= s1) e[r] = PB_PAD;
         }
         float x[PRI_ITEMS];
@@ -1260,7 +1271,7 @@ __global__ void k_pr_norm(const float *pr, float *rank, u32 V, const PrSlot *slo
 
 bool pr_bins_fit(u32 V) { return ((u64)V + PB_BIN - 1) / PB_BIN <= PB_MAX_BINS; }
 
-// the groups' rows follow the words
+// the groups' rows follow the words (groups of one word: stand beside them)
 static u64 pr_bins_rows_at(const PrBins &b) { return (b.words + b.group - 1) / b.group * b.group; }
 u64 pr_bins_edge_words(const PrBins &b) { return pr_bins_rows_at(b) / b.group * (b.group + 1) + b.group; }
 
@@ -1277,6 +1288,9 @@ PrBins pr_bins_plan(const DevState &d, u64 edges) {
     // Every run that holds an edge is padded to whole groups, and the offsets
     // of the words are 32-bit sums: runs whose padding could pass them, or could
     // take more memory than a row beside every word (8 B an edge), go unpadded.
+    // First iteration and each further one, unpadded against padded: 1.8*10^7
+    // edges on 2^24 vertices 1044 + 377 us (988 + 372), 4*10^6 562 + 195 (626 +
+    // 199), 4*10^6 on 2^22 214 + 72 (273 + 118).
     b.group = PB_CHUNK;
     b.words = std::min<u64>(edges * PB_CHUNK, edges + (u64)(PB_CHUNK - 1) * b.bins * b.parts);
     if (b.words >= 1ull << 32 || pr_bins_edge_words(b) > 2 * edges) {
