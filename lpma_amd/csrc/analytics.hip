@@ -1045,19 +1045,14 @@ __global__ __launch_bounds__(1024) void k_pb_chunks(const u32 *__restrict__ off,
     if (threadIdx.x == 0) cb[NB] = (u32)carry;
 }
 
-// Sums of contributions are kept in 64-bit fixed point of PR_FIX fractional
-// bits: the ranks of a vector sum to 1 (the recurrence keeps it), so a sum
-// stays below 2^(64 - PR_FIX), the adds are exact and their order does not
-// matter.  An FP32 contribution of 2^-39 or more converts exactly; a smaller
-// one loses less than 2^-62.  LDS adds 64-bit integers natively, where FP32
-// compensated by a compare-and-swap took 428 us an iteration at 6.4e7 edges.
-static constexpr u32 PR_FIX = 62;
-__device__ __forceinline__ u64 pr_fixed(float x) {
-    const u32 bits = __float_as_uint(x), e = bits >> 23;  // x >= 0
-    const u64 m = ((u64)((bits & 0x7FFFFFu) | 0x800000u)) << (PR_FIX - 23);  // mantissa, of value 1 at e = 127
-    return m >> min(127u - min(e, 127u), 63u);  // e = 0 (zero, denormal): shifted out
+// Sums of contributions are kept in 64 bits of floating point: an FP32
+// contribution of any size enters whole, and LDS adds such sums natively, where
+// FP32 compensated by a compare-and-swap took 428 us an iteration at 6.4e7
+// edges.
+__device__ __forceinline__ void pr_add(double *sum, float x) {
+    typedef __attribute__((address_space(3))) double lds_double;
+    (void)__builtin_amdgcn_ds_atomic_fadd_f64((lds_double *)sum, (double)x);
 }
-__device__ __forceinline__ float pr_float(u64 v) { return (float)((double)v * (1.0 / (double)(1ull << PR_FIX))); }
 
 // the host's word: (iteration, its L1 change)
 __device__ __forceinline__ void pr_report(const PrSlot &s, u32 it, u64 *host) {
@@ -1119,26 +1114,14 @@ __global__ __launch_bounds__(PR_TPB) void k_pr_start(DevState d, const u32 *__re
 // behind it return at once, which lets the host queue an iteration ahead; the
 // first kernel reports the change of the one before it to the host's word.
 
-// Waits for the LDS adds of f at e with both still in their registers.  A
-// 64-bit LDS add without a result has been seen here to pick up its operand
-// after a later instruction had overwritten the register, when many lanes add
-// to one word and the LDS falls behind (half-converted contributions then
-// ended up in the sums): the operands stay untouched until the adds are done.
-template <u32 N>
-__device__ __forceinline__ void lds_adds_done(const u64 (&f)[N], const u32 (&e)[N]) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-    for (u32 r = 0; r < N; ++r) asm volatile("" ::"v"(f[r]), "v"(e[r]));
-}
-
 // a vertex's new rank pr' = alpha * sum + gamma, gamma = (alpha * dangling +
 // (1 - alpha) * sum(pr)) / n, and what the next iteration needs of it
 struct PrMass {
     double dang, sum, delta;
 };
-__device__ __forceinline__ void pr_vertex(u32 v, u64 acc, float alpha, float gamma, const float *pr, float *out,
+__device__ __forceinline__ void pr_vertex(u32 v, double acc, float alpha, double gamma, const float *pr, float *out,
                                           const u32 *outdeg, float *cnext, PrMass &m) {
-    const float p = alpha * pr_float(acc) + gamma;
+    const float p = (float)((double)alpha * acc + gamma);
     const u32 od = outdeg[v];
     m.delta += (double)fabsf(p - pr[v]);
     m.sum += (double)p;
@@ -1146,8 +1129,8 @@ __device__ __forceinline__ void pr_vertex(u32 v, u64 acc, float alpha, float gam
     out[v] = p;
     cnext[v] = od ? p / (float)od : 0.f;
 }
-__device__ __forceinline__ float pr_gamma(const PrSlot &prev, float alpha, u32 V) {
-    return (alpha * (float)prev.dang + (1.f - alpha) * (float)prev.sum) / (float)V;
+__device__ __forceinline__ double pr_gamma(const PrSlot &prev, float alpha, u32 V) {
+    return ((double)alpha * prev.dang + (1.0 - (double)alpha) * prev.sum) / (double)V;
 }
 
 // Chunk k of a bin's edges (cb = chunks before each bin), in groups of G words.  A bin of one chunk
@@ -1167,9 +1150,9 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
                                                      const float *__restrict__ c, float *__restrict__ cnext,
                                                      const float *__restrict__ pr, float *__restrict__ out,
                                                      const u32 *__restrict__ outdeg, u32 V, float alpha, float tol,
-                                                     u32 it, PrSlot *slots, u64 *__restrict__ partial,
+                                                     u32 it, PrSlot *slots, double *__restrict__ partial,
                                                      u64 *__restrict__ host) {
-    extern __shared__ u64 pb_acc[];  // PB_BIN sums
+    extern __shared__ double pb_acc[];  // PB_BIN sums
     __shared__ double red[3 * PRI_TPB / 64];
     const PrSlot &prev = slots[(it - 1) % PR_SLOTS];
     if (blockIdx.x == 0 && threadIdx.x == 0 && it > 1) pr_report(prev, it - 1, host);
@@ -1187,7 +1170,7 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
     const u64 s0 = (u64)off[(u64)b * P] + (u64)(k - cb[b]) * chunk;
     const u64 s1 = min(e1, s0 + chunk);
     const u32 v0 = b << PB_BIN_LOG, nv = min(PB_BIN, V - v0);
-    for (u32 v = threadIdx.x; v < PB_BIN; v += PRI_TPB) pb_acc[v] = 0ull;
+    for (u32 v = threadIdx.x; v < PB_BIN; v += PRI_TPB) pb_acc[v] = 0.0;
     __syncthreads();
     for (u64 i0 = s0; i0 < s1; i0 += (u64)PRI_TPB * PRI_ITEMS) {
         u32 e[PRI_ITEMS], row0[PRI_ITEMS];
@@ -1208,21 +1191,16 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
         float x[PRI_ITEMS];
 #pragma unroll
         for (u32 r = 0; r < PRI_ITEMS; ++r) x[r] = c[e[r] == PB_PAD ? V : row0[r] + (e[r] >> PB_BIN_LOG)];
-        u64 f[PRI_ITEMS];
 #pragma unroll
-        for (u32 r = 0; r < PRI_ITEMS; ++r) f[r] = pr_fixed(x[r]);
-#pragma unroll
-        for (u32 r = 0; r < PRI_ITEMS; ++r)
-            atomicAdd((unsigned long long *)&pb_acc[e[r] & (PB_BIN - 1)], (unsigned long long)f[r]);
-        lds_adds_done(f, e);
+        for (u32 r = 0; r < PRI_ITEMS; ++r) pr_add(&pb_acc[e[r] & (PB_BIN - 1)], x[r]);
     }
     __syncthreads();
     if (nch > 1) {
-        u64 *to = partial + (u64)(cb[NB + 1 + b] + (k - cb[b])) * PB_BIN;
+        double *to = partial + (u64)(cb[NB + 1 + b] + (k - cb[b])) * PB_BIN;
         for (u32 v = threadIdx.x; v < nv; v += PRI_TPB) to[v] = pb_acc[v];
         return;
     }
-    const float gamma = pr_gamma(prev, alpha, V);
+    const double gamma = pr_gamma(prev, alpha, V);
     PrMass m{0.0, 0.0, 0.0};
     for (u32 v = threadIdx.x; v < nv; v += PRI_TPB)
         pr_vertex(v0 + v, pb_acc[v], alpha, gamma, pr, out, outdeg, cnext, m);
@@ -1231,7 +1209,7 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
 
 // the bins of several chunks: PB_BIN / PRI_TPB workgroups a bin, a thread a
 // vertex, the chunks' sums read PRI_ITEMS at a time
-__global__ __launch_bounds__(PRI_TPB) void k_pr_join(u32 NB, const u32 *__restrict__ cb, const u64 *__restrict__ partial,
+__global__ __launch_bounds__(PRI_TPB) void k_pr_join(u32 NB, const u32 *__restrict__ cb, const double *__restrict__ partial,
                                                      float *__restrict__ cnext, const float *__restrict__ pr,
                                                      float *__restrict__ out, const u32 *__restrict__ outdeg, u32 V,
                                                      float alpha, float tol, u32 it, PrSlot *slots) {
@@ -1246,10 +1224,10 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_join(u32 NB, const u32 *__restri
     const u32 v = (b << PB_BIN_LOG) + w;
     PrMass m{0.0, 0.0, 0.0};
     if (v < V) {
-        u64 acc = 0;
+        double acc = 0.0;
         u32 k = k0;
         for (; k + PRI_ITEMS <= k1; k += PRI_ITEMS) {
-            u64 t[PRI_ITEMS];
+            double t[PRI_ITEMS];
 #pragma unroll
             for (u32 r = 0; r < PRI_ITEMS; ++r) t[r] = partial[(u64)(k + r) * PB_BIN + w];
 #pragma unroll
@@ -1264,9 +1242,9 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_join(u32 NB, const u32 *__restri
 // rank = p / sum(p) of iteration `it`, and its report to the host
 __global__ void k_pr_norm(const float *pr, float *rank, u32 V, const PrSlot *slot, u32 it, u64 *host) {
     if (blockIdx.x == 0 && threadIdx.x == 0) pr_report(*slot, it, host);
-    const float inv = 1.f / (float)slot->sum;
+    const double inv = 1.0 / slot->sum;
     for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (u64)gridDim.x * blockDim.x)
-        rank[v] = pr[v] * inv;
+        rank[v] = (float)((double)pr[v] * inv);
 }
 
 bool pr_bins_fit(u32 V) { return ((u64)V + PB_BIN - 1) / PB_BIN <= PB_MAX_BINS; }
@@ -1340,9 +1318,9 @@ u64 pr_bins_partial_words(const PrBins &b) { return std::max<u64>(1, (u64)b.max_
 
 hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
                            const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
-                           float tol, u32 it, PrSlot *slots, u64 *partial, u64 *host, hipStream_t st) {
+                           float tol, u32 it, PrSlot *slots, double *partial, u64 *host, hipStream_t st) {
     const auto iter = b.group == PB_CHUNK ? k_pr_iter<PB_CHUNK> : k_pr_iter<1>;
-    iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(u64), st>>>(
+    iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(double), st>>>(
         words, words + pr_bins_rows_at(b), off, b.parts, b.bins, cb, b.chunk, c, cnext, pr, out, outdeg, d.V, alpha, tol, it,
         slots, partial, host);
     if (b.max_multi)

@@ -206,7 +206,7 @@ hipError_t pr_bins_start(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *o
 u64 pr_bins_partial_words(const PrBins &b);
 hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
                            const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
-                           float tol, u32 it, PrSlot *slots, u64 *partial, u64 *host, hipStream_t st);
+                           float tol, u32 it, PrSlot *slots, double *partial, u64 *host, hipStream_t st);
 hipError_t pr_bins_norm(const float *pr, float *rank, u32 V, u32 it, const PrSlot *slots, u64 *host, hipStream_t st);
 
 }  // namespace pma

@@ -247,7 +247,8 @@ struct lpma {
     // analytics scratch
     DBuf<u32> aq0, apoff, apcb, apwords;
     DBuf<float> af0, af1, af2, ared;
-    DBuf<u64> apart, aslots;
+    DBuf<double> apart;
+    DBuf<u64> aslots;
     u64 *h_word = nullptr;  // pinned: a word kernels report to
     u32 *d_err = nullptr;
 

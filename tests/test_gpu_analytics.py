@@ -354,3 +354,30 @@ def test_pagerank_runs_of_edges(V, E):
     want, _ = oracle.pagerank(keys, V, 0.85, 3)
     assert np.abs(pr.cpu().numpy().astype(np.float64) - want).sum() < 1e-6
     pma.close()
+
+
+@pytest.mark.parametrize("degree", [1000, 37])
+def test_pagerank_small_ranks(degree):
+    """Ranks far below 1/V keep FP32's relative precision: with damping 1 a
+    path whose vertices also lead to a cycle passes 1/degree of its rank on at
+    each step (1/V degree^-k after k of them).  A rank's value is rounded four
+    times an iteration and once when it is scaled, to 2^-24 each."""
+    say(f"pagerank small ranks degree={degree}")
+    from gpu_util import keys_of
+    V, steps = 5000, 6
+    cycle = np.arange(2000, V)
+    src, dst = [cycle], [np.roll(cycle, -1)]
+    for k in range(2000):
+        to = np.append(cycle[(np.arange(degree - 1) * 7 + k) % cycle.size], (k + 1) % 2000 if k < 1999 else 2000)
+        src.append(np.full(degree, k))
+        dst.append(to)
+    keys = oracle.sort_unique(keys_of(np.concatenate(src), np.concatenate(dst)))
+    pma = L.PMA(V)
+    pma.insert(keys)
+    for it in range(1, steps + 1):
+        got = pma.pagerank(1.0, 0.0, it)[0].cpu().numpy().astype(np.float64)
+        want, _ = oracle.pagerank(keys, V, 1.0, it)
+        there = want > 0
+        assert np.array_equal(got > 0, there)
+        assert np.max(np.abs(got[there] - want[there]) / want[there]) < (4 * it + 2) * 2.0 ** -24
+    pma.close()
