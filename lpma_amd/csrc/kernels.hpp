@@ -106,7 +106,8 @@ hipError_t rebalance_large(const Group &g, const BatchBufs &b, u64 *merged, u32 
 // root rebuild / resize of PMA pid: its keys after the batch (updates [u0, u1)
 // of the compacted batch) from src's arrays straight into dst's, spread evenly
 // (index: rebuild_index_words(src) words of scratch for the per-chunk update
-// starts and ranks; merged: room for the live keys where rebuild_merges())
+// starts and ranks; merged: room for the live keys to rebuild by merging them,
+// which pays where rebuild_merges(), or null)
 bool rebuild_merges(u64 live, u64 updates);
 hipError_t rebuild_scatter(const DevState &src, const DevState &dst, u32 pid, u32 u0, u32 u1, const BatchBufs &b,
                            u64 live, u64 m, u32 *index, u64 *merged, hipStream_t st);

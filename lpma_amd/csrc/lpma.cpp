@@ -827,7 +827,8 @@ int upload_table(Pipeline &pl, const Member *mem, u32 npma, u32 &pyr_blocks, hip
 // and that the pyramid's chunk levels are left owing to the next batch.
 //
 // Every fallible allocation of the round comes before its first change of a
-// PMA, so a round that fails with LPMA_ERR_OUT_OF_MEMORY changes nothing.  A
+// PMA, so a round that fails with LPMA_ERR_OUT_OF_MEMORY changes nothing (a
+// rebuild that cannot have the scratch to merge goes by chunks).  A
 // graph replay over several PMAs elects no windows at all when one of them
 // needs a rebuild (Group::defer_rebuild); the election then runs again here,
 // after the allocations.
@@ -869,6 +870,7 @@ int finish_round(Pipeline &pl, const Member *mem, u32 npma, const Group &g_in, u
     // election is still to come), and the new arrays of every member that
     // is rebuilt (a resize, or a root rebalance at the same height)
     std::vector<Geometry> geo(npma);
+    std::vector<char> merges(npma, 0);  // rebuilt by merging: the scratch is there
     auto undo = [&](int r) {
         for (u32 p = 0; p < npma; ++p) release_geometry(mem[p].h, geo[p]);
         return r;
@@ -883,10 +885,14 @@ int finish_round(Pipeline &pl, const Member *mem, u32 npma, const Group &g_in, u
         }
         for (u32 p = 0; !r && any_rebuild && p < npma; ++p)
             if (ps[p].flags & (FLAG_ROOT | FLAG_RESIZE)) {
-                if (rebuild_merges(mem[p].h->live, ps[p].u1 - ps[p].u0)) r = ensure(pl, pl.merged, mem[p].h->live);
-                if (!r) r = ensure(pl, pl.gpre, rebuild_index_words(mem[p].h->st));
+                r = ensure(pl, pl.gpre, rebuild_index_words(mem[p].h->st));
                 if (!r) r = alloc_geometry(mem[p].h, newH[p], geo[p], st);
             }
+        // after all that the round cannot do without
+        for (u32 p = 0; !r && any_rebuild && p < npma; ++p)
+            merges[p] = (ps[p].flags & (FLAG_ROOT | FLAG_RESIZE)) &&
+                        rebuild_merges(mem[p].h->live, ps[p].u1 - ps[p].u0) &&
+                        ensure(pl, pl.merged, mem[p].h->live) == LPMA_OK;
         if (r) return undo(r);
     }
     BatchBufs bb = batch_bufs(pl);
@@ -947,7 +953,7 @@ int finish_round(Pipeline &pl, const Member *mem, u32 npma, const Group &g_in, u
             if (!(ps[p].flags & (FLAG_ROOT | FLAG_RESIZE))) continue;
             lpma *h = mem[p].h;
             HIPUNDO(rebuild_scatter(h->st, state_with(h, newH[p], geo[p]), p, ps[p].u0, ps[p].u1, bb, h->live,
-                                    Mnew[p], pl.gpre.p, pl.merged.p, st));
+                                    Mnew[p], pl.gpre.p, merges[p] ? pl.merged.p : nullptr, st));
             const int r = pyramid_and_install(h, newH[p], geo[p], st);
             if (r) return undo(r);
             h->rebuilds++;

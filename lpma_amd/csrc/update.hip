@@ -2246,7 +2246,7 @@ hipError_t rebuild_scatter(const DevState &src, const DevState &dst, u32 pid, u3
     const u64 pb = (u64)pid << 32;
     const double spk = (double)nseg_of(dst) / (double)m;
     k_chunk_index<<<(u32)((nch + 1 + 3) / 4), 256, 0, st>>>(src, pb, u0, u1, b.cseg, cq, cob);
-    if (rebuild_merges(live, u1 - u0)) {
+    if (merged) {
         k_gather_live<<<(u32)nch, LGP_TPB, 0, st>>>(src, cob, merged);
         const u32 tiles = (u32)((live + (u1 - u0) + RM_TILE - 1) / RM_TILE);
         k_rebuild_merge<<<tiles, LGP_TPB, 0, st>>>(dst, merged, (u32)live, b.ckey + u0, b.pd + u0, u1 - u0, m, spk);

@@ -194,3 +194,31 @@ def test_pool_budget_exhausted_by_resize():
     case.apply()
     case.verify()
     case.close()
+
+
+def test_rebuild_without_merge_scratch():
+    """A batch of more than half of the live keys rebuilds by merging, which
+    takes a word a live key; where that is not to be had it rebuilds without."""
+    say("rebuild without merge scratch")
+    V = 1 << 12
+    keys = L.shuffle(L.gen_uniform(V, 1000000, 7), 7)
+    other = L.shuffle(L.gen_uniform(V, 50000, 8), 8)
+    case = Case([(V, keys, np.empty(0, dtype=np.uint64), keys[:600000].copy())] +
+                [(V, other, other[:1], other[1:2].copy())], group=True)
+    old = case.pmas[0].view()
+    empty = np.empty(0, dtype=np.uint64)
+    # the batch's own buffers: as many keys, without effect
+    case.group.update([s[1][:s[2].size + s[3].size] for s in case.specs], [empty] * 2)
+    torch.cuda.synchronize()
+    L.pool_trim()
+    # the new arrays: half as many slots, in segments of 32
+    arrays = int(old.capacity) // 2 * 9
+    assert 8 * int(old.live_keys) > arrays + (2 << 20)
+    try:
+        L.set_pool_budget(L.pool_reserved_bytes() + arrays + (2 << 20))
+        case.apply()
+    finally:
+        L.set_pool_budget(0)
+    case.verify()
+    assert case.pmas[0].view().capacity == old.capacity // 2
+    case.close()
