@@ -330,7 +330,8 @@ typedef struct {
     uint64_t snapshot_max_age_us; /* a BFS reuses the newest snapshot while younger, default 50000;
                                      0: every BFS sees the version current at its admission */
     uint32_t search_workgroups;   /* workgroups of each search's frontier expansion, default 256 of
-                                     the 2048 a lone search uses, so searches leave room for the writer */
+                                     the 1024 a lone search uses, so searches leave room for the writer;
+                                     0: 1024 */
 } lpma_server_config_t;
 
 typedef struct {

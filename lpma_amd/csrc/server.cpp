@@ -176,7 +176,9 @@ int grow_pin(Pin<T> &b, u64 n, hipStream_t st) {
 // device scratch of one search: per vertex two queues, an entry's two words
 // and the level (20 B) and a visited bit; one run entry per 256 slots (a
 // snapshot holds at least 8 B per slot, so snapshot bytes / 512 covers it);
-// the control words
+// the control words.  Searches run with a width of their own, which take no
+// lists of destinations (a word a slot, where there is memory for them).
+constexpr u32 SEARCH_FULL_WIDTH = 1024;  // the workgroups that fit the device, as a search without a width uses
 u64 bfs_bytes(u32 V, u64 snap_bytes) {
     return 20ull * ((u64)V + 2) + (u64)V / 8 + 64 + snap_bytes / 512 + (1ull << 20);
 }
@@ -380,7 +382,8 @@ void dispatch_bfs(lpma_server *s, std::unique_lock<std::mutex> &lk) {
                 s->cv_done.notify_all();
                 continue;
             }
-            lpma_snapshot_set_search_width(snap, s->cfg.search_workgroups);
+            lpma_snapshot_set_search_width(
+                snap, s->cfg.search_workgroups ? s->cfg.search_workgroups : SEARCH_FULL_WIDTH);
             Snap *p = new Snap();
             p->s = snap;
             p->applied = s->applied;

@@ -187,6 +187,31 @@ def test_bfs_admission_by_budget():
     pma.close()
 
 
+def test_full_width_search_within_its_charge():
+    """A server's search of the full width takes no more memory than admission
+    charges it: the snapshot, and 20 B and a bit a vertex and a word for 256
+    slots."""
+    say("server search at full width")
+    rng = np.random.default_rng(54)
+    V, E = 200000, 9500000
+    keys = oracle.sort_unique(rand_keys(rng, V, E))
+    pma = L.PMA(V)
+    pma.bulk_load(keys)
+    assert pma.view().capacity >= 1 << 24
+    snap = int(L.lib().lpma_snapshot_bytes(pma._h))
+    budget = snap + 20 * (V + 2) + V // 8 + 64 + snap // 512 + (1 << 20)
+    L.lib().lpma_pool_trim()
+    held = L.pool_reserved_bytes()
+    srv = L.Server(pma, bfs_workers=1, hbm_budget_bytes=budget, search_workgroups=0)
+    r = srv.wait(srv.submit_bfs(0))
+    srv.close()
+    want = oracle.bfs(keys, V, 0)
+    assert r["status"] == 0 and r["depth"] == int(want[want != 0xFFFFFFFF].max()) + 1
+    # blocks of the pool are up to twice what was asked for, large ones 16 MiB more
+    assert L.pool_reserved_bytes() - held <= snap + 2 * (budget - snap) + (32 << 20)
+    pma.close()
+
+
 def test_invalid_update_fails_alone():
     say("server invalid update")
     rng = np.random.default_rng(53)
