@@ -753,16 +753,20 @@ hipError_t device_excl_scan(const u32 *in, u64 n, u32 *out, u32 *scratch, hipStr
 // Keys a thread in a tile of the one-kernel passes: 4 up to one tile per CU, 8
 // beyond, for longer runs and fewer tiles to look back over (2*10^6 keys: 17.6
 // against 19.9 us a pass; 8.4*10^6: 55 and 54).
-static u32 os_items(u64 n) { return n <= (1ull << 20) ? 4 : 8; }
+static constexpr u64 OS_SMALL_N = 1ull << 20;
+static u32 os_items(u64 n) { return n <= OS_SMALL_N ? 4 : 8; }
 
 // digit width for a sort over `width` bits: as many passes as 8-bit digits take
 static u32 os_digit_bits(u32 width) { return (width + 7) / 8 * 7 >= width ? 7 : 8; }
 
+// of any batch of up to n keys (never less for more keys: a reserved scratch
+// serves the smaller batches too, whose tiles may be smaller and more)
 u64 sort_scratch_words(u64 n) {
-    const u64 tile = (u64)os_items(n) * OS_TPB;
-    const u64 look = 2 * ((n + tile - 1) / tile) * OS_MAX_R;
-    const u64 split = (u64)ss_buckets(n) * ss_tiles(n);
-    return OS_GH_WORDS + (n <= SS_MAX_N ? split : look);
+    auto tiles = [](u64 keys, u64 tile) { return (keys + tile - 1) / tile; };
+    const u64 small = std::min<u64>(n, OS_SMALL_N), ss = std::min<u64>(n, SS_MAX_N);
+    const u64 look = std::max(tiles(small, 4 * OS_TPB), n > OS_SMALL_N ? tiles(n, 8 * OS_TPB) : 0);
+    const u64 split = ss_buckets(ss) * std::min<u64>(SS_MAX_TILES, tiles(ss, SS_TPB));
+    return OS_GH_WORDS + std::max<u64>(2 * OS_MAX_R * look, split);
 }
 
 u32 sort_zero_words() { return OS_GH_WORDS; }

@@ -67,3 +67,13 @@ def test_pagerank_edge_words_memory(plans):
     sizes = pagerank_sizes()
     for size, (words, room, bins, parts) in zip(sizes, plans(["pagerank %d %d %d %d" % s for s in sizes])):
         assert room <= 2 * size[3] + 64, (size, room, bins, parts)
+
+
+def test_sort_scratch_grows_with_the_batch(plans):
+    """lpma_reserve(n) sizes the scratch of every batch of up to n keys."""
+    rng = random.Random(6)
+    edges = [1 << 10, 1 << 12, 1 << 16, 1 << 17, 1 << 18, 1 << 19, 1 << 20, 1 << 22]
+    ns = sorted({1, 2, 300} | {e + d for e in edges for d in (-1, 0, 1)} | {int(2 ** rng.uniform(0, 31)) for _ in range(500)})
+    got = [w for w, in plans(["sort %d" % n for n in ns])]
+    for (n, w), (n2, w2) in zip(zip(ns, got), list(zip(ns, got))[1:]):
+        assert w <= w2, (n, w, n2, w2)
