@@ -46,6 +46,7 @@ static constexpr u32 FLAG_INVALID_KEY = 1u;   // src or dst >= V
 static constexpr u32 FLAG_ROOT = 2u;          // a run chose the root window
 static constexpr u32 FLAG_RESIZE = 4u;        // the root window does not fit
 static constexpr u32 FLAG_SORT_STALL = 8u;    // a sort tile waited too long (the batch fails)
+static constexpr u32 FLAG_SORT_SKEW = 16u;    // not sorted: too skewed for buckets (the host runs the batch again)
 
 // most passes of the batch sort (8-bit digits over 64 bits)
 static constexpr u32 SORT_MAX_PASSES = 8;

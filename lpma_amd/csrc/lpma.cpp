@@ -978,8 +978,10 @@ int run_pipeline_graph(Pipeline &pl, const Member *mem, u32 npma, u64 n, u32 psh
 // One update round over the members (all on pl's device, same segment size,
 // ids fitting above the sort keys): sort + dedup + locate + density check +
 // election over every member at once, one host synchronisation, then the
-// rebalance classes, the pyramid, and root rebuilds / resizes per member.
-int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
+// rebalance classes, the pyramid, and root rebuilds / resizes per member.  A
+// batch that turns out too skewed for the sort's buckets (FLAG_SORT_SKEW) has
+// changed nothing and runs again, `skewed`.
+int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool skewed = false) {
     pl.cur_stream = st;
     u64 n = 0, nseg_total = 0;
     bool mixed = false;
@@ -987,7 +989,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     for (u32 p = 0; p < npma; ++p) {
         lpma *h = mem[p].h;
         h->cur_stream = st;
-        h->calls++;
+        if (!skewed) h->calls++;
         bool any_ins = false, any_del = false;
         for (u32 r = 0; r < mem[p].nreq; ++r) {
             const Req &q = mem[p].reqs[r];
@@ -1001,7 +1003,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
         vmax = std::max(vmax, h->vbits);
         nseg_total += 1ull << h->st.H;
     }
-    pl.rounds++;
+    if (!skewed) pl.rounds++;
     if (n == 0) {
         for (u32 p = 0; p < npma; ++p) mem[p].h->version++;
         return LPMA_OK;
@@ -1011,7 +1013,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     const u32 pshift = 2 * vmax + 1 + sbits;
     const u32 hi_bit = pshift + bits_for(npma);
     if (hi_bit > 64) return LPMA_ERR_TOO_LARGE;
-    if (pl.graph_on && maxreq <= 1) return run_pipeline_graph(pl, mem, npma, n, pshift, hi_bit, st);
+    if (pl.graph_on && maxreq <= 1 && !skewed) return run_pipeline_graph(pl, mem, npma, n, pshift, hi_bit, st);
     CHECKED(ensure_batch(pl, n, npma, nsegs, std::min<u64>(n, nseg_total)));
     // A lone PMA's single-segment and wave windows are queued before the
     // host reads the status (below): the large windows that may follow
@@ -1032,7 +1034,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
     CHECKED(upload_table(pl, mem, npma, pyr_blocks, st));
 
     // the sort carries the batch's first work and takes the sources as arguments
-    const bool carried = npma == 1 && sort_carries_first(n, nsegs);
+    const bool carried = npma == 1 && !skewed && sort_carries_first(n, nsegs);
     // batch sources: each request's deletes (op 0), then its inserts (op 1)
     {
         u64 off = 0;
@@ -1107,7 +1109,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
                 HIPCHECK(batch_begin(g, bb, pl.h_segs, nsegs <= ARG_SEGS ? nsegs : 0, pl.segs.p, pl.sort_scr.p,
                                      sort_zero_words(), st));
                 pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
-                                   pl.ukey.p, pl.sort_scr.p, &bb.status->flags, st);
+                                   pl.ukey.p, pl.sort_scr.p, &bb.status->flags, skewed, st);
             }
             HIPCHECK(hipGetLastError());
         }
@@ -1148,6 +1150,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st) {
         u64 w;
         CHECKED(wait_word(&pl.h_early->seq, st, w, [epoch](u64 x) { return x == epoch; }));
     }
+    if (((const Status *)pl.h_out)->flags & FLAG_SORT_SKEW) return run_pipeline(pl, mem, npma, st, true);
     return finish_round(pl, mem, npma, g, pyr_blocks, false, st, early);
 }
 
@@ -1244,7 +1247,7 @@ int graph_for(Pipeline &pl, u64 cap, u32 npma, u32 pshift, u32 hi_bit, u32 log2S
                   batch_begin(g, bb, nullptr, 0, pl.segs.p, pl.sort_scr.p, sort_zero_words(), cs) == hipSuccess;
         if (ok) {
             u64 *pk = pack_and_sort(pl.segs.p, nsegs, cap, &pl.rhdr.p->n, pshift, 0, 0, hi_bit, pl.pk0.p, pl.pk1.p,
-                                    pl.ukey.p, pl.sort_scr.p, &bb.status->flags, cs);
+                                    pl.ukey.p, pl.sort_scr.p, &bb.status->flags, false, cs);
             ok = hipGetLastError() == hipSuccess && locate_and_compact(g, pk, cap, bb, cs) == hipSuccess &&
                  density_check(g, cap, bb, cs) == hipSuccess && elect_windows(g, cap, bb, cs) == hipSuccess &&
                  rebalance_fixed(g, bb, (u32)cap, nullptr, cs) == hipSuccess &&
@@ -1315,6 +1318,7 @@ int run_pipeline_graph(Pipeline &pl, const Member *mem, u32 npma, u64 n, u32 psh
     }
     pl.graph_launches++;
     HIPCHECK(hipStreamSynchronize(st));
+    if (((const Status *)pl.h_out)->flags & FLAG_SORT_SKEW) return run_pipeline(pl, mem, npma, st, true);
     Group g = graph_group(pl, npma, pshift, log2S);
     g.epoch = epoch;  // a repeated election runs eagerly, outside the graph
     g.rh = nullptr;

@@ -11,7 +11,8 @@
 //   <= 2^19 keys   sample-split sort: two kernels, buckets chosen from a
 //                  sample, each sorted by a bitonic network;
 //   larger         LSD radix, one kernel per 7/8-bit digit (decoupled
-//                  look-back), the digit counts of every pass taken at pack.
+//                  look-back), the digit counts of every pass taken at pack;
+//                  also smaller batches found too skewed for the buckets.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "begin.hpp"
@@ -273,9 +274,17 @@ __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, 
 // between waves), and writes them at the bucket's offset.  A sample-chosen
 // split keeps buckets even under R-MAT skew, where a split on the top key bits
 // puts a hub's keys in one bucket.  A bucket beyond the workgroup's SB_CAP keys
-// (many equal keys) is LSD-radix-sorted through global memory, chunk by chunk,
-// on the bits on which its keys differ (AND / OR of the keys), with wave64
-// ranking (the k_os_pass scheme).
+// is LSD-radix-sorted through global memory, chunk by chunk, on the bits on
+// which its keys differ (AND / OR of the keys), with wave64 ranking (the
+// k_os_pass scheme): 3 us a chunk to gather and 8 a chunk and pass.  A splitter
+// that is repeated (a projection of more than an average bucket) has a bucket of
+// its own, so that a key repeated some thousand times is not mixed with others
+// and takes few passes or none.  A batch with a projection of SS_SKEW_KEYS keys
+// or more (a hub of a graph of so many vertices that its edges share
+// projections), or SS_SKEW_SAME copies of one key, is not sorted but flagged
+// FLAG_SORT_SKEW: the kernels after it do nothing, and the host runs it again
+// with the passes below, 50 us later.  Batches of 4*10^5 keys over 2^20 vertices,
+// one key half of them: 193 us, 1660 by one workgroup on mixed buckets.
 //
 // Bound: the sample's sort in every tile (vector issue: 1024 samples 5 us, 2048
 // 10 us with one tile a compute unit) and the largest bucket.  10^5 R-MAT keys:
@@ -299,11 +308,17 @@ static constexpr u32 SB_NW = SB_TPB / 64;
 // a tile's count entry: offset << 16 | count, bit 31 on bucket 0's entry
 // when the tile met an invalid key
 static constexpr u32 SS_BAD = 1u << 31;
+// and bit 30 on bucket 0's entry of tile 0 when the sample says that one
+// projection holds SS_SKEW_KEYS keys or more, or as many as SS_SKEW_SAME of
+// which all are one key
+static constexpr u32 SS_SKEW = 1u << 30;
+static constexpr u32 SS_SKEW_KEYS = 6144;
+static constexpr u32 SS_SKEW_SAME = 1u << 17;
 // keys a thread: 1 up to 2^18 keys, 2 above
 static int ss_items(u64 n) { return n <= (u64)SS_MAX_TILES * SS_TPB ? 1 : 2; }
 static u32 ss_tiles(u64 n) { return (u32)((n + ss_items(n) * SS_TPB - 1) / (ss_items(n) * SS_TPB)); }
-static_assert(SS_MAX_N <= 2ull * SS_MAX_TILES * SS_TPB && 2 * SS_TPB <= (1 << 15),
-              "the tiles hold a batch, and their offsets and counts stay below the bad-key bit");
+static_assert(SS_MAX_N <= 2ull * SS_MAX_TILES * SS_TPB && 2 * SS_TPB < (1 << 14),
+              "the tiles hold a batch, and their offsets and counts stay below the marks");
 
 // buckets of a batch of n keys, a power of two: of at most 256 keys on average
 // up to 2^18 keys, so that the largest of R-MAT keys (about four times the
@@ -386,14 +401,17 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
     // the sample's projections, sorted; its quantiles are the splitters
     const u32 ns = nb * SS_OVER;
     u32 sm[SS_SITEMS];
+    u64 sx[SS_SITEMS];
 #pragma unroll
     for (int r = 0; r < SS_SITEMS; ++r) {
         const u32 i = tid + r * SS_TPB;
         sm[r] = ~0u;
+        sx[r] = 0;
         if (i < ns) {
             const u64 p = ((2ull * i + 1) * n) / (2ull * ns);
             bool ignore = false;
-            sm[r] = (u32)(pack_element(segs[source_of(segs, nsegs, p)], p, pshift, sbits, ignore) >> psh);
+            sx[r] = pack_element(segs[source_of(segs, nsegs, p)], p, pshift, sbits, ignore);
+            sm[r] = (u32)(sx[r] >> psh);
         }
     }
     if (tid < SS_MAX_BUCKETS) cnt[tid] = 0;
@@ -405,20 +423,53 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
     }
     __syncthreads();
 
-    // bucket = number of splitters <= the key's projection
-    u32 bk[ITEMS], loc[ITEMS];
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-        const u32 x = (u32)(key[r] >> psh);
+    // bucket = number of splitters <= the key's projection, or one less where
+    // that is a repeated splitter
+    auto bucket_of = [&](u32 x) {
         u32 lo = 0, hi = nb - 1;
         while (lo < hi) {
             const u32 mid = (lo + hi) >> 1;
             if (spl[mid] <= x) lo = mid + 1; else hi = mid;
         }
-        bk[r] = lo;
-        loc[r] = valid[r] ? atomicAdd(&cnt[lo], 1u) : 0u;
+        return lo >= 2 && spl[lo - 2] == x ? lo - 1 : lo;
+    };
+    u32 bk[ITEMS], loc[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        bk[r] = bucket_of((u32)(key[r] >> psh));
+        loc[r] = valid[r] ? atomicAdd(&cnt[bk[r]], 1u) : 0u;
     }
     const bool tbad = __syncthreads_or(bad);
+    bool skew = false;
+    if (t == 0) {
+        // splitters `far` apart are 2 * far samples apart
+        static_assert(SS_OVER == 2, "sample keys a splitter");
+        auto holds = [&](u32 keys) {
+            const u32 far = (u32)(((u64)keys * nb + n - 1) / n);
+            return tid + far < nb - 1 && spl[tid] == spl[tid + far];
+        };
+        const bool many = holds(SS_SKEW_KEYS);
+        if (__syncthreads_or(many)) {
+            // the lowest and the highest of the samples' key bits below the projection
+            u32 *least = smp[0], *most = smp[1];
+            if (tid < nb) {
+                least[tid] = ~0u;
+                most[tid] = 0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < SS_SITEMS; ++r)
+                if (tid + r * SS_TPB < ns) {
+                    const u32 b = bucket_of((u32)(sx[r] >> psh));
+                    const u32 low = (u32)((sx[r] & ((1ull << psh) - 1)) >> (1 + sbits));
+                    atomicMin(&least[b], low);
+                    atomicMax(&most[b], low);
+                }
+            __syncthreads();
+            const u32 b = many ? bucket_of(spl[tid]) : 0u;
+            skew = __syncthreads_or(many && (least[b] != most[b] || holds(SS_SKEW_SAME)));
+        }
+    }
     if (tid < 64) {
         // exclusive scan of the bucket counts, four a lane
         constexpr u32 PER = SS_MAX_BUCKETS / 64;
@@ -440,7 +491,9 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
     for (int r = 0; r < ITEMS; ++r)
         if (valid[r]) tmp[tbase + base[bk[r]] + loc[r]] = key[r];
     static_assert(SS_MAX_BUCKETS <= (u32)SS_TPB, "one bucket a thread");
-    if (tid < nb) bc[(u64)tid * ntiles + t] = (base[tid] << 16) | cnt[tid] | (tid == 0 && tbad ? SS_BAD : 0u);
+    if (tid < nb)
+        bc[(u64)tid * ntiles + t] =
+            (base[tid] << 16) | cnt[tid] | (tid == 0 && tbad ? SS_BAD : 0u) | (tid == 0 && skew ? SS_SKEW : 0u);
 }
 
 // Keys of a workgroup are spread over every wave: with R = ceil(m / SB_TPB)
@@ -535,6 +588,7 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
         return;
     }
     if (b >= nb || ntiles == 0) return;
+    const bool skew = bc[0] & SS_SKEW;
     // where the bucket lies in each tile and inside the bucket; its offset in
     // the batch is the sum of its offsets in the tiles (a tile's keys of the
     // buckets before it)
@@ -545,7 +599,7 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
     if (tid < SS_MAX_TILES) {
         e = tid < ntiles ? bc[(u64)b * ntiles + tid] : 0u;
         inc = dpp_incl_scan32(e & 0xFFFFu);
-        const u32 off = wave_sum((e & ~SS_BAD) >> 16);
+        const u32 off = wave_sum((e & ~(SS_BAD | SS_SKEW)) >> 16);
         if (lane_id() == 63) {
             sums[0][tid >> 6] = inc;
             sums[1][tid >> 6] = off;
@@ -553,6 +607,10 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
     }
     __syncthreads();
     if (b == 0 && (e & SS_BAD)) atomicOr(flags, FLAG_INVALID_KEY);
+    if (skew) {
+        if (b == 0 && tid == 0) atomicOr(flags, FLAG_SORT_SKEW);
+        return;
+    }
     u32 m = 0, pre = 0;
     u64 obase = 0;
 #pragma unroll
@@ -563,7 +621,7 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
     }
     if (tid < ntiles) {
         toff[tid] = inc - (e & 0xFFFFu) + pre;
-        tb[tid] = (e & ~SS_BAD) >> 16;
+        tb[tid] = (e & ~(SS_BAD | SS_SKEW)) >> 16;
     }
     if (tid == 0) toff[ntiles] = m;
     if (m == 0) return;
@@ -606,11 +664,16 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
     // memory (from the output range to aux and back); each digit's running
     // offset carries across the chunks, which are taken in order (stable)
     u64 andv = ~0ull, orv = 0;
-    for (u32 j = tid; j < m; j += SB_TPB) {
-        const u64 x = tmp[addr_of(j)];
-        andv &= x;
-        orv |= x;
-        out[obase + j] = x;
+    for (u32 j0 = tid; j0 < m; j0 += SB_CAP) {
+        u64 x[SB_ITEMS];
+#pragma unroll
+        for (int r = 0; r < SB_ITEMS; ++r) x[r] = tmp[addr_of(min(j0 + r * SB_TPB, m - 1))];  // all in flight
+#pragma unroll
+        for (int r = 0; r < SB_ITEMS; ++r) {
+            andv &= x[r];
+            orv |= x[r];
+            if (j0 + r * SB_TPB < m) out[obase + j0 + r * SB_TPB] = x[r];
+        }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -798,11 +861,11 @@ static u64 *os_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u3
 // With n_dev the kernels read the element count from device memory and n
 // is only a capacity that sizes the grids (graph replays).  The first
 // sort_zero_words() words of `scratch` must be zero on entry (the batch's
-// first kernel clears them).
+// first kernel clears them).  skewed: by radix passes whatever the size.
 u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32 pshift, u32 sbits, u32 lo_bit,
-                   u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 *flags, hipStream_t st) {
+                   u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 *flags, bool skewed, hipStream_t st) {
     if (n == 0) return k0;
-    if (n <= SS_MAX_N) {
+    if (n <= SS_MAX_N && !skewed) {
         // sample-split sort: k1 holds the tiles grouped by bucket, k0 the
         // result, k2 the second buffer of oversized buckets; the tiles'
         // bucket counts go to the scratch after its cleared words

@@ -120,7 +120,7 @@ template <bool ONE, int ITEMS, u32 RANGE, bool FOUR>
 __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restrict__ pk, u64 n,
                                                     u64 *__restrict__ ukey, u64 *__restrict__ useg,
                                                     u64 *__restrict__ part, u64 *__restrict__ grp, u32 grp_log,
-                                                    u32 nb) {
+                                                    u32 nb, const Status *__restrict__ status) {
     __shared__ u64 ls[RANGE ? RANGE : 1];
     __shared__ u32 ends[2];
     __shared__ i32 tmp[2][ITEMS][LOC_TPB / 64];
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
     const u64 pmask = (1ull << g.pshift) - 1;
     const u32 ks = 1 + g.sbits;  // key (and pid) above the request order and op
     const u64 i0 = (u64)blockIdx.x * (LOC_TPB * ITEMS);
-    const u32 tid = threadIdx.x, wv = tid >> 6;
+    const u32 tid = threadIdx.x, wv = tid >> 6, flags = status->flags;
     u64 p[ITEMS];
     bool dup[ITEMS];
 #pragma unroll
@@ -183,6 +183,9 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
             seg[r] = locate_segment(d.sep, d.H, key[r]);
         }
     }
+    // nothing is sorted, and k_compact will find no updates (asked here, where
+    // the answer has come without a wait; the segments above lie in range)
+    if (flags & FLAG_SORT_SKEW) return;
     // presence: the items' searches step together (their loads are in
     // flight at once); an item without a key probes its PMA's first segment
     const u64 *base[ITEMS];
@@ -352,6 +355,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_compact(const Group g, const u64 *_
         inc[r] = dpp_incl_scan32(own[r]);
         if (lane_id() == 63) wt[r * NW + wv] = inc[r];
     }
+    if (status->flags & FLAG_SORT_SKEW) return;  // n_eff stays 0 (asked here, behind loads that had to be waited for)
     __syncthreads();
     i32 base_c = 0, base_d = 0, ta = 0, tb = 0;
     for (u32 w = 0; w < NW; ++w) {
@@ -423,17 +427,17 @@ hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchB
     const u32 grid = gl ? (nb + LOC_ITEMS - 1) / LOC_ITEMS : nb;
     if (gl && g.inline_one && n > 16 * nseg_of(g.one))
         k_locate<true, LOC_ITEMS, LOC_RANGE, false>
-            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb, b.status);
     else if (gl && g.inline_one)
         k_locate<true, LOC_ITEMS, LOC_RANGE, true>
-            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb, b.status);
     else if (gl)
         k_locate<false, LOC_ITEMS, LOC_RANGE, true>
-            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+            <<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb, b.status);
     else if (g.inline_one)
-        k_locate<true, 1, 0, false><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+        k_locate<true, 1, 0, false><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb, b.status);
     else
-        k_locate<false, 1, 0, false><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb);
+        k_locate<false, 1, 0, false><<<grid, LOC_TPB, 0, st>>>(g, pk, n, b.ukey, b.useg, part, grp, gl, nb, b.status);
     if (gl)
         k_compact<LOC_ITEMS><<<(nb + LOC_ITEMS - 1) / LOC_ITEMS, LOC_TPB, 0, st>>>(
             g, b.ukey, b.useg, n, part, grp, nb, gl, b.ckey, b.cseg, b.pd, b.wfirst, b.status);
@@ -832,7 +836,7 @@ __global__ __launch_bounds__(1024) void k_leaders(Group g, const u64 *__restrict
                           const u32 *__restrict__ rlevel, const uint4 *__restrict__ rwin, Work *w0, Work *w1,
                           Work *w2, Work *w3, Status *status) {
     // a lone PMA's rebuild leaves no windows
-    const u32 stop = FLAG_INVALID_KEY | FLAG_SORT_STALL |
+    const u32 stop = FLAG_INVALID_KEY | FLAG_SORT_STALL | FLAG_SORT_SKEW |
                      (g.defer_rebuild || g.npma == 1 ? FLAG_ROOT | FLAG_RESIZE : 0u);
     if (status->flags & stop) return;
     const u32 n_eff = status->n_eff;

@@ -363,3 +363,90 @@ def test_neighbor_lists_from_threads():
         x.join()
     assert not bad
     pma.close()
+
+
+# one key repeated: in a bucket of its workgroup's size and past it, and often
+# enough for the batch to leave the sample-split sort
+@pytest.mark.parametrize("n,copies", [(300001, 4000), (300001, 4600), (300001, 5500), (300001, 12000), (7000, 6500),
+                                      (9000, 8990), (131072, 131072), (1 << 19, 1 << 18)])
+@pytest.mark.parametrize("form", ["lone", "sequence", "group", "graph"])
+def test_repeated_key(n, copies, form):
+    rng = np.random.default_rng(n + copies)
+    say(f"repeated key n={n} copies={copies} {form}")
+    V = 1 << 14
+    ps = [L.PMA(V), L.PMA(50)] if form == "group" else [L.PMA(V)]
+    p = ps[0]
+    p.set_graph(form == "graph")
+    group = L.Group(ps) if form == "group" else None
+    ref = oracle.sort_unique(rand_keys(rng, V, 400000))
+    p.bulk_load(ref)
+    key = keys_of([V // 3], [V // 2])[0]
+    for r in range(2):
+        a = rand_keys(rng, V, n)
+        a[rng.choice(n, copies, replace=False)] = key
+        ins, dels = (a, ref[:100]) if r == 0 else (ref[100:200], a[: n - 100])
+        if form == "sequence":
+            parts = [(x, y) for x, y in zip(np.array_split(ins, 7), np.array_split(dels, 7))]
+            p.update_sequence(parts)
+        else:
+            parts = [(ins, dels)]
+            if group:
+                group.update([ins, rand_keys(rng, 50, 20)], [dels, None])
+            else:
+                p.update_mixed(ins, dels)
+        for x, y in parts:
+            ref = oracle.apply(ref, x, y)
+        ek, ro = p.export()
+        assert np.array_equal(L.to_host_u64(ek), ref)
+        assert np.array_equal(ro.cpu().numpy().view(np.uint32), oracle.row_offsets(ref, V))
+        assert p.check() == 0
+    if group:
+        group.close()
+    for q in ps:
+        q.close()
+
+
+def test_hub_of_a_wide_graph():
+    """A hub's edges in a graph of so many vertices that thousands of them share
+    a projection in the sort."""
+    rng = np.random.default_rng(8)
+    V, n = (1 << 26) + 3, 300000
+    say(f"hub V={V} n={n}")
+    p = L.PMA(V)
+    a = keys_of(np.full(n, V - 2), V - 1 - rng.integers(0, 1 << 22, n))
+    p.insert(a)
+    ref = oracle.sort_unique(a)
+    p.delete(a[::3])
+    ref = oracle.apply(ref, (), a[::3])
+    assert np.array_equal(L.to_host_u64(p.export()[0]), ref)
+    assert p.check() == 0
+    p.close()
+
+
+def test_repeated_key_costs_no_more_than_the_radix_sort():
+    """A batch of 4*10^5 keys, half of them one key, against one without
+    repeats: sorted by one workgroup it took ten times as long."""
+    import time
+    import torch
+    say("repeated key, time")
+    rng = np.random.default_rng(9)
+    V, n = 1 << 20, 400000
+    p = L.PMA(V)
+    p.bulk_load(rand_keys(rng, V, 2000000))
+    spread = rand_keys(rng, V, n)
+    repeated = np.where(rng.random(n) < 0.5, spread, keys_of([7], [9])[0])
+    took = []
+    for keys in (spread, repeated):
+        keys = L.to_device(keys, p.device)
+        times = []
+        for _ in range(9):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            p.insert(keys)
+            p.delete(keys)
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - t)
+        took.append(sorted(times)[4])
+    say(f"{took[0] * 1e6:.0f} us, half repeated {took[1] * 1e6:.0f} us")
+    assert took[1] < 3 * took[0]
+    p.close()
