@@ -301,6 +301,12 @@ uint64_t lpma_pool_reserved_bytes(void);
  * this call replaced (0: the earlier injection fired, or none was set). */
 int lpma_inject_alloc_failure(uint64_t nth, uint64_t *remaining);
 
+/* Fault injection for failure-path tests: in the next `sorts` radix sorts of
+ * batches no tile waits for the counts of the ones before it, as when they do
+ * not come in time.  Such a batch is run again, and one that meets it twice
+ * fails with LPMA_ERR_DEVICE and changes nothing.  Process-wide. */
+int lpma_inject_sort_stalls(uint64_t sorts);
+
 const char *lpma_strerror(int code);
 
 /* ---------------------------------------------------------------------------

@@ -149,6 +149,7 @@ SIGNATURES = [
     ("lpma_pool_trim", _int, []),
     ("lpma_pool_reserved_bytes", _u64, []),
     ("lpma_inject_alloc_failure", _int, [_u64, ctypes.POINTER(_u64)]),
+    ("lpma_inject_sort_stalls", _int, [_u64]),
     ("lpma_strerror", ctypes.c_char_p, [_int]),
     ("lpma_server_config_default", None, [ctypes.POINTER(ServerConfig)]),
     ("lpma_server_create", _int, [ctypes.POINTER(_vp), _vp, ctypes.POINTER(ServerConfig)]),

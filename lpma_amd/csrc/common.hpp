@@ -45,8 +45,9 @@ static constexpr u64 RK_SKIP = 1ull << 62;  // located, but without effect (set 
 static constexpr u32 FLAG_INVALID_KEY = 1u;   // src or dst >= V
 static constexpr u32 FLAG_ROOT = 2u;          // a run chose the root window
 static constexpr u32 FLAG_RESIZE = 4u;        // the root window does not fit
-static constexpr u32 FLAG_SORT_STALL = 8u;    // a sort tile waited too long (the batch fails)
+static constexpr u32 FLAG_SORT_STALL = 8u;    // not sorted: a tile waited too long (the host runs the batch again)
 static constexpr u32 FLAG_SORT_SKEW = 16u;    // not sorted: too skewed for buckets (the host runs the batch again)
+static constexpr u32 FLAG_UNSORTED = FLAG_SORT_STALL | FLAG_SORT_SKEW;
 
 // most passes of the batch sort (8-bit digits over 64 bits)
 static constexpr u32 SORT_MAX_PASSES = 8;

@@ -9,11 +9,17 @@ u64 scan_scratch_words(u64 n);
 hipError_t device_excl_scan(const u32 *in, u64 n, u32 *out, u32 *scratch, hipStream_t st);
 u64 sort_scratch_words(u64 n);
 u32 sort_zero_words();
+// how a batch is sorted: as its size asks, by radix passes (after
+// FLAG_SORT_SKEW), or by radix passes whose tiles cannot wait for one that has
+// not started (after FLAG_SORT_STALL)
+enum class SortBy { SIZE, RADIX, ORDERED_TILES };
 // k0, k1, k2: n keys each (k2 only for batches of up to 2^19 keys, as the
-// second buffer of an oversized bucket).  Such a batch may come back unsorted,
-// with FLAG_SORT_SKEW in flags, unless `skewed` says that it has
+// second buffer of an oversized bucket).  A batch that comes back unsorted has
+// FLAG_SORT_SKEW or FLAG_SORT_STALL in flags
 u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32 pshift, u32 sbits, u32 lo_bit,
-                   u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 *flags, bool skewed, hipStream_t st);
+                   u32 hi_bit, u64 *k0, u64 *k1, u64 *k2, u32 *scratch, u32 *flags, SortBy by, hipStream_t st);
+// the next `sorts` radix sorts give up waiting at once (tests)
+void inject_sort_stalls(u64 sorts);
 
 // update.hip
 struct BatchBufs {

@@ -975,13 +975,24 @@ int finish_round(Pipeline &pl, const Member *mem, u32 npma, const Group &g_in, u
 
 int run_pipeline_graph(Pipeline &pl, const Member *mem, u32 npma, u64 n, u32 pshift, u32 hi_bit, hipStream_t st);
 
+// Whether the batch whose outcome is on the host came back unsorted and shall
+// run again, `by` then saying how.
+bool sort_again(const Pipeline &pl, SortBy &by) {
+    const u32 flags = ((const Status *)pl.h_out)->flags;
+    if (flags & FLAG_INVALID_KEY) return false;
+    if ((flags & FLAG_SORT_STALL) && by != SortBy::ORDERED_TILES) by = SortBy::ORDERED_TILES;
+    else if ((flags & FLAG_SORT_SKEW) && by == SortBy::SIZE) by = SortBy::RADIX;
+    else return false;
+    return true;
+}
+
 // One update round over the members (all on pl's device, same segment size,
 // ids fitting above the sort keys): sort + dedup + locate + density check +
 // election over every member at once, one host synchronisation, then the
 // rebalance classes, the pyramid, and root rebuilds / resizes per member.  A
-// batch that turns out too skewed for the sort's buckets (FLAG_SORT_SKEW) has
-// changed nothing and runs again, `skewed`.
-int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool skewed = false) {
+// batch that came back unsorted has changed nothing and runs again (sort_again).
+int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, SortBy by = SortBy::SIZE) {
+    const bool first = by == SortBy::SIZE;
     pl.cur_stream = st;
     u64 n = 0, nseg_total = 0;
     bool mixed = false;
@@ -989,7 +1000,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool
     for (u32 p = 0; p < npma; ++p) {
         lpma *h = mem[p].h;
         h->cur_stream = st;
-        if (!skewed) h->calls++;
+        if (first) h->calls++;
         bool any_ins = false, any_del = false;
         for (u32 r = 0; r < mem[p].nreq; ++r) {
             const Req &q = mem[p].reqs[r];
@@ -1003,7 +1014,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool
         vmax = std::max(vmax, h->vbits);
         nseg_total += 1ull << h->st.H;
     }
-    if (!skewed) pl.rounds++;
+    if (first) pl.rounds++;
     if (n == 0) {
         for (u32 p = 0; p < npma; ++p) mem[p].h->version++;
         return LPMA_OK;
@@ -1013,7 +1024,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool
     const u32 pshift = 2 * vmax + 1 + sbits;
     const u32 hi_bit = pshift + bits_for(npma);
     if (hi_bit > 64) return LPMA_ERR_TOO_LARGE;
-    if (pl.graph_on && maxreq <= 1 && !skewed) return run_pipeline_graph(pl, mem, npma, n, pshift, hi_bit, st);
+    if (pl.graph_on && maxreq <= 1 && first) return run_pipeline_graph(pl, mem, npma, n, pshift, hi_bit, st);
     CHECKED(ensure_batch(pl, n, npma, nsegs, std::min<u64>(n, nseg_total)));
     // A lone PMA's single-segment and wave windows are queued before the
     // host reads the status (below): the large windows that may follow
@@ -1034,7 +1045,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool
     CHECKED(upload_table(pl, mem, npma, pyr_blocks, st));
 
     // the sort carries the batch's first work and takes the sources as arguments
-    const bool carried = npma == 1 && !skewed && sort_carries_first(n, nsegs);
+    const bool carried = npma == 1 && first && sort_carries_first(n, nsegs);
     // batch sources: each request's deletes (op 0), then its inserts (op 1)
     {
         u64 off = 0;
@@ -1109,7 +1120,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool
                 HIPCHECK(batch_begin(g, bb, pl.h_segs, nsegs <= ARG_SEGS ? nsegs : 0, pl.segs.p, pl.sort_scr.p,
                                      sort_zero_words(), st));
                 pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
-                                   pl.ukey.p, pl.sort_scr.p, &bb.status->flags, skewed, st);
+                                   pl.ukey.p, pl.sort_scr.p, &bb.status->flags, by, st);
             }
             HIPCHECK(hipGetLastError());
         }
@@ -1150,7 +1161,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, bool
         u64 w;
         CHECKED(wait_word(&pl.h_early->seq, st, w, [epoch](u64 x) { return x == epoch; }));
     }
-    if (((const Status *)pl.h_out)->flags & FLAG_SORT_SKEW) return run_pipeline(pl, mem, npma, st, true);
+    if (sort_again(pl, by)) return run_pipeline(pl, mem, npma, st, by);
     return finish_round(pl, mem, npma, g, pyr_blocks, false, st, early);
 }
 
@@ -1247,7 +1258,7 @@ int graph_for(Pipeline &pl, u64 cap, u32 npma, u32 pshift, u32 hi_bit, u32 log2S
                   batch_begin(g, bb, nullptr, 0, pl.segs.p, pl.sort_scr.p, sort_zero_words(), cs) == hipSuccess;
         if (ok) {
             u64 *pk = pack_and_sort(pl.segs.p, nsegs, cap, &pl.rhdr.p->n, pshift, 0, 0, hi_bit, pl.pk0.p, pl.pk1.p,
-                                    pl.ukey.p, pl.sort_scr.p, &bb.status->flags, false, cs);
+                                    pl.ukey.p, pl.sort_scr.p, &bb.status->flags, SortBy::SIZE, cs);
             ok = hipGetLastError() == hipSuccess && locate_and_compact(g, pk, cap, bb, cs) == hipSuccess &&
                  density_check(g, cap, bb, cs) == hipSuccess && elect_windows(g, cap, bb, cs) == hipSuccess &&
                  rebalance_fixed(g, bb, (u32)cap, nullptr, cs) == hipSuccess &&
@@ -1318,7 +1329,8 @@ int run_pipeline_graph(Pipeline &pl, const Member *mem, u32 npma, u64 n, u32 psh
     }
     pl.graph_launches++;
     HIPCHECK(hipStreamSynchronize(st));
-    if (((const Status *)pl.h_out)->flags & FLAG_SORT_SKEW) return run_pipeline(pl, mem, npma, st, true);
+    SortBy by = SortBy::SIZE;
+    if (sort_again(pl, by)) return run_pipeline(pl, mem, npma, st, by);
     Group g = graph_group(pl, npma, pshift, log2S);
     g.epoch = epoch;  // a repeated election runs eagerly, outside the graph
     g.rh = nullptr;
@@ -2288,6 +2300,11 @@ int lpma_inject_alloc_failure(uint64_t nth, uint64_t *remaining) {
     long long prev =
         g_fail_countdown.exchange(nth > (uint64_t)LLONG_MAX ? LLONG_MAX : (long long)nth, std::memory_order_relaxed);
     if (remaining) *remaining = prev > 0 ? (uint64_t)prev : 0;  // -1: it fired
+    return LPMA_OK;
+}
+
+int lpma_inject_sort_stalls(uint64_t sorts) {
+    inject_sort_stalls(sorts);
     return LPMA_OK;
 }
 

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_locate(Group g, const u64 *__restri
     }
     // nothing is sorted, and k_compact will find no updates (asked here, where
     // the answer has come without a wait; the segments above lie in range)
-    if (flags & FLAG_SORT_SKEW) return;
+    if (flags & FLAG_UNSORTED) return;
     // presence: the items' searches step together (their loads are in
     // flight at once); an item without a key probes its PMA's first segment
     const u64 *base[ITEMS];
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(LOC_TPB) void k_compact(const Group g, const u64 *_
         inc[r] = dpp_incl_scan32(own[r]);
         if (lane_id() == 63) wt[r * NW + wv] = inc[r];
     }
-    if (status->flags & FLAG_SORT_SKEW) return;  // n_eff stays 0 (asked here, behind loads that had to be waited for)
+    if (status->flags & FLAG_UNSORTED) return;  // n_eff stays 0 (asked here, behind loads that had to be waited for)
     __syncthreads();
     i32 base_c = 0, base_d = 0, ta = 0, tb = 0;
     for (u32 w = 0; w < NW; ++w) {
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(1024) void k_leaders(Group g, const u64 *__restrict
                           const u32 *__restrict__ rlevel, const uint4 *__restrict__ rwin, Work *w0, Work *w1,
                           Work *w2, Work *w3, Status *status) {
     // a lone PMA's rebuild leaves no windows
-    const u32 stop = FLAG_INVALID_KEY | FLAG_SORT_STALL | FLAG_SORT_SKEW |
+    const u32 stop = FLAG_INVALID_KEY | FLAG_UNSORTED |
                      (g.defer_rebuild || g.npma == 1 ? FLAG_ROOT | FLAG_RESIZE : 0u);
     if (status->flags & stop) return;
     const u32 n_eff = status->n_eff;

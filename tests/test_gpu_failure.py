@@ -222,3 +222,30 @@ def test_rebuild_without_merge_scratch():
     case.verify()
     assert case.pmas[0].view().capacity == old.capacity // 2
     case.close()
+
+
+@pytest.mark.parametrize("form", ["lone", "group"])
+@pytest.mark.parametrize("n", [600000, (1 << 22) + 1])
+def test_sort_stall(n, form):
+    """A sort whose tiles give up waiting for the ones before them: the batch
+    runs again and equals the oracle; twice, it fails and changes nothing."""
+    say(f"sort stall n={n} {form}")
+    rng = np.random.default_rng(n)
+    V = 1 << 16
+    bulk = L.shuffle(L.gen_uniform(V, 300000, 9), 9)
+    small = (50, rand_keys(rng, 50, 100), rand_keys(rng, 50, 9), rand_keys(rng, 50, 9))
+    case = Case([(V, bulk, rand_keys(rng, V, n - 1000), bulk[:1000].copy())] + [small] * (form == "group"),
+                group=form == "group")
+    before = case.snaps()
+    try:
+        assert L.lib().lpma_inject_sort_stalls(2) == 0
+        with pytest.raises(L.LpmaError) as e:
+            case.apply()
+        assert e.value.code == 4  # LPMA_ERR_DEVICE
+        assert all(same(a, b) for a, b in zip(before, case.snaps()))
+        assert L.lib().lpma_inject_sort_stalls(1) == 0
+        case.apply()
+    finally:
+        L.lib().lpma_inject_sort_stalls(0)
+    case.verify()
+    case.close()
