@@ -171,7 +171,7 @@ struct Pipeline {
     u32 h_tab_n = 0;
     std::vector<PmaEntry> tab_shadow;  // what the device table holds
     const PmaEntry *tab_shadow_at = nullptr;
-    BatchSeg *h_segs = nullptr;
+    BatchSeg *h_segs = nullptr;  // pinned: more sources than kernel arguments take, or a graph's
     u32 h_segs_n = 0;
     unsigned char *h_out = nullptr;
     u64 h_out_bytes = 0;
@@ -636,9 +636,10 @@ int ensure_batch(Pipeline &pl, u64 n, u32 npma, u32 nsegs, u64 runs) {
         return r;
     for (int c = 0; c < NUM_CLASSES; ++c)
         if ((r = ensure(pl, pl.work[c], runs))) return r;
-    if ((r = ensure_host(pl.h_tab, pl.h_tab_n, npma, pl.cur_stream)) ||
-        (r = ensure_host(pl.h_segs, pl.h_segs_n, nsegs, pl.cur_stream)))
-        return r;
+    if ((r = ensure_host(pl.h_tab, pl.h_tab_n, npma, pl.cur_stream))) return r;
+    // (up to ARG_SEGS sources travel as kernel arguments: growing pinned memory
+    // for them took 380 us of a handle's first merged run)
+    if ((nsegs > ARG_SEGS || pl.graph_on) && (r = ensure_host(pl.h_segs, pl.h_segs_n, nsegs, pl.cur_stream))) return r;
     if (!pl.h_out || pl.h_out_bytes < out_words * 8) {
         if (injected_failure()) return LPMA_ERR_OUT_OF_MEMORY;
         if (pl.h_early) {
@@ -1047,6 +1048,8 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, Sort
     // the sort carries the batch's first work and takes the sources as arguments
     const bool carried = npma == 1 && first && sort_carries_first(n, nsegs);
     // batch sources: each request's deletes (op 0), then its inserts (op 1)
+    BatchSeg arg_segs[ARG_SEGS];
+    BatchSeg *const hsegs = nsegs <= ARG_SEGS ? arg_segs : pl.h_segs;
     {
         u64 off = 0;
         u32 k = 0;
@@ -1058,7 +1061,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, Sort
                     const u64 *keys = op ? q.ins : q.del;
                     u64 cnt = op ? q.nins : q.ndel;
                     if (!cnt) continue;
-                    BatchSeg &b = pl.h_segs[k++];
+                    BatchSeg &b = hsegs[k++];
                     memset(&b, 0, sizeof(b));
                     b.keys = keys;
                     b.n = cnt;
@@ -1073,7 +1076,7 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, Sort
             }
         }
         if (nsegs > ARG_SEGS) {
-            HIPCHECK(hipMemcpyAsync(pl.segs.p, pl.h_segs, nsegs * sizeof(BatchSeg), hipMemcpyHostToDevice, st));
+            HIPCHECK(hipMemcpyAsync(pl.segs.p, hsegs, nsegs * sizeof(BatchSeg), hipMemcpyHostToDevice, st));
         }
     }
 
@@ -1100,7 +1103,8 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, Sort
         PhaseTimer t(pl, st, PH_SORT);
         lpma *h0 = mem[0].h;
         const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
-        HIPCHECK(small_batch(g, bb, seg_args<INLINE_SEGS>(pl.h_segs, nsegs), n, chunks, (u32 *)(pl.d_stats + ST_ROWS * ST_NUM), pl.h_early, st));
+        HIPCHECK(small_batch(g, bb, seg_args<INLINE_SEGS>(hsegs, nsegs), n, chunks,
+                             (u32 *)(pl.d_stats + ST_ROWS * ST_NUM), pl.h_early, st));
         h0->pyr_owed = false;
     } else {
         // bit 0 of a packed key is the operation (with the request order above
@@ -1112,12 +1116,12 @@ int run_pipeline(Pipeline &pl, const Member *mem, u32 npma, hipStream_t st, Sort
             if (carried) {
                 lpma *h0 = mem[0].h;
                 const u32 chunks = h0->pyr_owed ? pyramid_blocks(h0->st.H) : 0u;
-                pk = pack_and_sort_first(g, bb.status, bb.wfirst, pl.h_segs, nsegs, n, pshift, sbits, hi_bit, pl.pk0.p,
+                pk = pack_and_sort_first(g, bb.status, bb.wfirst, hsegs, nsegs, n, pshift, sbits, hi_bit, pl.pk0.p,
                                          pl.pk1.p, pl.ukey.p, pl.sort_scr.p, chunks, st);
                 h0->pyr_owed = false;
             } else {
                 HIPCHECK(pay_owed_pyramids(mem, npma, st));
-                HIPCHECK(batch_begin(g, bb, pl.h_segs, nsegs <= ARG_SEGS ? nsegs : 0, pl.segs.p, pl.sort_scr.p,
+                HIPCHECK(batch_begin(g, bb, hsegs, nsegs <= ARG_SEGS ? nsegs : 0, pl.segs.p, pl.sort_scr.p,
                                      sort_zero_words(), st));
                 pk = pack_and_sort(pl.segs.p, nsegs, n, nullptr, pshift, sbits, lo_bit, hi_bit, pl.pk0.p, pl.pk1.p,
                                    pl.ukey.p, pl.sort_scr.p, &bb.status->flags, by, st);

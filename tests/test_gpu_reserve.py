@@ -59,6 +59,31 @@ def test_reserved_growth_allocates_nothing(seed):
     p.close()
 
 
+def test_first_merged_run_allocates_nothing():
+    """After reserve, 32 merged requests with as many keys as it names: their 64
+    sources travel as kernel arguments and take no pinned memory."""
+    say("first merged run")
+    rng = np.random.default_rng(4)
+    V = 1 << 14
+    keys = L.shuffle(L.gen_uniform(V, 300000, 3), 3)
+    p = L.PMA(V)
+    p.bulk_load(keys)
+    p.reserve_capacity(310000)
+    p.reserve(1 << 17)
+    torch.cuda.synchronize()
+    ref = oracle.apply(np.empty(0, dtype=np.uint64), keys)
+    batches = [(L.gen_uniform(V, 200, 100 + r), rng.choice(keys, 150, replace=False)) for r in range(32)]
+    try:
+        L.inject_alloc_failure(1)  # any allocation from here on would fail
+        p.update_sequence(batches)
+    finally:
+        assert L.inject_alloc_failure(0) == 1, "the merged run allocated"
+    for a, d in batches:
+        ref = oracle.apply(ref, a, d)
+    check(p, ref, V)
+    p.close()
+
+
 def check(p, ref, V):
     ek, ro = p.export()
     assert np.array_equal(L.to_host_u64(ek), ref)
