@@ -381,3 +381,35 @@ def test_pagerank_small_ranks(degree):
         assert np.array_equal(got > 0, there)
         assert np.max(np.abs(got[there] - want[there]) / want[there]) < (4 * it + 2) * 2.0 ** -24
     pma.close()
+
+
+# a bitmap of less than a window, of one and a few vertices, and past the last one
+@pytest.mark.parametrize("V,listed", [(4100, True), (5000, True), ((1 << 20) + 1, True), ((1 << 22) + 1, False)])
+def test_bfs_levels_that_take_lists(V, listed):
+    """Graphs of 2^24 slots and up to 2^22 vertices have lists (a word a slot of
+    the pool), which a level of 2^22 places goes through."""
+    from gpu_util import keys_of
+    say(f"bfs levels through lists V={V}")
+    rng = np.random.default_rng(V)
+    E = 9500000
+    keys = oracle.sort_unique(keys_of(rng.integers(0, V, E), rng.integers(0, V, E)))
+    while keys.size < 9000000:
+        keys = oracle.sort_unique(np.append(keys, keys_of(rng.integers(0, V, E), rng.integers(0, V, E))))[:E]
+    keys = np.sort(rng.permutation(keys)[:9000000])
+    pma = L.PMA(V)
+    pma.bulk_load(keys)
+    slots = int(pma.view().capacity)
+    assert slots >= 1 << 24
+    row_off = pma.copy_view()[1].cpu().numpy().view(np.uint32).astype(np.int64)
+    places = np.diff(row_off)
+    want = oracle.bfs(keys, V, 0)
+    widest = max(int(places[want == k].sum()) for k in range(int(want[want != 0xFFFFFFFF].max()) + 1))
+    assert widest >= 1 << 22 or not listed
+    L.lib().lpma_pool_trim()
+    held = L.pool_reserved_bytes()
+    lv, depth, scanned = pma.bfs(0)
+    assert (L.pool_reserved_bytes() - held >= 4 * slots) == listed
+    assert np.array_equal(lv.cpu().numpy().view(np.uint32), want)
+    deg = np.diff(oracle.csr_of(keys, V)[0].astype(np.int64))
+    assert depth == int(want[want != 0xFFFFFFFF].max()) + 1 and scanned == int(deg[want != 0xFFFFFFFF].sum())
+    pma.close()
