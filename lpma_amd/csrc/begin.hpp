@@ -219,7 +219,12 @@ __device__ __forceinline__ void row_lines(const u64 *a, u64 at, u32 w, u64 (&v)[
 template <int J0, bool LE>
 __device__ __forceinline__ void row_counts(const u64 (&v)[8], u64 key, u32 &mine) {
     const u32 gl = lane_id() & 15, sh = lane_id() & 48;
-#define LPMA_COUNT(K)                                                                                    {                                                                                                        const u64 k = row_lane<J0 + K>(key);                                                                 const u32 c = (u32)__popc((u32)(__ballot(LE ? v[K] <= k : v[K] == k) >> sh) & 0xFFFFu);             if (gl == J0 + K) mine = c;                                                                      }
+#define LPMA_COUNT(K)                                                                                       \
+    {                                                                                                       \
+        const u64 k = row_lane<J0 + K>(key);                                                                \
+        const u32 c = (u32)__popc((u32)(__ballot(LE ? v[K] <= k : v[K] == k) >> sh) & 0xFFFFu);             \
+        if (gl == J0 + K) mine = c;                                                                         \
+    }
     LPMA_COUNT(0) LPMA_COUNT(1) LPMA_COUNT(2) LPMA_COUNT(3) LPMA_COUNT(4) LPMA_COUNT(5) LPMA_COUNT(6) LPMA_COUNT(7)
 #undef LPMA_COUNT
 }

@@ -318,17 +318,10 @@ __device__ __forceinline__ u32 dpp_incl_scan32(u32 v) {
     return v;
 }
 
-// AND / OR of a 64-bit value over the wave, the same in every lane (the
-// DPP scan pattern with the operation's identity for lanes out of a row;
+// OR of a value over the wave, the same in every lane (the DPP scan pattern;
 // lane 63 ends with the whole wave's result)
-template <bool AND>
-__device__ __forceinline__ u32 dpp_reduce32(u32 v) {
-    const int id = AND ? -1 : 0;
-#define LPMA_DPP_STEP(ctrl, rows)                                                           \
-    {                                                                                       \
-        const u32 t = (u32)__builtin_amdgcn_update_dpp(id, (int)v, ctrl, rows, 0xF, false); \
-        v = AND ? (v & t) : (v | t);                                                        \
-    }
+__device__ __forceinline__ u32 dpp_or32(u32 v) {
+#define LPMA_DPP_STEP(ctrl, rows) v |= (u32)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false);
     LPMA_DPP_STEP(0x111, 0xF)
     LPMA_DPP_STEP(0x112, 0xF)
     LPMA_DPP_STEP(0x114, 0xF)
@@ -337,13 +330,6 @@ __device__ __forceinline__ u32 dpp_reduce32(u32 v) {
     LPMA_DPP_STEP(0x143, 0xC)
 #undef LPMA_DPP_STEP
     return (u32)__builtin_amdgcn_readlane((int)v, 63);
-}
-
-__device__ __forceinline__ u64 wave_and64(u64 v) {
-    return ((u64)dpp_reduce32<true>((u32)(v >> 32)) << 32) | dpp_reduce32<true>((u32)v);
-}
-__device__ __forceinline__ u64 wave_or64(u64 v) {
-    return ((u64)dpp_reduce32<false>((u32)(v >> 32)) << 32) | dpp_reduce32<false>((u32)v);
 }
 
 template <typename T>

@@ -156,7 +156,7 @@ hipError_t bfs_init(u32 *levels, u32 V, u32 src, u32 *queue, u32 *ctl, u32 *visi
 u64 bfs_run_words(u64 slots);
 // a search's large levels through lists (list null: none)
 static constexpr u32 BFS_WIN_LOG = 20;  // vertices of a window of the bitmap: 128 KB of LDS
-static constexpr u32 BFS_WINDOWS = 4;
+static constexpr u32 BFS_WINDOWS = 4;   // what a wave of the expansion has LDS for; larger graphs go without lists
 static constexpr u64 BFS_LIST_SLOTS = 1ull << 24;
 struct BfsLists {
     u32 *list;   // destinations, in extents
@@ -170,8 +170,9 @@ u32 bfs_list_waves();  // of the default expansion
 u64 bfs_list_extents(u64 slots, u32 waves);
 u64 bfs_list_words(u64 extents);
 u64 bfs_part_words();
-// host: pinned; [0] level + 1 and the size of its frontier (low half), stored
-// last; [1] live edges scanned and [2] levels with a frontier before it
+// host: pinned; [0] level + 1 and the size of its frontier (low half; 1 for any
+// after a level through lists), stored last; [1] live edges scanned and [2]
+// levels with a frontier before it
 hipError_t bfs_level(const DevState &d, const u32 *q, u32 *off, u32 *adj, u32 *runs, u32 *levels, u32 *visited,
                      u32 level, u32 *qnext, u32 *ctl, const BfsLists &ls, u64 *host, u32 expand_grid, hipStream_t st);
 hipError_t pr_outdeg(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *outdeg, hipStream_t st);

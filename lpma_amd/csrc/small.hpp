@@ -116,7 +116,7 @@ __device__ __forceinline__ void small_settle(const Group &g, const BatchBufs &bb
                       (unsigned long long)(tag | (u64)(~j)));
         }
     }
-    const u32 f = dpp_reduce32<false>(myflags), mk = dpp_reduce32<false>(mymask);
+    const u32 f = dpp_or32(myflags), mk = dpp_or32(mymask);
     if (lane_id() == 0) {
         if (f) atomicOr(&S.flags, f);
         if (mk) atomicOr(&S.mask, mk);

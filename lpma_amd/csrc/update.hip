@@ -411,15 +411,12 @@ hipError_t locate_and_compact(const Group &g, const u64 *pk, u64 n, const BatchB
     u32 nb = locate_blocks(n);
     const u32 gl = locate_group_log(nb);
     u64 *grp = gl ? b.part : nullptr, *part = b.part + LOC_GROUPS;
-    // Large batches take LOC_ITEMS keys a thread (more probes in flight, a
-    // narrower range for each key).  Small ones over many segments (a lone
-    // PMA's, where the height is known here) skip the range: 1000 keys over
-    // 2^19 segments would stage 2^17 separators a tile.
-    // Large batches: LOC_ITEMS keys a thread, searching their tile's staged
-    // range (8.4 M keys into 2^15 segments: 142 -> 73 us; 2 M into 2^19: 54
-    // -> 52-59, the probes' lines bound it).  Below, one key a thread over
-    // all separators: more waves hide the latency (160 K keys over 2^21
-    // segments: 31 us against 35 us, 10^5 over 2^19: 9.2 against 18).
+    // Large batches: LOC_ITEMS keys a thread (more probes in flight), searching
+    // their tile's staged range (8.4 M keys into 2^15 segments: 142 -> 73 us; 2 M
+    // into 2^19: 54 -> 52-59, the probes' lines bound it).  Below, one key a
+    // thread over all separators: more waves hide the latency (160 K keys over
+    // 2^21 segments: 31 us against 35 us, 10^5 over 2^19: 9.2 against 18), and a
+    // tile's range would be wide (1000 keys over 2^19: 2^17 separators).
     // The presence probes of large batches go four ways at a step where the keys
     // spread over the segments (2*10^6 keys into 2^19: 58 -> 47 us), two ways
     // where many share a segment, whose lines are at hand (8.4*10^6 into 2^15:
@@ -781,7 +778,7 @@ __global__ __launch_bounds__(256) void k_density(Group g, const u64 *__restrict_
     // PMA the flags and the claimed levels: lanes of the first PMA in the
     // wave combine theirs, the others (rare) go alone (the levels into the
     // workgroup's replica of the PMA's mask)
-    const u32 f = dpp_reduce32<false>(local_flags);
+    const u32 f = dpp_or32(local_flags);
     if (lone) {
         __shared__ u32 s_flags;
         if (threadIdx.x == 0) s_flags = 0;
@@ -798,8 +795,8 @@ __global__ __launch_bounds__(256) void k_density(Group g, const u64 *__restrict_
     }
     const u32 pid0 = __shfl(pid, 0, 64);
     const u32 rep = blockIdx.x & (LV_REPL - 1);
-    const u32 lv = dpp_reduce32<false>(pid == pid0 ? lvbit : 0u);
-    const u32 pf = dpp_reduce32<false>(pid == pid0 ? local_flags : 0u);
+    const u32 lv = dpp_or32(pid == pid0 ? lvbit : 0u);
+    const u32 pf = dpp_or32(pid == pid0 ? local_flags : 0u);
     if (lane_id() == 0 && pid0 != 0xFFFFFFFFu) {
         if (lv) atomicOr(&g.lvmask[(u64)pid0 * LV_REPL + rep], lv);
         if (pf) atomicOr(&g.pstat[pid0].flags, pf);
@@ -2135,7 +2132,9 @@ static constexpr u32 RM_TILE = 2048;  // merged items of a tile
 static constexpr u32 RM_PER = RM_TILE / LGP_TPB;
 
 // live keys among the first D items of the merge of A and U (equal keys: the
-// live key first), by one whole wave
+// live key first), by one whole wave: a search along the merge's D-th diagonal
+// (Odeh, Green, Mwassi, Shmueli, Birk, "Merge path - parallel merging made
+// simple", IPDPSW 2012)
 __device__ __forceinline__ u32 merge_split(const u64 *__restrict__ A, u32 na, const u64 *__restrict__ U, u32 nu,
                                            u64 D) {
     const u32 lane = lane_id();

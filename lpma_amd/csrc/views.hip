@@ -138,7 +138,7 @@ hipError_t export_compacted(const DevState &d, u32 *sums, u64 *edge_keys, u32 *r
 // call on a device shares that device's copy: calls that overlap on one device
 // race.  Nothing in it needs clearing: every word is written before it is read.
 
-static constexpr u64 EXPORT_STATIC_MAX_SEGS = 1ull << 21;
+static constexpr u64 EXPORT_STATIC_MAX_SEGS = 1ull << 21;  // what callers are promised (the scratch would serve any)
 static __device__ __align__(256) u32 scratch[EX_TILES];
 
 static constexpr int EXPORT_STATIC_MAX_DEVICES = 64;
