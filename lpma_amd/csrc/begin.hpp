@@ -23,20 +23,23 @@ __device__ __forceinline__ void put(T *p, T v) {
 }
 
 // Levels 1..PYR_CHL of one chunk of 2^PYR_CHL segments (all levels of a
-// smaller PMA), by one workgroup, through LDS (v0: PYR_CH words, v1: half).
+// smaller PMA), by nt threads of a workgroup (this one tid of them), through
+// LDS (v0: PYR_CH words, v1: half).  Every thread of the workgroup calls it; one
+// without a chunk (a place past the last) only meets the others' barriers.
 template <bool COH = false>
-__device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1) {
+__device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1, u32 tid, u32 nt) {
     const u64 nseg = nseg_of(d);
     const u32 levels = d.H < PYR_CHL ? d.H : PYR_CHL;
-    const u32 n = (u32)(nseg < PYR_CH ? nseg : PYR_CH);
-    const u64 c0 = chunk * n;
-    for (u32 i = threadIdx.x; i < n; i += blockDim.x) v0[i] = d.cnt[c0 + i];
+    const u32 size = (u32)(nseg < PYR_CH ? nseg : PYR_CH);
+    const u64 c0 = chunk * size;
+    const u32 n = c0 < nseg ? size : 0;
+    for (u32 i = tid; i < n; i += nt) v0[i] = d.cnt[c0 + i];
     __syncthreads();
     u32 *in = v0, *tmp = v1;
     for (u32 l = 1; l <= levels; ++l) {
         u32 nw = n >> l;
         u32 *out = d.pyr + pyr_off(nseg, l) + (c0 >> l);
-        for (u32 x = threadIdx.x; x < nw; x += blockDim.x) {
+        for (u32 x = tid; x < nw; x += nt) {
             u32 s = in[2 * x] + in[2 * x + 1];
             tmp[x] = s;
             put<COH>(&out[x], s);
@@ -44,6 +47,11 @@ __device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1)
         __syncthreads();
         u32 *sw = in; in = tmp; tmp = sw;
     }
+}
+
+template <bool COH = false>
+__device__ inline void pyr_chunk(const DevState &d, u64 chunk, u32 *v0, u32 *v1) {
+    pyr_chunk<COH>(d, chunk, v0, v1, threadIdx.x, blockDim.x);
 }
 
 // Levels above the chunk levels, by one workgroup.  Up to PYR_TOP_LDS

@@ -312,6 +312,7 @@ __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, 
 // against 14 + 5 * 15 in the one-kernel passes below.
 
 static constexpr int SS_TPB = 1024;
+static constexpr u32 SS_PYR = 4;          // pyramid chunks a workgroup sums side by side
 static constexpr u32 SS_MAX_TILES = 256;  // a tile a compute unit: every tile sorts the sample
 static constexpr u32 SS_MAX_BUCKETS = 1024;
 static constexpr u32 SS_LSEGS = 128;                 // sources staged in LDS
@@ -353,9 +354,11 @@ static u32 ss_buckets(u64 n) {
 // non-decreasing splitters give a correct split.
 // FIRST: a lone PMA's batch of at most FIRST sources, whose first work (status,
 // update index) one more workgroup, past the tiles, does here instead of a
-// kernel of its own, and the next pyr_chunks workgroups the count pyramid's
-// chunk levels the last batch left owing (its top levels follow in the
-// bucket kernel); the sources come from the kernel arguments.  A tile that
+// kernel of its own, and the next ones the count pyramid's chunk levels the last
+// batch left owing, SS_PYR chunks each (its top levels follow in the bucket
+// kernel); the sources come from the kernel arguments.  (A chunk is eleven
+// barriers: one by a whole workgroup, two of which fill a compute unit, took the
+// kernel to 32 us over 2^23 segments; 21 with four side by side.)  A tile that
 // met an invalid key marks its count of bucket 0 (bit 31): the bucket
 // kernel raises the flag, after the status is cleared.
 template <u32 FIRST, int ITEMS>
@@ -364,12 +367,14 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
                                                       u64 *__restrict__ tmp, u32 *__restrict__ bc,
                                                       SegArgs<FIRST ? FIRST : 1> in, Group g, Status *status, u32 *wfirst) {
     constexpr u32 TILE = SS_TPB * ITEMS;
-    __shared__ u32 smp[2][SS_MAX_SAMPLE];
-    __shared__ u32 spl[SS_MAX_BUCKETS];
-    __shared__ u32 cnt[SS_MAX_BUCKETS];
-    __shared__ u32 base[SS_MAX_BUCKETS];
+    __shared__ union {
+        struct {
+            u32 smp[2][SS_MAX_SAMPLE], spl[SS_MAX_BUCKETS], cnt[SS_MAX_BUCKETS], base[SS_MAX_BUCKETS];
+        };
+        u32 pyr[FIRST ? SS_PYR : 1][PYR_CH + PYR_CH / 2];
+    } L;
+    u32(*const smp)[SS_MAX_SAMPLE] = L.smp, *const spl = L.spl, *const cnt = L.cnt, *const base = L.base;
     __shared__ BatchSeg lsegs[FIRST ? FIRST : SS_LSEGS];
-    __shared__ u32 pyr_v0[FIRST ? PYR_CH : 1], pyr_v1[FIRST ? PYR_CH / 2 : 1];
     if (n_dev) n = *n_dev;
     const u32 t = blockIdx.x;
     const u32 ntiles = (u32)((n + TILE - 1) / TILE);
@@ -378,8 +383,11 @@ __global__ __launch_bounds__(SS_TPB) void k_ss_split(const BatchSeg *__restrict_
         if (t >= ntiles) {
             if (t == ntiles)
                 batch_first_work(g, status, 0, nullptr, 0, wfirst, nullptr);
-            else
-                pyr_chunk(pma_of(g, 0), t - ntiles - 1, pyr_v0, pyr_v1);
+            else {
+                const u32 q = tid / (SS_TPB / SS_PYR);
+                pyr_chunk(pma_of(g, 0), (u64)(t - ntiles - 1) * SS_PYR + q, L.pyr[q], L.pyr[q] + PYR_CH,
+                          tid % (SS_TPB / SS_PYR), SS_TPB / SS_PYR);
+            }
             return;
         }
         if (tid < in.n) lsegs[tid] = in.s[tid];
@@ -954,7 +962,7 @@ u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const Batc
     u32 *bc = scratch + OS_ZERO_WORDS;
     const u32 ks = 1 + sbits;
     const u32 psh = hi_bit > 32 + ks ? hi_bit - 32 : ks;
-    const u32 grid = ss_tiles(n) + 1 + pyr_chunks;
+    const u32 grid = ss_tiles(n) + 1 + (pyr_chunks + SS_PYR - 1) / SS_PYR;
     if (nsegs <= INLINE_SEGS)
         ss_split_first<INLINE_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
     else

@@ -66,3 +66,24 @@ def test_owed_pyramid_paid_on_every_path():
     g.close()
     t.close()
     other.close()
+
+
+# a PMA smaller than a chunk, of one chunk, of two, of as many as a workgroup of
+# the sort sums side by side, and of more
+@pytest.mark.parametrize("H", [3, 11, 12, 13, 15])
+def test_owed_pyramid_chunks(H):
+    S, V = 2, 500
+    n = int(0.6 * (S << H))
+    say(f"owed pyramid over 2^{H} segments")
+    rng = np.random.default_rng(H)
+    t = Triple(V if n > 2 * V else 2, segment_slots=S)
+    V = t.V
+    pairs = rng.permutation(V * V)[: n - V]
+    t.insert(keys_of(pairs // V, pairs % V))
+    for _ in range(4):
+        # (2049 keys or more go through the sort, with repeats in a small PMA)
+        ins, dels = rand_keys(rng, V, 1500), t.ref[rng.integers(0, t.ref.size, 1500)]
+        t.mixed(ins, np.setdiff1d(dels, ins)[rng.integers(0, max(1, np.setdiff1d(dels, ins).size), 1500)]
+                if np.setdiff1d(dels, ins).size else dels)
+        t.compare()
+    t.close()
