@@ -233,7 +233,8 @@ int lpma_snapshot_set_search_width(lpma_snapshot_t *s, uint32_t workgroups);
 /* PageRank over the gapped layout with nvGraph's formulation
  * (include/pagerank.hxx:66-88): from the uniform vector, until the L1 change
  * is below `tolerance` or `max_iter` iterations, then L1-normalised.  FP32
- * values; sums in FP64 (V <= 2^27) or compensated FP32.
+ * values; sums of contributions in 64 bits that hold each whole (V <= 2^27) or
+ * in compensated FP32.
  * The host waits for every iteration's L1 change, and for the stream at the
  * end.  d_rank has V entries.  Device scratch (V <= 2^27): 5 to 8 B per edge
  * and 32 B per vertex, 4 B for each part of 2^12 to 2^18 slots and 8192

@@ -548,7 +548,6 @@ __device__ __forceinline__ void atomic_add2(float *hi, float *lo, float x) {
 // sum over a workgroup of PR_TPB threads (every thread gets it); tmp holds
 // PR_TPB / 64 floats of LDS
 static constexpr u32 PR_TPB = 256;
-static constexpr u32 PR_GRID = 2048;  // vector passes: few enough blocks for one atomic each
 __device__ __forceinline__ float block_sum(float v, float *tmp) {
     v = wave_sum(v);
     __syncthreads();  // tmp may still be read from a previous call
@@ -1045,13 +1044,36 @@ __global__ __launch_bounds__(1024) void k_pb_chunks(const u32 *__restrict__ off,
     if (threadIdx.x == 0) cb[NB] = (u32)carry;
 }
 
-// Sums of contributions are kept in 64 bits of floating point: an FP32
-// contribution of any size enters whole, and LDS adds such sums natively, where
-// FP32 compensated by a compare-and-swap took 428 us an iteration at 6.4e7
-// edges.
-__device__ __forceinline__ void pr_add(double *sum, float x) {
-    typedef __attribute__((address_space(3))) double lds_double;
-    (void)__builtin_amdgcn_ds_atomic_fadd_f64((lds_double *)sum, (double)x);
+// Sums of contributions are kept in 64 bits, in floating or in fixed point of
+// PR_FIX fractional bits.  FP64 takes a contribution of any size whole.  Fixed
+// point does so from 2^(23 - PR_FIX) on, and then its adds are exact; a sum stays
+// below 2, as the ranks of a vector sum to 1 (the recurrence keeps it).  LDS adds
+// integers faster where many lanes meet on one address, until the reads of the
+// contributions hide that: 10^7 edges on 6*10^5 vertices 78 us an iteration, FP64
+// 94; 3.4*10^7 on 2^21 104 and 109; 6.4*10^7 on 2^22 the same.  So integers take the
+// sums where no contribution can be smaller (pr_fits_fixed).
+static constexpr u32 PR_FIX = 63;
+// A rank is at least an equal share of (1 - alpha) of the mass, a contribution
+// at least that over the largest out-degree; a hundredth of it is more than
+// roundings take.
+bool pr_fits_fixed(u32 V, u64 degree, float alpha) {
+    return (1.0 - (double)alpha) * 0.99 * (double)(1ull << (PR_FIX - 23)) >= (double)V * (double)degree;
+}
+// x to a word of LDS
+template <bool FIXED>
+__device__ __forceinline__ void pr_add(u64 *sum, float x) {
+    if constexpr (FIXED) {
+        const u32 bits = __float_as_uint(x), e = bits >> 23;  // x is 0, or of [2^(23 - PR_FIX), 2)
+        const u64 m = ((u64)((bits & 0x7FFFFFu) | 0x800000u)) << (PR_FIX - 23);  // mantissa, of value 1 at e = 127
+        atomicAdd((unsigned long long *)sum, (unsigned long long)(m >> min(127u - min(e, 127u), 63u)));
+    } else {
+        typedef __attribute__((address_space(3))) double lds_double;
+        (void)__builtin_amdgcn_ds_atomic_fadd_f64((lds_double *)sum, (double)x);
+    }
+}
+template <bool FIXED>
+__device__ __forceinline__ double pr_sum(u64 sum) {
+    return FIXED ? (double)sum * (0.5 / (double)(1ull << (PR_FIX - 1))) : __longlong_as_double((long long)sum);
 }
 
 // the host's word: (iteration, its L1 change)
@@ -1060,6 +1082,11 @@ __device__ __forceinline__ void pr_report(const PrSlot &s, u32 it, u64 *host) {
                        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+__device__ __forceinline__ u32 wave_max(u32 v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, (u32)__shfl_xor((int)v, o, 64));
+    return v;
+}
 static __device__ __forceinline__ double wave_sum_d(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -1082,11 +1109,14 @@ __device__ __forceinline__ void pr_reduce(double dang, double sum, double delta,
 }
 
 // start vector 1/V, out-degrees (from marker ranks), contributions, dangling
-// mass
+// mass, and each workgroup's largest out-degree (PR_GRID words after the slots:
+// an atomic maximum by every wave took 26 us)
 __global__ __launch_bounds__(PR_TPB) void k_pr_start(DevState d, const u32 *__restrict__ gpre,
                                                      u32 *__restrict__ outdeg, float *__restrict__ pr,
                                                      float *__restrict__ c0, float *__restrict__ c1, PrSlot *slot) {
     __shared__ double lds[3 * PR_TPB / 64];
+    __shared__ u32 s_most[PR_TPB / 64];
+    u32 most = 0;
     const u32 V = d.V, Smask = (1u << d.log2S) - 1;
     const float p = 1.f / (float)V;
     double dang = 0.0;
@@ -1100,12 +1130,19 @@ __global__ __launch_bounds__(PR_TPB) void k_pr_start(DevState d, const u32 *__re
         pr[r] = p;
         c0[r] = od ? p / (float)od : 0.f;
         if (!od) dang += p;
+        most = max(most, od);
     }
+    most = wave_max(most);
+    if (lane_id() == 0) s_most[threadIdx.x >> 6] = most;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         c0[V] = c1[V] = 0.f;  // the padding words' source
         slot->sum = 1.0;
     }
-    pr_reduce(dang, 0.0, 0.0, slot, lds);
+    pr_reduce(dang, 0.0, 0.0, slot, lds);  // (a barrier inside)
+    if (threadIdx.x == 0) {
+        for (u32 w = 0; w < PR_TPB / 64; ++w) most = max(most, s_most[w]);
+        ((u32 *)(slot + PR_SLOTS))[blockIdx.x] = most;
+    }
 }
 
 // Iteration `it` (from 1) is two kernels.  It reads the masses of iteration
@@ -1143,19 +1180,26 @@ __device__ __forceinline__ double pr_gamma(const PrSlot &prev, float alpha, u32 
 // 1340 us when every iteration binned contributions and summed them by LDS
 // compare-and-swap; with 8-byte edges 235 us.  The LDS adds are hidden: without
 // them the kernel takes the same time.
-template <u32 G>
+template <u32 G, bool FIXED>
 __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ words,
                                                      const u32 *__restrict__ rows, const u32 *__restrict__ off, u32 P,
                                                      u32 NB, const u32 *__restrict__ cb, u32 chunk,
                                                      const float *__restrict__ c, float *__restrict__ cnext,
                                                      const float *__restrict__ pr, float *__restrict__ out,
                                                      const u32 *__restrict__ outdeg, u32 V, float alpha, float tol,
-                                                     u32 it, PrSlot *slots, double *__restrict__ partial,
+                                                     u32 it, PrSlot *slots, u32 starts, double *__restrict__ partial,
                                                      u64 *__restrict__ host) {
-    extern __shared__ double pb_acc[];  // PB_BIN sums
+    extern __shared__ u64 pb_acc[];  // PB_BIN sums
     __shared__ double red[3 * PRI_TPB / 64];
     const PrSlot &prev = slots[(it - 1) % PR_SLOTS];
     if (blockIdx.x == 0 && threadIdx.x == 0 && it > 1) pr_report(prev, it - 1, host);
+    if (blockIdx.x == 0 && it == 1 && threadIdx.x < 64) {
+        // the largest out-degree, for the host's choice of later iterations
+        u32 most = 0;
+        for (u32 i = threadIdx.x; i < starts; i += 64) most = max(most, ((const u32 *)(slots + PR_SLOTS))[i]);
+        most = wave_max(most);
+        if (threadIdx.x == 0) __hip_atomic_store(host + 1, (u64)most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     if (it > 1 && (float)prev.delta < tol) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) slots[(it + 1) % PR_SLOTS] = PrSlot{0.0, 0.0, 0.0};
     const u32 k = blockIdx.x;
@@ -1170,7 +1214,7 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
     const u64 s0 = (u64)off[(u64)b * P] + (u64)(k - cb[b]) * chunk;
     const u64 s1 = min(e1, s0 + chunk);
     const u32 v0 = b << PB_BIN_LOG, nv = min(PB_BIN, V - v0);
-    for (u32 v = threadIdx.x; v < PB_BIN; v += PRI_TPB) pb_acc[v] = 0.0;
+    for (u32 v = threadIdx.x; v < PB_BIN; v += PRI_TPB) pb_acc[v] = 0ull;
     __syncthreads();
     for (u64 i0 = s0; i0 < s1; i0 += (u64)PRI_TPB * PRI_ITEMS) {
         u32 e[PRI_ITEMS], row0[PRI_ITEMS];
@@ -1192,18 +1236,18 @@ __global__ __launch_bounds__(PRI_TPB) void k_pr_iter(const u32 *__restrict__ wor
 #pragma unroll
         for (u32 r = 0; r < PRI_ITEMS; ++r) x[r] = c[e[r] == PB_PAD ? V : row0[r] + (e[r] >> PB_BIN_LOG)];
 #pragma unroll
-        for (u32 r = 0; r < PRI_ITEMS; ++r) pr_add(&pb_acc[e[r] & (PB_BIN - 1)], x[r]);
+        for (u32 r = 0; r < PRI_ITEMS; ++r) pr_add<FIXED>(&pb_acc[e[r] & (PB_BIN - 1)], x[r]);
     }
     __syncthreads();
     if (nch > 1) {
         double *to = partial + (u64)(cb[NB + 1 + b] + (k - cb[b])) * PB_BIN;
-        for (u32 v = threadIdx.x; v < nv; v += PRI_TPB) to[v] = pb_acc[v];
+        for (u32 v = threadIdx.x; v < nv; v += PRI_TPB) to[v] = pr_sum<FIXED>(pb_acc[v]);
         return;
     }
     const double gamma = pr_gamma(prev, alpha, V);
     PrMass m{0.0, 0.0, 0.0};
     for (u32 v = threadIdx.x; v < nv; v += PRI_TPB)
-        pr_vertex(v0 + v, pb_acc[v], alpha, gamma, pr, out, outdeg, cnext, m);
+        pr_vertex(v0 + v, pr_sum<FIXED>(pb_acc[v]), alpha, gamma, pr, out, outdeg, cnext, m);
     pr_reduce(m.dang, m.sum, m.delta, &slots[it % PR_SLOTS], red);
 }
 
@@ -1318,11 +1362,12 @@ u64 pr_bins_partial_words(const PrBins &b) { return std::max<u64>(1, (u64)b.max_
 
 hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
                            const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
-                           float tol, u32 it, PrSlot *slots, double *partial, u64 *host, hipStream_t st) {
-    const auto iter = b.group == PB_CHUNK ? k_pr_iter<PB_CHUNK> : k_pr_iter<1>;
-    iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(double), st>>>(
+                           float tol, u32 it, bool fixed, PrSlot *slots, double *partial, u64 *host, hipStream_t st) {
+    const auto iter = b.group == PB_CHUNK ? (fixed ? k_pr_iter<PB_CHUNK, true> : k_pr_iter<PB_CHUNK, false>)
+                                          : (fixed ? k_pr_iter<1, true> : k_pr_iter<1, false>);
+    iter<<<b.max_chunks, PRI_TPB, PB_BIN * sizeof(u64), st>>>(
         words, words + pr_bins_rows_at(b), off, b.parts, b.bins, cb, b.chunk, c, cnext, pr, out, outdeg, d.V, alpha, tol, it,
-        slots, partial, host);
+        slots, grid_for(d.V, PR_TPB, PR_GRID), partial, host);
     if (b.max_multi)
         k_pr_join<<<b.bins * (PB_BIN / PRI_TPB), PRI_TPB, 0, st>>>(b.bins, cb, partial, cnext, pr, out, outdeg, d.V,
                                                                    alpha, tol, it, slots);

@@ -199,6 +199,8 @@ struct PrSlot {
     double dang, sum, delta;
 };
 static constexpr u32 PR_SLOTS = 4;
+static constexpr u32 PR_GRID = 2048;  // workgroups of vector passes: few enough for one atomic each
+static constexpr u64 PR_SLOT_WORDS = PR_SLOTS * sizeof(PrSlot) / 8 + PR_GRID / 2;  // and the workgroups' largest out-degrees
 bool pr_bins_fit(u32 V);
 PrBins pr_bins_plan(const DevState &d, u64 edges);
 u64 pr_bins_count_words(const PrBins &b);
@@ -211,11 +213,14 @@ hipError_t pr_bins_start(const DevState &d, u32 *gpre, u32 *scan_scratch, u32 *o
                          PrSlot *slots, hipStream_t st);
 // iteration `it` = 1, 2, ...; does nothing once an earlier L1 change is below
 // tol.  (it - 1) << 32 | its L1 change reaches `host`; pr_bins_norm reports the
-// last one's.
+// last one's.  The first leaves the largest out-degree in host[1].  fixed: sums in
+// fixed point, where pr_fits_fixed says of a bound on the out-degrees that they
+// are exact.
+bool pr_fits_fixed(u32 V, u64 degree, float alpha);
 u64 pr_bins_partial_words(const PrBins &b);
 hipError_t pr_bins_iterate(const DevState &d, const PrBins &b, const u32 *words, const u32 *off, const u32 *cb,
                            const float *c, float *cnext, const float *pr, float *out, const u32 *outdeg, float alpha,
-                           float tol, u32 it, PrSlot *slots, double *partial, u64 *host, hipStream_t st);
+                           float tol, u32 it, bool fixed, PrSlot *slots, double *partial, u64 *host, hipStream_t st);
 hipError_t pr_bins_norm(const float *pr, float *rank, u32 V, u32 it, const PrSlot *slots, u64 *host, hipStream_t st);
 
 }  // namespace pma

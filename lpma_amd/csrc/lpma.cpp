@@ -1935,7 +1935,7 @@ static int pagerank_binned(lpma *h, float damping, float tolerance, u32 max_iter
     CHECKED(ensure(h, h->apwords, pr_bins_edge_words(bins)));
     CHECKED(ensure(h, h->apart, pr_bins_partial_words(bins)));
     CHECKED(ensure(h, h->af1, V + 1));  // with af0: contributions, and the padding's
-    CHECKED(ensure(h, h->aslots, (PR_SLOTS * sizeof(PrSlot) + 7) / 8));
+    CHECKED(ensure(h, h->aslots, PR_SLOT_WORDS));
     if (!h->h_word) {
         if (injected_failure()) return LPMA_ERR_OUT_OF_MEMORY;
         if (hipHostMalloc((void **)&h->h_word, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
@@ -1951,10 +1951,11 @@ static int pagerank_binned(lpma *h, float damping, float tolerance, u32 max_iter
     HIPCHECK(pr_bins_start(h->st, h->pl.gpre.p, h->pl.scan_scr.p, h->aq0.p, vec[0], c[0], c[1], slots, st));
     // an iteration reports the L1 change of the one before it, so one more is
     // always queued (it returns at once when it was not wanted)
+    bool fixed = pr_fits_fixed(h->V, std::min<u64>(V, h->live - V), damping);
     auto queue = [&](u32 i) {
         const int a = (i - 1) & 1;
         return pr_bins_iterate(h->st, bins, h->apwords.p, h->apoff.p, h->apcb.p, c[a], c[a ^ 1], vec[a], vec[a ^ 1],
-                               h->aq0.p, damping, tolerance, i, slots, h->apart.p, h->h_word, st);
+                               h->aq0.p, damping, tolerance, i, fixed, slots, h->apart.p, h->h_word, st);
     };
     u64 w = 0;
     HIPCHECK(queue(1));
@@ -1965,6 +1966,9 @@ static int pagerank_binned(lpma *h, float damping, float tolerance, u32 max_iter
         const u32 bits = (u32)w;
         memcpy(&delta, &bits, sizeof(delta));
         if (delta < tolerance) break;
+        // from the third iteration on by the graph's own degrees (and not for so
+        // long that roundings could move the mass)
+        fixed = it < 65536 && pr_fits_fixed(h->V, __atomic_load_n(h->h_word + 1, __ATOMIC_RELAXED), damping);
     }
     HIPCHECK(pr_bins_norm(vec[it & 1], d_rank, h->V, it, slots, h->h_word, st));
     HIPCHECK(hipStreamSynchronize(st));

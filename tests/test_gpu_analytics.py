@@ -414,3 +414,23 @@ def test_bfs_levels_that_take_lists(V, listed):
     deg = np.diff(oracle.csr_of(keys, V)[0].astype(np.int64))
     assert depth == int(want[want != 0xFFFFFFFF].max()) + 1 and scanned == int(deg[want != 0xFFFFFFFF].sum())
     pma.close()
+
+
+# sums in fixed point where no contribution can fall below what it holds whole
+# (by V * V, or from the third iteration on by V and the largest out-degree), else
+# in FP64: a hub of every vertex at the rule's edges, and one of a tenth
+@pytest.mark.parametrize("V,hub", [(403000, 403000), (405000, 405000), (700000, 233000), (700000, 234000), (50, 50)])
+def test_pagerank_smallest_contributions(V, hub):
+    say(f"pagerank smallest contributions V={V} hub={hub}")
+    from gpu_util import keys_of
+    rng = np.random.default_rng(V)
+    keys = oracle.sort_unique(keys_of(np.concatenate([np.full(hub, 3), np.arange(V), rng.integers(0, V, 2 * V)]),
+                                      np.concatenate([np.arange(hub), (np.arange(V) + 1) % V, rng.integers(0, V, 2 * V)])))
+    pma = L.PMA(V)
+    pma.insert(keys)
+    for it in (1, 2, 5):
+        got = pma.pagerank(0.85, 0.0, it)[0].cpu().numpy().astype(np.float64)
+        want, _ = oracle.pagerank(keys, V, float(np.float32(0.85)), it)
+        # four roundings an iteration and one of the final scale
+        assert np.max(np.abs(got - want) / want) < (4 * it + 2) * 2.0 ** -24
+    pma.close()
