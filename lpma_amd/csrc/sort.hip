@@ -292,17 +292,20 @@ __global__ __launch_bounds__(OS_TPB) void k_os_pass(const u64 *__restrict__ in, 
 // between waves), and writes them at the bucket's offset.  A sample-chosen
 // split keeps buckets even under R-MAT skew, where a split on the top key bits
 // puts a hub's keys in one bucket.  A bucket beyond the workgroup's SB_CAP keys
-// is LSD-radix-sorted through global memory, chunk by chunk, on the bits on
-// which its keys differ (AND / OR of the keys), with wave64 ranking (the
-// k_os_pass scheme): 3 us a chunk to gather and 8 a chunk and pass.  A splitter
-// that is repeated (a projection of more than an average bucket) has a bucket of
-// its own, so that a key repeated some thousand times is not mixed with others
-// and takes few passes or none.  A batch with a projection of SS_SKEW_KEYS keys
-// or more (a hub of a graph of so many vertices that its edges share
-// projections), or SS_SKEW_SAME copies of one key, is not sorted but flagged
-// FLAG_SORT_SKEW: the kernels after it do nothing, and the host runs it again
-// with the passes below, 50 us later.  Batches of 4*10^5 keys over 2^20 vertices,
-// one key half of them: 193 us, 1660 by one workgroup on mixed buckets.
+// is read for the bits on which its keys differ (AND / OR of the keys), 3 us a
+// chunk of SB_CAP: if that is one key, its last element is written for all (the
+// update asks only for that one); else the bucket is gathered and LSD-radix-sorted
+// through global memory on those bits, chunk by chunk, with wave64 ranking (the
+// k_os_pass scheme), 8 us a chunk and pass.  A splitter that is repeated (a
+// projection of more than an average bucket) has a bucket of its own, so that a
+// key repeated some thousand times is not mixed with others.  A batch with a
+// projection of SS_SKEW_KEYS keys or more (a hub of a graph of so many vertices
+// that its edges share projections), or SS_SKEW_SAME copies of one key, is not
+// sorted but flagged FLAG_SORT_SKEW: the kernels after it do nothing, and the host
+// runs it again with the passes above, 50 us later.  Batches over 2^20 vertices:
+// 4*10^5 keys, one key half of them, 197 us (1660 by one workgroup on mixed
+// buckets); 10^5 121 (473); 32 requests of 4*10^5 of one key 235 (1240), of 10^5
+// 162 (350).
 //
 // Bound: the sample's sort in every tile (vector issue: 1024 samples 5 us, 2048
 // 10 us with one tile a compute unit) and the largest bucket.  10^5 R-MAT keys:
@@ -332,7 +335,7 @@ static constexpr u32 SS_BAD = 1u << 31;
 // which all are one key
 static constexpr u32 SS_SKEW = 1u << 30;
 static constexpr u32 SS_SKEW_KEYS = 6144;
-static constexpr u32 SS_SKEW_SAME = 1u << 17;
+static constexpr u32 SS_SKEW_SAME = 160000;
 // keys a thread: 1 up to 2^18 keys, 2 above
 static int ss_items(u64 n) { return n <= (u64)SS_MAX_TILES * SS_TPB ? 1 : 2; }
 static u32 ss_tiles(u64 n) { return (u32)((n + ss_items(n) * SS_TPB - 1) / (ss_items(n) * SS_TPB)); }
@@ -585,10 +588,11 @@ __device__ __forceinline__ void sb_rank(const u64 (&x)[SB_ITEMS], u32 m, u32 R, 
     __syncthreads();
 }
 
+// ks: bits below the key (request order, operation).
 // top: one more workgroup, past the buckets, sums the lone PMA's pyramid
 // top levels (after the split kernel's chunk levels)
 __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tmp, u64 *__restrict__ out,
-                                                       u64 *__restrict__ aux, u64 n, const u64 *n_dev, u32 tile, u32 nb,
+                                                       u64 *__restrict__ aux, u64 n, const u64 *n_dev, u32 tile, u32 nb, u32 ks,
                                                        const u32 *__restrict__ bc, u32 *__restrict__ flags,
                                                        bool top, DevState topd) {
     // the bucket's sort, or an oversized bucket's radix passes, or the
@@ -602,7 +606,7 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
     } L;
     __shared__ u32 toff[SS_MAX_TILES + 1], tb[SS_MAX_TILES];
     __shared__ u32 stmp[SB_NW + 1];
-    __shared__ u64 red[2][SB_NW];
+    __shared__ u64 red[3][SB_NW];
     u32(*const whist)[256] = L.whist;
     u32 *const dofs = L.dofs, *const run = L.run;
     if (n_dev) n = *n_dev;
@@ -685,33 +689,44 @@ __global__ __launch_bounds__(SB_TPB) void k_ss_bucket(const u64 *__restrict__ tm
         return;
     }
 
-    // beyond the LDS (many equal keys): gathered into the output range, then
-    // LSD passes over the bits that vary, chunk by chunk through global
-    // memory (from the output range to aux and back); each digit's running
-    // offset carries across the chunks, which are taken in order (stable)
-    u64 andv = ~0ull, orv = 0;
-    for (u32 j0 = tid; j0 < m; j0 += SB_CAP) {
-        u64 x[SB_ITEMS];
+    // beyond the LDS: the bits that vary, and the last key in order
+    u64 andv = ~0ull, orv = 0, last = 0;
+    constexpr u32 FLY = 16;  // loads of a thread in flight
+    for (u32 j0 = tid; j0 < m; j0 += SB_TPB * FLY) {
+        u64 x[FLY];
 #pragma unroll
-        for (int r = 0; r < SB_ITEMS; ++r) x[r] = tmp[addr_of(min(j0 + r * SB_TPB, m - 1))];  // all in flight
+        for (u32 r = 0; r < FLY; ++r) x[r] = tmp[addr_of(min(j0 + r * SB_TPB, m - 1))];
 #pragma unroll
-        for (int r = 0; r < SB_ITEMS; ++r) {
+        for (u32 r = 0; r < FLY; ++r) {
             andv &= x[r];
             orv |= x[r];
-            if (j0 + r * SB_TPB < m) out[obase + j0 + r * SB_TPB] = x[r];
+            last = max(last, x[r]);
         }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         andv &= __shfl_xor(andv, o, 64);
         orv |= __shfl_xor(orv, o, 64);
+        last = max(last, (u64)__shfl_xor(last, o, 64));
     }
-    if (lane == 0) { red[0][w] = andv; red[1][w] = orv; }
-    __syncthreads();  // also makes the gather's stores visible to the workgroup
+    if (lane == 0) { red[0][w] = andv; red[1][w] = orv; red[2][w] = last; }
+    __syncthreads();
     andv = ~0ull;
     orv = 0;
 #pragma unroll
-    for (u32 q = 0; q < SB_NW; ++q) { andv &= red[0][q]; orv |= red[1][q]; }
+    for (u32 q = 0; q < SB_NW; ++q) { andv &= red[0][q]; orv |= red[1][q]; last = max(last, red[2][q]); }
+    if (((andv ^ orv) >> ks) == 0) {
+        // one key: its last element decides, and the ones before it only have to
+        // be that key's, so it stands for all
+        for (u32 j = tid; j < m; j += SB_TPB) out[obase + j] = last;
+        return;
+    }
+    // several: gathered into the output range, then LSD passes over the bits
+    // that vary, chunk by chunk through global memory (from the output range to
+    // aux and back); each digit's running offset carries across the chunks, which
+    // are taken in order (stable)
+    for (u32 j = tid; j < m; j += SB_TPB) out[obase + j] = tmp[addr_of(j)];
+    __syncthreads();  // makes the gather's stores visible to the workgroup
     const u64 diff = andv ^ orv;
     const u32 lo_bit = diff ? (u32)__builtin_ctzll(diff) : 64u;
     const u32 hi_bit = diff ? 64u - (u32)__builtin_clzll(diff) : 0u;
@@ -919,7 +934,7 @@ u64 *pack_and_sort(const BatchSeg *segs, u32 nsegs, u64 n, const u64 *n_dev, u32
         else
             k_ss_split<0, 2><<<ntiles, SS_TPB, 0, st>>>(segs, nsegs, n, n_dev, pshift, sbits, psh, nb, k1, bc,
                                                              SegArgs<1>{}, Group{}, nullptr, nullptr);
-        k_ss_bucket<<<nb, SB_TPB, 0, st>>>(k1, k0, k2, n, n_dev, (u32)ss_items(n) * SS_TPB, nb, bc, flags, false,
+        k_ss_bucket<<<nb, SB_TPB, 0, st>>>(k1, k0, k2, n, n_dev, (u32)ss_items(n) * SS_TPB, nb, ks, bc, flags, false,
                                            DevState{});
         return k0;
     }
@@ -967,7 +982,7 @@ u64 *pack_and_sort_first(const Group &g, Status *status, u32 *wfirst, const Batc
         ss_split_first<INLINE_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
     else
         ss_split_first<ARG_SEGS>(grid, g, status, wfirst, segs, nsegs, n, pshift, sbits, psh, nb, k1, bc, st);
-    k_ss_bucket<<<nb + 1, SB_TPB, 0, st>>>(k1, k0, k2, n, nullptr, (u32)ss_items(n) * SS_TPB, nb, bc, &status->flags,
+    k_ss_bucket<<<nb + 1, SB_TPB, 0, st>>>(k1, k0, k2, n, nullptr, (u32)ss_items(n) * SS_TPB, nb, ks, bc, &status->flags,
                                            true, g.one);
     return k0;
 }
