@@ -450,3 +450,27 @@ def test_repeated_key_costs_no_more_than_the_radix_sort():
     say(f"{took[0] * 1e6:.0f} us, half repeated {took[1] * 1e6:.0f} us")
     assert took[1] < 3 * took[0]
     p.close()
+
+
+@pytest.mark.parametrize("copies", [16, 18, 22])
+def test_bucket_of_many_keys_of_one_projection(copies):
+    """256 neighboring keys, repeated, share a projection (2^20 vertices: 41 bits,
+    of which 32 are compared) and a bucket, of 4096 keys and of more than its
+    workgroup holds; inserted and deleted at once."""
+    rng = np.random.default_rng(copies)
+    V, n = 1 << 20, 300000
+    say(f"bucket of 256 keys x {copies}")
+    p = L.PMA(V)
+    ref = np.empty(0, dtype=np.uint64)
+    near = keys_of(np.full(256 * copies, 70000), 5 * 256 + np.tile(np.arange(256), copies))
+    for _ in range(2):
+        ins = np.concatenate([near, rand_keys(rng, V, n)])
+        p.insert(rng.permutation(ins))
+        ref = oracle.apply(ref, ins)
+        assert np.array_equal(L.to_host_u64(p.export()[0]), ref)
+        ins, dels = np.concatenate([near[::3], rand_keys(rng, V, n // 2)]), np.concatenate([near, ref[::5][: n // 2]])
+        p.update_mixed(rng.permutation(ins), rng.permutation(dels))
+        ref = oracle.apply(ref, ins, dels)
+        assert np.array_equal(L.to_host_u64(p.export()[0]), ref)
+    assert p.check() == 0
+    p.close()
